@@ -3,11 +3,13 @@ and the pybind11 module cuhnsw_bind that wraps it.
 
   python -m cuhnsw_amd.build
 """
+import concurrent.futures
 import json
 import os
 import subprocess
 import sys
 import sysconfig
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -41,13 +43,11 @@ def _demangle(names):
     return names
 
 
-def build_lib():
-  """Compiles the library and records, from the compiler's resource-usage remarks of this very build, what
-  every kernel in it takes: registers, spills, scratch bytes, wavefronts per SIMD (profiles/kernel_resources.json;
-  `python -m cuhnsw_amd.kernel_report` adds where in the first-pass kernels the scratch accesses sit)."""
-  from cuhnsw_amd import kernel_report
-  srcs = [os.path.join(CSRC, "engine.hip"), os.path.join(CSRC, "index_file.cpp")]
-  cmd = [HIPCC] + HIP_FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-x", "hip"] + srcs + ["-o", LIB]
+def _compile(job):
+  """One object of the library; returns what the compiler said on stderr."""
+  src, defines, obj = job
+  cmd = [HIPCC] + [f for f in HIP_FLAGS if f != "-shared"] + defines + [
+      "-Rpass-analysis=kernel-resource-usage", "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
   print("+", " ".join(cmd), flush=True)
   r = subprocess.run(cmd, stderr=subprocess.PIPE, text=True)
   other = [l for l in r.stderr.split("\n") if "kernel-resource-usage" not in l and "not a recognized feature" not in l
@@ -57,7 +57,25 @@ def build_lib():
     print("\n".join(l for l in other if l.strip()), file=sys.stderr)
   if r.returncode != 0:
     raise subprocess.CalledProcessError(r.returncode, cmd)
-  usage = kernel_report.parse_remarks(r.stderr)
+  return r.stderr
+
+
+def build_lib():
+  """Compiles the library -- the templated kernels one object per distance and row width, side by side -- and
+  records, from the compiler's resource-usage remarks of this very build, what every kernel in it takes: registers,
+  spills, scratch bytes, wavefronts per SIMD (profiles/kernel_resources.json; `python -m cuhnsw_amd.kernel_report`
+  adds where in the first-pass kernels the scratch accesses sit)."""
+  from cuhnsw_amd import kernel_report
+  with tempfile.TemporaryDirectory(prefix="cuhnsw_build_") as tmp:
+    # (the objects that take longest first)
+    jobs = [("instances.hip", ["-DCUHNSW_DT=" + dt, "-DCUHNSW_QR=%d" % qr], os.path.join(tmp, "%s_%d.o" % (dt, qr)))
+            for qr in (4, 2, 0, 1) for dt in ("DIST_DOT", "DIST_L2")]
+    jobs += [(name, [], os.path.join(tmp, name + ".o")) for name in ("engine.hip", "index_file.cpp")]
+    workers = max(1, min(len(jobs), len(os.sched_getaffinity(0)), int(os.environ.get("MAX_JOBS") or 8)))
+    with concurrent.futures.ThreadPoolExecutor(workers) as pool:
+      said = "\n".join(pool.map(_compile, jobs))
+    _run([HIPCC] + HIP_FLAGS + [obj for _, _, obj in jobs] + ["-o", LIB])
+  usage = kernel_report.parse_remarks(said)
   names = sorted(usage)
   table = {plain: usage[mangled] for mangled, plain in zip(names, _demangle(names))}
   try:

@@ -1,0 +1,669 @@
+// Host engine of libcuhnsw_amd.so: options, data, index files and what surrounds the kernel launches.  (The C ABI is
+// in engine.hip, the launches of the templated kernels are in instances.hip.)
+//
+// Counterpart of the reference's host class cuhnsw::CuHNSW
+// (cpp/include/cuhnsw.hpp:61-112, cpp/src/cuhnsw_base.cu, cpp/src/cuhnsw_build.cu).
+// Differences by design: the whole multi-level index stays resident in HBM in flat
+// fixed-stride rows (the reference re-flattens and re-uploads the graph on every
+// search call, cpp/src/cuhnsw_build.cu:226-253, and once per upper level for the
+// descent, :25-94); there is no per-level host graph container; HIP runtime calls
+// are made directly (no Thrust).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <cstdio>
+#include <cstring>
+#include <mutex>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "index_file.h"
+#include "kernels.h"
+#include "options.h"
+
+namespace cuhnsw_amd {
+
+#define HIP_CHECK(expr)                                                                              \
+  do {                                                                                               \
+    hipError_t err_ = (expr);                                                                        \
+    if (err_ != hipSuccess)                                                                          \
+      throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(err_) + " at " #expr); \
+  } while (0)
+
+inline bool device_present() {
+  int n = 0;
+  hipError_t e = hipGetDeviceCount(&n);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return n > 0;
+}
+
+// ---- scratch of the entry point that allocates nothing (cuhnsw_search_knn_device_noalloc) ----------
+// Everything the two search kernels need beyond the caller's buffers, at fixed maximum sizes, in one
+// array that lives in the code object: each GPU the library runs on holds its own copy from the moment
+// the code object is loaded there until the process ends.  Host code never uses the array's name as an
+// address (it is a host-side stand-in); the device address is looked up once per device
+// (static_scratch_for_current_device) and handed to the kernels like any other buffer.
+constexpr int kStaticMaxQueries = 131072;  // entries of the list of queries the first pass gives up
+constexpr int kStaticMaxEf = 512;          // the sorted set in registers holds up to 512 entries
+constexpr int kStaticSlots = 128;          // wavefronts of the literal pass
+constexpr int kStaticGlobCap = 4096;       // per wavefront: overflow of its candidate queue beyond the LDS share
+constexpr int kStaticLogCap = 8192;        // per wavefront: log of accepted entries
+struct StaticScratch {
+  int ctl[128];
+  int redo[kStaticMaxQueries];
+  HeapEnt cand_glob[(size_t)kStaticSlots * kStaticGlobCap];
+  HeapEnt log[(size_t)kStaticSlots * kStaticLogCap];
+};
+constexpr int kMaxDevices = 64;
+extern std::atomic_flag g_static_busy[kMaxDevices];  // set while a no-allocation search uses the device's array
+// device address of this device's copy of the array; looked up on first use, then kept
+StaticScratch* static_scratch_for_current_device(int* device = nullptr);
+// One no-allocation search at a time per GPU: every engine of the process shares that GPU's array.
+struct StaticScratchLease {
+  int dev;
+  explicit StaticScratchLease(int d) : dev(d) {
+    if (g_static_busy[dev].test_and_set(std::memory_order_acquire))
+      throw std::runtime_error("search_knn (no allocation): another no-allocation search is running on this GPU "
+                               "(all engines of a process share the GPU's scratch array; serialise the calls)");
+  }
+  ~StaticScratchLease() { g_static_busy[dev].clear(std::memory_order_release); }
+  StaticScratchLease(const StaticScratchLease&) = delete;
+  StaticScratchLease& operator=(const StaticScratchLease&) = delete;
+};
+
+template <typename T>
+struct DevBuf {
+  T* p = nullptr;
+  size_t n = 0;
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  // grows (never shrinks); contents are not preserved
+  void reserve(size_t want) {
+    if (want <= n) return;
+    release();
+    HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&p), want * sizeof(T)));
+    n = want;
+  }
+  // the same for a buffer the caller can do without: false (and an empty buffer) when the memory is not there
+  bool try_reserve(size_t want) {
+    if (want <= n) return true;
+    release();
+    if (hipMalloc(reinterpret_cast<void**>(&p), want * sizeof(T)) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      return false;
+    }
+    n = want;
+    return true;
+  }
+  ~DevBuf() { release(); }
+};
+
+class Engine {
+ public:
+  Options opt;
+  int dist_type = DIST_DOT;
+  HostIndex host;
+  bool have_data = false, have_levels = false, have_graph = false;
+  bool host_links_stale = false;  // device links are newer than host.links0 / linksU
+  bool has_device = false;
+  int num_cus = 0;
+  hipStream_t stream = nullptr;
+  hipStream_t stream2 = nullptr;  // the literal pass, while the sorted-set pass runs on `stream`
+  hipEvent_t ev_side0 = nullptr, ev_side1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  std::string err;
+  double last_build_seconds = 0.0;
+
+  // tunables
+  int level_first = 1;     // build: a batch hands out its nodes with upper levels first
+  int build_literal = 0;   // build: 1 = the literal search (queues / sorted list in LDS) whatever ef_construction (tests)
+  int build_batch = 0;     // nodes inserted per batch at most; 0 = by the size of the graph (batch_at)
+  int search_slots = 0;
+  int cand_lds_override = 0;
+  int hnswlib_dist = 0;
+  int spin_limit_override = -1;  // polls a waiting literal wavefront may spend (-1 = automatic)
+  int side_per_cu = 0;         // its wavefronts per CU (0 = from the share of queries the last search gave up)
+  bool share_known = false;               // last_repeat_share comes from a search of this index
+  double last_repeat_share = 0.0;         // its wavefronts per CU
+  int concurrent_literal = 1;  // run the literal pass beside the sorted-set pass (0: after it)
+  // A literal wavefront whose bounded wait ran out (the two streams did not run side by side: a profiler that
+  // serialises kernels, a saturated device) makes the next kSequentialSearches searches run their passes one
+  // after the other; then the concurrent schedule is tried again.  The caller's setting above is left alone.
+  static constexpr int kSequentialSearches = 8;
+  int sequential_left = 0;       // searches still to run one pass after the other
+  int literal_fallbacks = 0;     // how often that happened on this index
+  int last_side_by_side = 0;     // the last search ran its literal pass beside the first pass
+  bool trails_unavailable = false;  // the trail buffers could not be allocated: searches go on without trails
+  int filter_entries = 0;  // entries of the sorted-set search's visited filter (0 = automatic)
+  int first_pass_waves = 0;  // wavefronts per CU of the first pass (0 = as many as fit)
+  int query_order = 1;     // first pass of 1.5 to 32 rounds of wavefronts: longest queries first (0: caller's order)
+  bool fast_suspended = false;  // this index ties too often for the sorted-set search to pay (integer data)
+  int lean_literal = 1;  // literal pass: 0 = always the exact visited bitmap, 1 = automatic, 2 = always the LDS filter
+  bool storage_half = false;  // vectors live in HBM as fp16 (set before set_data / load_index)
+  bool tight_rows = false;    // rows padded to 16-byte chunks only, not to 128-byte lines (set before set_data / load_index)
+  int fast_path = 1;     // 0: search with the literal queues only; 1: sorted-set pass first when the batch is
+                         // larger than one round of literal wavefronts; 2: always
+  int last_repeats = 0;  // queries of the last search that were repeated with the literal queues
+  int last_trails = 0;   // how many of them came with the first pass's trail
+  int count_build_work = 0;    // count the work of a build on the device (cuhnsw_last_build_counters)
+  unsigned long long build_counters[10] = {};
+  int last_build_dropped = 0;  // reverse links of the last build that found no room in an inbox
+  int keep_link_keys = 0;      // keep the keys stored with the level-0 links after a build (debugging aid)
+  std::vector<float> link_keys0;  // N x max_m0, only with keep_link_keys
+  int newcomer_shortcut = 1;  // build: a link row that the selection rule produced is re-selected with the shortcut for newcomers
+  int own_links0 = 0;  // links a new node selects for itself on level 0: 0 = max_m0 (as the reference), else min(value, max_m0); hnswlib uses max_m
+  int spill_cap = 0;  // first size of the per-slot queue overflow area (0 = automatic); the accept log is twice that
+  int visited_cache = 0;  // entries of the LDS visited cache: 0 = automatic, < 0 = none
+
+  // resident index
+  int Dp = 0;
+  DevBuf<float> d_vectors;
+  DevBuf<uint64_t> d_labels;
+  DevBuf<uint32_t> d_deleted;  // one bit per element: hnswlib's delete marks of a loaded file (used while host.n_deleted > 0)
+  DevBuf<uint32_t> d_links0, d_linksU;
+  DevBuf<int64_t> d_upper_off;
+  DevBuf<int> d_levels;
+  // per-wavefront slots
+  DevBuf<uint32_t> d_bitmaps, d_undo;
+  DevBuf<HeapEnt> d_cand_glob, d_log;
+  SlotPool pool{};
+  int pool_slots = 0;
+  DevBuf<int> d_ctl;  // [0] work counter, [1] status, [2] dirty count, [32] queries given up by the
+                      // sorted-set pass, [64] queries it has finished with, [96] work counter of a concurrent literal pass
+  DevBuf<int> d_redo;  // their indices
+  DevBuf<uint4> d_trail;      // trails of the sorted-set pass: one buffer per wavefront and the spares,
+  DevBuf<int4> d_redo_trail;  // and which of them goes with which entry of d_redo
+  int trails = 1;             // 0 = the literal pass searches every handed-over query from its entry point
+  int trail_cap = 2048;       // records (accepted entries) per trail; a search that outgrows it leaves none
+  int trail_spares = 1024;    // hand-overs with a trail per batch; the ones after that leave none
+  DevBuf<uint4> d_entry;      // longest queries first: level-0 entry of every query of the batch,
+  DevBuf<int> d_order_hist;   // bucket counters,
+  DevBuf<int> d_order;        // and the order the first pass takes the queries in
+  // staging for the host-pointer search entry point
+  DevBuf<float> d_q, d_dist;
+  DevBuf<int> d_nns, d_found;
+  StaticScratch* static_scratch = nullptr;  // this device's copy (device address)
+  int device_ordinal = 0;
+  int* h_ctl = nullptr;                     // pinned: control words read back without staging
+  long long wall_clock_khz = 100000;        // ticks of wall_clock64() per millisecond
+
+  Engine() {
+    has_device = device_present();
+    if (has_device) {
+      int dev = 0;
+      HIP_CHECK(hipGetDevice(&dev));
+      hipDeviceProp_t prop;
+      HIP_CHECK(hipGetDeviceProperties(&prop, dev));
+      num_cus = prop.multiProcessorCount;
+      int khz = 0;
+      if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0) wall_clock_khz = khz;
+      else (void)hipGetLastError();
+      static_scratch = static_scratch_for_current_device(&device_ordinal);
+      HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_ctl), 64 * sizeof(int), hipHostMallocDefault));
+      HIP_CHECK(hipStreamCreate(&stream));
+      HIP_CHECK(hipEventCreate(&ev0));
+      HIP_CHECK(hipEventCreate(&ev1));
+      d_ctl.reserve(128);
+      HIP_CHECK(hipStreamCreate(&stream2));
+      HIP_CHECK(hipEventCreate(&ev_side0));
+      HIP_CHECK(hipEventCreate(&ev_side1));
+    }
+  }
+  ~Engine() {
+    if (ev0) (void)hipEventDestroy(ev0);
+    if (ev1) (void)hipEventDestroy(ev1);
+    if (ev_side0) (void)hipEventDestroy(ev_side0);
+    if (ev_side1) (void)hipEventDestroy(ev_side1);
+    if (stream2) (void)hipStreamDestroy(stream2);
+    if (stream) (void)hipStreamDestroy(stream);
+    if (h_ctl) (void)hipHostFree(h_ctl);
+  }
+
+  void need_device() const {
+    if (!has_device) throw std::runtime_error("no HIP device available: this call needs a GPU");
+  }
+
+  int qr() const { return query_regs(Dp); }
+
+  DevIndex dev_index(float* dists0 = nullptr, float* distsU = nullptr) const {
+    DevIndex ix;
+    ix.vectors = d_vectors.p;
+    ix.labels = host.labelled ? d_labels.p : nullptr;
+    ix.links0 = d_links0.p;
+    ix.linksU = d_linksU.p;
+    ix.upper_off = d_upper_off.p;
+    ix.levels = d_levels.p;
+    ix.dists0 = dists0;
+    ix.distsU = distsU;
+    ix.half = storage_half ? 1 : 0;
+    ix.N = host.N; ix.D = host.D; ix.Dp = Dp; ix.S0 = host.S0; ix.SU = host.SU;
+    ix.max_m = host.max_m; ix.max_m0 = host.max_m0; ix.maxlevel = host.maxlevel;
+    ix.enterpoint = host.enterpoint;
+    return ix;
+  }
+
+  // ---- option / data / level plumbing -------------------------------------------------
+  int init(const char* path) {
+    Options o;
+    int dt = DIST_DOT;
+    std::string why;
+    int rc = load_options(path ? path : "", o, dt, why);
+    if (rc == 0) {
+      opt = o;
+      dist_type = dt;
+    }
+    err = why;  // empty after a successful call
+    return rc;
+  }
+
+  // vectors go up as one contiguous copy (a pitched copy from pageable memory crawls row by
+  // row); rows that need padding are spread out by a small kernel on the device
+  // With fp16 storage the host copy is rounded to the stored values first: everything downstream
+  // (the saved file, a CPU search of that file) then sees exactly the vectors the kernels see.
+  void upload_vectors() {
+    Dp = padded_dims(host.D, tight_rows);
+    const size_t n = (size_t)host.N;
+    if (storage_half) {
+      for (float& x : host.vectors) x = (float)(_Float16)x;
+      d_vectors.reserve((n * Dp + 1) / 2);
+      DevBuf<float> raw;
+      raw.reserve(n * host.D);
+      HIP_CHECK(hipMemcpyAsync(raw.p, host.vectors.data(), n * host.D * sizeof(float), hipMemcpyHostToDevice, stream));
+      HIP_CHECK(hipMemsetAsync(d_vectors.p, 0, n * Dp * sizeof(_Float16), stream));
+      const long long work = (long long)n * host.D;
+      hipLaunchKernelGGL(pad_rows_half_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, raw.p,
+                         reinterpret_cast<_Float16*>(d_vectors.p), (long long)n, host.D, Dp);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipStreamSynchronize(stream));
+      return;
+    }
+    d_vectors.reserve(n * Dp);
+    if (Dp == host.D) {
+      HIP_CHECK(hipMemcpyAsync(d_vectors.p, host.vectors.data(), n * Dp * sizeof(float), hipMemcpyHostToDevice, stream));
+      HIP_CHECK(hipStreamSynchronize(stream));
+      return;
+    }
+    DevBuf<float> raw;
+    raw.reserve(n * host.D);
+    HIP_CHECK(hipMemcpyAsync(raw.p, host.vectors.data(), n * host.D * sizeof(float), hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipMemsetAsync(d_vectors.p, 0, n * Dp * sizeof(float), stream));
+    const long long work = (long long)n * host.D;
+    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, raw.p, d_vectors.p,
+                       (long long)n, host.D, Dp);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+
+  void set_data(const float* data, int n, int d) {
+    if (!data || n <= 0 || d <= 0) throw std::runtime_error("set_data: empty data");
+    host = HostIndex();
+    host.N = n;
+    host.D = d;
+    host.vectors.assign(data, data + (size_t)n * d);
+    have_levels = have_graph = host_links_stale = false;
+    forget_search_history();
+    pool_slots = 0;  // the slot pool is sized by N: rebuild it lazily
+    pool = SlotPool{};
+    if (has_device) upload_vectors();  // without a GPU only the host-side calls remain usable
+    have_data = true;
+  }
+
+  void upload_structure() {
+    d_levels.reserve((size_t)host.N);
+    d_upper_off.reserve((size_t)host.N);
+    d_links0.reserve((size_t)host.N * host.S0);
+    d_linksU.reserve(std::max<size_t>((size_t)host.upper_rows * host.SU, 1));
+    HIP_CHECK(hipMemcpyAsync(d_levels.p, host.levels.data(), (size_t)host.N * 4, hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipMemcpyAsync(d_upper_off.p, host.upper_off.data(), (size_t)host.N * 8, hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  void upload_links() {
+    HIP_CHECK(hipMemcpyAsync(d_links0.p, host.links0.data(), host.links0.size() * 4, hipMemcpyHostToDevice, stream));
+    if (!host.linksU.empty())
+      HIP_CHECK(hipMemcpyAsync(d_linksU.p, host.linksU.data(), host.linksU.size() * 4, hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  void download_links() {
+    HIP_CHECK(hipMemcpyAsync(host.links0.data(), d_links0.p, host.links0.size() * 4, hipMemcpyDeviceToHost, stream));
+    if (!host.linksU.empty())
+      HIP_CHECK(hipMemcpyAsync(host.linksU.data(), d_linksU.p, host.linksU.size() * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    host_links_stale = false;
+  }
+
+  void set_random_levels(const int* levels, int n) {
+    if (!have_data) throw std::runtime_error("set_random_levels: call set_data first");
+    if (n != host.N) throw std::runtime_error("set_random_levels: length differs from the number of data rows");
+    host.max_m = opt.max_m;
+    host.max_m0 = opt.max_m0;
+    host.M = opt.max_m;
+    host.ef_construction = opt.ef_construction;
+    host.mult = opt.level_mult;
+    host.set_levels(levels, n);
+    host.layout_links();
+    host.labelled = false;
+    host.labels.clear();
+    host.deleted.clear();  // a graph built anew holds every element
+    host.n_deleted = 0;
+    have_levels = true;
+    have_graph = false;
+    if (has_device) upload_structure();
+  }
+
+  // What a search learns about an index (how many of its queries tie, whether the two passes ran side by
+  // side) belongs to that index: forgotten whenever another one takes its place.
+  void forget_search_history() {
+    fast_suspended = false;
+    share_known = false;
+    last_repeat_share = 0.0;
+    sequential_left = 0;
+    literal_fallbacks = 0;
+    last_side_by_side = 0;
+    last_repeats = last_trails = 0;
+  }
+
+  // Buffers of a search that do not depend on the batch are allocated when the index becomes resident, not
+  // inside the first search that wants them: the trails of the sorted-set pass (one buffer per wavefront the
+  // GPU can hold plus the spares).  They are an optimisation: if the memory is not there the searches go on
+  // without trails.
+  size_t trail_records_wanted(int slots) const { return (size_t)(slots + trail_spares) * (size_t)trail_cap; }
+  void reserve_trails(int slots) {
+    if (!trails || trails_unavailable) return;
+    if (!d_trail.try_reserve(trail_records_wanted(slots))) trails_unavailable = true;
+  }
+  void prepare_search_buffers() {
+    if (!has_device) return;
+    trails_unavailable = false;
+    reserve_trails(28 * num_cus);  // seven wavefronts per SIMD: what the sorted-set pass holds at most where it keeps trails
+  }
+
+  // ---- slots -----------------------------------------------------------------------------
+  void ensure_pool(int slots, int cand_glob_cap, int log_cap) {
+    const int words = (host.N + 31) / 32;
+    const int undo_cap = std::min(32768, std::max(host.N, 64));
+    if (slots <= pool_slots && words == pool.bitmap_words && cand_glob_cap <= pool.cand_glob_cap &&
+        log_cap <= pool.log_cap && undo_cap == pool.undo_cap)
+      return;
+    slots = std::max(slots, pool_slots);
+    cand_glob_cap = std::max(cand_glob_cap, pool.cand_glob_cap);
+    log_cap = std::max(log_cap, pool.log_cap);
+    d_bitmaps.release();
+    d_bitmaps.reserve((size_t)slots * words);
+    HIP_CHECK(hipMemsetAsync(d_bitmaps.p, 0, (size_t)slots * words * 4, stream));
+    d_undo.reserve((size_t)slots * undo_cap);
+    d_cand_glob.reserve((size_t)slots * cand_glob_cap);
+    d_log.reserve((size_t)slots * log_cap);
+    pool.log = d_log.p;
+    pool.log_cap = log_cap;
+    pool.bitmaps = d_bitmaps.p;
+    pool.bitmap_words = words;
+    pool.undo = d_undo.p;
+    pool.undo_cap = undo_cap;
+    pool.cand_glob = d_cand_glob.p;
+    pool.cand_glob_cap = cand_glob_cap;
+    pool_slots = slots;
+  }
+  // a failed kernel may leave bits set: start over with clean bitmaps
+  void scrub_pool() {
+    HIP_CHECK(hipMemsetAsync(d_bitmaps.p, 0, (size_t)pool_slots * pool.bitmap_words * 4, stream));
+  }
+
+  // slots of sorted result keys per lane: the result set lives in registers while
+  // ef < 64 * NS; 0 selects the literal LDS heap for larger ef
+  static int key_slots(int ef) { return ef <= 128 ? 2 : (ef < 320 ? 5 : (ef <= 512 ? 8 : (ef < 1024 ? 16 : 0))); }
+
+  // LDS entries of the candidate queue.  With the result keys in registers the queue is the
+  // only large LDS user: 2*ef entries hold it in nearly every query (the rest spills to the
+  // slot's global area) and keep ~30 wavefronts per CU resident at ef = 300.
+  int auto_cand_lds(int ef, int ns, int floor_entries, size_t fixed_bytes) const {
+    if (cand_lds_override > 0) return std::max(cand_lds_override, floor_entries);
+    if (ns > 0) return std::max(floor_entries, std::min(std::max(2 * ef, 128), 1024));
+    const size_t budget = 10240;  // ~16 resident wavefronts per CU out of 160 KB LDS
+    size_t used = fixed_bytes + (size_t)(ef + 1) * 8;
+    int c = used < budget ? (int)((budget - used) / 8) : 0;
+    return std::max(c, std::max(floor_entries, 128));
+  }
+
+  // log2 entries of the LDS visited cache (16-bit tags: usable while N >> bits fits 16 bits
+  // with 0xFFFF to spare)
+  int auto_vc_bits() const {
+    if (visited_cache < 0) return 0;
+    int want = visited_cache > 0 ? visited_cache : 1024;
+    int bits = 8;
+    while ((1 << bits) < want && bits < 14) ++bits;
+    if (((unsigned)host.N >> bits) >= 0xFFFFu) return 0;
+    return bits;
+  }
+
+  // log2 of the size in 32-bit words (two 16-bit tags each; a set is two words, four ways) of
+  // the LDS visited filter of the sorted-set search.  A search at ef = 300 evaluates 1 100 to
+  // 1 300 distinct nodes on the million-point sets (max_m0 24 and 32 alike), about 800 at
+  // ef = 100; the filter gets 4 * ef + 512 entries rounded up to a power of two (1 024 up to
+  // ef = 128, 2 048 = 4 KB up to ef = 384), and twice as much when a repeated evaluation is
+  // expensive (rows of 2 KB and more).  More costs occupancy and is slower, less repeats more.
+  // 0 when ids do not fit the tags.
+  int auto_fc_bits(int ef) const {
+    long long want = filter_entries > 0 ? filter_entries : 4ll * ef + 512;
+    if (filter_entries <= 0 && Dp >= 512) want *= 2;
+    int bits = 8;
+    while ((2ll << bits) < want && bits < 13) ++bits;
+    if (((unsigned)host.N >> (bits - 1)) >= 0xFFFFu) return 0;  // tags are 16 bits wide, sets 64
+    return bits;
+  }
+
+  template <typename K>
+  int resident_slots(K kernel, size_t lds) const {
+    int per_cu = 0;
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, lds));
+    per_cu = std::max(1, std::min(per_cu, 32));
+    return per_cu * num_cus;
+  }
+
+  // ---- search ------------------------------------------------------------------------------
+  // (defined in instances.hip, one object per distance and row width)
+  template <int DT, int QR, int NS>
+  void launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_override, float* ms);
+  template <int DT, int QR, int NS>
+  void launch_search_static(const DevIndex& ix, SearchArgs& a, float* ms);
+  template <int DT, int QR>
+  void launch_search_ns(int ns, const DevIndex& ix, SearchArgs& a, float* ms);
+  template <int DT>
+  void launch_search_qr(int q, int ns, const DevIndex& ix, SearchArgs& a, float* ms) {
+    switch (q) {
+      case 1: launch_search_ns<DT, 1>(ns, ix, a, ms); break;
+      case 2: launch_search_ns<DT, 2>(ns, ix, a, ms); break;
+      case 4: launch_search_ns<DT, 4>(ns, ix, a, ms); break;
+      default: launch_search_ns<DT, 0>(ns, ix, a, ms); break;
+    }
+  }
+
+  bool use_static = false;  // the running search is the one that allocates nothing
+
+  void search_device(const float* d_qdata, int nq, int k, int ef, int* d_nns_out, float* d_dist_out, int* d_found_out,
+                     int* d_stats, float* ms, bool no_alloc = false) {
+    need_device();
+    if (!have_graph) throw std::runtime_error("search_knn: no index (call build_graph or load_index first)");
+    if (nq <= 0) return;
+    if (k <= 0) throw std::runtime_error("search_knn: topk must be positive");
+    ef = std::max(ef, k);
+    use_static = no_alloc;
+    if (no_alloc) {
+      if (nq > kStaticMaxQueries)
+        throw std::runtime_error("search_knn (no allocation): at most " + std::to_string(kStaticMaxQueries) + " queries per call");
+      if (ef > kStaticMaxEf)
+        throw std::runtime_error("search_knn (no allocation): max(topk, ef_search) must not exceed " + std::to_string(kStaticMaxEf));
+      if (auto_fc_bits(ef) == 0)
+        throw std::runtime_error("search_knn (no allocation): the index has too many points for the LDS visited filter");
+    }
+    DevIndex ix = dev_index();
+    SearchArgs a{};
+    a.q = d_qdata; a.nq = nq; a.k = k; a.ef = ef;
+    a.nns = d_nns_out; a.dists = d_dist_out; a.found = d_found_out; a.stats = d_stats;
+    a.hnswlib_dist = hnswlib_dist;
+    a.lcap = (std::max(std::max(host.S0, host.SU), std::max(k, 64)) + 63) / 64 * 64;
+    const int q = qr();
+    size_t fixed = (size_t)a.lcap * 8 + (q == 0 ? (size_t)query_lds_chunks(Dp) * 16 : 0);
+    int ns = key_slots(ef);
+    a.vc_bits = auto_vc_bits();
+    a.fast_path = no_alloc ? 2 : (fast_suspended ? 0 : fast_path);
+    a.reverse = opt.reverse_cand ? 1 : 0;
+    // An index with deleted elements (hnswlib's marks in a loaded file) is searched by hnswlib's rule for them:
+    // walked through, never returned.  Only the search on the literal queues in LDS states that rule; it takes
+    // every query of such an index.
+    if (host.n_deleted > 0) {
+      if (no_alloc) throw std::runtime_error("search_knn (no allocation): the index holds deleted elements");
+      if (a.reverse) throw std::runtime_error("search_knn: reverse_cand is not defined on an index with deleted elements");
+      ns = 0;
+      a.fast_path = 0;
+      a.deleted = d_deleted.p;
+    }
+    // reverse_cand: the sorted set in registers expands its farthest entry; beyond its capacity (ef >= 1024) the
+    // literal pass does, on a sorted list in LDS
+    if (a.reverse) a.fast_path = ns > 0 ? 2 : 0;
+    if (a.reverse && no_alloc && ns == 0) throw std::runtime_error("search_knn (no allocation): reverse_cand needs ef_search below 1024");
+    a.fc_bits = (ns > 0 && a.fast_path) ? auto_fc_bits(ef) : 0;
+    if (a.reverse && ns > 0 && a.fc_bits == 0)
+      throw std::runtime_error("search_knn: reverse_cand needs fewer than 2^28 points");
+    // with the keys in registers the queue's LDS share doubles as result buffer (lcap entries,
+    // then lcap label slots) and as the replay heap (ef + 1 entries)
+    const int floor_entries = ns > 0 ? std::max(ef + 1, 2 * a.lcap) : std::max(k, 64);
+    a.cand_lds = auto_cand_lds(ef, ns, floor_entries, fixed);
+    if (dist_type == DIST_DOT) launch_search_qr<DIST_DOT>(q, ns, ix, a, ms);
+    else launch_search_qr<DIST_L2>(q, ns, ix, a, ms);
+  }
+
+  void search_host(const float* q, int nq, int k, int ef, int* nns, float* dists, int* found) {
+    need_device();
+    if (nq <= 0) return;
+    if (!q || !nns || !dists || !found) throw std::runtime_error("search_knn: null argument");
+    if (k <= 0) throw std::runtime_error("search_knn: topk must be positive");
+    d_q.reserve((size_t)nq * host.D);
+    d_nns.reserve((size_t)nq * k);
+    d_dist.reserve((size_t)nq * k);
+    d_found.reserve((size_t)nq);
+    HIP_CHECK(hipMemcpyAsync(d_q.p, q, (size_t)nq * host.D * 4, hipMemcpyHostToDevice, stream));
+    search_device(d_q.p, nq, k, ef, d_nns.p, d_dist.p, d_found.p, nullptr, nullptr);
+    HIP_CHECK(hipMemcpyAsync(nns, d_nns.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipMemcpyAsync(dists, d_dist.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipMemcpyAsync(found, d_found.p, (size_t)nq * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+
+  // ---- build ---------------------------------------------------------------------------------
+  // (defined in instances.hip)
+  template <int DT, int QR, int NS>
+  void build_levels();
+  template <int DT, int QR>
+  void build_ns(int ns);
+  template <int DT>
+  void build_qr(int q, int ns) {
+    switch (q) {
+      case 1: build_ns<DT, 1>(ns); break;
+      case 2: build_ns<DT, 2>(ns); break;
+      case 4: build_ns<DT, 4>(ns); break;
+      default: build_ns<DT, 0>(ns); break;
+    }
+  }
+
+  void build_graph() {
+    need_device();
+    if (!have_data || !have_levels) throw std::runtime_error("build_graph: call set_data and set_random_levels first");
+    HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 4 * sizeof(int), stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    auto t0 = std::chrono::steady_clock::now();
+    const int q = qr();
+    const int ns = build_literal ? 0 : key_slots(opt.ef_construction);
+    if (dist_type == DIST_DOT) build_qr<DIST_DOT>(q, ns);
+    else build_qr<DIST_L2>(q, ns);
+    last_build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    have_graph = true;
+    forget_search_history();
+    prepare_search_buffers();
+    host_links_stale = true;
+  }
+
+  // ---- measurement aid --------------------------------------------------------------------------------
+  // random row gathers over the resident vectors (gather_probe_kernel): returns rows fetched, ms taken
+  void gather_probe(int waves_per_cu, int rows_in_flight, int dependent, double* rows, float* ms) {
+    need_device();
+    if (!have_data) throw std::runtime_error("gather probe: no vectors (call set_data or load_index first)");
+    const int waves = std::max(1, std::min(waves_per_cu, 32)) * num_cus;
+    const int batches = 2048;
+    const int U = rows_in_flight >= 16 ? 4 : (rows_in_flight >= 8 ? 2 : 1);
+    DevBuf<float> sink;
+    sink.reserve((size_t)waves);
+    DevIndex ix = dev_index();
+    float best = 0.f;
+    for (int it = 0; it < 3; ++it) {
+      HIP_CHECK(hipEventRecord(ev0, stream));
+      if (U == 4) hipLaunchKernelGGL(gather_probe_kernel<4>, dim3(waves), dim3(64), 0, stream, ix, batches, dependent, sink.p);
+      else if (U == 2) hipLaunchKernelGGL(gather_probe_kernel<2>, dim3(waves), dim3(64), 0, stream, ix, batches, dependent, sink.p);
+      else hipLaunchKernelGGL(gather_probe_kernel<1>, dim3(waves), dim3(64), 0, stream, ix, batches, dependent, sink.p);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipEventRecord(ev1, stream));
+      HIP_CHECK(hipEventSynchronize(ev1));
+      float t = 0.f;
+      HIP_CHECK(hipEventElapsedTime(&t, ev0, ev1));
+      if (it == 0 || t < best) best = t;
+    }
+    if (rows) *rows = (double)waves * 4.0 * U * batches;
+    if (ms) *ms = best;
+  }
+
+  // ---- index file --------------------------------------------------------------------------------
+  void save_index(const char* path) {
+    if (!have_graph) throw std::runtime_error("save_index: no index to save");
+    if (host_links_stale) download_links();
+    write_index_file(host, path);
+  }
+  void load_index(const char* path) {
+    HostIndex fresh;
+    read_index_file(fresh, path);
+    if (fresh.N <= 0) throw std::runtime_error("load_index: empty index");
+    host = std::move(fresh);
+    have_data = have_levels = have_graph = true;
+    forget_search_history();
+    host_links_stale = false;
+    if (has_device) {
+      upload_vectors();
+      upload_structure();
+      upload_links();
+      d_labels.reserve((size_t)host.N);
+      HIP_CHECK(hipMemcpyAsync(d_labels.p, host.labels.data(), (size_t)host.N * 8, hipMemcpyHostToDevice, stream));
+      std::vector<uint32_t> marks;
+      if (host.n_deleted > 0) {
+        marks.assign(((size_t)host.N + 31) / 32, 0u);
+        for (int i = 0; i < host.N; ++i)
+          if (host.deleted[i]) marks[(size_t)i >> 5] |= 1u << (i & 31);
+        d_deleted.reserve(marks.size());
+        HIP_CHECK(hipMemcpyAsync(d_deleted.p, marks.data(), marks.size() * 4, hipMemcpyHostToDevice, stream));
+      }
+      HIP_CHECK(hipStreamSynchronize(stream));
+      pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
+      pool = SlotPool{};
+      prepare_search_buffers();
+    }
+  }
+};
+
+
+// every instance has an object of its own (instances.hip)
+#define CUHNSW_EXTERN(DT, QR)                                                                                  \
+  extern template void Engine::launch_search_ns<DT, QR>(int, const DevIndex&, SearchArgs&, float*);            \
+  extern template void Engine::build_ns<DT, QR>(int);
+CUHNSW_EXTERN(DIST_DOT, 0) CUHNSW_EXTERN(DIST_DOT, 1) CUHNSW_EXTERN(DIST_DOT, 2) CUHNSW_EXTERN(DIST_DOT, 4)
+CUHNSW_EXTERN(DIST_L2, 0) CUHNSW_EXTERN(DIST_L2, 1) CUHNSW_EXTERN(DIST_L2, 2) CUHNSW_EXTERN(DIST_L2, 4)
+#undef CUHNSW_EXTERN
+
+}  // namespace cuhnsw_amd

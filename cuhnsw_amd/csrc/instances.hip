@@ -1,0 +1,536 @@
+// Launches of the templated kernels, compiled once per distance and row width: the build passes CUHNSW_DT (DistType)
+// and CUHNSW_QR (kernels.h, query_regs), so that the objects compile side by side.
+#include "engine.h"
+
+namespace cuhnsw_amd {
+
+// (the no-allocation search clears its control words with this kernel: it issues no memset)
+static __global__ void __launch_bounds__(128) fill_ints_kernel(int* p, int n, int value) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = value;
+}
+// Everything a two-pass search needs cleared, in one launch: the control words (0), the list the first pass
+// appends to (-1 = "no entry yet", which the literal wavefronts poll for) and, for a batch taken longest
+// first, the counters of the counting sort (0).
+static __global__ void __launch_bounds__(256) prepare_search_kernel(int* ctl, int n_ctl, int* redo, int n_redo, int* hist, int n_hist) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_ctl) ctl[i] = 0;
+  if (i < n_redo) redo[i] = -1;
+  if (i < n_hist) hist[i] = 0;
+}
+
+// Two passes: every query on the sorted set in registers (search_fast_kernel); the queries
+// in which equal keys met, and every query when ef exceeds the set's capacity, with the
+// literal priority queues (search_kernel).  The literal pass normally runs at the same time
+// on a second stream, on one wavefront per SIMD, and picks the given-up queries off a list
+// as the first pass appends them; should it report a problem (its bounded wait ran out, or a
+// queue overflowed) the list is answered again after the first pass.  ms covers everything.
+template <int DT, int QR, int NS>
+void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_override, float* ms) {
+  a.counter = d_ctl.p;
+  a.status = d_ctl.p + 1;
+  a.repeats = d_ctl.p + 32;   // the counters of the two passes sit in separate 128-byte lines
+  a.done = d_ctl.p + 64;
+  a.redo = nullptr;
+  a.live = 0;
+  a.nq_total = a.nq;
+  a.slot_base = 0;
+  // a literal wavefront beside the first pass waits at most 2 ms for that pass to start (it is launched
+  // microseconds later unless something serialises the two streams) and accepts no progress of a
+  // started first pass for 100 ms (its queries finish every few microseconds)
+  a.spin_limit = spin_limit_override;
+  a.start_ticks = 2 * wall_clock_khz;
+  a.stall_ticks = 100 * wall_clock_khz;
+  a.nq_dev = nullptr;
+  a.entry = nullptr;
+  a.order_hist = nullptr;
+  a.order = nullptr;
+  a.trail = nullptr;
+  a.redo_trail = nullptr;
+  a.trail_next = nullptr;
+  a.trail_cap = a.trail_first_spare = a.trail_spares = 0;
+  last_repeats = 0;
+  last_trails = 0;
+  if (use_static) {
+    launch_search_static<DT, QR, NS>(ix, a, ms);
+    return;
+  }
+  HIP_CHECK(hipEventRecord(ev0, stream));
+  // the literal pass runs on the sorted set with ids and the LDS filter (no bitmap) unless the
+  // caller asked for literal queues only, which also means exact evaluation counters
+  // ...and unless the visited bitmaps of the wavefronts at work fit the L2 caches (32 MB) together:
+  // there the bitmap's atomics are cheap and the literal search with them is the faster one
+  const size_t bitmap_bytes = (size_t)std::min(num_cus * 24, a.nq) * ((host.N + 31) / 32) * 4;
+  const bool want_lean = lean_literal == 1 ? bitmap_bytes > ((size_t)32 << 20) : lean_literal > 1;
+  a.lean = (NS > 0 && fast_path != 0 && want_lean) ? auto_fc_bits(a.ef) : 0;
+  if (a.lean && filter_entries <= 0) {
+    // a batch of few queries leaves most of each CU's LDS unused: give the filter what is there
+    // (up to 32 KB), so that it forgets next to nothing
+    const int per_cu = (a.nq + num_cus - 1) / num_cus;
+    const size_t room = per_cu > 0 ? (size_t)(150 * 1024) / per_cu : 0;
+    const size_t other = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, 0, 0, 0).total + 256;
+    while (a.lean < 13 && other + ((size_t)4 << (a.lean + 1)) <= std::min<size_t>(room, 60 * 1024) &&
+           (((unsigned)host.N >> a.lean) < 0xFFFFu))
+      ++a.lean;
+  }
+  const LdsPlan lp = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean);
+  auto kernel = search_kernel<DT, QR, NS>;
+  int lit_slots = resident_slots(kernel, lp.total);
+  if (max_slots_override > 0) lit_slots = max_slots_override;
+  int glob_cap = spill_cap > 0 ? spill_cap : std::max(4096, 8 * a.ef);
+  int n_literal = a.nq;
+  bool answered = false;
+  bool timed = false;  // ev1 has been recorded after the last kernel of this search
+  // A batch that fits the machine in one round of literal wavefronts is latency-bound: where the literal
+  // search has its exact bitmaps, two passes would only add the second pass's latency to the first's, and
+  // the literal pass answers alone.  Where the bitmaps do not fit the L2 (the literal search then runs on
+  // the sorted set with the LDS filter) the first pass is the same search without the literal candidate
+  // queue, and the faster choice even with a hand-over.
+  // (Long rows — the query in LDS — go to the first pass whatever the batch: there the literal search takes twice
+  // the first pass's time per expanded candidate, 2.0 against 1.0 ms for a single query on 1 M x 960.)
+  if (NS > 0 && a.fast_path && a.fc_bits > 0 &&
+      (a.fast_path > 1 || a.nq > lit_slots || (a.lean && a.nq > 1) || QR == 0)) {  // (reverse_cand: fast_path is 2)
+    d_redo.reserve((size_t)a.nq);
+    a.redo = d_redo.p;
+    auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
+    auto fast_lds = [&](int bits) -> size_t { return plan_fast_lds(QR, ix.Dp, a.lcap, bits).total; };
+    auto fast_slots = [&](int bits) -> int { return resident_slots(fast_kernel, fast_lds(bits)); };
+    // the filter must not be what limits the wavefronts per CU: half the filter repeats more
+    // evaluations but is the faster choice wherever it buys 15 % more wavefronts
+    while (filter_entries <= 0 && a.fc_bits > 9) {
+      const int now = fast_slots(a.fc_bits);
+      const int with_half = fast_slots(a.fc_bits - 1);
+      if (with_half * 20 < now * 23) break;  // less than 15 % more
+      --a.fc_bits;
+    }
+    const size_t fast_lds_bytes = fast_lds(a.fc_bits);
+    int slots = fast_slots(a.fc_bits);
+    const bool side = concurrent_literal && sequential_left == 0 && max_slots_override <= 0;
+    last_side_by_side = side ? 1 : 0;
+    int side_slots = 0;
+    // few queries need the literal pass: one wavefront per CU serves them without taking room from
+    // the first pass; two when the last search handed over 2 % and more (a literal wavefront's LDS
+    // is that of one and a half wavefronts of the first pass, so more of them cost more than they serve)
+    const int per_cu = side_per_cu > 0 ? side_per_cu : (last_repeat_share < 0.02 ? 1 : 2);
+    if (side) {
+      side_slots = std::min(num_cus * per_cu, a.nq);
+      // an index that hands over next to nothing (the last search: under one query in a thousand) gets one
+      // literal wavefront per four CUs, and the first pass the room of the others
+      if (side_per_cu <= 0 && share_known && last_repeat_share < 0.001) side_slots = std::min(std::max(num_cus / 4, 1), a.nq);
+      ensure_pool(std::max(side_slots, 1), glob_cap, 2 * glob_cap);
+      slots = std::max(num_cus, slots - std::min(side_slots, num_cus * per_cu));  // leave the literal wavefronts their room
+    }
+    if (max_slots_override > 0) slots = max_slots_override;
+    if (first_pass_waves > 0) slots = std::min(slots, first_pass_waves * num_cus);
+    slots = std::max(1, std::min(slots, a.nq));
+    // (every allocation before the literal pass is launched: growing a buffer frees the old one, and
+    // hipFree waits for the device, on which that pass would be waiting for the first pass to start)
+    const long long resident = slots;  // queries at work at a time
+    // A handed-over query is not searched again from its entry point: the first pass leaves the entries it
+    // accepted, hop by hop, and the literal pass (on the sorted set with ids: it needs no visited bitmap
+    // brought up to date) replays its queue operations from them up to where the two may part.  One query per
+    // wavefront, link rows of one pass of 64 lanes, and batches of under three rounds of wavefronts: keeping
+    // the trail costs the first pass 9 % (the kernel instance with the trail code 4 %, writing the records the
+    // rest), which only a batch short enough to wait for its last hand-over gets back.  trails = 2: whatever
+    // the batch.
+    bool keep_trails = (QR == 1 || QR == 2) && trails && !a.reverse && a.lean && host.S0 <= 63 &&
+                       (trails > 1 || 4 * (long long)a.nq <= 11 * resident);
+    if (keep_trails) {
+      // (normally there since the index became resident; a changed trail_cap / trail_spares asks again)
+      if (d_trail.n < trail_records_wanted(slots)) {
+        trails_unavailable = false;
+        reserve_trails(slots);
+      }
+      keep_trails = !trails_unavailable && d_trail.n >= trail_records_wanted(slots);
+    }
+    // (with trails a late hand-over costs less, and the order pays from one round on)
+    const bool in_order = query_order && (query_order > 1 ? a.nq > resident
+                                                           : (keep_trails ? a.nq > resident : 2 * a.nq >= 3 * resident) &&
+                                                                 a.nq <= 32 * resident);
+    if (in_order) {
+      d_entry.reserve((size_t)a.nq);
+      d_order.reserve((size_t)a.nq);
+      d_order_hist.reserve((size_t)kOrderBuckets);
+    }
+    if (keep_trails) {
+      d_redo_trail.reserve((size_t)a.nq);
+      a.trail = d_trail.p;
+      a.trail_cap = trail_cap;
+      a.trail_first_spare = slots;
+      a.trail_spares = trail_spares;
+      a.trail_next = d_ctl.p + 48;
+      a.redo_trail = d_redo_trail.p;
+    }
+    {
+      const int n_hist = in_order ? kOrderBuckets : 0;
+      const int n_fill = std::max(std::max(a.nq, n_hist), 128);
+      hipLaunchKernelGGL(prepare_search_kernel, dim3((unsigned)((n_fill + 255) / 256)), dim3(256), 0, stream, d_ctl.p, 128,
+                         d_redo.p, a.nq, in_order ? d_order_hist.p : nullptr, n_hist);
+      HIP_CHECK(hipGetLastError());
+    }
+    if (side) {
+      SearchArgs b = a;
+      b.live = 1;
+      b.entry = in_order ? d_entry.p : nullptr;  // (a query reaches that pass after the batch's descents are done)
+      b.counter = d_ctl.p + 96;
+      b.pool = pool;
+      // one or two of these wavefronts per CU: LDS for a candidate queue that never spills costs the first
+      // pass nothing (the queue of a long search outgrows 2 * ef entries)
+      if (NS > 0) b.cand_lds = std::max(a.cand_lds, 1024);
+      const LdsPlan lp_side = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, b.cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean);
+      // (the first pass starts after the batch's descents when its queries are put in order: 0.1 ms per
+      // 10 000 queries of the 1.18 M x 50 set; allow ten times that on top of the usual 2 ms)
+      b.start_ticks += (long long)wall_clock_khz * (a.nq / 10000 + 1);
+      HIP_CHECK(hipEventRecord(ev_side0, stream));
+      HIP_CHECK(hipStreamWaitEvent(stream2, ev_side0, 0));
+      hipLaunchKernelGGL(kernel, dim3(side_slots), dim3(64), lp_side.total, stream2, ix, b);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipEventRecord(ev_side1, stream2));
+    }
+    // more than one round of wavefronts: the batch's descents first, then its queries longest first.  (The
+    // literal pass has been launched by now: launched after the first pass it would find no room until the
+    // first of that pass's wavefronts leave, a third of the way through the batch.)
+    if (in_order) {
+      a.entry = d_entry.p;
+      a.order = d_order.p;
+      a.order_hist = d_order_hist.p;
+      if constexpr (QR == 1 || QR == 2) {
+        // four queries per wavefront, one per group of 16 lanes
+        auto k_entry = entry4_kernel<DT, QR>;
+        const int entry_grid = std::max(1, std::min((a.nq + 3) / 4, resident_slots(k_entry, 0)));
+        hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), 0, stream, ix, a);
+      } else {
+        auto k_entry = entry_kernel<DT, QR>;
+        const size_t entry_lds = plan_fast_lds(QR, ix.Dp, a.lcap, 0).total;
+        const int entry_grid = std::max(1, std::min(a.nq, resident_slots(k_entry, entry_lds)));
+        hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), entry_lds, stream, ix, a);
+      }
+      HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(order_prefix_kernel, dim3(1), dim3(1024), 0, stream, d_order_hist.p);
+      HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(order_scatter_kernel, dim3((unsigned)((a.nq + 1023) / 1024)), dim3(1024), 0, stream, d_entry.p,
+                         a.nq, d_order_hist.p, d_order.p);
+      HIP_CHECK(hipGetLastError());
+    }
+    if constexpr (QR == 1 || QR == 2) {
+      if (keep_trails) hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
+      else hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
+    } else {
+      hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
+    }
+    HIP_CHECK(hipGetLastError());
+    if (side) {
+      HIP_CHECK(hipStreamWaitEvent(stream, ev_side1, 0));
+    }
+    HIP_CHECK(hipEventRecord(ev1, stream));  // (recorded again further down if the list has to be answered after all)
+    timed = true;
+    int* ctl = h_ctl;  // pinned: read back without a staging copy
+    HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, 49 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    n_literal = last_repeats = ctl[32];
+    last_trails = ctl[48];
+    last_repeat_share = (double)n_literal / a.nq;
+    share_known = true;
+    if (!side && sequential_left > 0) --sequential_left;
+    // an index whose distances tie all the time (integer-valued data) sends most queries
+    // through both passes: stop trying the sorted set on it
+    if (a.nq >= 256 && (long long)n_literal * 3 > a.nq) fast_suspended = true;
+    if (side) {
+      answered = ctl[1] == 0;
+      if (!answered) {
+        scrub_pool();
+        if (ctl[1] & 1) glob_cap *= 4;
+        // the wait ran out: the streams of this process do not run side by side at present (a profiler
+        // collecting counters, a saturated device); the next searches run one pass after the other
+        if (ctl[1] & 2) {
+          sequential_left = kSequentialSearches;
+          ++literal_fallbacks;
+        }
+      }
+    }
+  }
+  if (n_literal > 0 && !answered) {
+    timed = false;
+    SearchArgs b = a;
+    b.nq = n_literal;
+    int slots = std::max(1, std::min(lit_slots, b.nq));
+    bool done = false;
+    for (int attempt = 0; attempt < 8 && !done; ++attempt) {
+      ensure_pool(slots, glob_cap, 2 * glob_cap);
+      b.pool = pool;
+      HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 3 * sizeof(int), stream));
+      hipLaunchKernelGGL(kernel, dim3(slots), dim3(64), lp.total, stream, ix, b);
+      HIP_CHECK(hipGetLastError());
+      int ctl[2];
+      HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, sizeof(ctl), hipMemcpyDeviceToHost, stream));
+      HIP_CHECK(hipStreamSynchronize(stream));
+      done = ctl[1] == 0;
+      if (!done) {
+        scrub_pool();
+        glob_cap *= 4;  // a candidate queue or accept log overflowed its global area: retry with more room
+      }
+    }
+    if (!done) throw std::runtime_error("search: candidate queue overflow");
+  }
+  if (!timed) {
+    HIP_CHECK(hipEventRecord(ev1, stream));
+    HIP_CHECK(hipEventSynchronize(ev1));
+  }
+  if (ms) HIP_CHECK(hipEventElapsedTime(ms, ev0, ev1));
+}
+// The search of the entry point that allocates nothing: the sorted-set pass over every query, then the
+// literal pass over the list it left, one after the other on the engine's stream.  The length of the
+// list stays on the device (the literal kernel reads it there), so nothing is read back in between;
+// control words, list and the literal wavefronts' queue overflow and log areas live in this device's
+// copy of the static scratch array.  No hipMalloc, no hipFree, no memset: a fill kernel clears the
+// control words, the list needs no clearing (the pass after reads only the entries the count vouches
+// for).  Calls that overlap on one GPU would share the array and race.
+template <int DT, int QR, int NS>
+void Engine::launch_search_static(const DevIndex& ix, SearchArgs& a, float* ms) {
+  if constexpr (NS > 0) {
+    StaticScratchLease lease(device_ordinal);  // released on every way out of this function
+    StaticScratch* sc = static_scratch;
+    a.counter = sc->ctl;
+    a.status = sc->ctl + 1;
+    a.repeats = sc->ctl + 32;
+    a.done = sc->ctl + 64;
+    a.redo = sc->redo;
+    a.fast_path = 2;
+    a.lean = a.fc_bits;  // literal searches keep the LDS filter and the sorted set with ids: no bitmap in HBM
+    auto kernel = search_kernel<DT, QR, NS>;
+    auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
+    while (filter_entries <= 0 && a.fc_bits > 9) {  // (as in the allocating search: the filter must not cost occupancy)
+      const int now = resident_slots(fast_kernel, plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits).total);
+      const int with_half = resident_slots(fast_kernel, plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits - 1).total);
+      if (with_half * 20 < now * 23) break;
+      --a.fc_bits;
+    }
+    const FastLdsPlan fp = plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits);
+    const LdsPlan lp = plan_lds(QR, ix.Dp, -1, a.cand_lds, a.lcap, 0, 0, 0, 0, a.lean);
+    const int slots = std::max(1, std::min(resident_slots(fast_kernel, fp.total), a.nq));
+    const int lit_slots = std::max(1, std::min(std::min(resident_slots(kernel, lp.total), kStaticSlots), a.nq));
+    HIP_CHECK(hipEventRecord(ev0, stream));
+    hipLaunchKernelGGL(fill_ints_kernel, dim3(1), dim3(128), 0, stream, sc->ctl, 128, 0);
+    HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fp.total, stream, ix, a);
+    HIP_CHECK(hipGetLastError());
+    SearchArgs b = a;
+    b.nq = 0;
+    b.nq_dev = sc->ctl + 32;
+    b.counter = sc->ctl + 96;
+    b.pool = SlotPool{};
+    b.pool.cand_glob = sc->cand_glob;
+    b.pool.cand_glob_cap = kStaticGlobCap;
+    b.pool.log = sc->log;
+    b.pool.log_cap = kStaticLogCap;
+    hipLaunchKernelGGL(kernel, dim3(lit_slots), dim3(64), lp.total, stream, ix, b);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipEventRecord(ev1, stream));
+    HIP_CHECK(hipMemcpyAsync(h_ctl, sc->ctl, 33 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    last_repeats = h_ctl[32];
+    if (ms) HIP_CHECK(hipEventElapsedTime(ms, ev0, ev1));
+    if (h_ctl[1] != 0)
+      throw std::runtime_error("search_knn (no allocation): a literal search outgrew its share of the static scratch "
+                               "(candidate queue or accept log); use cuhnsw_search_knn_device for this batch");
+  } else {
+    (void)ix; (void)a; (void)ms;
+    throw std::runtime_error("search_knn (no allocation): ef_search beyond the sorted set's capacity");
+  }
+}
+
+template <int DT, int QR>
+void Engine::launch_search_ns(int ns, const DevIndex& ix, SearchArgs& a, float* ms) {
+  switch (ns) {
+    case 2: launch_search<DT, QR, 2>(ix, a, search_slots, ms); break;
+    case 5: launch_search<DT, QR, 5>(ix, a, search_slots, ms); break;
+    case 8: launch_search<DT, QR, 8>(ix, a, search_slots, ms); break;
+    case 16: launch_search<DT, QR, 16>(ix, a, search_slots, ms); break;
+    default: launch_search<DT, QR, 0>(ix, a, search_slots, ms); break;
+  }
+}
+
+// ---- build ---------------------------------------------------------------------------------
+template <int DT, int QR, int NS>
+void Engine::build_levels() {
+  const int N = host.N;
+  const int cap_in = 32;
+  const int bmax = build_batch > 0 ? build_batch : std::min(std::max(N, 1), 65536);
+  const int m_max = std::max(host.max_m, host.max_m0);
+  const size_t up_rows = std::max<size_t>((size_t)host.upper_rows, 1);
+  DevBuf<float> d_dists0, d_distsU, d_sel0_keys, d_selU_keys;
+  DevBuf<uint32_t> d_sel0_ids, d_selU_ids;
+  DevBuf<unsigned long long> d_dirty;
+  DevBuf<int> d_sel0_cnt, d_selU_cnt, d_inbox0_cnt, d_inboxU_cnt;
+  DevBuf<HeapEnt> d_inbox0, d_inboxU;
+  DevBuf<unsigned char> d_selected;  // per link row: the row is an output of the selection rule (kernels.h, BuildArgs)
+  d_dists0.reserve((size_t)N * host.S0);
+  d_distsU.reserve(up_rows * host.SU);
+  d_sel0_ids.reserve((size_t)bmax * host.max_m0);
+  d_sel0_keys.reserve((size_t)bmax * host.max_m0);
+  d_sel0_cnt.reserve((size_t)bmax);
+  d_selU_ids.reserve(up_rows * host.max_m);
+  d_selU_keys.reserve(up_rows * host.max_m);
+  d_selU_cnt.reserve(up_rows);
+  // a batch node posts at most max_m0 links on level 0 and max_m on each upper level
+  d_dirty.reserve((size_t)bmax * ((size_t)host.max_m0 + (size_t)std::max(host.maxlevel, 1) * host.max_m));
+  d_inbox0.reserve((size_t)N * cap_in);
+  d_inbox0_cnt.reserve((size_t)N);
+  d_inboxU.reserve(up_rows * cap_in);
+  d_inboxU_cnt.reserve(up_rows);
+  if (newcomer_shortcut) {
+    d_selected.reserve((size_t)N + up_rows);
+    HIP_CHECK(hipMemsetAsync(d_selected.p, 0, (size_t)N + up_rows, stream));
+  }
+  HIP_CHECK(hipMemsetAsync(d_inbox0_cnt.p, 0, (size_t)N * 4, stream));
+  HIP_CHECK(hipMemsetAsync(d_inboxU_cnt.p, 0, up_rows * 4, stream));
+  HIP_CHECK(hipMemsetAsync(d_links0.p, 0xFF, (size_t)N * host.S0 * 4, stream));
+  if (host.upper_rows > 0) HIP_CHECK(hipMemsetAsync(d_linksU.p, 0xFF, (size_t)host.upper_rows * host.SU * 4, stream));
+
+  DevIndex ix = dev_index(d_dists0.p, d_distsU.p);
+  auto k_search = build_search_kernel<DT, QR, NS>;
+  auto k_reverse = reverse_kernel<DT, QR>;
+  const int efc = opt.ef_construction;
+  const int glob_cap = std::max(4096, 8 * efc);
+
+  BuildArgs a{};
+  a.efc = efc;
+  // (the reference multiplies in single precision: `const int nn_num = max_m * heuristic_coef` with a
+  // float coefficient, cpp/include/cuda_build_kernels.cuh:77,101)
+  a.nn_num0 = (int)((float)host.max_m0 * (float)opt.heuristic_coef);
+  a.nn_numU = (int)((float)host.max_m * (float)opt.heuristic_coef);
+  a.save_remains = opt.save_remains ? 1 : 0;
+  a.reverse = opt.reverse_cand ? 1 : 0;
+  a.own_cap0 = own_links0 > 0 ? std::min(own_links0, host.max_m0) : host.max_m0;
+  a.sel0_ids = d_sel0_ids.p; a.sel0_keys = d_sel0_keys.p; a.sel0_cnt = d_sel0_cnt.p;
+  a.selU_ids = d_selU_ids.p; a.selU_keys = d_selU_keys.p; a.selU_cnt = d_selU_cnt.p;
+  a.counter = d_ctl.p; a.status = d_ctl.p + 1;
+  a.inbox0 = d_inbox0.p; a.inbox0_cnt = d_inbox0_cnt.p;
+  a.inboxU = d_inboxU.p; a.inboxU_cnt = d_inboxU_cnt.p;
+  a.cap_in = cap_in;
+  a.dirty = d_dirty.p; a.dirty_cnt = d_ctl.p + 2;
+  a.dropped = d_ctl.p + 3;
+  a.selected0 = newcomer_shortcut ? d_selected.p : nullptr;
+  a.selectedU = newcomer_shortcut ? d_selected.p + N : nullptr;
+  DevBuf<unsigned long long> d_work;
+  if (count_build_work) {
+    d_work.reserve(10);
+    HIP_CHECK(hipMemsetAsync(d_work.p, 0, 10 * sizeof(unsigned long long), stream));
+  }
+  a.counters = d_work.p;
+  const int s_max = std::max(host.S0, host.SU);
+  a.lcap = (std::max(s_max, 64) + 63) / 64 * 64;
+  size_t fixed = (size_t)a.lcap * 8 + (size_t)efc * 8 + (size_t)m_max * 8 + 64 +
+                 (QR == 0 ? (size_t)query_lds_chunks(Dp) * 16 : 0);
+  a.fc_bits = NS > 0 ? auto_fc_bits(efc) : 0;
+  const bool sorted_set = NS > 0 && a.fc_bits > 0;  // then neither queue nor literal cache is needed
+  if (a.reverse && NS > 0 && !sorted_set) throw std::runtime_error("build_graph: reverse_cand needs fewer than 2^28 points");
+  a.cand_lds = sorted_set ? 0 : auto_cand_lds(efc, NS, 64, fixed);
+  a.vc_bits = sorted_set ? 0 : auto_vc_bits();
+  const LdsPlan lp1 = plan_lds(QR, Dp, sorted_set ? -1 : efc, a.cand_lds, a.lcap, efc, m_max, a.vc_bits, a.fc_bits);
+  const LdsPlan lp3 = plan_lds(QR, Dp, s_max + cap_in, 0, a.lcap, s_max + cap_in, std::max(m_max, cap_in));
+  const int slots1 = resident_slots(k_search, lp1.total);
+  const int slots3 = resident_slots(k_reverse, lp3.total);
+  // the sorted-set search needs no per-wavefront global memory (no bitmap, no undo list, no log)
+  if (!sorted_set) ensure_pool(slots1, glob_cap, 2 * glob_cap);
+  a.pool = pool;
+
+  // Nodes go in by ascending id, as hnswlib inserts them.  The graph a batch sees is the
+  // one of all earlier batches: its entry point is the first node that reached the highest
+  // level so far.  Batches grow with the graph — a quarter of what is already in, up to 16 384 nodes, so
+  // that early nodes, which wire the long-range links, see each other; beyond half a million nodes a
+  // thirty-second of the graph, up to 65 536 — because the nodes of a batch do not see each other (recall
+  // falls when the share of new nodes grows), and a launch of several rounds of wavefronts loses less to
+  // its last, partly filled round.
+  // build_batch > 0 replaces the two caps by one.
+  auto batch_at = [&](int in) {
+    if (build_batch > 0) return std::max(1, std::min(build_batch, in / 4));
+    return std::max(1, std::min(in / 4, std::max(16384, std::min(65536, in / 32))));
+  };
+  // within a batch the nodes with upper levels are handed out first (highest level first, then by id)
+  DevBuf<int> d_order;
+  {
+    std::vector<int> order((size_t)N);
+    for (int p0 = 0; p0 < N;) {
+      const int b = std::min(batch_at(p0), N - p0);
+      int* o = order.data() + p0;
+      int n_up = 0;
+      for (int i = 0; i < b; ++i)
+        if (host.levels[p0 + i] > 0) o[n_up++] = i;
+      std::stable_sort(o, o + n_up, [&](int x, int y) { return host.levels[p0 + x] > host.levels[p0 + y]; });
+      for (int i = 0, w = n_up; i < b; ++i)
+        if (host.levels[p0 + i] <= 0) o[w++] = i;
+      p0 += b;
+    }
+    d_order.reserve((size_t)N);
+    HIP_CHECK(hipMemcpyAsync(d_order.p, order.data(), (size_t)N * sizeof(int), hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  a.order = level_first ? d_order.p : nullptr;
+  int cur_ep = 0, cur_max = -1;
+  int pos = 0;
+  while (pos < N) {
+    int b = batch_at(pos);
+    b = std::min(b, N - pos);
+    a.begin = pos;
+    a.count = b;
+    a.cur_ep = cur_ep;
+    a.cur_max = cur_max;
+    // counter and dirty count back to zero; the status word is sticky
+    HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, sizeof(int), stream));
+    HIP_CHECK(hipMemsetAsync(d_ctl.p + 2, 0, sizeof(int), stream));
+    hipLaunchKernelGGL(k_search, dim3(std::min(b, slots1)), dim3(64), lp1.total, stream, ix, a);
+    HIP_CHECK(hipGetLastError());
+    if (cur_max >= 0) {
+      long long work = (long long)b * m_max;
+      hipLaunchKernelGGL(apply_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, ix, a);
+      HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(k_reverse, dim3((unsigned)std::min<long long>(work, slots3)), dim3(64), lp3.total, stream, ix, a);
+      HIP_CHECK(hipGetLastError());
+    }
+    for (int i = pos; i < pos + b; ++i)
+      if (host.levels[i] > cur_max) {
+        cur_max = host.levels[i];
+        cur_ep = i;
+      }
+    pos += b;
+  }
+  int ctl[4];
+  HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, sizeof(ctl), hipMemcpyDeviceToHost, stream));
+  HIP_CHECK(hipStreamSynchronize(stream));
+  if (ctl[1] != 0) {
+    scrub_pool();
+    throw std::runtime_error("build_graph: candidate queue overflow");
+  }
+  last_build_dropped = ctl[3];
+  std::memset(build_counters, 0, sizeof(build_counters));
+  if (count_build_work) {
+    HIP_CHECK(hipMemcpyAsync(build_counters, d_work.p, sizeof(build_counters), hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  if (keep_link_keys) {
+    // debugging aid: the key stored with every level-0 link, for a validator to recompute
+    std::vector<float> strided((size_t)N * host.S0);
+    HIP_CHECK(hipMemcpyAsync(strided.data(), d_dists0.p, strided.size() * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    link_keys0.assign((size_t)N * host.max_m0, 0.f);
+    for (int i = 0; i < N; ++i)
+      std::memcpy(&link_keys0[(size_t)i * host.max_m0], &strided[(size_t)i * host.S0], (size_t)host.max_m0 * 4);
+  }
+}
+
+template <int DT, int QR>
+void Engine::build_ns(int ns) {
+  switch (ns) {
+    case 2: build_levels<DT, QR, 2>(); break;
+    case 5: build_levels<DT, QR, 5>(); break;
+    case 8: build_levels<DT, QR, 8>(); break;
+    case 16: build_levels<DT, QR, 16>(); break;
+    default: build_levels<DT, QR, 0>(); break;
+  }
+}
+
+template void Engine::launch_search_ns<CUHNSW_DT, CUHNSW_QR>(int, const DevIndex&, SearchArgs&, float*);
+template void Engine::build_ns<CUHNSW_DT, CUHNSW_QR>(int);
+
+}  // namespace cuhnsw_amd

@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(64) entry4_kernel(DevIndex ix, SearchArgs a) {
   else entry4_body<DT, QR, false>(ix, a);
 }
 // counters -> first position of every bucket (exclusive prefix sum; one workgroup of 1024)
-__global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist) {
+static __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist) {
   __shared__ int part[1024];
   constexpr int per = kOrderBuckets / 1024;
   const int t = threadIdx.x;
@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist) {
     run += local[i];
   }
 }
-__global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4* entry, int nq, int* cursor, int* order) {
+static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4* entry, int nq, int* cursor, int* order) {
   // The keys of a batch fall into a few dozen buckets: a workgroup ranks its 1024 queries in LDS and takes one
   // range per bucket it met from the global cursors (the order inside a bucket is free).
   __shared__ int cnt[kOrderBuckets];
@@ -1098,7 +1098,7 @@ __device__ __forceinline__ float* dist_row_mut(const DevIndex& ix, uint32_t node
 
 // Phase 2: write the selected rows and post the reverse links.  Thread (b, j) handles slot j
 // of node b on each of its levels.
-__global__ void __launch_bounds__(256) apply_kernel(DevIndex ix, BuildArgs a) {
+static __global__ void __launch_bounds__(256) apply_kernel(DevIndex ix, BuildArgs a) {
   const int m_max = ix.max_m0 > ix.max_m ? ix.max_m0 : ix.max_m;
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (long long)a.count * m_max) return;
@@ -1391,7 +1391,7 @@ __global__ void __launch_bounds__(64) gather_probe_kernel(DevIndex ix, int batch
 }
 
 // Upload helper for fp16 storage: N x D floats into rows of Dp halves (the padding was zeroed before).
-__global__ void __launch_bounds__(256) pad_rows_half_kernel(const float* src, _Float16* dst, long long n, int D, int Dp) {
+static __global__ void __launch_bounds__(256) pad_rows_half_kernel(const float* src, _Float16* dst, long long n, int D, int Dp) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n * D) return;
   const long long row = i / D;
@@ -1400,7 +1400,7 @@ __global__ void __launch_bounds__(256) pad_rows_half_kernel(const float* src, _F
 }
 
 // Upload helper: copies N x D floats into rows of Dp floats (the padding was zeroed before).
-__global__ void __launch_bounds__(256) pad_rows_kernel(const float* src, float* dst, long long n, int D, int Dp) {
+static __global__ void __launch_bounds__(256) pad_rows_kernel(const float* src, float* dst, long long n, int D, int Dp) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n * D) return;
   const long long row = i / D;
