@@ -100,5 +100,10 @@ def random_levels(n, level_mult, seed=777):
   """Level stream of the Python wrapper (cuhnsw/pyhnsw.py:65-71 in the
   reference): legacy MT19937 uniform draws, truncated -ln(u) * mult."""
   np.random.seed(seed)
-  u = np.maximum(np.random.uniform(size=n), 1e-10)
-  return (-np.log(u) * level_mult).astype(np.int32)
+  u = np.random.uniform(size=n)
+  levels = np.zeros(n, np.int32)
+  # only draws below exp(-1 / level_mult) reach level 1: one in max_m with the default multiplier, and the
+  # logarithm is taken of those alone (a hair's breadth more of them, so that its rounding decides)
+  some = np.flatnonzero(u <= np.exp(-1.0 / level_mult) * (1.0 + 1e-9)) if level_mult > 0 else np.arange(n)
+  levels[some] = (-np.log(np.maximum(u[some], 1e-10)) * level_mult).astype(np.int32)
+  return levels
