@@ -94,7 +94,7 @@ def build_bind():
       "-I" + sysconfig.get_paths()["include"],
       "-I" + os.path.join(HERE, "..", "include"),
   ]
-  _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden"] +
+  _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", "-fvisibility=hidden"] +
        inc + [os.path.join(CSRC, "bindings.cc"), "-o", BIND,
               "-L" + HERE, "-lcuhnsw_amd", "-Wl,-rpath,$ORIGIN"])
   return BIND

@@ -4,8 +4,15 @@
 #include <pybind11/numpy.h>
 #include <pybind11/pybind11.h>
 
+#include <sched.h>
+
+#include <algorithm>
+#include <cstring>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
+#include <vector>
 
 #include "cuhnsw_amd.h"
 
@@ -91,7 +98,33 @@ class CuHNSWBind {
   cuhnsw_engine* obj_ = nullptr;
 };
 
+// dst[:] = src[:] for two C-contiguous arrays of the same number of bytes, on several threads: a copy into fresh memory
+// is bound by the page faults of the thread that makes it (236 MB: 45 ms on one thread, 8 ms on eight).
+static void CopyBytes(py::array dst, py::array src) {
+  if (!(dst.flags() & py::array::c_style) || !(src.flags() & py::array::c_style) || dst.nbytes() != src.nbytes())
+    throw std::runtime_error("copy_bytes: two contiguous arrays of one size are wanted");
+  char* to = static_cast<char*>(dst.mutable_data());
+  const char* from = static_cast<const char*>(src.data());
+  const size_t total = (size_t)src.nbytes(), step = ((total + 7) / 8 + 4095) & ~(size_t)4095;
+  py::gil_scoped_release release;
+  cpu_set_t set;
+  CPU_ZERO(&set);
+  const bool several = sched_getaffinity(0, sizeof(set), &set) == 0 && CPU_COUNT(&set) > 1;
+  std::vector<std::thread> threads;
+  size_t at = 0;
+  for (; several && at + step < total; at += step) {
+    try {
+      threads.emplace_back([=] { std::memcpy(to + at, from + at, step); });
+    } catch (const std::system_error&) {
+      break;  // no more threads to be had
+    }
+  }
+  std::memcpy(to + at, from + at, total - at);
+  for (std::thread& t : threads) t.join();
+}
+
 PYBIND11_MODULE(cuhnsw_bind, m) {
+  m.def("copy_bytes", &CopyBytes, py::arg("dst"), py::arg("src"));
   m.def("has_device", []() { return cuhnsw_has_device() != 0; });
   py::class_<CuHNSWBind>(m, "CuHNSWBind")
       .def(py::init())

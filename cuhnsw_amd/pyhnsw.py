@@ -29,7 +29,7 @@ import numpy as np
 from cuhnsw_amd import aux, datasets
 
 try:
-  from cuhnsw_amd.cuhnsw_bind import CuHNSWBind
+  from cuhnsw_amd.cuhnsw_bind import CuHNSWBind, copy_bytes
 except ImportError as exc:  # pragma: no cover
   raise ImportError(
       "cuhnsw_amd: the native extension is missing (%s); build it with "
@@ -64,6 +64,15 @@ def _option_file(opt):
     os.remove(path)
 
 
+def _copy_of(data):
+  """data.copy(), on several threads where that pays."""
+  if type(data) is not np.ndarray or data.nbytes < 8 << 20 or not data.flags.c_contiguous or data.dtype.hasobject:
+    return data.copy()
+  rows = np.empty(data.shape, data.dtype)
+  copy_bytes(rows, data)
+  return rows
+
+
 class CuHNSW:
   """HNSW index built and searched on the GPU."""
 
@@ -78,7 +87,7 @@ class CuHNSW:
 
   # -- data ------------------------------------------------------------------------------------
   def set_data(self, data):
-    rows = data.copy()
+    rows = _copy_of(data)
     if self.opt.nrz:
       if self.opt.dist_type == "l2":
         self.logger.warning("it is not common to set nrz = True and dist_type = l2")
