@@ -21,18 +21,12 @@
 #include <string>
 #include <vector>
 
+#include "host_staging.h"
 #include "index_file.h"
 #include "kernels.h"
 #include "options.h"
 
 namespace cuhnsw_amd {
-
-#define HIP_CHECK(expr)                                                                              \
-  do {                                                                                               \
-    hipError_t err_ = (expr);                                                                        \
-    if (err_ != hipSuccess)                                                                          \
-      throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(err_) + " at " #expr); \
-  } while (0)
 
 inline bool device_present() {
   int n = 0;
@@ -115,7 +109,6 @@ class Engine {
   int dist_type = DIST_DOT;
   HostIndex host;
   bool have_data = false, have_levels = false, have_graph = false;
-  bool host_links_stale = false;  // device links are newer than host.links0 / linksU
   bool has_device = false;
   int num_cus = 0;
   hipStream_t stream = nullptr;
@@ -193,6 +186,8 @@ class Engine {
   // staging for the host-pointer search entry point
   DevBuf<float> d_q, d_dist;
   DevBuf<int> d_nns, d_found;
+  HostStaging staging;
+  static constexpr size_t kPiece = (size_t)512 << 20;  // device memory an index file is packed in, piece by piece
   StaticScratch* static_scratch = nullptr;  // this device's copy (device address)
   int device_ordinal = 0;
   int* h_ctl = nullptr;                     // pinned: control words read back without staging
@@ -267,41 +262,39 @@ class Engine {
     return rc;
   }
 
-  // vectors go up as one contiguous copy (a pitched copy from pageable memory crawls row by
-  // row); rows that need padding are spread out by a small kernel on the device
-  // With fp16 storage the host copy is rounded to the stored values first: everything downstream
-  // (the saved file, a CPU search of that file) then sees exactly the vectors the kernels see.
-  void upload_vectors() {
+  // Between host memory and device memory everything large goes through the pinned blocks of `staging`
+  // (host_staging.h), filled and emptied by several threads while the copy engine runs.  Vectors, links and labels live
+  // in device memory only; an index file is packed and unpacked there.
+  void reserve_vectors() {
     Dp = padded_dims(host.D, tight_rows);
-    const size_t n = (size_t)host.N;
-    if (storage_half) {
-      for (float& x : host.vectors) x = (float)(_Float16)x;
-      d_vectors.reserve((n * Dp + 1) / 2);
-      DevBuf<float> raw;
-      raw.reserve(n * host.D);
-      HIP_CHECK(hipMemcpyAsync(raw.p, host.vectors.data(), n * host.D * sizeof(float), hipMemcpyHostToDevice, stream));
-      HIP_CHECK(hipMemsetAsync(d_vectors.p, 0, n * Dp * sizeof(_Float16), stream));
-      const long long work = (long long)n * host.D;
-      hipLaunchKernelGGL(pad_rows_half_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, raw.p,
-                         reinterpret_cast<_Float16*>(d_vectors.p), (long long)n, host.D, Dp);
-      HIP_CHECK(hipGetLastError());
-      HIP_CHECK(hipStreamSynchronize(stream));
-      return;
-    }
-    d_vectors.reserve(n * Dp);
-    if (Dp == host.D) {
-      HIP_CHECK(hipMemcpyAsync(d_vectors.p, host.vectors.data(), n * Dp * sizeof(float), hipMemcpyHostToDevice, stream));
-      HIP_CHECK(hipStreamSynchronize(stream));
-      return;
-    }
-    DevBuf<float> raw;
-    raw.reserve(n * host.D);
-    HIP_CHECK(hipMemcpyAsync(raw.p, host.vectors.data(), n * host.D * sizeof(float), hipMemcpyHostToDevice, stream));
-    HIP_CHECK(hipMemsetAsync(d_vectors.p, 0, n * Dp * sizeof(float), stream));
-    const long long work = (long long)n * host.D;
-    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, raw.p, d_vectors.p,
-                       (long long)n, host.D, Dp);
-    HIP_CHECK(hipGetLastError());
+    const size_t n = (size_t)host.N * Dp;
+    d_vectors.reserve(storage_half ? (n + 1) / 2 : n);
+  }
+  // (with fp16 storage the rows are rounded to nearest even on their way into the index: everything downstream,
+  // the saved file and a CPU search of that file, then sees exactly the vectors the kernels see)
+  void upload_vectors(const float* rows) {
+    reserve_vectors();
+    const size_t row_bytes = (size_t)host.D * sizeof(float), total = (size_t)host.N * row_bytes;
+    const bool plain = Dp == host.D && !storage_half;
+    staging.reserve(row_bytes, !plain);
+    const size_t block = staging.block() / row_bytes * row_bytes;  // whole rows
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(rows);
+    unsigned char* dst = reinterpret_cast<unsigned char*>(d_vectors.p);
+    staging.send(stream, total, block, [&](unsigned char* to, size_t at, size_t n) { std::memcpy(to, src + at, n); },
+                 [&](size_t at, size_t) { return plain ? dst + at : nullptr; },
+                 [&](unsigned char* there, size_t at, size_t n) {
+                   if (plain) return;
+                   const long long first = (long long)(at / row_bytes), count = (long long)(n / row_bytes);
+                   const dim3 grid((unsigned)((count * (Dp / 4) + 255) / 256));
+                   const float* from = reinterpret_cast<const float*>(there);
+                   if (storage_half)
+                     hipLaunchKernelGGL(pad_rows_kernel<_Float16>, grid, dim3(256), 0, stream, from,
+                                        reinterpret_cast<_Float16*>(d_vectors.p) + first * Dp, count, host.D, Dp);
+                   else
+                     hipLaunchKernelGGL(pad_rows_kernel<float>, grid, dim3(256), 0, stream, from, d_vectors.p + first * Dp,
+                                        count, host.D, Dp);
+                   HIP_CHECK(hipGetLastError());
+                 });
     HIP_CHECK(hipStreamSynchronize(stream));
   }
 
@@ -310,12 +303,12 @@ class Engine {
     host = HostIndex();
     host.N = n;
     host.D = d;
-    host.vectors.assign(data, data + (size_t)n * d);
-    have_levels = have_graph = host_links_stale = false;
+    have_levels = have_graph = false;
     forget_search_history();
     pool_slots = 0;  // the slot pool is sized by N: rebuild it lazily
     pool = SlotPool{};
-    if (has_device) upload_vectors();  // without a GPU only the host-side calls remain usable
+    if (has_device) upload_vectors(data);
+    else host.vectors.assign(data, data + (size_t)n * d);  // without a GPU only the host-side calls remain usable
     have_data = true;
   }
 
@@ -328,20 +321,6 @@ class Engine {
     HIP_CHECK(hipMemcpyAsync(d_upper_off.p, host.upper_off.data(), (size_t)host.N * 8, hipMemcpyHostToDevice, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
   }
-  void upload_links() {
-    HIP_CHECK(hipMemcpyAsync(d_links0.p, host.links0.data(), host.links0.size() * 4, hipMemcpyHostToDevice, stream));
-    if (!host.linksU.empty())
-      HIP_CHECK(hipMemcpyAsync(d_linksU.p, host.linksU.data(), host.linksU.size() * 4, hipMemcpyHostToDevice, stream));
-    HIP_CHECK(hipStreamSynchronize(stream));
-  }
-  void download_links() {
-    HIP_CHECK(hipMemcpyAsync(host.links0.data(), d_links0.p, host.links0.size() * 4, hipMemcpyDeviceToHost, stream));
-    if (!host.linksU.empty())
-      HIP_CHECK(hipMemcpyAsync(host.linksU.data(), d_linksU.p, host.linksU.size() * 4, hipMemcpyDeviceToHost, stream));
-    HIP_CHECK(hipStreamSynchronize(stream));
-    host_links_stale = false;
-  }
-
   void set_random_levels(const int* levels, int n) {
     if (!have_data) throw std::runtime_error("set_random_levels: call set_data first");
     if (n != host.N) throw std::runtime_error("set_random_levels: length differs from the number of data rows");
@@ -351,7 +330,8 @@ class Engine {
     host.ef_construction = opt.ef_construction;
     host.mult = opt.level_mult;
     host.set_levels(levels, n);
-    host.layout_links();
+    if (has_device) host.layout_upper();
+    else host.layout_links();
     host.labelled = false;
     host.labels.clear();
     host.deleted.clear();  // a graph built anew holds every element
@@ -590,7 +570,6 @@ class Engine {
     have_graph = true;
     forget_search_history();
     prepare_search_buffers();
-    host_links_stale = true;
   }
 
   // ---- measurement aid --------------------------------------------------------------------------------
@@ -622,38 +601,109 @@ class Engine {
   }
 
   // ---- index file --------------------------------------------------------------------------------
+  // The level-0 block leaves device memory as the file's own bytes: packed by pack_records_kernel, piece by piece,
+  // copied into the pinned blocks and from there into the file by the threads that wait for them.
   void save_index(const char* path) {
     if (!have_graph) throw std::runtime_error("save_index: no index to save");
-    if (host_links_stale) download_links();
-    write_index_file(host, path);
+    if (!has_device) {
+      write_index_file(host, path);
+      return;
+    }
+    IndexWriter out(host, path);
+    const size_t rec = (size_t)out.layout.record;
+    const size_t piece_rows = std::max<size_t>(1, std::min<size_t>((size_t)host.N, kPiece / rec));
+    DevBuf<unsigned char> packed;
+    packed.reserve(piece_rows * rec);
+    staging.reserve(0, false);
+    if (host.n_deleted > 0) upload_marks();
+    std::vector<uint32_t> up((size_t)host.upper_rows * host.SU);
+    if (!up.empty()) HIP_CHECK(hipMemcpyAsync(up.data(), d_linksU.p, up.size() * 4, hipMemcpyDeviceToHost, stream));
+    const DevIndex ix = dev_index();
+    for (size_t first = 0; first < (size_t)host.N; first += piece_rows) {
+      const size_t rows = std::min(piece_rows, (size_t)host.N - first);
+      hipLaunchKernelGGL(pack_records_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, ix, (int)first, (int)rows,
+                         host.n_deleted > 0 ? d_deleted.p : nullptr, reinterpret_cast<uint32_t*>(packed.p));
+      HIP_CHECK(hipGetLastError());
+      const uint64_t file_at = FileLayout::kHeader + (uint64_t)first * rec;
+      staging.fetch(stream, packed.p, rows * rec, out.parallel(),
+                    [&](const unsigned char* from, size_t at, size_t n) { out.write(file_at + at, from, n); });
+    }
+    HIP_CHECK(hipStreamSynchronize(stream));
+    out.write_upper(host, up.data());
+    out.finish();
   }
+  void upload_marks() {
+    std::vector<uint32_t> marks(((size_t)host.N + 31) / 32, 0u);
+    for (int i = 0; i < host.N; ++i)
+      if (host.deleted[i]) marks[(size_t)i >> 5] |= 1u << (i & 31);
+    d_deleted.reserve(marks.size());
+    HIP_CHECK(hipMemcpyAsync(d_deleted.p, marks.data(), marks.size() * 4, hipMemcpyHostToDevice, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  // The way back: the level-0 block goes up as it stands in the file and is checked there; only once the whole file
+  // has been found good do its records take the place of the index that was resident before.
   void load_index(const char* path) {
     HostIndex fresh;
-    read_index_file(fresh, path);
-    if (fresh.N <= 0) throw std::runtime_error("load_index: empty index");
+    if (!has_device) {
+      read_index_file(fresh, path);
+      if (fresh.N <= 0) throw std::runtime_error("load_index: empty index");
+      host = std::move(fresh);
+      have_data = have_levels = have_graph = true;
+      forget_search_history();
+      return;
+    }
+    IndexReader in(fresh, path);
+    const size_t rec = (size_t)in.layout.record, n = (size_t)fresh.N;
+    DevBuf<unsigned char> raw, marks;
+    raw.reserve(std::max<size_t>(n * rec, 1));
+    marks.reserve(std::max<size_t>(n, 1));
+    staging.reserve(0, false);
+    std::string upper_error;
+    HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 2 * sizeof(int), stream));
+    staging.send(stream, n * rec, staging.block(),
+                 [&](unsigned char* to, size_t at, size_t len) { in.read(FileLayout::kHeader + at, to, len, "level-0 block"); },
+                 [&](size_t at, size_t) { return raw.p + at; }, [](unsigned char*, size_t, size_t) {},
+                 [&] {  // (on this thread, beside the others)
+                   try {
+                     in.read_upper(fresh);
+                   } catch (const std::exception& ex) {
+                     upper_error = ex.what();
+                   }
+                 });
+    if (n > 0) {
+      hipLaunchKernelGGL(check_records_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
+                         reinterpret_cast<const uint32_t*>(raw.p), (int)n, fresh.D, fresh.max_m0, marks.p, d_ctl.p);
+      HIP_CHECK(hipGetLastError());
+    }
+    HIP_CHECK(hipMemcpyAsync(h_ctl, d_ctl.p, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
+    if (h_ctl[0] & 1) throw std::runtime_error("index file: link count above max_m0");
+    if (h_ctl[0] & 2) throw std::runtime_error("index file: link id out of range");
+    if (!upper_error.empty()) throw std::runtime_error(upper_error);
+    if (n == 0) throw std::runtime_error("load_index: empty index");
+    fresh.n_deleted = h_ctl[1];
+    if (fresh.n_deleted > 0) {
+      fresh.deleted.resize(n);
+      HIP_CHECK(hipMemcpyAsync(fresh.deleted.data(), marks.p, n, hipMemcpyDeviceToHost, stream));
+      HIP_CHECK(hipStreamSynchronize(stream));
+    }
     host = std::move(fresh);
     have_data = have_levels = have_graph = true;
     forget_search_history();
-    host_links_stale = false;
-    if (has_device) {
-      upload_vectors();
-      upload_structure();
-      upload_links();
-      d_labels.reserve((size_t)host.N);
-      HIP_CHECK(hipMemcpyAsync(d_labels.p, host.labels.data(), (size_t)host.N * 8, hipMemcpyHostToDevice, stream));
-      std::vector<uint32_t> marks;
-      if (host.n_deleted > 0) {
-        marks.assign(((size_t)host.N + 31) / 32, 0u);
-        for (int i = 0; i < host.N; ++i)
-          if (host.deleted[i]) marks[(size_t)i >> 5] |= 1u << (i & 31);
-        d_deleted.reserve(marks.size());
-        HIP_CHECK(hipMemcpyAsync(d_deleted.p, marks.data(), marks.size() * 4, hipMemcpyHostToDevice, stream));
-      }
-      HIP_CHECK(hipStreamSynchronize(stream));
-      pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
-      pool = SlotPool{};
-      prepare_search_buffers();
-    }
+    reserve_vectors();
+    upload_structure();
+    d_labels.reserve(n);
+    hipLaunchKernelGGL(unpack_records_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
+                       reinterpret_cast<const uint32_t*>(raw.p), dev_index(), d_labels.p);
+    HIP_CHECK(hipGetLastError());
+    if (!host.linksU.empty())
+      HIP_CHECK(hipMemcpyAsync(d_linksU.p, host.linksU.data(), host.linksU.size() * 4, hipMemcpyHostToDevice, stream));
+    if (host.n_deleted > 0) upload_marks();
+    HIP_CHECK(hipStreamSynchronize(stream));
+    std::vector<uint32_t>().swap(host.linksU);
+    pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
+    pool = SlotPool{};
+    prepare_search_buffers();
   }
 };
 

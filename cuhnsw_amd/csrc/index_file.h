@@ -36,14 +36,74 @@ struct HostIndex {
 
   static int stride0(int max_m0) { return (max_m0 + 31) / 32 * 32; }
   static int strideU(int max_m) { return (max_m + 15) / 16 * 16; }
-  // sizes strides, offsets and empty link tables from N, levels, max_m, max_m0
+  // strides, offsets and number of upper rows from N, levels, max_m, max_m0
+  void layout_upper();
+  // the same, and empty link tables on the host (an engine with a GPU keeps its links there)
   void layout_links();
   // max level and entry point from levels: the first node that reaches the
   // maximal level (cpp/src/cuhnsw_base.cu:133-141; node 0 if every level is 0)
   void set_levels(const int* lv, int n);
 };
 
-// Both throw std::runtime_error with a message on I/O or format errors.
+constexpr uint32_t kDeleteMark = 0x00010000u;  // hnswlib's DELETE_MARK as a bit of the level-0 count word
+
+// Where things sit in an index file: a header, N level-0 records, the upper block.
+struct FileLayout {
+  static constexpr uint64_t kHeader = 96;
+  uint64_t links0_bytes = 0;  // bytes of a record's link part = offset of its vector
+  uint64_t linksU_bytes = 0;  // bytes of one upper-level link list
+  uint64_t label_offset = 0;  // offset of a record's label
+  uint64_t record = 0;        // bytes of a record
+  FileLayout() {}
+  FileLayout(uint64_t max_m, uint64_t max_m0, uint64_t D)
+      : links0_bytes(max_m0 * 4 + 4), linksU_bytes(max_m * 4 + 4), label_offset(links0_bytes + D * 4), record(label_offset + 8) {}
+};
+
+// An index file opened for reading.  The constructor checks the header; read() is safe to call from several
+// threads and throws "index file: truncated <what>" where the file ends early.
+class IndexReader {
+ public:
+  IndexReader(HostIndex& ix, const std::string& path);  // fills the header's fields of ix
+  ~IndexReader();
+  IndexReader(const IndexReader&) = delete;
+  IndexReader& operator=(const IndexReader&) = delete;
+  void read(uint64_t offset, void* dst, size_t n, const char* what) const;
+  // levels, offsets and upper links (on the host) of ix from the block behind the records; links are checked
+  void read_upper(HostIndex& ix) const;
+  FileLayout layout;
+
+ private:
+  int fd_ = -1;
+  std::vector<unsigned char> memory_;  // the whole file where it cannot be read by position (a pipe)
+  bool in_memory_ = false;
+  uint64_t size_ = 0;
+  uint64_t upper_at_ = 0;
+};
+
+// An index file opened for writing; its size is known from the start.  write() may be called from several threads
+// where parallel() says so, else in ascending order without gaps.  finish() makes the file as long as it has to be.
+class IndexWriter {
+ public:
+  IndexWriter(const HostIndex& ix, const std::string& path);  // writes the header
+  ~IndexWriter();
+  IndexWriter(const IndexWriter&) = delete;
+  IndexWriter& operator=(const IndexWriter&) = delete;
+  bool parallel() const { return regular_; }
+  void write(uint64_t offset, const void* src, size_t n);
+  // the upper block from ix.levels / upper_off and the link rows given (upper_rows x SU)
+  void write_upper(const HostIndex& ix, const uint32_t* linksU);
+  void finish();
+  FileLayout layout;
+
+ private:
+  int fd_ = -1;
+  bool regular_ = false;
+  unsigned char* map_ = nullptr;
+  uint64_t size_ = 0, upper_at_ = 0;
+};
+
+// Both throw std::runtime_error with a message on I/O or format errors.  (Host tables only: an engine with a GPU
+// moves records between the file and device memory itself, engine.h.)
 void write_index_file(const HostIndex& ix, const std::string& path);
 void read_index_file(HostIndex& ix, const std::string& path);
 

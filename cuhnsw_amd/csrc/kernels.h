@@ -1390,22 +1390,86 @@ __global__ void __launch_bounds__(64) gather_probe_kernel(DevIndex ix, int batch
   if (acc == 7654321.0f) sink[blockIdx.x] = acc;
 }
 
-// Upload helper for fp16 storage: N x D floats into rows of Dp halves (the padding was zeroed before).
-static __global__ void __launch_bounds__(256) pad_rows_half_kernel(const float* src, _Float16* dst, long long n, int D, int Dp) {
+// Upload helper: N rows of D floats into rows of Dp elements, zero padded; a thread writes four of them.  (fp16: to
+// nearest even.)
+template <typename T>
+__global__ void __launch_bounds__(256) pad_rows_kernel(const float* src, T* dst, long long n, int D, int Dp) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * D) return;
-  const long long row = i / D;
-  const int col = (int)(i - row * D);
-  dst[row * Dp + col] = (_Float16)src[i];  // round to nearest even; the host rounds its copy the same way
+  const int chunks = Dp >> 2;
+  if (i >= n * chunks) return;
+  const long long row = i / chunks;
+  const int col = 4 * (int)(i - row * chunks);
+  const float* from = src + row * D + col;
+  struct __attribute__((aligned(4 * sizeof(T)))) Four { T v[4]; } out;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) out.v[j] = col + j < D ? (T)from[j] : (T)0.f;
+  *reinterpret_cast<Four*>(dst + row * Dp + col) = out;
 }
 
-// Upload helper: copies N x D floats into rows of Dp floats (the padding was zeroed before).
-static __global__ void __launch_bounds__(256) pad_rows_kernel(const float* src, float* dst, long long n, int D, int Dp) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * D) return;
-  const long long row = i / D;
-  const int col = (int)(i - row * D);
-  dst[row * Dp + col] = src[i];
+// ---- level-0 records of an index file: [count | max_m0 ids | D floats | label], 32-bit words ------------------------
+// One wavefront per record, four per workgroup: a record is read and written in whole lines whatever its length.
+static __global__ void __launch_bounds__(256) pack_records_kernel(DevIndex ix, int first, int rows, const uint32_t* deleted,
+                                                                  uint32_t* out) {
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const int i = first + r;
+  uint32_t* rec = out + (size_t)r * (size_t)(1 + ix.max_m0 + ix.D + 2);
+  const uint32_t* row = ix.links0 + (size_t)i * ix.S0;
+  uint32_t deg = 0;
+  for (int base = 0; base < ix.max_m0; base += 64) {
+    const int k = base + lane;
+    const uint32_t id = k < ix.max_m0 ? row[k] : kEmpty;
+    deg += (uint32_t)__popcll(__ballot(id != kEmpty));
+    if (k < ix.max_m0) rec[1 + k] = id != kEmpty ? id : 0u;  // unused link slots are zeros in the file
+  }
+  float* vec = reinterpret_cast<float*>(rec + 1 + ix.max_m0);
+  const size_t at = (size_t)i * ix.Dp;
+  for (int k = lane; k < ix.D; k += 64)
+    vec[k] = ix.half ? (float)reinterpret_cast<const _Float16*>(ix.vectors)[at + k] : reinterpret_cast<const float*>(ix.vectors)[at + k];
+  if (lane == 0) {
+    const uint64_t label = ix.labels ? ix.labels[i] : (uint64_t)i;
+    const bool marked = deleted && ((deleted[i >> 5] >> (i & 31)) & 1u) != 0u;
+    rec[0] = deg | (marked ? kDeleteMark : 0u);
+    rec[1 + ix.max_m0 + ix.D] = (uint32_t)label;
+    rec[2 + ix.max_m0 + ix.D] = (uint32_t)(label >> 32);
+  }
+}
+// status[0]: 1 = a link count above max_m0, 2 = a link id out of range; status[1] counts the delete marks (marks: one
+// byte per record).  hnswlib keeps the count in the low 16 bits of its word and flags above: markDelete sets bit 0 of
+// the third byte, the others are unknown and dropped.
+static __global__ void __launch_bounds__(256) check_records_kernel(const uint32_t* raw, int n, int D, int max_m0,
+                                                                   unsigned char* marks, int* status) {
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= n) return;
+  const uint32_t* rec = raw + (size_t)i * (size_t)(1 + max_m0 + D + 2);
+  const uint32_t word = rec[0];
+  const uint32_t deg = word & 0xffffu;
+  int wrong = deg > (uint32_t)max_m0 ? 1 : 0;
+  for (int k = lane; k < max_m0; k += 64) wrong |= ((uint32_t)k < deg && rec[1 + k] >= (uint32_t)n) ? 2 : 0;
+  if (wrong) atomicOr(status, wrong);
+  if (lane == 0) {
+    const bool marked = (word & kDeleteMark) != 0u;
+    marks[i] = marked ? 1 : 0;
+    if (marked) atomicAdd(status + 1, 1);
+  }
+}
+static __global__ void __launch_bounds__(256) unpack_records_kernel(const uint32_t* raw, DevIndex ix, uint64_t* labels) {
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= ix.N) return;
+  const uint32_t* rec = raw + (size_t)i * (size_t)(1 + ix.max_m0 + ix.D + 2);
+  const int deg = (int)(rec[0] & 0xffffu);
+  for (int k = lane; k < ix.S0; k += 64) ix.links0[(size_t)i * ix.S0 + k] = k < deg ? rec[1 + k] : kEmpty;
+  const float* vec = reinterpret_cast<const float*>(rec + 1 + ix.max_m0);
+  const size_t at = (size_t)i * ix.Dp;
+  for (int k = lane; k < ix.Dp; k += 64) {
+    const float x = k < ix.D ? vec[k] : 0.f;
+    if (ix.half) const_cast<_Float16*>(reinterpret_cast<const _Float16*>(ix.vectors))[at + k] = (_Float16)x;
+    else const_cast<float*>(reinterpret_cast<const float*>(ix.vectors))[at + k] = x;
+  }
+  if (lane == 0) labels[i] = (uint64_t)rec[1 + ix.max_m0 + ix.D] | ((uint64_t)rec[2 + ix.max_m0 + ix.D] << 32);
 }
 
 }  // namespace cuhnsw_amd
