@@ -456,7 +456,7 @@ def main():
       "bound": "hbm", "achieved": build_bytes / build_s / 1e9, "peak": 8000.0, "unit": "GB/s",
       "frac": build_bytes / build_s / 1e9 / 8000.0, "algorithmic_bytes": int(build_bytes),
       "counters": {"names": ["distance evaluations (searches, descents)", "link rows read", "heuristic pair tests",
-                             "heuristic candidate rows", "link rows written"], "level0": lv0, "upper_levels": up},
+                             "heuristic pick rows", "link rows written"], "level0": lv0, "upper_levels": up},
       "note": "vector rows x %d B + link rows x %d B (level 0) / %d B (upper levels), over build_seconds" % (row_bytes, s0, su),
   }
 

@@ -163,7 +163,7 @@ class Engine:
 
   def build_counters(self):
     """Work of the last build counted on the device (needs tunable build_counters): dict of two lists
-    [evaluations, link rows read, heuristic pair tests, heuristic candidate rows, link rows written]."""
+    [evaluations, link rows read, heuristic pair tests, heuristic pick rows, link rows written]."""
     out = np.zeros(10, dtype=np.uint64)
     if self._l.cuhnsw_last_build_counters(self._h, out.ctypes.data, 10) != 0:
       raise RuntimeError("cuhnsw_last_build_counters failed")

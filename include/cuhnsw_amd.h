@@ -147,7 +147,7 @@ int cuhnsw_debug_gather_probe(cuhnsw_engine* e, int waves_per_cu, int rows_in_fl
 /* Work of the last cuhnsw_build_graph, counted on the device when tunable "build_counters" = 1 was set before it
  * (all zero otherwise); the reference counts its visited nodes per level the same way
  * (cpp/src/cuhnsw_build.cu:191-195).  out[0..4] level 0, out[5..9] upper levels: distance evaluations of the
- * searches and descents, link rows read, pair tests of the selection heuristic, candidates the heuristic loaded
+ * searches and descents, link rows read, pair tests of the selection heuristic, picks the heuristic loaded
  * to test them, link rows written.  n must be at least 10. */
 int cuhnsw_last_build_counters(cuhnsw_engine* e, unsigned long long* out, int n);
 /* Debugging aid: the key (ordering distance) the build stored with every level-0 link, row-major
