@@ -166,7 +166,7 @@ __host__ __device__ inline LdsPlan plan_lds(int qr, int Dp, int ef, int cand_lds
   p.sorted_key = o; o = align16(o + (size_t)n_sorted * 4);
   p.out_id = o; o = align16(o + (size_t)n_out * 4);
   p.out_key = o; o = align16(o + (size_t)n_out * 4);
-  p.nbuf = o; o = align16(o + (size_t)lcap * 4);
+  p.nbuf = o; o = align16(o + (size_t)nbuf_words(lcap) * 4);
   p.dbuf = o; o = align16(o + (size_t)lcap * 4);
   p.lfilter = o; o = align16(o + (lf_bits > 0 ? ((size_t)4 << lf_bits) : 0));
   p.total = o;
@@ -194,7 +194,7 @@ __host__ __device__ inline FastLdsPlan plan_fast_lds(int qr, int Dp, int lcap, i
   p.qlds = o;
   if (qr == 0) o += (size_t)query_lds_chunks(Dp) * 16;
   p.fcache = o; o = align16(o + ((size_t)4 << fc_bits));
-  p.nbuf = o; o = align16(o + (size_t)lcap * 4);
+  p.nbuf = o; o = align16(o + (size_t)nbuf_words(lcap) * 4);
   p.dbuf = o; o = align16(o + (size_t)lcap * 4);
   p.total = o;
   return p;
@@ -383,6 +383,24 @@ static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4*
   if (qi < nq) order[cnt[bucket] + rank] = qi;
 }
 
+// A kernel's arguments read afresh from where the launch put them.  The compiler loads every argument once, when the
+// kernel starts, and keeps it: fifty scalar registers for what is needed once per query, and what does not fit is parked
+// in lanes of vector registers.  Through a pointer it cannot see through the fields are loaded where they are used.
+// (Kernels here take a DevIndex, then their own arguments.)
+template <typename T>
+__device__ __forceinline__ const T& fresh_kernel_args(size_t offset) {
+  typedef const __attribute__((address_space(4))) char* kernarg_t;
+  kernarg_t p = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const T*)(const __attribute__((address_space(4))) T*)(p + offset);
+}
+__device__ __forceinline__ const DevIndex& fresh_index() { return fresh_kernel_args<DevIndex>(0); }
+template <typename Args>
+__device__ __forceinline__ const Args& fresh_args() {
+  static_assert(alignof(Args) == 8 && alignof(DevIndex) == 8, "second argument right after the first");
+  return fresh_kernel_args<Args>((sizeof(DevIndex) + 7) / 8 * 8);
+}
+
 // First pass of a search batch: every query on the sorted set in registers (ef < 64*NS).
 // A query in which two equal keys meet is not answered here: its index is appended to
 // a.redo (a.repeats counts them) and the literal search_kernel answers it afterwards.
@@ -394,60 +412,64 @@ static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4*
 // this instance for batches of a round or two of wavefronts, where a query handed over late is a good part of the
 // batch's time, and the instance without the trail code otherwise).
 template <int DT, int QR, int NS, bool TRAILS>
-__global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS == 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix, SearchArgs a) {
+__global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS == 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x;
-  const FastLdsPlan lp = plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits);
+  const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
   Scratch s;
   s.vcache = reinterpret_cast<uint16_t*>(smem + lp.fcache);
-  s.vc_bits = a.fc_bits;
+  s.vc_bits = a0.fc_bits;
   s.qlds = reinterpret_cast<float4*>(smem + lp.qlds);
   s.nbuf = reinterpret_cast<uint32_t*>(smem + lp.nbuf);
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
   // tells a literal pass waiting beside this one that the two kernels do run at the same time
-  if (blockIdx.x == 0 && lane == 0) __hip_atomic_store(a.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  int trail_buf = (TRAILS && a.trail) ? (int)blockIdx.x : -1;  // the buffer this wavefront's trails go to
+  if (blockIdx.x == 0 && lane == 0) __hip_atomic_store(a0.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int trail_buf = (TRAILS && a0.trail) ? (int)blockIdx.x : -1;  // the buffer this wavefront's trails go to
 
   for (;;) {
+    const SearchArgs& in = fresh_args<SearchArgs>();
+    const DevIndex& from = fresh_index();
     int qi = 0;
     if (lane == 0) {
-      qi = atomicAdd(a.counter, 1);
-      if (qi < a.nq && a.order) qi = a.order[qi];
+      qi = atomicAdd(in.counter, 1);
+      if (qi < in.nq && in.order) qi = in.order[qi];
     }
     qi = __builtin_amdgcn_readfirstlane(qi);
-    if (qi >= a.nq) break;
+    if (qi >= in.nq) break;
     Trail tr;
     if (TRAILS && trail_buf >= 0) {
-      tr.rec = a.trail + (size_t)trail_buf * a.trail_cap;
-      tr.cap = a.trail_cap;
+      tr.rec = in.trail + (size_t)trail_buf * in.trail_cap;
+      tr.cap = in.trail_cap;
       tr.on = true;
     }
     QVec<QR> qv;
-    load_query<QR>(qv, s.qlds, a.q + (size_t)qi * ix.D, ix.D, ix.Dp, lane);
+    load_query<QR>(qv, s.qlds, in.q + (size_t)qi * from.D, from.D, from.Dp, lane);
     SearchState st;
     st.top_size = 0; st.cand_size = 0; st.n_acc = 0; st.lower = 0.f; st.maxkey = -INFINITY; st.undo_cnt = 0;
-    st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0;
+    st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0; st.ahead = 1;
 
-    uint32_t cur = ix.enterpoint;
-    if (a.entry) {  // the descent through the upper levels has been done for the whole batch
-      const uint4 en = a.entry[qi];
+    uint32_t cur = from.enterpoint;
+    if (in.entry) {  // the descent through the upper levels has been done for the whole batch
+      const uint4 en = in.entry[qi];
       cur = (uint32_t)__builtin_amdgcn_readfirstlane((int)en.x);
       st.n_dist_upper = __builtin_amdgcn_readfirstlane((int)en.z);
       st.n_sweeps = __builtin_amdgcn_readfirstlane((int)en.w);
     } else {
-      float dcur = dist_single<DT, QR>(ix, qv, cur, s, lane);
-      descend<DT, QR>(ix, qv, ix.maxlevel, 0, cur, dcur, s, st, lane);
+      float dcur = dist_single<DT, QR>(from, qv, cur, s, lane);
+      descend<DT, QR>(from, qv, from.maxlevel, 0, cur, dcur, s, st, lane);
     }
 
     Frontier<NS> fr;
-    frontier_init<NS>(fr, a.ef, lane);
+    frontier_init<NS>(fr, a0.ef, lane);
     filter_reset(s, lane);
     visit_lossy_single(s, cur, lane);
     if (lane == 0) s.nbuf[0] = cur;
     wave_sync();
     // (the flag is made wavefront-uniform explicitly and both outcomes are plain branches)
     const int how =
-        __builtin_amdgcn_readfirstlane(search_level_fast<DT, QR, NS, false, TRAILS>(ix, qv, 0, a.ef, s, st, fr, 1, lane, a.reverse != 0, a.k >= a.ef, TRAILS ? &tr : nullptr));
+        __builtin_amdgcn_readfirstlane(search_level_fast<DT, QR, NS, false, TRAILS>(ix0, qv, 0, a0.ef, s, st, fr, 1, lane, a0.reverse != 0, a0.k >= a0.ef, TRAILS ? &tr : nullptr));
+    const SearchArgs& a = fresh_args<SearchArgs>();
+    const DevIndex& ix = fresh_index();
     const int T0 = st.top_size < a.k ? st.top_size : a.k;
     // Equal keys across the cut at k: which of them stays is up to the result heap, which the
     // literal search reproduces.  Equal keys among the k best: the answer lists them by label.
@@ -634,7 +656,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
     load_query<QR>(qv, s.qlds, a.q + (size_t)qi * ix.D, ix.D, ix.Dp, lane);
     SearchState st;
     st.top_size = 0; st.cand_size = 0; st.n_acc = 0; st.lower = 0.f; st.maxkey = -INFINITY; st.undo_cnt = 0;
-    st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0;
+    st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0; st.ahead = 1;
     TopKeys<NS> tk;
     topkeys_init<NS>(tk, a.ef, lane);
 
@@ -1015,7 +1037,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
       QVec<QR> qv;
       load_node_query<QR>(qv, s.qlds, ix, x, lane);
       SearchState st;
-      st.undo_cnt = 0; st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0;
+      st.undo_cnt = 0; st.n_dist = 0; st.n_hops = 0; st.n_dist_upper = 0; st.n_sweeps = 0; st.fail = 0; st.ahead = 1;
 
       // hnswlib addPoint: greedy descent from the entry point down to the node's top level,
       // then search + select on every level it has, entering each level at the closest
@@ -1027,7 +1049,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
       }
       for (int level = top_level; level >= 0; --level) {
         const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
-        st.top_size = 0; st.cand_size = 0; st.n_acc = 0; st.lower = 0.f; st.maxkey = -INFINITY;
+        st.top_size = 0; st.cand_size = 0; st.n_acc = 0; st.lower = 0.f; st.maxkey = -INFINITY; st.ahead = 1;
         const int evals_before = st.n_dist, hops_before = st.n_hops;
         int T;
         if (sorted_set) {
