@@ -127,8 +127,9 @@ class Engine {
   int hnswlib_dist = 0;
   int spin_limit_override = -1;  // polls a waiting literal wavefront may spend (-1 = automatic)
   int side_per_cu = 0;         // its wavefronts per CU (0 = from the share of queries the last search gave up)
-  bool share_known = false;               // last_repeat_share comes from a search of this index
-  double last_repeat_share = 0.0;         // its wavefronts per CU
+  bool share_known = false;               // repeat_share comes from searches of this index
+  double repeat_share = 0.0;              // share of the last queries (256 or more, once there are so many) that were given up
+  long long share_queries = 0, share_repeats = 0;  // the batches too small to judge by, taken together
   int concurrent_literal = 1;  // run the literal pass beside the sorted-set pass (0: after it)
   // A literal wavefront whose bounded wait ran out (the two streams did not run side by side: a profiler that
   // serialises kernels, a saturated device) makes the next kSequentialSearches searches run their passes one
@@ -187,6 +188,19 @@ class Engine {
   DevBuf<float> d_q, d_dist;
   DevBuf<int> d_nns, d_found;
   HostStaging staging;
+  // pinned memory that small batches are read from and answered into (kernels address it)
+  static constexpr size_t kDirectQueries = (size_t)64 << 10, kDirectAnswers = (size_t)1 << 20;
+  unsigned char* h_io = nullptr;
+  size_t h_io_bytes = 0;
+  void reserve_io(size_t bytes) {
+    if (bytes <= h_io_bytes) return;
+    bytes = std::max(bytes, (size_t)64 << 10);
+    if (h_io) HIP_CHECK(hipHostFree(h_io));
+    h_io = nullptr;
+    h_io_bytes = 0;
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_io), bytes, hipHostMallocDefault));
+    h_io_bytes = bytes;
+  }
   static constexpr size_t kPiece = (size_t)512 << 20;  // device memory an index file is packed in, piece by piece
   StaticScratch* static_scratch = nullptr;  // this device's copy (device address)
   int device_ordinal = 0;
@@ -223,6 +237,7 @@ class Engine {
     if (stream2) (void)hipStreamDestroy(stream2);
     if (stream) (void)hipStreamDestroy(stream);
     if (h_ctl) (void)hipHostFree(h_ctl);
+    if (h_io) (void)hipHostFree(h_io);
   }
 
   void need_device() const {
@@ -346,11 +361,38 @@ class Engine {
   void forget_search_history() {
     fast_suspended = false;
     share_known = false;
-    last_repeat_share = 0.0;
+    repeat_share = 0.0;
+    share_queries = share_repeats = 0;
     sequential_left = 0;
     literal_fallbacks = 0;
     last_side_by_side = 0;
     last_repeats = last_trails = 0;
+  }
+
+  // An index whose distances tie all the time (integer-valued data) sends most queries through both passes: where more
+  // than a third of 256 or more queries were given up the sorted set is tried no more.  Smaller batches are judged
+  // together (not where the caller asked for the first pass whatever the batch).
+  void learn_share(long long nq, long long given_up) {
+    if (nq < 256 && fast_path == 1) {
+      nq = share_queries += nq;
+      given_up = share_repeats += given_up;
+      if (nq >= 256) share_queries = share_repeats = 0;
+    }
+    repeat_share = (double)given_up / (double)nq;
+    share_known = true;
+    if (nq >= 256 && given_up * 3 > nq) fast_suspended = true;
+  }
+  // control words (as d_ctl) of a search that needs nothing else cleared: cleared kControlBlocks at a time
+  static constexpr int kControlBlocks = 64;
+  DevBuf<int> d_ctl_blocks;
+  int ctl_block = kControlBlocks;
+  int* next_control_block() {
+    if (ctl_block == kControlBlocks) {
+      d_ctl_blocks.reserve((size_t)kControlBlocks * 128);
+      HIP_CHECK(hipMemsetAsync(d_ctl_blocks.p, 0, (size_t)kControlBlocks * 128 * sizeof(int), stream));
+      ctl_block = 0;
+    }
+    return d_ctl_blocks.p + (size_t)128 * ctl_block++;
   }
 
   // Buffers of a search that do not depend on the batch are allocated when the index becomes resident, not
@@ -442,11 +484,22 @@ class Engine {
     return bits;
   }
 
+  // (asked of the runtime once per kernel and LDS size: a search wants to know half a dozen of them)
+  struct Resident {
+    const void* kernel;
+    size_t lds;
+    int slots;
+  };
+  std::vector<Resident> resident_known;
   template <typename K>
-  int resident_slots(K kernel, size_t lds) const {
+  int resident_slots(K kernel, size_t lds) {
+    for (const Resident& r : resident_known)
+      if (r.kernel == reinterpret_cast<const void*>(kernel) && r.lds == lds) return r.slots;
     int per_cu = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, lds));
     per_cu = std::max(1, std::min(per_cu, 32));
+    if (resident_known.size() >= 64) resident_known.clear();
+    resident_known.push_back({reinterpret_cast<const void*>(kernel), lds, per_cu * num_cus});
     return per_cu * num_cus;
   }
 
@@ -528,12 +581,32 @@ class Engine {
     if (nq <= 0) return;
     if (!q || !nns || !dists || !found) throw std::runtime_error("search_knn: null argument");
     if (k <= 0) throw std::runtime_error("search_knn: topk must be positive");
-    d_q.reserve((size_t)nq * host.D);
+    // Small traffic skips the copy engine, of which every copy is 15 to 40 us with what surrounds it: the kernels read
+    // few queries where they lie in pinned memory, and write the answers there (each is written once).
+    const size_t q_bytes = (size_t)nq * host.D * 4, out_bytes = ((size_t)nq * k * 2 + nq) * 4;
+    const bool direct_q = q_bytes <= kDirectQueries, direct_out = out_bytes <= kDirectAnswers;
+    if (direct_q || direct_out) reserve_io((direct_q ? q_bytes : 0) + (direct_out ? out_bytes : 0));
+    int* out = reinterpret_cast<int*>(h_io + (direct_q ? q_bytes : 0));
+    const float* q_there;
+    if (direct_q) {
+      std::memcpy(h_io, q, q_bytes);
+      q_there = reinterpret_cast<const float*>(h_io);
+    } else {
+      d_q.reserve((size_t)nq * host.D);
+      HIP_CHECK(hipMemcpyAsync(d_q.p, q, q_bytes, hipMemcpyHostToDevice, stream));
+      q_there = d_q.p;
+    }
+    if (direct_out) {
+      search_device(q_there, nq, k, ef, out, reinterpret_cast<float*>(out + (size_t)nq * k), out + (size_t)nq * k * 2, nullptr, nullptr);
+      std::memcpy(nns, out, (size_t)nq * k * 4);
+      std::memcpy(dists, out + (size_t)nq * k, (size_t)nq * k * 4);
+      std::memcpy(found, out + (size_t)nq * k * 2, (size_t)nq * 4);
+      return;
+    }
     d_nns.reserve((size_t)nq * k);
     d_dist.reserve((size_t)nq * k);
     d_found.reserve((size_t)nq);
-    HIP_CHECK(hipMemcpyAsync(d_q.p, q, (size_t)nq * host.D * 4, hipMemcpyHostToDevice, stream));
-    search_device(d_q.p, nq, k, ef, d_nns.p, d_dist.p, d_found.p, nullptr, nullptr);
+    search_device(q_there, nq, k, ef, d_nns.p, d_dist.p, d_found.p, nullptr, nullptr);
     HIP_CHECK(hipMemcpyAsync(nns, d_nns.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipMemcpyAsync(dists, d_dist.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipMemcpyAsync(found, d_found.p, (size_t)nq * 4, hipMemcpyDeviceToHost, stream));

@@ -49,13 +49,15 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   a.redo_trail = nullptr;
   a.trail_next = nullptr;
   a.trail_cap = a.trail_first_spare = a.trail_spares = 0;
+  a.waiting = 0;
+  a.report = nullptr;
   last_repeats = 0;
   last_trails = 0;
   if (use_static) {
     launch_search_static<DT, QR, NS>(ix, a, ms);
     return;
   }
-  HIP_CHECK(hipEventRecord(ev0, stream));
+  if (ms) HIP_CHECK(hipEventRecord(ev0, stream));
   // the literal pass runs on the sorted set with ids and the LDS filter (no bitmap) unless the
   // caller asked for literal queues only, which also means exact evaluation counters
   // ...and unless the visited bitmaps of the wavefronts at work fit the L2 caches (32 MB) together:
@@ -81,15 +83,11 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   int n_literal = a.nq;
   bool answered = false;
   bool timed = false;  // ev1 has been recorded after the last kernel of this search
-  // A batch that fits the machine in one round of literal wavefronts is latency-bound: where the literal
-  // search has its exact bitmaps, two passes would only add the second pass's latency to the first's, and
-  // the literal pass answers alone.  Where the bitmaps do not fit the L2 (the literal search then runs on
-  // the sorted set with the LDS filter) the first pass is the same search without the literal candidate
-  // queue, and the faster choice even with a hand-over.
-  // (Long rows — the query in LDS — go to the first pass whatever the batch: there the literal search takes twice
-  // the first pass's time per expanded candidate, 2.0 against 1.0 ms for a single query on 1 M x 960.)
-  if (NS > 0 && a.fast_path && a.fc_bits > 0 &&
-      (a.fast_path > 1 || a.nq > lit_slots || (a.lean && a.nq > 1) || QR == 0)) {  // (reverse_cand: fast_path is 2)
+  // The first pass takes every batch, however small: it needs half the literal search's time per expanded candidate, so
+  // that it is the faster way even for a query that has to be handed over now and then (100 000 x 50, ef 300: one query
+  // 0.81 -> 0.37 ms, 1 000 queries 1.69 -> 0.76; a 200 000 x 128 integer set, ef 128, 32 queries: 0.75 -> 0.61 on average,
+  // 1.06 where one of them is handed over).
+  if (NS > 0 && a.fast_path && a.fc_bits > 0) {  // (reverse_cand: fast_path is 2)
     d_redo.reserve((size_t)a.nq);
     a.redo = d_redo.p;
     auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
@@ -105,18 +103,22 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     }
     const size_t fast_lds_bytes = fast_lds(a.fc_bits);
     int slots = fast_slots(a.fc_bits);
-    const bool side = concurrent_literal && sequential_left == 0 && max_slots_override <= 0;
+    // A batch of at most one wavefront per SIMD that is not expected to hand anything over does without the second
+    // stream: its events and the wait for the waiting wavefronts are 60 us of a search of a few hundred.
+    const bool alone = fast_path == 1 && !a.reverse && a.nq <= std::min(4 * num_cus, slots) && first_pass_waves == 0 &&
+                       max_slots_override <= 0 && repeat_share * a.nq < 0.5;
+    const bool side = concurrent_literal && sequential_left == 0 && max_slots_override <= 0 && !alone;
     last_side_by_side = side ? 1 : 0;
     int side_slots = 0;
     // few queries need the literal pass: one wavefront per CU serves them without taking room from
     // the first pass; two when the last search handed over 2 % and more (a literal wavefront's LDS
     // is that of one and a half wavefronts of the first pass, so more of them cost more than they serve)
-    const int per_cu = side_per_cu > 0 ? side_per_cu : (last_repeat_share < 0.02 ? 1 : 2);
+    const int per_cu = side_per_cu > 0 ? side_per_cu : (repeat_share < 0.02 ? 1 : 2);
     if (side) {
       side_slots = std::min(num_cus * per_cu, a.nq);
       // an index that hands over next to nothing (the last search: under one query in a thousand) gets one
       // literal wavefront per four CUs, and the first pass the room of the others
-      if (side_per_cu <= 0 && share_known && last_repeat_share < 0.001) side_slots = std::min(std::max(num_cus / 4, 1), a.nq);
+      if (side_per_cu <= 0 && share_known && repeat_share < 0.001) side_slots = std::min(std::max(num_cus / 4, 1), a.nq);
       ensure_pool(std::max(side_slots, 1), glob_cap, 2 * glob_cap);
       slots = std::max(num_cus, slots - std::min(side_slots, num_cus * per_cu));  // leave the literal wavefronts their room
     }
@@ -161,7 +163,16 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       a.trail_next = d_ctl.p + 48;
       a.redo_trail = d_redo_trail.p;
     }
-    {
+    a.waiting = side_slots;
+    a.report = side ? nullptr : h_ctl;  // (beside a literal pass the host needs that pass's status as well)
+    if (alone) {
+      // control words of its own, cleared with those of the next searches of this kind (the list is not: nobody polls it)
+      int* ctl = next_control_block();
+      a.counter = ctl;
+      a.repeats = ctl + 32;
+      a.done = ctl + 64;
+      if (keep_trails) a.trail_next = ctl + 48;
+    } else {
       const int n_hist = in_order ? kOrderBuckets : 0;
       const int n_fill = std::max(std::max(a.nq, n_hist), 128);
       hipLaunchKernelGGL(prepare_search_kernel, dim3((unsigned)((n_fill + 255) / 256)), dim3(256), 0, stream, d_ctl.p, 128,
@@ -222,19 +233,15 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     if (side) {
       HIP_CHECK(hipStreamWaitEvent(stream, ev_side1, 0));
     }
-    HIP_CHECK(hipEventRecord(ev1, stream));  // (recorded again further down if the list has to be answered after all)
+    if (ms) HIP_CHECK(hipEventRecord(ev1, stream));  // (recorded again further down if the list has to be answered after all)
     timed = true;
-    int* ctl = h_ctl;  // pinned: read back without a staging copy
-    HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, 49 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    int* ctl = h_ctl;  // pinned
+    if (side) HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, 49 * sizeof(int), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
-    n_literal = last_repeats = ctl[32];
-    last_trails = ctl[48];
-    last_repeat_share = (double)n_literal / a.nq;
-    share_known = true;
+    n_literal = last_repeats = side ? ctl[32] : ctl[0];
+    last_trails = side ? ctl[48] : ctl[1];
     if (!side && sequential_left > 0) --sequential_left;
-    // an index whose distances tie all the time (integer-valued data) sends most queries
-    // through both passes: stop trying the sorted set on it
-    if (a.nq >= 256 && (long long)n_literal * 3 > a.nq) fast_suspended = true;
+    learn_share(a.nq, n_literal);
     if (side) {
       answered = ctl[1] == 0;
       if (!answered) {
@@ -258,6 +265,8 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     for (int attempt = 0; attempt < 8 && !done; ++attempt) {
       ensure_pool(slots, glob_cap, 2 * glob_cap);
       b.pool = pool;
+      b.counter = d_ctl.p;
+      b.status = d_ctl.p + 1;
       HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 3 * sizeof(int), stream));
       hipLaunchKernelGGL(kernel, dim3(slots), dim3(64), lp.total, stream, ix, b);
       HIP_CHECK(hipGetLastError());
@@ -272,7 +281,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     }
     if (!done) throw std::runtime_error("search: candidate queue overflow");
   }
-  if (!timed) {
+  if (!timed && ms) {
     HIP_CHECK(hipEventRecord(ev1, stream));
     HIP_CHECK(hipEventSynchronize(ev1));
   }
@@ -309,7 +318,7 @@ void Engine::launch_search_static(const DevIndex& ix, SearchArgs& a, float* ms) 
     const LdsPlan lp = plan_lds(QR, ix.Dp, -1, a.cand_lds, a.lcap, 0, 0, 0, 0, a.lean);
     const int slots = std::max(1, std::min(resident_slots(fast_kernel, fp.total), a.nq));
     const int lit_slots = std::max(1, std::min(std::min(resident_slots(kernel, lp.total), kStaticSlots), a.nq));
-    HIP_CHECK(hipEventRecord(ev0, stream));
+    if (ms) HIP_CHECK(hipEventRecord(ev0, stream));
     hipLaunchKernelGGL(fill_ints_kernel, dim3(1), dim3(128), 0, stream, sc->ctl, 128, 0);
     HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fp.total, stream, ix, a);
@@ -325,7 +334,7 @@ void Engine::launch_search_static(const DevIndex& ix, SearchArgs& a, float* ms) 
     b.pool.log_cap = kStaticLogCap;
     hipLaunchKernelGGL(kernel, dim3(lit_slots), dim3(64), lp.total, stream, ix, b);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipEventRecord(ev1, stream));
+    if (ms) HIP_CHECK(hipEventRecord(ev1, stream));
     HIP_CHECK(hipMemcpyAsync(h_ctl, sc->ctl, 33 * sizeof(int), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     last_repeats = h_ctl[32];

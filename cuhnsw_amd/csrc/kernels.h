@@ -27,6 +27,9 @@
 
 namespace cuhnsw_amd {
 
+// what the entries of the list of given-up queries hold that never come: the first pass is through
+constexpr int kListEnds = -2;
+
 struct SlotPool {
   uint32_t* bitmaps;
   int bitmap_words;
@@ -53,6 +56,8 @@ struct SearchArgs {
                  // by the first wavefront of that pass to start
   int live;      // literal pass only: 1 = the sorted-set pass is running at the same time and a.redo is
                  // still being filled (entries start at -1); a.nq_total queries will pass through it
+  int waiting;   // sorted-set pass only: how many literal wavefronts wait beside it (they are told when it is through)
+  int* report;   // sorted-set pass only: host memory that gets the number of given-up queries and of spare trails taken
   int nq_total;
   int spin_limit;  // >= 0: polls of a live literal wavefront before it leaves with status 2 (tests force the
                    // fall-back with 0); < 0: no bound in polls, the two bounds in time below apply
@@ -534,8 +539,20 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS 
     // reads (its list entry, its trail): there the count is raised with release order, after them; an answered
     // query's results are the host's to read, after the kernel.
     if (lane == 0) {
-      if (gave_up) __hip_atomic_fetch_add(a.done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      else __hip_atomic_fetch_add(a.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int before = gave_up ? __hip_atomic_fetch_add(a.done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT)
+                                 : __hip_atomic_fetch_add(a.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (before == a.nq - 1) {
+        // the batch's last query: the list is complete.  The wavefronts that wait for further entries are told through
+        // the entries they poll (at most a.waiting of them), the host through its own memory.
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        const int n_list = __hip_atomic_load(a.repeats, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.report) {
+          a.report[0] = n_list;
+          a.report[1] = a.trail_next ? __hip_atomic_load(a.trail_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        }
+        for (int i = n_list; i < a.nq && i < n_list + a.waiting; ++i)
+          __hip_atomic_store(&a.redo[i], kListEnds, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
     wave_sync();
   }
@@ -585,7 +602,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
         // after start_ticks (the two streams are being serialised, as under a counter-collecting
         // profiler), or has made no progress for stall_ticks, the wavefront leaves with status 2
         // and the host answers the rest after the first pass.
-        int got = -1;
+        int got = kListEnds;
         if (qi < a.nq_total) {
           const long long t_begin = wall_clock64();
           long long t_progress = t_begin;
@@ -593,17 +610,18 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
           // (relaxed agent-scope loads: they read the L2 and, unlike acquire loads, do not
           // invalidate this CU's vector cache on every poll; the list entry is the only thing
           // read from the other pass, and it is read after the count that vouches for it)
-          // every waiter polls its own list entry; the shared count is looked at only now and
-          // then, and the pauses grow, so that the waiting does not crowd the memory channel
-          // of the counters the other pass is working with
+          // every waiter polls its own list entry, which is where it also learns that the first pass
+          // is through (kListEnds); the shared count is looked at only now and then, for the bounds
+          // in time, so that the waiting does not crowd the memory channel of the counters the other
+          // pass is working with
           for (int spins = 0;; ++spins) {
             got = __hip_atomic_load(&a.redo[qi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (got >= 0) break;
+            if (got != -1) break;
             if (a.spin_limit >= 0 && spins >= a.spin_limit) {
               atomicOr(a.status, 2);
               break;
             }
-            if ((spins & 3) == 3) {
+            if ((spins & 15) == 15) {
               const int done_now = __hip_atomic_load(a.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
               if (done_now >= a.nq_total) {
                 got = __hip_atomic_load(&a.redo[qi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -620,13 +638,8 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
                 break;
               }
             }
-            if (spins < 16) {
-              __builtin_amdgcn_s_sleep(32);
-            } else {
-              __builtin_amdgcn_s_sleep(127);
-              __builtin_amdgcn_s_sleep(127);
-              __builtin_amdgcn_s_sleep(127);
-            }
+            if (spins < 16) __builtin_amdgcn_s_sleep(32);  // 0.9 us
+            else __builtin_amdgcn_s_sleep(127);            // 3.5 us
           }
         }
         qi = got;

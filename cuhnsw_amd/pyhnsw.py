@@ -113,7 +113,7 @@ class CuHNSW:
 
   # -- search ----------------------------------------------------------------------------------
   def search_knn(self, qdata, topk, ef_search):
-    queries = np.asarray(qdata).astype(np.float32)
+    queries = np.ascontiguousarray(qdata, dtype=np.float32)
     rows = 1 if queries.ndim == 1 else queries.shape[0]
     out = (np.empty((rows, topk), np.int32), np.empty((rows, topk), np.float32), np.empty(rows, np.int32))
     self.obj.search_knn(queries, topk, max(topk, ef_search), *out)
