@@ -103,6 +103,41 @@ struct DevBuf {
   ~DevBuf() { release(); }
 };
 
+// Device memory that a build, a save or a load needs while it runs, in one allocation that the engine keeps for the next
+// of them: parts are asked for one after the other, reserve() makes room for all of them.
+class Workspace {
+ public:
+  template <typename T>
+  struct Part {
+    size_t offset;
+  };
+  void begin() { used_ = 0; }
+  template <typename T>
+  Part<T> part(size_t n) {
+    const Part<T> p{used_};
+    used_ += (n * sizeof(T) + 255) & ~(size_t)255;
+    return p;
+  }
+  void reserve() { memory_.reserve(std::max<size_t>(used_, 256)); }
+  template <typename T>
+  T* at(Part<T> p) const {
+    return reinterpret_cast<T*>(memory_.p + p.offset);
+  }
+  template <typename T>
+  size_t bytes_from(Part<T> p) const {
+    return used_ - p.offset;
+  }
+  // more than this is not kept (the largest builds need a tenth of the GPU's memory, which a search may want)
+  void end() {
+    if (memory_.n > kKept) memory_.release();
+  }
+
+ private:
+  static constexpr size_t kKept = (size_t)2 << 30;
+  DevBuf<unsigned char> memory_;
+  size_t used_ = 0;
+};
+
 class Engine {
  public:
   Options opt;
@@ -188,6 +223,7 @@ class Engine {
   DevBuf<float> d_q, d_dist;
   DevBuf<int> d_nns, d_found;
   HostStaging staging;
+  Workspace workspace;
   // pinned memory that small batches are read from and answered into (kernels address it)
   static constexpr size_t kDirectQueries = (size_t)64 << 10, kDirectAnswers = (size_t)1 << 20;
   unsigned char* h_io = nullptr;
@@ -639,6 +675,7 @@ class Engine {
     const int ns = build_literal ? 0 : key_slots(opt.ef_construction);
     if (dist_type == DIST_DOT) build_qr<DIST_DOT>(q, ns);
     else build_qr<DIST_L2>(q, ns);
+    workspace.end();
     last_build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     have_graph = true;
     forget_search_history();
@@ -685,24 +722,31 @@ class Engine {
     IndexWriter out(host, path);
     const size_t rec = (size_t)out.layout.record;
     const size_t piece_rows = std::max<size_t>(1, std::min<size_t>((size_t)host.N, kPiece / rec));
-    DevBuf<unsigned char> packed;
-    packed.reserve(piece_rows * rec);
+    workspace.begin();
+    const auto p_packed = workspace.part<unsigned char>(piece_rows * rec);
+    workspace.reserve();
+    unsigned char* const packed = workspace.at(p_packed);
     staging.reserve(0, false);
     if (host.n_deleted > 0) upload_marks();
     std::vector<uint32_t> up((size_t)host.upper_rows * host.SU);
     if (!up.empty()) HIP_CHECK(hipMemcpyAsync(up.data(), d_linksU.p, up.size() * 4, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
     const DevIndex ix = dev_index();
     for (size_t first = 0; first < (size_t)host.N; first += piece_rows) {
       const size_t rows = std::min(piece_rows, (size_t)host.N - first);
       hipLaunchKernelGGL(pack_records_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, ix, (int)first, (int)rows,
-                         host.n_deleted > 0 ? d_deleted.p : nullptr, reinterpret_cast<uint32_t*>(packed.p));
+                         host.n_deleted > 0 ? d_deleted.p : nullptr, reinterpret_cast<uint32_t*>(packed));
       HIP_CHECK(hipGetLastError());
       const uint64_t file_at = FileLayout::kHeader + (uint64_t)first * rec;
-      staging.fetch(stream, packed.p, rows * rec, out.parallel(),
-                    [&](const unsigned char* from, size_t at, size_t n) { out.write(file_at + at, from, n); });
+      staging.fetch(stream, packed, rows * rec, out.parallel(),
+                    [&](const unsigned char* from, size_t at, size_t n) { out.write(file_at + at, from, n); },
+                    [&] {  // (beside the others, where the file may be written in any order)
+                      if (out.parallel() && first + rows == (size_t)host.N) out.write_upper(host, up.data());
+                    });
     }
     HIP_CHECK(hipStreamSynchronize(stream));
-    out.write_upper(host, up.data());
+    workspace.end();
+    if (!out.parallel()) out.write_upper(host, up.data());
     out.finish();
   }
   void upload_marks() {
@@ -727,15 +771,17 @@ class Engine {
     }
     IndexReader in(fresh, path);
     const size_t rec = (size_t)in.layout.record, n = (size_t)fresh.N;
-    DevBuf<unsigned char> raw, marks;
-    raw.reserve(std::max<size_t>(n * rec, 1));
-    marks.reserve(std::max<size_t>(n, 1));
+    workspace.begin();
+    const auto p_raw = workspace.part<unsigned char>(n * rec);
+    const auto p_marks = workspace.part<unsigned char>(n);
+    workspace.reserve();
+    unsigned char *const raw = workspace.at(p_raw), *const marks = workspace.at(p_marks);
     staging.reserve(0, false);
     std::string upper_error;
     HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 2 * sizeof(int), stream));
     staging.send(stream, n * rec, staging.block(),
                  [&](unsigned char* to, size_t at, size_t len) { in.read(FileLayout::kHeader + at, to, len, "level-0 block"); },
-                 [&](size_t at, size_t) { return raw.p + at; }, [](unsigned char*, size_t, size_t) {},
+                 [&](size_t at, size_t) { return raw + at; }, [](unsigned char*, size_t, size_t) {},
                  [&] {  // (on this thread, beside the others)
                    try {
                      in.read_upper(fresh);
@@ -745,7 +791,7 @@ class Engine {
                  });
     if (n > 0) {
       hipLaunchKernelGGL(check_records_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
-                         reinterpret_cast<const uint32_t*>(raw.p), (int)n, fresh.D, fresh.max_m0, marks.p, d_ctl.p);
+                         reinterpret_cast<const uint32_t*>(raw), (int)n, fresh.D, fresh.max_m0, marks, d_ctl.p);
       HIP_CHECK(hipGetLastError());
     }
     HIP_CHECK(hipMemcpyAsync(h_ctl, d_ctl.p, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -757,7 +803,7 @@ class Engine {
     fresh.n_deleted = h_ctl[1];
     if (fresh.n_deleted > 0) {
       fresh.deleted.resize(n);
-      HIP_CHECK(hipMemcpyAsync(fresh.deleted.data(), marks.p, n, hipMemcpyDeviceToHost, stream));
+      HIP_CHECK(hipMemcpyAsync(fresh.deleted.data(), marks, n, hipMemcpyDeviceToHost, stream));
       HIP_CHECK(hipStreamSynchronize(stream));
     }
     host = std::move(fresh);
@@ -767,12 +813,13 @@ class Engine {
     upload_structure();
     d_labels.reserve(n);
     hipLaunchKernelGGL(unpack_records_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
-                       reinterpret_cast<const uint32_t*>(raw.p), dev_index(), d_labels.p);
+                       reinterpret_cast<const uint32_t*>(raw), dev_index(), d_labels.p);
     HIP_CHECK(hipGetLastError());
     if (!host.linksU.empty())
       HIP_CHECK(hipMemcpyAsync(d_linksU.p, host.linksU.data(), host.linksU.size() * 4, hipMemcpyHostToDevice, stream));
     if (host.n_deleted > 0) upload_marks();
     HIP_CHECK(hipStreamSynchronize(stream));
+    workspace.end();
     std::vector<uint32_t>().swap(host.linksU);
     pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
     pool = SlotPool{};

@@ -119,9 +119,9 @@ class HostStaging {
   }
 
   // Device to host: drain(from, at, n) takes bytes [at, at + n) of the transfer out of pinned memory, on several threads
-  // at once if `side_by_side`, else in ascending order on one.
-  template <typename Drain>
-  void fetch(hipStream_t stream, const unsigned char* source, size_t total, bool side_by_side, Drain&& drain) {
+  // at once if `side_by_side`, else in ascending order on one.  `meanwhile` runs on the calling thread.
+  template <typename Drain, typename Meanwhile>
+  void fetch(hipStream_t stream, const unsigned char* source, size_t total, bool side_by_side, Drain&& drain, Meanwhile&& meanwhile) {
     int device = 0;
     HIP_CHECK(hipGetDevice(&device));
     const size_t block = block_;
@@ -143,7 +143,7 @@ class HostStaging {
         HIP_CHECK(hipEventSynchronize(event_[slot]));
         drain(host_ + (size_t)slot * block_, at, std::min(block, total - at));
       }
-    }, [] {});
+    }, meanwhile);
   }
 
  private:

@@ -93,9 +93,8 @@ struct SearchArgs {
 
 struct BuildArgs {
   int begin, count;        // batch = nodes begin .. begin+count-1
-  const int* order;        // N entries or null: the i-th node a batch hands out is begin + order[begin + i] (the
-                           // nodes with upper levels first: they take several searches, and a launch ends when
-                           // its last node does)
+  const int* upper;        // the batch's nodes with upper levels (highest first, offsets from begin): handed out before
+  int n_upper;             // the others (they take several searches, and a launch ends when its last node does); 0 = by id
   int cur_ep, cur_max;     // entry point and top level of the graph before this batch (cur_max < 0: empty)
   int efc, nn_num0, nn_numU, save_remains;
   int reverse;   // expand the farthest waiting candidate (reverse_cand)
@@ -1033,20 +1032,24 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
   wave_sync();
 
   for (;;) {
+    // first the n_upper nodes of the list, then all by id, the ones of the list passed over
     int b = 0;
     if (lane == 0) {
       b = atomicAdd(a.counter, 1);
-      if (b < a.count && a.order) b = a.order[a.begin + b];
+      b = b < a.n_upper ? a.upper[b] : b - a.n_upper + (1 << 30);
     }
     b = __builtin_amdgcn_readfirstlane(b);
+    const bool listed = b < (1 << 30);
+    b &= (1 << 30) - 1;
     if (b >= a.count) break;
     const uint32_t x = (uint32_t)(a.begin + b);
     const int lx = ix.levels[x];
     const int top_level = lx < a.cur_max ? lx : a.cur_max;  // levels x shares with the graph so far
-    if (lane == 0) a.sel0_cnt[b] = 0;
+    const bool here = listed || a.n_upper == 0 || lx <= 0;
+    if (lane == 0 && here) a.sel0_cnt[b] = 0;
     // (the very first node has nothing to link to; a plain branch, not a `continue` after the
     // one-lane store above, keeps the control flow simple for the compiler)
-    if (top_level >= 0) {
+    if (here && top_level >= 0) {
       QVec<QR> qv;
       load_node_query<QR>(qv, s.qlds, ix, x, lane);
       SearchState st;
