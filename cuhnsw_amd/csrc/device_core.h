@@ -133,6 +133,12 @@ __device__ __forceinline__ float reduce16(float x) {
 __device__ __forceinline__ float uni(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
 }
+// The same number, which the compiler takes for a new one: what is computed from it is computed here, not ahead of the
+// loops around and kept in registers through them.
+__device__ __forceinline__ int fresh(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 // how many lanes below this one have their bit set in a wavefront-uniform mask (v_mbcnt: no lane masks in registers)
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
@@ -858,6 +864,83 @@ __device__ __forceinline__ void frontier_insert_distinct(Frontier<NS>& f, float 
     f.v[j] = before_this ? (before_lower ? lo_v : id) : f.v[j];
   }
 }
+// All n offers of a list (lane i < n: the i-th; in the other lanes any key) into a set that has room for them.  Each set entry
+// counts the offers before it, each offer the entries and offers before it, and every entry goes to its new place through
+// LDS: the counting has no dependent steps (15 vector instructions per offer at ef 300, where an insert of its own is 39
+// and 0.25 us of latency), the rest is paid once.  `room`: 64 * NS words of LDS, whose contents are put back.  Returns
+// false, with nothing done, if two keys are equal (or the node is in the set already): those go in one by one, by the rules
+// for them.  last_key: the set's largest key afterwards.
+// (1.18 M x 50, ef 300, 10 000 queries: 1.51 -> 1.45 ms; 1 M x 96, ef 256, 100 000 queries: 10.28 -> 9.96; one query on
+// 100 000 x 50: 0.304 -> 0.288; 200 003 x 128 indexed: 73.6 -> 71.5 ms)
+template <int NS>
+__device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, int n, int size, int ef, float my_key, uint32_t my_id, uint32_t* room,
+                                                    float& last_key, int lane) {
+  constexpr int N = NS > 0 ? NS : 1;
+  lane = fresh(lane);
+  int before[N];  // offers that go before each of this lane's entries
+#pragma unroll
+  for (int j = 0; j < N; ++j) before[j] = 0;
+  int place = 0, less = 0;  // this lane's offer: entries and offers before it
+  unsigned long long equal = 0ull;
+  for (int i = 0; i < n; ++i) {
+    const float key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_key), i));
+    int above = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      above += __popcll(__ballot(key < f.k[j]));
+      before[j] += key < f.k[j] ? 1 : 0;
+    }
+    const unsigned long long self = 1ull << i;
+    place = __builtin_amdgcn_inverse_ballot_w64(self) ? 64 * N - above : place;
+    less += key < my_key ? 1 : 0;
+    equal |= __ballot(key == my_key) & ~self;
+  }
+  const unsigned long long offers = n < 64 ? (1ull << n) - 1ull : ~0ull;
+  if ((equal & offers) != 0ull) return false;
+  // (keys first, then ids: half the registers, of which the search has none to spare)
+  uint32_t kept[N];
+  const bool mine = __builtin_amdgcn_inverse_ballot_w64(offers);
+#pragma unroll
+  for (int j = 0; j < N; ++j) kept[j] = room[64 * j + lane];
+  wave_sync();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int to = lane * N + j + before[j];
+    if (to < 64 * N) room[to] = __float_as_uint(f.k[j]);  // (what is pushed out is padding)
+  }
+  if (mine) room[place + less] = __float_as_uint(my_key);
+  wave_sync();
+  // an offer equal to an entry comes right after it (the padding on both sides is infinite)
+  unsigned long long twins = 0ull;
+  float key[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) key[j] = __uint_as_float(room[lane * N + j]);
+  const float last = __uint_as_float(room[64 * N - ef + size + n - 1]);
+  const float prev_last = __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, key[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    twins |= __ballot(key[j] == (j > 0 ? key[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(key[j]) < INFINITY);
+  if (twins == 0ull) {
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int to = lane * N + j + before[j];
+      if (to < 64 * N) room[to] = f.v[j];
+      f.k[j] = key[j];
+    }
+    if (mine) room[place + less] = my_id;
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < N; ++j) f.v[j] = room[lane * N + j];
+    last_key = uni(last);
+  }
+  wave_sync();
+#pragma unroll
+  for (int j = 0; j < N; ++j) room[64 * j + lane] = kept[j];
+  wave_sync();
+  return twins == 0ull;
+}
 template <int NS>
 __device__ __forceinline__ float frontier_max(const Frontier<NS>& f) {
   constexpr int N = NS > 0 ? NS : 1;
@@ -1380,6 +1463,8 @@ template <int DT, int QR, int NS, bool FULL, bool TRAILS, bool WATCH, bool BUILD
 __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>& qv, int level, int ef, int S, Scratch& s,
                                               SearchState& st, Frontier<NS>& fr, int& n, int& hop_cid, int& resume_at,
                                               unsigned long long& accepted, Trail& tr, const TieWatch& watch, int lane) {
+  constexpr int N = NS > 0 ? NS : 1;
+  constexpr int kInsertAllFrom = 4;  // shorter lists go in one by one
   constexpr int kWide = (QR == 0 && !BUILD && NS <= 8) ? 2 : 1;  // (the search on long rows: dist_long)
   constexpr int K = FULL && (BUILD || NS > 2) ? (QR == 1 ? kAhead : 6) : 1;  // (longer rows: registers)
   // (said to be wavefront-uniform, so that they sit in scalar registers through the loop)
@@ -1412,6 +1497,16 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
     int row_end = K > 1 ? (int)(ends & 0xFFu) : n;
     int good = rows;                                        // candidates of the batch that are expanded for good
     const int acc_before = st.n_acc;
+    if (!FULL && (BUILD || NS > 2) && n >= kInsertAllFrom && st.n_acc + n <= ef && 64 * N <= (1 << s.vc_bits)) {
+      float last_key = 0.f;
+      if (frontier_insert_all<NS>(fr, n, st.n_acc, ef, my_key, my_id, reinterpret_cast<uint32_t*>(s.vcache), last_key, lane)) {
+        if (TRAILS) accepted |= todo;
+        st.n_acc = st.n_acc + n;
+        st.maxkey = last_key;
+        st.lower = last_key;
+        todo = 0ull;
+      }
+    }
     if (K > 1)
       tie_free_offers<NS, FULL, TRAILS, WATCH, BUILD, true>(st, fr, todo, my_key, my_id, ef, w_hi, cand, ends, hop_cid, r, row_end, good,
                                                             resume_at, accepted, tr, lane);

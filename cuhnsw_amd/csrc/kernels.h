@@ -418,7 +418,6 @@ __device__ __forceinline__ const Args& fresh_args() {
 template <int DT, int QR, int NS, bool TRAILS>
 __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS == 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int lane = threadIdx.x;
   const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
   Scratch s;
   s.vcache = reinterpret_cast<uint16_t*>(smem + lp.fcache);
@@ -427,10 +426,11 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS 
   s.nbuf = reinterpret_cast<uint32_t*>(smem + lp.nbuf);
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
   // tells a literal pass waiting beside this one that the two kernels do run at the same time
-  if (blockIdx.x == 0 && lane == 0) __hip_atomic_store(a0.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(a0.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int trail_buf = (TRAILS && a0.trail) ? (int)blockIdx.x : -1;  // the buffer this wavefront's trails go to
 
   for (;;) {
+    int lane = fresh((int)threadIdx.x);
     const SearchArgs& in = fresh_args<SearchArgs>();
     const DevIndex& from = fresh_index();
     int qi = 0;
@@ -463,6 +463,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS 
       descend<DT, QR>(from, qv, from.maxlevel, 0, cur, dcur, s, st, lane);
     }
 
+    lane = fresh(lane);
     Frontier<NS> fr;
     frontier_init<NS>(fr, a0.ef, lane);
     filter_reset(s, lane);
@@ -472,6 +473,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS 
     // (the flag is made wavefront-uniform explicitly and both outcomes are plain branches)
     const int how =
         __builtin_amdgcn_readfirstlane(search_level_fast<DT, QR, NS, false, TRAILS>(ix0, qv, 0, a0.ef, s, st, fr, 1, lane, a0.reverse != 0, a0.k >= a0.ef, TRAILS ? &tr : nullptr));
+    lane = fresh(lane);
     const SearchArgs& a = fresh_args<SearchArgs>();
     const DevIndex& ix = fresh_index();
     const int T0 = st.top_size < a.k ? st.top_size : a.k;
@@ -1006,7 +1008,7 @@ __device__ __forceinline__ int select_neighbors(const DevIndex& ix, const uint32
 template <int DT, int QR, int NS>
 __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR == 2) ? 5 : 1)) build_search_kernel(DevIndex ix, BuildArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int lane = threadIdx.x;
+  int lane = threadIdx.x;
   const int m_max = ix.max_m0 > ix.max_m ? ix.max_m0 : ix.max_m;
   const bool sorted_set = NS > 0 && a.fc_bits > 0;
   const LdsPlan lp = plan_lds(QR, ix.Dp, sorted_set ? -1 : a.efc, a.cand_lds, a.lcap, a.efc, m_max, a.vc_bits, a.fc_bits);
@@ -1033,6 +1035,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
 
   for (;;) {
     // first the n_upper nodes of the list, then all by id, the ones of the list passed over
+    lane = fresh(lane);
     int b = 0;
     if (lane == 0) {
       b = atomicAdd(a.counter, 1);
@@ -1064,6 +1067,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
         descend<DT, QR>(ix, qv, a.cur_max, lx, cur, dcur, s, st, lane);
       }
       for (int level = top_level; level >= 0; --level) {
+        lane = fresh(lane);
         const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
         st.top_size = 0; st.cand_size = 0; st.n_acc = 0; st.lower = 0.f; st.maxkey = -INFINITY; st.ahead = 1;
         const int evals_before = st.n_dist, hops_before = st.n_hops;
@@ -1117,6 +1121,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
           rank_sort(s.top, nullptr, T, sid, skey, lane);
           wave_sync();
         }
+        lane = fresh(lane);
         unsigned int* level_work = a.counters ? work + (level == 0 ? 0 : 5) : nullptr;
         const int deg = select_neighbors<DT, QR>(ix, sid, skey, T, level == 0 ? a.own_cap0 : m_cap,
                                                  level == 0 ? a.nn_num0 : a.nn_numU, a.save_remains, oid, okey, s, lane,
