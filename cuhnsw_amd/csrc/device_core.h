@@ -301,9 +301,13 @@ __device__ __forceinline__ void dist_pass(const void* rows, uint32_t rowlen, uin
     for (int k = 0; k < R; ++k) acc4<DT>(q[k], v[u][k], ax, ay, az, aw);
     s[u] = (ax + ay) + (az + aw);
   }
-  const float key = finish_rows<DT, RAW, U>(s, sub);
-  const int mine = r + 4 * sub + g;
-  if (sub < U && mine < n) out[mine] = key;
+#pragma unroll
+  for (int u = 0; u < U; u += 4) {
+    constexpr int H = U < 4 ? U : 4;
+    const float key = finish_rows<DT, RAW, H>(s + u, sub);
+    const int mine = r + 4 * (u + sub) + g;
+    if (sub < H && mine < n) out[mine] = key;
+  }
   // (the lanes meet again here, not at the caller's loop end: see trail_mark)
   __builtin_amdgcn_wave_barrier();
 }
@@ -385,7 +389,10 @@ __device__ __forceinline__ void dist_long(const void* rows, int rowlen, int used
                                           int n, float* out, int g, int sub) {
   int r = 0;
   while (r < n) {
-    if (U >= 2 && n - r > 4) {
+    if (U >= 4 && n - r > 8) {
+      dist_long_pass<DT, RAW, HALF, (U >= 4 ? 4 : 1), kLongB>(rows, rowlen, used, qlds, ids, r, n, out, g, sub);
+      r += 16;
+    } else if (U >= 2 && n - r > 4) {
       dist_long_pass<DT, RAW, HALF, (U >= 2 ? 2 : 1), kLongB>(rows, rowlen, used, qlds, ids, r, n, out, g, sub);
       r += 8;
     } else {
@@ -405,11 +412,15 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
   const void* rows = ix.vectors;
   if (QR > 0) {
     constexpr int R = QR > 0 ? QR : 1;
-    constexpr int UMAX = R == 1 ? 4 : (R == 2 ? 2 * WIDE : 1);  // groups of 4 rows in flight
+    // groups of 4 rows in flight
+    constexpr int UMAX = R == 1 ? (WIDE >= 4 ? 8 : 4) : (R == 2 ? (WIDE >= 2 ? 4 : 2) : (WIDE >= 4 ? 2 : 1));
     int r = 0;
     while (r < n) {
       const int rem = n - r;
-      if (UMAX >= 4 && rem > 8) {
+      if (UMAX >= 8 && rem > 16) {
+        dist_pass<DT, R, (UMAX >= 8 ? 8 : 1), RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
+        r += 32;
+      } else if (UMAX >= 4 && rem > 8) {
         dist_pass<DT, R, (UMAX >= 4 ? 4 : 1), RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
         r += 16;
       } else if (UMAX >= 2 && rem > 4) {
@@ -425,7 +436,8 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
   }
 }
 // (the element type of the stored vectors is a property of the index: one scalar branch per list)
-// WIDE: groups of four rows in flight on long rows (dist_long); 2 doubles them where the query takes two registers
+// WIDE: how many rows are in flight; 1 = as many as registers allow beside a full machine's wavefronts, 4 = as a
+// wavefront with a SIMD to itself can have
 template <int DT, int QR, bool RAW, int WIDE = 1>
 __device__ __forceinline__ void dist_list(const DevIndex& ix, const QVec<QR>& qv, const float4* qlds,
                                           const uint32_t* ids, int n, float* out, int lane) {
@@ -1459,7 +1471,7 @@ __device__ __forceinline__ void tie_free_offers(SearchState& st, Frontier<NS>& f
 // ef <= 128: with as many accepted offers as hops a batch seldom holds (40 000 queries on 1.18 M x 50, ef 64: 1.77 ms
 // without, 1.81 with).  1.18 M x 50, ef 300, 10 000 / 40 000 queries: 1.76 -> 1.53, 5.08 -> 4.54 ms; 1 M x 96, topk 100,
 // ef 256, 100 000 queries: 11.06 -> 9.99 ms; 100 000 x 960, ef 300, 1 000 queries: 1.44 -> 1.36 ms.
-template <int DT, int QR, int NS, bool FULL, bool TRAILS, bool WATCH, bool BUILD = false>
+template <int DT, int QR, int NS, bool FULL, bool TRAILS, bool WATCH, bool BUILD = false, bool FEW = false>
 __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>& qv, int level, int ef, int S, Scratch& s,
                                               SearchState& st, Frontier<NS>& fr, int& n, int& hop_cid, int& resume_at,
                                               unsigned long long& accepted, Trail& tr, const TieWatch& watch, int lane) {
@@ -1467,8 +1479,8 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   constexpr int kInsertAllFrom = 4;  // shorter lists go in one by one
   // more rows in flight: the search on long rows (dist_long), and small sets, which leave the registers for it (56 of 72;
   // 345 678 x 101 in fp16, ef 77, 5 003 queries: 0.85 -> 0.71 ms)
-  constexpr int kWide = !BUILD && ((QR == 0 && NS <= 8) || (QR == 2 && NS == 2)) ? 2 : 1;
-  constexpr int K = FULL && (BUILD || NS > 2) ? (QR == 1 ? kAhead : 6) : 1;  // (longer rows: registers)
+  constexpr int kWide = FEW ? 4 : (!BUILD && ((QR == 0 && NS <= 8) || (QR == 2 && NS == 2)) ? 2 : 1);
+  constexpr int K = FULL && (BUILD || FEW || NS > 2) ? (QR == 1 || FEW ? kAhead : 6) : 1;  // (longer rows: registers)
   // (said to be wavefront-uniform, so that they sit in scalar registers through the loop)
   const int w0 = WATCH ? uni(watch.id0) : -1, w1 = WATCH ? uni(watch.id1) : -1;
   const int w2 = WATCH ? uni(watch.id2) : -1, w3 = WATCH ? uni(watch.id3) : -1;
@@ -1499,7 +1511,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
     int row_end = K > 1 ? (int)(ends & 0xFFu) : n;
     int good = rows;                                        // candidates of the batch that are expanded for good
     const int acc_before = st.n_acc;
-    if (!FULL && (BUILD || NS > 2) && n >= kInsertAllFrom && st.n_acc + n <= ef && 64 * N <= (1 << s.vc_bits)) {
+    if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && st.n_acc + n <= ef && 64 * N <= (1 << s.vc_bits)) {
       float last_key = 0.f;
       if (frontier_insert_all<NS>(fr, n, st.n_acc, ef, my_key, my_id, reinterpret_cast<uint32_t*>(s.vcache), last_key, lane)) {
         if (TRAILS) accepted |= todo;
@@ -1632,12 +1644,12 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
 // far: expand the farthest waiting entry instead of the closest (the reference's
 // reverse_cand); that is no hnswlib search any more, equal keys simply keep their order of
 // arrival and nothing is ever given up.  BUILD likewise never gives up.
-template <int DT, int QR, int NS, bool BUILD, bool TRAILS = false>
+template <int DT, int QR, int NS, bool BUILD, bool TRAILS = false, bool FEW = false>
 __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<QR>& qv, int level, int ef, Scratch& s,
                                                   SearchState& st, Frontier<NS>& fr, int n_seed, int lane,
                                                   bool far = false, bool whole_set = false, Trail* trail = nullptr) {
   const int S = row_stride(ix, level);
-  constexpr int kWide = (QR == 0 && !BUILD && NS <= 8) ? 2 : 1;  // (the search on long rows: dist_long)
+  constexpr int kWide = FEW ? 4 : ((QR == 0 && !BUILD && NS <= 8) ? 2 : 1);  // (rows in flight: dist_list)
   int n = n_seed;
   const bool exact = !BUILD && !far;  // the outcome has to be hnswlib's
   Trail no_trail;
@@ -1666,11 +1678,11 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
       } else if (!have_tie) {
-        if (how == 0) how = tie_free_phase<DT, QR, NS, false, TRAILS, false>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
-        if (how == 2) how = tie_free_phase<DT, QR, NS, true, TRAILS, false>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
+        if (how == 0) how = tie_free_phase<DT, QR, NS, false, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
+        if (how == 2) how = tie_free_phase<DT, QR, NS, true, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
       } else {
         // (after equal keys have met, the tie-free loop takes over again only once the set is full: how == 2)
-        how = tie_free_phase<DT, QR, NS, true, TRAILS, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
+        how = tie_free_phase<DT, QR, NS, true, TRAILS, true, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
       }
       st.top_size = st.n_acc < ef ? st.n_acc : ef;
       if (how == 0) {

@@ -135,7 +135,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     // the trail costs the first pass 9 % (the kernel instance with the trail code 4 %, writing the records the
     // rest), which only a batch short enough to wait for its last hand-over gets back.  trails = 2: whatever
     // the batch.
-    bool keep_trails = (QR == 1 || QR == 2) && trails && !a.reverse && a.lean && host.S0 <= 63 &&
+    bool keep_trails = !alone && (QR == 1 || QR == 2) && trails && !a.reverse && a.lean && host.S0 <= 63 &&
                        (trails > 1 || 4 * (long long)a.nq <= 11 * resident);
     if (keep_trails) {
       // (normally there since the index became resident; a changed trail_cap / trail_spares asks again)
@@ -171,7 +171,6 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       a.counter = ctl;
       a.repeats = ctl + 32;
       a.done = ctl + 64;
-      if (keep_trails) a.trail_next = ctl + 48;
     } else {
       const int n_hist = in_order ? kOrderBuckets : 0;
       const int n_fill = std::max(std::max(a.nq, n_hist), 128);
@@ -223,7 +222,9 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
                          a.nq, d_order_hist.p, d_order.p);
       HIP_CHECK(hipGetLastError());
     }
-    if constexpr (QR == 1 || QR == 2) {
+    if (alone) {
+      hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, false, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
+    } else if constexpr (QR == 1 || QR == 2) {
       if (keep_trails) hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
       else hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
     } else {
