@@ -75,6 +75,18 @@ int row_degree(const uint32_t* row, int cap) {
   return d;
 }
 
+void write_at(int fd, uint64_t offset, const void* src, size_t n) {
+  const unsigned char* p = static_cast<const unsigned char*>(src);
+  while (n > 0) {
+    const ssize_t got = ::pwrite(fd, p, n, (off_t)offset);
+    if (got < 0 && errno == EINTR) continue;
+    if (got <= 0) throw std::runtime_error("index file: write failed");
+    p += got;
+    offset += (uint64_t)got;
+    n -= (size_t)got;
+  }
+}
+
 void write_all(int fd, const void* src, size_t n) {
   const unsigned char* p = static_cast<const unsigned char*>(src);
   while (n > 0) {
@@ -206,7 +218,7 @@ void IndexReader::read_upper(HostIndex& ix) const {
 
 // ---- writing -------------------------------------------------------------------------------------------
 IndexWriter::IndexWriter(const HostIndex& ix, const std::string& path)
-    : layout((uint64_t)ix.max_m, (uint64_t)ix.max_m0, (uint64_t)ix.D) {
+    : layout((uint64_t)ix.max_m, (uint64_t)ix.max_m0, (uint64_t)ix.D), path_(path) {
   upper_at_ = FileLayout::kHeader + (uint64_t)ix.N * layout.record;
   size_ = upper_at_ + (uint64_t)ix.N * 4 + (uint64_t)ix.upper_rows * layout.linksU_bytes;
   // A file that is there is written over in place and cut to its new length at the end: its pages need not be
@@ -227,6 +239,7 @@ IndexWriter::IndexWriter(const HostIndex& ix, const std::string& path)
       do rc = ::fallocate(fd_, 0, 0, (off_t)size_);
       while (rc != 0 && errno == EINTR);
       if (rc != 0 && (errno == ENOSPC || errno == EDQUOT || errno == EFBIG)) {
+        (void)!::ftruncate(fd_, st.st_size);  // (the file that is there stays as it was)
         ::close(fd_);
         throw std::runtime_error("index file: write failed");
       }
@@ -250,8 +263,11 @@ IndexWriter::IndexWriter(const HostIndex& ix, const std::string& path)
   h.put<uint64_t>(kM, (uint64_t)ix.M);
   h.put<double>(kMult, ix.mult);
   h.put<uint64_t>(kEfConstruction, (uint64_t)ix.ef_construction);
+  std::memcpy(header_, h.bytes, sizeof(header_));
   try {
-    write(0, h.bytes, sizeof(h.bytes));
+    static const unsigned char none[FileLayout::kHeader] = {};
+    if (regular_) write_at(fd_, 0, none, sizeof(none));  // from here on the file is no index, until finish() says so
+    else write_all(fd_, header_, sizeof(header_));
   } catch (...) {
     if (map_) ::munmap(map_, size_);
     ::close(fd_);
@@ -261,7 +277,9 @@ IndexWriter::IndexWriter(const HostIndex& ix, const std::string& path)
 
 IndexWriter::~IndexWriter() {
   if (map_) ::munmap(map_, size_);
-  if (fd_ >= 0) ::close(fd_);
+  if (fd_ < 0) return;
+  if (regular_) (void)!::ftruncate(fd_, 0);  // not finished
+  ::close(fd_);
 }
 
 void IndexWriter::write(uint64_t offset, const void* src, size_t n) {
@@ -269,19 +287,8 @@ void IndexWriter::write(uint64_t offset, const void* src, size_t n) {
     std::memcpy(map_ + offset, src, n);
     return;
   }
-  if (!regular_) {
-    write_all(fd_, src, n);
-    return;
-  }
-  const unsigned char* p = static_cast<const unsigned char*>(src);
-  while (n > 0) {
-    const ssize_t got = ::pwrite(fd_, p, n, (off_t)offset);
-    if (got < 0 && errno == EINTR) continue;
-    if (got <= 0) throw std::runtime_error("index file: write failed");
-    p += got;
-    offset += (uint64_t)got;
-    n -= (size_t)got;
-  }
+  if (regular_) write_at(fd_, offset, src, n);
+  else write_all(fd_, src, n);
 }
 
 void IndexWriter::write_upper(const HostIndex& ix, const uint32_t* linksU) {
@@ -307,10 +314,16 @@ void IndexWriter::finish() {
     ::munmap(map_, size_);
     map_ = nullptr;
   }
-  if (regular_ && ::ftruncate(fd_, (off_t)size_) != 0) throw std::runtime_error("index file: write failed");
+  if (regular_) {
+    if (::ftruncate(fd_, (off_t)size_) != 0) throw std::runtime_error("index file: write failed");
+    write_at(fd_, 0, header_, sizeof(header_));
+  }
   const int fd = fd_;
   fd_ = -1;
-  if (::close(fd) != 0) throw std::runtime_error("index file: write failed");
+  if (::close(fd) != 0) {  // (where what was written leaves for a server only now)
+    if (regular_) (void)!::truncate(path_.c_str(), 0);
+    throw std::runtime_error("index file: write failed");
+  }
 }
 
 // ---- host tables <-> file ------------------------------------------------------------------------------

@@ -81,10 +81,12 @@ class IndexReader {
 };
 
 // An index file opened for writing; its size is known from the start.  write() may be called from several threads
-// where parallel() says so, else in ascending order without gaps.  finish() makes the file as long as it has to be.
+// where parallel() says so, else in ascending order without gaps.  A regular file has no header until finish() puts it
+// there, as the last thing of all: a save that does not get that far, for whatever reason, leaves nothing that loads (and
+// an empty file where the destructor still runs).
 class IndexWriter {
  public:
-  IndexWriter(const HostIndex& ix, const std::string& path);  // writes the header
+  IndexWriter(const HostIndex& ix, const std::string& path);
   ~IndexWriter();
   IndexWriter(const IndexWriter&) = delete;
   IndexWriter& operator=(const IndexWriter&) = delete;
@@ -100,6 +102,8 @@ class IndexWriter {
   bool regular_ = false;
   unsigned char* map_ = nullptr;
   uint64_t size_ = 0, upper_at_ = 0;
+  unsigned char header_[FileLayout::kHeader];
+  std::string path_;
 };
 
 // Both throw std::runtime_error with a message on I/O or format errors.  (Host tables only: an engine with a GPU
