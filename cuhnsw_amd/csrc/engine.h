@@ -799,6 +799,7 @@ class Engine {
     if (h_ctl[0] & 1) throw std::runtime_error("index file: link count above max_m0");
     if (h_ctl[0] & 2) throw std::runtime_error("index file: link id out of range");
     if (!upper_error.empty()) throw std::runtime_error(upper_error);
+    in.check_unchanged();
     if (n == 0) throw std::runtime_error("load_index: empty index");
     fresh.n_deleted = h_ctl[1];
     if (fresh.n_deleted > 0) {

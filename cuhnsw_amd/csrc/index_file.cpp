@@ -108,6 +108,8 @@ IndexReader::IndexReader(HostIndex& ix, const std::string& path) {
     struct stat st;
     if (::fstat(fd_, &st) == 0 && S_ISREG(st.st_mode)) {
       size_ = (uint64_t)st.st_size;
+      seconds_ = st.st_mtim.tv_sec;
+      nanoseconds_ = st.st_mtim.tv_nsec;
     } else {
       in_memory_ = true;
       size_t have = 0;
@@ -123,6 +125,7 @@ IndexReader::IndexReader(HostIndex& ix, const std::string& path) {
     }
     HeaderField h;
     read(0, h.bytes, sizeof(h.bytes), "header");
+    std::memcpy(header_, h.bytes, sizeof(header_));
     const uint64_t count = h.get<uint64_t>(kCount), max_elements = h.get<uint64_t>(kMaxElements);
     const uint64_t max_m = h.get<uint64_t>(kMaxM), max_m0 = h.get<uint64_t>(kMaxM0);
     const uint64_t offset_data = h.get<uint64_t>(kOffsetData), label_offset = h.get<uint64_t>(kLabelOffset);
@@ -172,6 +175,16 @@ void IndexReader::read(uint64_t offset, void* dst, size_t n, const char* what) c
     offset += (uint64_t)got;
     n -= (size_t)got;
   }
+}
+
+void IndexReader::check_unchanged() const {
+  if (in_memory_) return;
+  struct stat st;
+  unsigned char now[FileLayout::kHeader];
+  const bool same = ::fstat(fd_, &st) == 0 && (uint64_t)st.st_size == size_ && st.st_mtim.tv_sec == seconds_ &&
+                    st.st_mtim.tv_nsec == nanoseconds_ && ::pread(fd_, now, sizeof(now), 0) == (ssize_t)sizeof(now) &&
+                    std::memcmp(now, header_, sizeof(now)) == 0;
+  if (!same) throw std::runtime_error("index file: written to while it was read");
 }
 
 void IndexReader::read_upper(HostIndex& ix) const {
@@ -390,6 +403,7 @@ void read_index_file(HostIndex& ix, const std::string& path) {
     }
   }
   in.read_upper(ix);
+  in.check_unchanged();
 }
 
 }  // namespace cuhnsw_amd

@@ -70,6 +70,9 @@ class IndexReader {
   void read(uint64_t offset, void* dst, size_t n, const char* what) const;
   // levels, offsets and upper links (on the host) of ix from the block behind the records; links are checked
   void read_upper(HostIndex& ix) const;
+  // Once everything has been read: throws if the file was written to meanwhile (a save goes over a file in place: what
+  // was read may be part of one index and part of another).
+  void check_unchanged() const;
   FileLayout layout;
 
  private:
@@ -78,6 +81,8 @@ class IndexReader {
   bool in_memory_ = false;
   uint64_t size_ = 0;
   uint64_t upper_at_ = 0;
+  long long seconds_ = 0, nanoseconds_ = 0;  // when the file was last written, as it was opened
+  unsigned char header_[FileLayout::kHeader];
 };
 
 // An index file opened for writing; its size is known from the start.  write() may be called from several threads

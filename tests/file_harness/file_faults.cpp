@@ -91,6 +91,7 @@ int main(int argc, char** argv) {
       write_index_file(ix, path);
       in.read(FileLayout::kHeader + bytes, buf.data(), bytes, "level-0 block");
       in.read_upper(got);
+      in.check_unchanged();
       std::printf("accepted\n");
     } else {
       return 2;

@@ -4,6 +4,7 @@ import os
 import shutil
 import subprocess
 import tempfile
+import time
 
 import pytest
 
@@ -48,3 +49,10 @@ def test_an_unfinished_save_leaves_nothing_that_loads(harness, path, mode, befor
   assert call(harness, "read", path).startswith("refused: index file:")
   call(harness, "write", path, "3")                # and the path is as good as before
   assert call(harness, "read", path) == "3 3"
+
+
+def test_a_file_saved_over_while_it_is_read_is_refused(harness, path):
+  call(harness, "write", path, "1")
+  time.sleep(0.05)                                 # (a file's time stamp moves in steps of a few milliseconds)
+  assert call(harness, "overtaken", path, "2") == "refused: index file: written to while it was read"
+  assert call(harness, "read", path) == "2 2"
