@@ -6,8 +6,11 @@
 
 #include <errno.h>
 #include <fcntl.h>
+#include <linux/magic.h>
 #include <sys/mman.h>
 #include <sys/stat.h>
+#include <sys/uio.h>
+#include <sys/vfs.h>
 #include <unistd.h>
 
 #include <algorithm>
@@ -244,20 +247,23 @@ IndexWriter::IndexWriter(const HostIndex& ix, const std::string& path)
   if (fd_ < 0) throw std::runtime_error("cannot open index file for writing: " + path);
   regular_ = ::fstat(fd_, &st) == 0 && S_ISREG(st.st_mode);
   if (readable && regular_) {
-    // Written through a mapping where the file system reserves the room beforehand (a mapping cannot report a
-    // full disk): write() holds the file's lock, pages of a mapping are filled by several threads side by side.
+    // Room first, where the file system can say that there is none: a file that is there stays as it was then.
     const bool there = (uint64_t)st.st_size >= size_ && (uint64_t)st.st_blocks * 512 >= size_;
     int rc = 0;
     if (!there) {
       do rc = ::fallocate(fd_, 0, 0, (off_t)size_);
       while (rc != 0 && errno == EINTR);
       if (rc != 0 && (errno == ENOSPC || errno == EDQUOT || errno == EFBIG)) {
-        (void)!::ftruncate(fd_, st.st_size);  // (the file that is there stays as it was)
+        (void)!::ftruncate(fd_, st.st_size);
         ::close(fd_);
         throw std::runtime_error("index file: write failed");
       }
     }
-    if (rc == 0) {
+    // In memory (tmpfs) the file is written through a mapping: write() holds the file's lock, pages of a mapping are
+    // filled by several threads side by side (364 MB over a file that is there: 7 ms, 20 to 25 with pwrite on one thread
+    // or eight).  On a disk's file system a mapping costs more than it saves (61 ms, 13 with pwrite).
+    struct statfs fs;
+    if (rc == 0 && ::fstatfs(fd_, &fs) == 0 && fs.f_type == TMPFS_MAGIC) {
       void* p = ::mmap(nullptr, size_, PROT_READ | PROT_WRITE, MAP_SHARED, fd_, 0);
       if (p != MAP_FAILED) map_ = static_cast<unsigned char*>(p);
     }
@@ -297,8 +303,23 @@ IndexWriter::~IndexWriter() {
 
 void IndexWriter::write(uint64_t offset, const void* src, size_t n) {
   if (map_) {
-    std::memcpy(map_ + offset, src, n);
-    return;
+    // The kernel makes the copy: a page that cannot be had (no room for it, the file cut off by somebody else) is an
+    // error there, where a store of this process would end it with a bus error.
+    const unsigned char* from = static_cast<const unsigned char*>(src);
+    while (n > 0) {
+      struct iovec local = {const_cast<unsigned char*>(from), n}, remote = {map_ + offset, n};
+      const ssize_t got = ::process_vm_writev(::getpid(), &local, 1, &remote, 1, 0);
+      if (got <= 0) {
+        if (got < 0 && (errno == EINTR || errno == EAGAIN)) continue;
+        if (got < 0 && (errno == ENOSYS || errno == EPERM)) break;  // (not allowed here: pwrite below)
+        throw std::runtime_error("index file: write failed");
+      }
+      from += got;
+      offset += (uint64_t)got;
+      n -= (size_t)got;
+    }
+    src = from;
+    if (n == 0) return;
   }
   if (regular_) write_at(fd_, offset, src, n);
   else write_all(fd_, src, n);

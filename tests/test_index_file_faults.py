@@ -56,3 +56,10 @@ def test_a_file_saved_over_while_it_is_read_is_refused(harness, path):
   time.sleep(0.05)                                 # (a file's time stamp moves in steps of a few milliseconds)
   assert call(harness, "overtaken", path, "2") == "refused: index file: written to while it was read"
   assert call(harness, "read", path) == "2 2"
+
+
+def test_a_file_cut_off_while_it_is_written_does_not_end_the_process(harness, path):
+  """(Through a mapping an ordinary store to what is no longer there would be a bus error.)"""
+  call(harness, "cut", path, "1")                  # refused, or written as far as it goes: but it returns
+  call(harness, "write", path, "2")
+  assert call(harness, "read", path) == "2 2"
