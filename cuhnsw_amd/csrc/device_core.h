@@ -179,12 +179,26 @@ __device__ __forceinline__ float4 load_chunk_f16(const void* base, uint64_t chun
 }
 
 // RAW = false: ordering key (1 - dot | squared L2); RAW = true: API value (-dot | squared L2)
+//
+// The distance of two finite vectors can overflow to an infinity.  An ordering key never is one: it stops at the largest
+// finite number, so that no entry of a set is ever equal to the set's padding (-inf below, +inf above), which keeps its
+// place by comparisons alone -- an infinite key would be lost among the padding and the padding's id taken for its
+// node's.  The order is the same (only a key that is exactly the largest number is no longer told from an overflow), and
+// what a search returns is computed without the stop, or freed of it (answer_key).
+constexpr float kLargestKey = 3.402823466e+38f;
+template <int DT, bool RAW>
+__device__ __forceinline__ float finish_sum(float s) {
+  if (DT == DIST_DOT) return RAW ? -s : __builtin_amdgcn_fmed3f(1.0f - s, -kLargestKey, kLargestKey);
+  return RAW ? s : fminf(s, kLargestKey);
+}
+__device__ __forceinline__ float answer_key(float key) {
+  return __builtin_fabsf(key) < kLargestKey ? key : __builtin_copysignf(INFINITY, key);
+}
 template <int DT, bool RAW>
 __device__ __forceinline__ float finish16(float ax, float ay, float az, float aw) {
   float s = (ax + ay) + (az + aw);
   s = reduce16(s);
-  if (DT == DIST_DOT) return RAW ? -s : 1.0f - s;
-  return s;
+  return finish_sum<DT, RAW>(s);
 }
 
 // The same for U rows at once (s[u]: this lane's partial sum of row u): lane `sub` < U of each group of 16 gets row sub's
@@ -220,8 +234,7 @@ __device__ __forceinline__ float finish_rows(const float* s, int sub) {
   }
   x = x + dpp_move_zero<0x104>(x);  // row_shl:4 (from the lane four above)
   x = x + dpp_move_zero<0x108>(x);  // row_shl:8
-  if (DT == DIST_DOT) return RAW ? -x : 1.0f - x;
-  return x;
+  return finish_sum<DT, RAW>(x);
 }
 
 // Query kept in registers: lane `sub` of each 16-lane group holds float4 chunks

@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
         if (r < T) {
           const uint32_t id = s.nbuf[r];
           out_id = ix.labels ? (int)ix.labels[id] : (int)id;
-          out_d = s.dbuf[r];
+          out_d = a.hnswlib_dist ? answer_key(s.dbuf[r]) : s.dbuf[r];
         }
         a.nns[(size_t)qi * a.k + r] = out_id;
         a.dists[(size_t)qi * a.k + r] = out_d;
@@ -850,7 +850,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
       if (r < T) {
         uint32_t id = s.nbuf[r];
         out_id = ix.labels ? (int)ix.labels[id] : (int)id;
-        out_d = s.dbuf[r];
+        out_d = a.hnswlib_dist ? answer_key(s.dbuf[r]) : s.dbuf[r];
       }
       a.nns[(size_t)qi * a.k + r] = out_id;
       a.dists[(size_t)qi * a.k + r] = out_d;

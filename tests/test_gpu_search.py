@@ -42,8 +42,8 @@ def _check_parity(oracle, ix, e, q, k, ef, counters=True, dup_bound=3.0):
   LDS-only visited filter; queries that meet equal keys are repeated with literal queues)
   and the literal queues alone (fast_path = 0)."""
   o_ids, o_d, o_f, o_cnt = ix.search(q, k, ef, counters=True)
-  # 2 = sorted-set pass whatever the batch size; 1 = default (a batch this small goes to the literal
-  # pass on the sorted set with ids and the LDS filter); 0 = literal queues with the exact bitmap
+  # 2 = sorted-set pass with the literal pass beside it; 1 = default (a batch this small takes the sorted-set pass
+  # alone and what that hands over afterwards); 0 = literal queues with the exact bitmap
   for fast in (2, 1, 0):
     e.set_tunable("fast_path", fast)
     e.set_tunable("lean_literal", 2 if fast else 1)   # small test indexes would otherwise choose the bitmap
@@ -566,6 +566,42 @@ def test_tiny_batches_on_long_rows(oracle, tmp_path):
           assert (stats[:, 1:] == o_cnt[:, 1:4]).all()
           handed += e.last_search_repeats
     assert handed > 0
+
+
+@pytest.mark.parametrize("dist", ["dot", "l2"])
+@pytest.mark.parametrize("d", [50, 100, 200, 300])
+def test_distances_that_overflow(oracle, tmp_path, dist, d):
+  """Finite vectors whose distances are infinite: one such row, and a quarter of them.  Searches answer as the oracle
+  does, whichever pass takes them, and a build on such data gives a valid graph."""
+  n, mult = 400, 1 / np.log(8)
+  q = gauss_mixture(30, d, seed=71)
+  q[-5:] = np.abs(q[-5:]) * np.float32(1e20)
+  q[-8:-5] = -np.abs(q[-8:-5]) * np.float32(1e20)
+  for many in (1, 100):
+    x = gauss_mixture(n, d, seed=72)
+    # (of one sign, so that a product's terms overflow to one side)
+    x[7:7 + many] = np.abs(x[7:7 + many]) * np.float32(1e20)
+    ix = oracle.OracleIndex(dist).build(x, _levels(n, mult, 73), 8, 24, 60, mult)
+    p = str(tmp_path / "o.idx")
+    ix.save(p)
+    e = _engine(tmp_path, dist_type=dist, max_m=8, max_m0=24, ef_construction=60)
+    e.load_index(p)
+    for k, ef in ((n, n), (10, 300), (250, 300), (10, 100), (n, 600), (10, 1100)):
+      _check_parity(oracle, ix, e, q, k, ef, dup_bound=None)
+    if dist == "l2":
+      e.set_tunable("hnswlib_dist", 1)
+      ids, dd, found = e.search_knn(q, n, n)
+      o_ids, o_d, o_f = ix.search(q, n, n)
+      assert (found == o_f).all() and (ids == o_ids).all() and (dd == o_d).all() and np.isinf(dd[:, -1]).any()
+    built = _engine(tmp_path, dist_type=dist, max_m=8, max_m0=24, ef_construction=60)
+    built.set_data(x)
+    built.set_random_levels(_levels(n, mult, 73))
+    built.build_graph()
+    p = str(tmp_path / "g.idx")
+    built.save_index(p)
+    iy = oracle.OracleIndex(dist).load(p)
+    assert iy.validate() == 0
+    _check_parity(oracle, iy, built, q, 10, 300, dup_bound=None)
 
 
 def test_errors(tmp_path):
