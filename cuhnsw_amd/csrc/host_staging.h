@@ -22,8 +22,10 @@ namespace cuhnsw_amd {
 #define HIP_CHECK(expr)                                                                              \
   do {                                                                                               \
     hipError_t err_ = (expr);                                                                        \
-    if (err_ != hipSuccess)                                                                          \
+    if (err_ != hipSuccess) {                                                                        \
+      (void)hipGetLastError(); /* reported here, not by the next launch of a later call */           \
       throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(err_) + " at " #expr); \
+    }                                                                                                \
   } while (0)
 
 // threads worth using for `bytes` of host-side bulk work in steps of `block`

@@ -19,6 +19,11 @@ def _engine(tmp_path, **opt):
   return e
 
 
+def capi_lib():
+  from cuhnsw_amd import capi
+  return capi.load()
+
+
 def _levels(n, mult, seed):
   rng = np.random.default_rng(seed)
   return (-np.log(np.maximum(rng.uniform(size=n), 1e-10)) * mult).astype(np.int32)
@@ -611,6 +616,20 @@ def test_errors(tmp_path):
     e.search_knn(np.zeros((1, 4), np.float32), 1, 1)
   with pytest.raises(RuntimeError, match="set_random_levels first"):
     e.build_graph()
+
+
+def _ask_for_too_much(e):
+  import ctypes
+  small = np.zeros(4, np.float32)
+  rc = capi_lib().cuhnsw_set_data(e._h, small.ctypes.data_as(ctypes.c_void_p), 100, 2_000_000_000)   # 800 GB
+  assert rc != 0 and b"memory" in capi_lib().cuhnsw_last_error(e._h)
+
+
+def test_an_error_is_reported_once(tmp_path):
+  """Not again by the first launch of a call that has nothing to do with it."""
+  e, other = _engine(tmp_path), _engine(tmp_path)
+  _ask_for_too_much(e)
+  other.set_data(gauss_mixture(300, 20, seed=81))
 
 
 @pytest.mark.parametrize("name,n,d,dist,max_m,max_m0,kind", [CASES[0], CASES[2], CASES[4], CASES[6]],
