@@ -351,15 +351,21 @@ class Engine {
 
   void set_data(const float* data, int n, int d) {
     if (!data || n <= 0 || d <= 0) throw std::runtime_error("set_data: empty data");
+    // (a call that fails leaves nothing behind that a later one could mistake for data or a graph)
+    have_data = have_levels = have_graph = false;
     host = HostIndex();
     host.N = n;
     host.D = d;
-    have_levels = have_graph = false;
     forget_search_history();
     pool_slots = 0;  // the slot pool is sized by N: rebuild it lazily
     pool = SlotPool{};
-    if (has_device) upload_vectors(data);
-    else host.vectors.assign(data, data + (size_t)n * d);  // without a GPU only the host-side calls remain usable
+    try {
+      if (has_device) upload_vectors(data);
+      else host.vectors.assign(data, data + (size_t)n * d);  // without a GPU only the host-side calls remain usable
+    } catch (...) {
+      host = HostIndex();
+      throw;
+    }
     have_data = true;
   }
 
@@ -375,11 +381,13 @@ class Engine {
   void set_random_levels(const int* levels, int n) {
     if (!have_data) throw std::runtime_error("set_random_levels: call set_data first");
     if (n != host.N) throw std::runtime_error("set_random_levels: length differs from the number of data rows");
+    if (std::any_of(levels, levels + n, [](int l) { return l < 0; })) throw std::runtime_error("levels must be non-negative");
     host.max_m = opt.max_m;
     host.max_m0 = opt.max_m0;
     host.M = opt.max_m;
     host.ef_construction = opt.ef_construction;
     host.mult = opt.level_mult;
+    have_levels = have_graph = false;
     host.set_levels(levels, n);
     if (has_device) host.layout_upper();
     else host.layout_links();
@@ -387,9 +395,8 @@ class Engine {
     host.labels.clear();
     host.deleted.clear();  // a graph built anew holds every element
     host.n_deleted = 0;
-    have_levels = true;
-    have_graph = false;
     if (has_device) upload_structure();
+    have_levels = true;
   }
 
   // What a search learns about an index (how many of its queries tie, whether the two passes ran side by
@@ -673,6 +680,7 @@ class Engine {
     auto t0 = std::chrono::steady_clock::now();
     const int q = qr();
     const int ns = build_literal ? 0 : key_slots(opt.ef_construction);
+    have_graph = false;
     if (dist_type == DIST_DOT) build_qr<DIST_DOT>(q, ns);
     else build_qr<DIST_L2>(q, ns);
     workspace.end();
@@ -719,8 +727,7 @@ class Engine {
       write_index_file(host, path);
       return;
     }
-    IndexWriter out(host, path);
-    const size_t rec = (size_t)out.layout.record;
+    const size_t rec = (size_t)FileLayout((uint64_t)host.max_m, (uint64_t)host.max_m0, (uint64_t)host.D).record;
     const size_t piece_rows = std::max<size_t>(1, std::min<size_t>((size_t)host.N, kPiece / rec));
     workspace.begin();
     const auto p_packed = workspace.part<unsigned char>(piece_rows * rec);
@@ -732,6 +739,7 @@ class Engine {
     if (!up.empty()) HIP_CHECK(hipMemcpyAsync(up.data(), d_linksU.p, up.size() * 4, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     const DevIndex ix = dev_index();
+    IndexWriter out(host, path);  // (after everything that may find no memory: the file that is there goes with it)
     for (size_t first = 0; first < (size_t)host.N; first += piece_rows) {
       const size_t rows = std::min(piece_rows, (size_t)host.N - first);
       hipLaunchKernelGGL(pack_records_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, ix, (int)first, (int)rows,
@@ -807,8 +815,8 @@ class Engine {
       HIP_CHECK(hipMemcpyAsync(fresh.deleted.data(), marks, n, hipMemcpyDeviceToHost, stream));
       HIP_CHECK(hipStreamSynchronize(stream));
     }
+    have_data = have_levels = have_graph = false;  // until all of it is there
     host = std::move(fresh);
-    have_data = have_levels = have_graph = true;
     forget_search_history();
     reserve_vectors();
     upload_structure();
@@ -824,6 +832,7 @@ class Engine {
     std::vector<uint32_t>().swap(host.linksU);
     pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
     pool = SlotPool{};
+    have_data = have_levels = have_graph = true;
     prepare_search_buffers();
   }
 };

@@ -632,6 +632,29 @@ def test_an_error_is_reported_once(tmp_path):
   other.set_data(gauss_mixture(300, 20, seed=81))
 
 
+def test_calls_that_find_no_memory_leave_nothing_to_run_on(tmp_path):
+  """After a set_data that could not have its memory there are no vectors: the calls that would run on them refuse."""
+  e = _engine(tmp_path)
+  x = gauss_mixture(300, 20, seed=81)
+  e.set_data(x)
+  e.set_random_levels(np.zeros(300, np.int32))
+  e.build_graph()
+  e.search_knn(x[:3], 2, 10)
+  _ask_for_too_much(e)
+  with pytest.raises(RuntimeError, match="set_data first"):
+    e.set_random_levels(np.zeros(100, np.int32))
+  with pytest.raises(RuntimeError, match="set_data"):
+    e.build_graph()
+  with pytest.raises(RuntimeError, match="dimension"):
+    e.search_knn(x[:3], 2, 10)
+  assert e.num_data == 0
+  e.set_data(x)
+  e.set_random_levels(np.zeros(300, np.int32))
+  e.build_graph()
+  ids, _, _ = e.search_knn(x[:3], 1, 50)
+  assert list(ids[:, 0]) == [0, 1, 2]
+
+
 @pytest.mark.parametrize("name,n,d,dist,max_m,max_m0,kind", [CASES[0], CASES[2], CASES[4], CASES[6]],
                          ids=[CASES[i][0] for i in (0, 2, 4, 6)])
 def test_reverse_cand_search_parity(oracle, tmp_path, name, n, d, dist, max_m, max_m0, kind):

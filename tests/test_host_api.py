@@ -136,3 +136,15 @@ def test_datasets_are_seeded_and_shaped():
   assert (r == c2).all() and qr.shape == (40, 50) and rs["topk"] == 100
   np.testing.assert_allclose(np.linalg.norm(qr, axis=1), 1.0, rtol=1e-5)
   assert abs(float(qr.mean())) < 0.05
+
+
+def test_levels_that_are_refused_leave_the_index_as_it_was(tmp_path):
+  from test_index_file import expected_bytes
+  p, q = str(tmp_path / "a.idx"), str(tmp_path / "b.idx")
+  open(p, "wb").write(expected_bytes())
+  e = capi.Engine()
+  e.load_index(p)
+  with pytest.raises(RuntimeError, match="non-negative"):
+    e.set_random_levels(np.array([0, 2, -1], np.int32))
+  e.save_index(q)
+  assert open(q, "rb").read() == expected_bytes()
