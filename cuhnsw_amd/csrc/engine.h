@@ -127,15 +127,23 @@ class Workspace {
   size_t bytes_from(Part<T> p) const {
     return used_ - p.offset;
   }
-  // more than this is not kept (the largest builds need a tenth of the GPU's memory, which a search may want)
-  void end() {
-    if (memory_.n > kKept) memory_.release();
+  // The call that needed it is over: what the next one may use stays.  (More than kKept does not: the largest builds need
+  // a tenth of the GPU's memory, which a search may want.  Nor does what goes beyond the process's bound, nor anything
+  // with keep = false.)
+  void end(bool keep) {
+    if (keep && memory_.n == counted_) return;
+    kept_device_memory.give_back(counted_);
+    counted_ = 0;
+    if (keep && memory_.n <= kKept && kept_device_memory.take(memory_.n)) counted_ = memory_.n;
+    else memory_.release();
   }
+  ~Workspace() { kept_device_memory.give_back(counted_); }
 
  private:
   static constexpr size_t kKept = (size_t)2 << 30;
   DevBuf<unsigned char> memory_;
   size_t used_ = 0;
+  size_t counted_ = 0;  // bytes of it that count as kept
 };
 
 class Engine {
@@ -224,6 +232,16 @@ class Engine {
   DevBuf<int> d_nns, d_found;
   HostStaging staging;
   Workspace workspace;
+  int keep_workspace = 1;  // 0: neither stays allocated after the call that needed it
+  struct CallEnd {         // (also where the call ends with an exception)
+    Engine& e;
+    explicit CallEnd(Engine& engine) : e(engine) {}
+    ~CallEnd() { e.give_back_workspace(); }
+  };
+  void give_back_workspace() {
+    workspace.end(keep_workspace != 0);
+    staging.end(keep_workspace != 0);
+  }
   // pinned memory that small batches are read from and answered into (kernels address it)
   static constexpr size_t kDirectQueries = (size_t)64 << 10, kDirectAnswers = (size_t)1 << 20;
   unsigned char* h_io = nullptr;
@@ -351,6 +369,7 @@ class Engine {
 
   void set_data(const float* data, int n, int d) {
     if (!data || n <= 0 || d <= 0) throw std::runtime_error("set_data: empty data");
+    const CallEnd at_end(*this);
     // (a call that fails leaves nothing behind that a later one could mistake for data or a graph)
     have_data = have_levels = have_graph = false;
     host = HostIndex();
@@ -675,6 +694,7 @@ class Engine {
   void build_graph() {
     need_device();
     if (!have_data || !have_levels) throw std::runtime_error("build_graph: call set_data and set_random_levels first");
+    const CallEnd at_end(*this);
     HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 4 * sizeof(int), stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     auto t0 = std::chrono::steady_clock::now();
@@ -683,7 +703,6 @@ class Engine {
     have_graph = false;
     if (dist_type == DIST_DOT) build_qr<DIST_DOT>(q, ns);
     else build_qr<DIST_L2>(q, ns);
-    workspace.end();
     last_build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     have_graph = true;
     forget_search_history();
@@ -729,6 +748,7 @@ class Engine {
     }
     const size_t rec = (size_t)FileLayout((uint64_t)host.max_m, (uint64_t)host.max_m0, (uint64_t)host.D).record;
     const size_t piece_rows = std::max<size_t>(1, std::min<size_t>((size_t)host.N, kPiece / rec));
+    const CallEnd at_end(*this);
     workspace.begin();
     const auto p_packed = workspace.part<unsigned char>(piece_rows * rec);
     workspace.reserve();
@@ -753,7 +773,6 @@ class Engine {
                     });
     }
     HIP_CHECK(hipStreamSynchronize(stream));
-    workspace.end();
     if (!out.parallel()) out.write_upper(host, up.data());
     out.finish();
   }
@@ -779,6 +798,7 @@ class Engine {
     }
     IndexReader in(fresh, path);
     const size_t rec = (size_t)in.layout.record, n = (size_t)fresh.N;
+    const CallEnd at_end(*this);
     workspace.begin();
     const auto p_raw = workspace.part<unsigned char>(n * rec);
     const auto p_marks = workspace.part<unsigned char>(n);
@@ -828,7 +848,6 @@ class Engine {
       HIP_CHECK(hipMemcpyAsync(d_linksU.p, host.linksU.data(), host.linksU.size() * 4, hipMemcpyHostToDevice, stream));
     if (host.n_deleted > 0) upload_marks();
     HIP_CHECK(hipStreamSynchronize(stream));
-    workspace.end();
     std::vector<uint32_t>().swap(host.linksU);
     pool_slots = 0;  // N may have changed: rebuild the slot pool lazily
     pool = SlotPool{};

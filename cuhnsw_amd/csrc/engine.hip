@@ -162,6 +162,10 @@ int cuhnsw_set_tunable(cuhnsw_engine* e, const char* name, double value) {
   else if (n == "literal_spin_limit") e->impl.spin_limit_override = (int)value;
   else if (n == "literal_per_cu") e->impl.side_per_cu = std::max(0, std::min(8, (int)value));
   else if (n == "spill_cap") e->impl.spill_cap = (int)value;
+  else if (n == "keep_workspace") {
+    e->impl.keep_workspace = value != 0.0;
+    e->impl.give_back_workspace();
+  }
   else if (n == "keep_link_keys") e->impl.keep_link_keys = value != 0.0;
   else if (n == "build_counters") e->impl.count_build_work = value != 0.0;
   else if (n == "tight_rows") {

@@ -3,12 +3,13 @@
 // A copy from pageable memory runs at 29 GB/s here and one thread fills or empties fresh pages at 3 to 6 GB/s, while
 // the copy engine moves 57 GB/s out of pinned memory.  So the data pass through a few pinned blocks: each of several
 // threads takes every k-th block of the transfer and fills one of its two blocks while the other one is on its way.
-// The blocks belong to an engine and are given back with it.
+// The blocks belong to an engine and are given back with it at the latest.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <sched.h>
 
 #include <algorithm>
+#include <atomic>
 #include <exception>
 #include <mutex>
 #include <stdexcept>
@@ -27,6 +28,25 @@ namespace cuhnsw_amd {
       throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(err_) + " at " #expr); \
     }                                                                                                \
   } while (0)
+
+// What engines keep between calls so that the next one finds it allocated is bounded for the process as a whole: an
+// engine that would go beyond keeps nothing and allocates anew each time.
+class KeptMemory {
+ public:
+  explicit constexpr KeptMemory(size_t limit) : limit_(limit) {}
+  bool take(size_t n) {
+    if (total_.fetch_add(n) + n <= limit_) return true;
+    total_ -= n;
+    return false;
+  }
+  void give_back(size_t n) { total_ -= n; }
+
+ private:
+  const size_t limit_;
+  std::atomic<size_t> total_{0};
+};
+inline KeptMemory kept_device_memory((size_t)4 << 30);  // (of 288 GB, on whichever GPUs)
+inline KeptMemory kept_pinned_memory((size_t)256 << 20);
 
 // threads worth using for `bytes` of host-side bulk work in steps of `block`
 inline int host_threads(size_t bytes, size_t block) {
@@ -89,6 +109,22 @@ class HostStaging {
     if (on_device && !device_) HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&device_), block_ * kBlocks));
   }
   size_t block() const { return block_; }
+  // The call that needed the blocks is over: they stay for the next one, within the process's bounds.  (keep = false:
+  // they do not.)
+  void end(bool keep) {
+    if (!host_) return;
+    const size_t pinned = block_ * kBlocks, device = device_ ? pinned : 0;
+    if (keep && pinned == counted_pinned_ && device == counted_device_) return;
+    uncount();
+    if (keep && kept_pinned_memory.take(pinned)) {
+      counted_pinned_ = pinned;
+      if (device == 0 || kept_device_memory.take(device)) {
+        counted_device_ = device;
+        return;
+      }
+    }
+    release();
+  }
 
   // Host to device, `block` bytes at a time: fill(to, at, n) puts bytes [at, at + n) of the transfer into pinned memory;
   // they are copied to target(at, n), or to the block's counterpart in device memory where that is null; after(there,
@@ -165,7 +201,13 @@ class HostStaging {
       throw;
     }
   }
+  void uncount() {
+    kept_pinned_memory.give_back(counted_pinned_);
+    kept_device_memory.give_back(counted_device_);
+    counted_pinned_ = counted_device_ = 0;
+  }
   void release() {
+    uncount();
     for (hipEvent_t& e : event_) {
       if (e) (void)hipEventDestroy(e);
       e = nullptr;
@@ -179,6 +221,7 @@ class HostStaging {
   unsigned char* host_ = nullptr;
   unsigned char* device_ = nullptr;
   size_t block_ = 0;
+  size_t counted_pinned_ = 0, counted_device_ = 0;
   hipEvent_t event_[kBlocks] = {};
 };
 

@@ -209,6 +209,10 @@ int cuhnsw_trails_available(cuhnsw_engine* e);
  *                   it leaves and the host answers the remaining queries afterwards (-1 = no bound in
  *                   polls: it leaves when the first pass has not started within 2 ms or stalls for
  *                   100 ms; see cuhnsw_literal_fallbacks for what follows)
+ *   "keep_workspace" 1 (default) = the device and pinned memory that set_data, build_graph, save_index and
+ *                   load_index work in (up to 2 GB and up to 32 MB of each) stays with the engine for the next of
+ *                   these calls, up to 4 GB of device and 256 MB of pinned memory for all engines of a process;
+ *                   0 = it is given back, what is held now at once
  *   "build_counters" 1 = count the work of the next builds on the device (cuhnsw_last_build_counters)
  *   "keep_link_keys" 1 = keep the keys stored with the level-0 links after build_graph for
  *                   cuhnsw_debug_link_keys0
