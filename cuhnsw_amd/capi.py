@@ -19,7 +19,7 @@ SYMBOLS = [
     "cuhnsw_search_knn_device_noalloc", "cuhnsw_last_build_dropped_links", "cuhnsw_debug_link_keys0",
     "cuhnsw_last_build_counters", "cuhnsw_debug_gather_probe", "cuhnsw_last_search_trails",
     "cuhnsw_last_search_side_by_side", "cuhnsw_literal_fallbacks", "cuhnsw_trails_available",
-    "cuhnsw_num_deleted",
+    "cuhnsw_num_deleted", "cuhnsw_search_knn_taking",
 ]
 
 _lib = None
@@ -46,6 +46,7 @@ def load():
   l.cuhnsw_save_index.argtypes = [vp, ctypes.c_char_p]
   l.cuhnsw_load_index.argtypes = [vp, ctypes.c_char_p]
   l.cuhnsw_search_knn.argtypes = [vp, vp, ci, ci, ci, vp, vp, vp]
+  l.cuhnsw_search_knn_taking.argtypes = [vp, vp, ci, ci, ci, ci, vp, vp, vp, vp, vp]
   l.cuhnsw_search_knn_device.argtypes = [vp, vp, ci, ci, ci, vp, vp, vp, vp, ctypes.POINTER(ctypes.c_float)]
   l.cuhnsw_search_knn_device_noalloc.argtypes = [vp, vp, ci, ci, ci, vp, vp, vp, ctypes.POINTER(ctypes.c_float)]
   l.cuhnsw_last_build_dropped_links.argtypes = [vp]

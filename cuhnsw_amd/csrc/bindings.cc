@@ -71,12 +71,13 @@ class CuHNSWBind {
     int* out_nns = _nns.mutable_data(0);
     float* out_distances = _distances.mutable_data(0);
     int* out_found = _found_cnt.mutable_data(0);
-    int rc;
-    {
-      // plain pointers from here on: other Python threads may run while the GPU searches
-      py::gil_scoped_release release;
-      rc = cuhnsw_search_knn(obj_, q, num_queries, topk, ef_search, out_nns, out_distances, out_found);
-    }
+    // Other Python threads may run while the GPU searches: from the moment the engine has read the queries, which are the
+    // caller's own memory, to the end of the call.
+    PyThreadState* released = nullptr;
+    const int rc = cuhnsw_search_knn_taking(
+        obj_, q, num_queries, dims, topk, ef_search, out_nns, out_distances, out_found,
+        [](void* p) { *static_cast<PyThreadState**>(p) = PyEval_SaveThread(); }, &released);
+    if (released) PyEval_RestoreThread(released);
     Check(rc);
   }
   // not in the reference: engine facts and tuning knobs

@@ -244,6 +244,7 @@ class Engine {
   }
   // pinned memory that small batches are read from and answered into (kernels address it)
   static constexpr size_t kDirectQueries = (size_t)64 << 10, kDirectAnswers = (size_t)1 << 20;
+  static constexpr size_t kQueryBlock = (size_t)512 << 10, kQueryThreadsFrom = (size_t)16 << 20;
   unsigned char* h_io = nullptr;
   size_t h_io_bytes = 0;
   void reserve_io(size_t bytes) {
@@ -638,7 +639,9 @@ class Engine {
     else launch_search_qr<DIST_L2>(q, ns, ix, a, ms);
   }
 
-  void search_host(const float* q, int nq, int k, int ef, int* nns, float* dists, int* found) {
+  // taken() is called once the queries have been read for the last time
+  template <typename Taken>
+  void search_host(const float* q, int nq, int k, int ef, int* nns, float* dists, int* found, Taken&& taken) {
     need_device();
     if (nq <= 0) return;
     if (!q || !nns || !dists || !found) throw std::runtime_error("search_knn: null argument");
@@ -655,9 +658,19 @@ class Engine {
       q_there = reinterpret_cast<const float*>(h_io);
     } else {
       d_q.reserve((size_t)nq * host.D);
-      HIP_CHECK(hipMemcpyAsync(d_q.p, q, q_bytes, hipMemcpyHostToDevice, stream));
       q_there = d_q.p;
+      if (staging.block() > 0) {
+        const unsigned char* src = reinterpret_cast<const unsigned char*>(q);
+        unsigned char* dst = reinterpret_cast<unsigned char*>(d_q.p);
+        staging.send(stream, q_bytes, kQueryBlock, [&](unsigned char* to, size_t at, size_t n) { std::memcpy(to, src + at, n); },
+                     [&](size_t at, size_t) { return dst + at; }, [](unsigned char*, size_t, size_t) {}, [] {},
+                     q_bytes < kQueryThreadsFrom ? 1 : HostStaging::kBlocks / 2);
+      } else {  // (no pinned blocks are kept: one copy out of the caller's memory, waited for)
+        HIP_CHECK(hipMemcpyAsync(d_q.p, q, q_bytes, hipMemcpyHostToDevice, stream));
+        HIP_CHECK(hipStreamSynchronize(stream));
+      }
     }
+    taken();
     if (direct_out) {
       search_device(q_there, nq, k, ef, out, reinterpret_cast<float*>(out + (size_t)nq * k), out + (size_t)nq * k * 2, nullptr, nullptr);
       std::memcpy(nns, out, (size_t)nq * k * 4);

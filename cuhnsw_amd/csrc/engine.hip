@@ -38,9 +38,7 @@ namespace {
 thread_local std::string g_create_error;
 
 template <typename F>
-int guarded(cuhnsw_engine* e, F&& f) {
-  if (!e) return -1;
-  std::lock_guard<std::mutex> lock(e->mutex);
+int locked(cuhnsw_engine* e, F&& f) {  // (the engine's lock is held)
   try {
     e->impl.err.clear();
     f(e->impl);
@@ -52,6 +50,12 @@ int guarded(cuhnsw_engine* e, F&& f) {
     e->impl.err = "unknown error";
     return -1;
   }
+}
+template <typename F>
+int guarded(cuhnsw_engine* e, F&& f) {
+  if (!e) return -1;
+  std::lock_guard<std::mutex> lock(e->mutex);
+  return locked(e, f);
 }
 }  // namespace
 
@@ -94,7 +98,32 @@ int cuhnsw_load_index(cuhnsw_engine* e, const char* fpath) {
 }
 int cuhnsw_search_knn(cuhnsw_engine* e, const float* qdata, int num_queries, int topk, int ef_search, int* nns,
                       float* distances, int* found_cnt) {
-  return guarded(e, [&](Engine& g) { g.search_host(qdata, num_queries, topk, ef_search, nns, distances, found_cnt); });
+  return guarded(e, [&](Engine& g) { g.search_host(qdata, num_queries, topk, ef_search, nns, distances, found_cnt, [] {}); });
+}
+int cuhnsw_search_knn_taking(cuhnsw_engine* e, const float* qdata, int num_queries, int num_dims, int topk, int ef_search,
+                             int* nns, float* distances, int* found_cnt, void (*taken)(void*), void* arg) {
+  if (!e || !taken) return -1;
+  // (an engine that is at work is not waited for with the queries still in the caller's memory)
+  std::vector<float> own;
+  bool told = false;
+  std::unique_lock<std::mutex> lock(e->mutex, std::try_to_lock);
+  if (!lock.owns_lock()) {
+    try {
+      if (qdata && num_queries > 0 && num_dims > 0) own.assign(qdata, qdata + (size_t)num_queries * num_dims);
+    } catch (const std::exception&) {
+      return -1;
+    }
+    if (qdata) qdata = own.data();
+    taken(arg);
+    told = true;
+    lock.lock();
+  }
+  return locked(e, [&](Engine& g) {
+    if (num_dims != g.host.D) throw std::runtime_error("query dimension differs from the index dimension");
+    g.search_host(qdata, num_queries, topk, ef_search, nns, distances, found_cnt, [&] {
+      if (!told) taken(arg);
+    });
+  });
 }
 int cuhnsw_search_knn_device(cuhnsw_engine* e, const float* d_qdata, int num_queries, int topk, int ef_search, int* d_nns,
                              float* d_distances, int* d_found_cnt, int* d_stats, float* kernel_ms) {

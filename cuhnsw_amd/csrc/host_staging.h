@@ -130,10 +130,11 @@ class HostStaging {
   // they are copied to target(at, n), or to the block's counterpart in device memory where that is null; after(there,
   // at, n) may launch work on them.  `meanwhile` runs on the calling thread.  Everything is on `stream` on return.
   template <typename Fill, typename Target, typename After, typename Meanwhile>
-  void send(hipStream_t stream, size_t total, size_t block, Fill&& fill, Target&& target, After&& after, Meanwhile&& meanwhile) {
+  void send(hipStream_t stream, size_t total, size_t block, Fill&& fill, Target&& target, After&& after, Meanwhile&& meanwhile,
+            int most_threads = kBlocks / 2) {
     int device = 0;
     HIP_CHECK(hipGetDevice(&device));
-    const int threads = std::min(host_threads(total, block), kBlocks / 2);
+    const int threads = std::min(host_threads(total, block), most_threads);
     run(threads, total, stream, [&](int t) {
       HIP_CHECK(hipSetDevice(device));
       int use = 0;

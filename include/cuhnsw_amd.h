@@ -84,6 +84,13 @@ int cuhnsw_load_index(cuhnsw_engine* e, const char* fpath);
  * (cuhnsw/pyhnsw.py:80 does the same before the call). */
 int cuhnsw_search_knn(cuhnsw_engine* e, const float* qdata, int num_queries, int topk, int ef_search,
                       int* nns, float* distances, int* found_cnt);
+/* The same for callers whose other threads may reuse the memory of the queries while the search is under way (a
+ * language binding that gives up its interpreter's lock meanwhile; the reference's binding keeps it throughout,
+ * cuhnsw/bindings.cc:18-71): taken(arg) is called, on this thread and at most once, when the queries have been read for
+ * the last time -- before the search, and before waiting for a call of another thread on the same engine.  It is not
+ * called where the arguments are refused first.  num_dims is the length of a query and must be the index's. */
+int cuhnsw_search_knn_taking(cuhnsw_engine* e, const float* qdata, int num_queries, int num_dims, int topk, int ef_search,
+                             int* nns, float* distances, int* found_cnt, void (*taken)(void*), void* arg);
 
 /* Same search with queries and outputs already in device memory (HBM); nothing
  * is copied.  Counterpart of the kernel launch inside CuHNSW::SearchGraph

@@ -618,6 +618,66 @@ def test_errors(tmp_path):
     e.build_graph()
 
 
+@pytest.mark.parametrize("nq,keep", [(3, 1), (700, 1), (60_000, 1), (700, 0)],
+                         ids=["read in place", "one thread", "several threads", "no pinned blocks"])
+def test_queries_may_be_reused_once_they_are_taken(tmp_path, nq, keep):
+  """The caller's memory is overwritten the moment the engine says that it has read it; so is that of a second search,
+  which finds the engine at work and says so before it waits."""
+  import ctypes
+  import threading
+  n, d, k = 3000, 72, 5
+  x = gauss_mixture(n, d, seed=95)
+  e = _engine(tmp_path, max_m=8, max_m0=16, ef_construction=40)
+  e.set_data(x)
+  e.set_random_levels(_levels(n, 0.4, 96))
+  e.build_graph()
+  e.set_tunable("keep_workspace", keep)
+  lib, vp = capi_lib(), ctypes.c_void_p
+  told_type = ctypes.CFUNCTYPE(None, vp)
+
+  def search(q, told):
+    out = (np.empty((nq, k), np.int32), np.empty((nq, k), np.float32), np.empty(nq, np.int32))
+    mine = q.copy()
+    calls = []
+
+    def taken(_):
+      calls.append(1)
+      mine[:] = np.nan
+      told()
+
+    keep_alive = told_type(taken)
+    rc = lib.cuhnsw_search_knn_taking(e._h, mine.ctypes.data_as(vp), nq, d, k, 50, *[o.ctypes.data_as(vp) for o in out],
+                                      ctypes.cast(keep_alive, vp), None)
+    assert rc == 0 and calls == [1]
+    return out
+
+  qa, qb = gauss_mixture(nq, d, seed=97), gauss_mixture(nq, d, seed=98)
+  want_a, want_b = e.search_knn(qa, k, 50), e.search_knn(qb, k, 50)
+  second = []
+  waiting = threading.Event()
+
+  def other():
+    second.append(search(qb, waiting.set))
+
+  t = threading.Thread(target=other)
+
+  def start_second():   # (the first search holds the engine: the second one tells before it gets it)
+    t.start()
+    assert waiting.wait(30)
+
+  got_a = search(qa, start_second)
+  t.join(30)
+  for got, want in ((got_a, want_a), (second[0], want_b)):
+    for g, w in zip(got, want):
+      np.testing.assert_array_equal(g, w)
+  # refused before anything is taken
+  calls = []
+  none = told_type(lambda _: calls.append(1))
+  assert lib.cuhnsw_search_knn_taking(e._h, qa.ctypes.data_as(vp), 1, d + 1, k, 50, qa.ctypes.data_as(vp), qa.ctypes.data_as(vp),
+                                      qa.ctypes.data_as(vp), ctypes.cast(none, vp), None) != 0
+  assert calls == [] and b"dimension" in lib.cuhnsw_last_error(e._h)
+
+
 def _ask_for_too_much(e):
   import ctypes
   small = np.zeros(4, np.float32)
