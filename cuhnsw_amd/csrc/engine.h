@@ -242,9 +242,15 @@ class Engine {
     workspace.end(keep_workspace != 0);
     staging.end(keep_workspace != 0);
   }
-  // pinned memory that small batches are read from and answered into (kernels address it)
-  static constexpr size_t kDirectQueries = (size_t)64 << 10, kDirectAnswers = (size_t)1 << 20;
-  static constexpr size_t kQueryBlock = (size_t)512 << 10, kQueryThreadsFrom = (size_t)16 << 20;
+  // Pinned memory that small batches are read from and answered into (kernels address it).  How small was measured on
+  // searches of next to no work (ef 8, 20 000 rows), through copies -> directly:
+  //   queries 128 KB 84 -> 72 us (128 x 256), 256 KB 95 -> 80 us (128 x 512), 125 -> 113 us (960 x 66), 750 KB 261 -> 229 us
+  //           (32 x 6 000), 1 MB 171 -> 147 us (960 x 266), 194 -> 177 us (128 x 2 000);
+  //   answers 0.1 MB 272 -> 196 us (128 x topk 100), 0.5 MB 285 -> 240 us, 1 MB 450 -> 395 us, 2 MB 532 -> 456 us,
+  //           3.9 MB 728 -> 633 us.
+  // Beyond, the copies run at the bus's rate while a search's own reads and writes wait for it.
+  static constexpr size_t kDirectQueries = (size_t)1 << 20, kDirectAnswers = (size_t)4 << 20;
+  static constexpr size_t kQueryBlock = (size_t)512 << 10;
   unsigned char* h_io = nullptr;
   size_t h_io_bytes = 0;
   void reserve_io(size_t bytes) {
@@ -662,9 +668,13 @@ class Engine {
       if (staging.block() > 0) {
         const unsigned char* src = reinterpret_cast<const unsigned char*>(q);
         unsigned char* dst = reinterpret_cast<unsigned char*>(d_q.p);
-        staging.send(stream, q_bytes, kQueryBlock, [&](unsigned char* to, size_t at, size_t n) { std::memcpy(to, src + at, n); },
+        // (each copy is 15 us, whatever its size; threads pay from a megabyte each on.  10 000 x 128: 0.60 ms, 0.63 on one
+        // thread, 0.61 to 0.67 in blocks of 1 or 0.5 MB; out of the caller's own memory in one copy that is waited for
+        // 0.63; 100 000 x 128: 3.46, 3.89, 3.77 to 4.45 and 3.98 ms)
+        const bool small = q_bytes <= staging.block();
+        staging.send(stream, q_bytes, small ? kQueryBlock : staging.block(), [&](unsigned char* to, size_t at, size_t n) { std::memcpy(to, src + at, n); },
                      [&](size_t at, size_t) { return dst + at; }, [](unsigned char*, size_t, size_t) {}, [] {},
-                     q_bytes < kQueryThreadsFrom ? 1 : HostStaging::kBlocks / 2);
+                     small ? 1 : (int)std::min<size_t>(q_bytes >> 20, HostStaging::kBlocks / 2), true);
       } else {  // (no pinned blocks are kept: one copy out of the caller's memory, waited for)
         HIP_CHECK(hipMemcpyAsync(d_q.p, q, q_bytes, hipMemcpyHostToDevice, stream));
         HIP_CHECK(hipStreamSynchronize(stream));

@@ -128,10 +128,11 @@ class HostStaging {
 
   // Host to device, `block` bytes at a time: fill(to, at, n) puts bytes [at, at + n) of the transfer into pinned memory;
   // they are copied to target(at, n), or to the block's counterpart in device memory where that is null; after(there,
-  // at, n) may launch work on them.  `meanwhile` runs on the calling thread.  Everything is on `stream` on return.
+  // at, n) may launch work on them.  `meanwhile` runs on the calling thread, which with caller_too is one of the threads
+  // as well.  Everything is on `stream` on return.
   template <typename Fill, typename Target, typename After, typename Meanwhile>
   void send(hipStream_t stream, size_t total, size_t block, Fill&& fill, Target&& target, After&& after, Meanwhile&& meanwhile,
-            int most_threads = kBlocks / 2) {
+            int most_threads = kBlocks / 2, bool caller_too = false) {
     int device = 0;
     HIP_CHECK(hipGetDevice(&device));
     const int threads = std::min(host_threads(total, block), most_threads);
@@ -150,7 +151,7 @@ class HostStaging {
         after(to, at, n);
         HIP_CHECK(hipEventRecord(event_[slot], stream));
       }
-    }, meanwhile);
+    }, meanwhile, caller_too);
   }
   template <typename Fill, typename Target, typename After>
   void send(hipStream_t stream, size_t total, size_t block, Fill&& fill, Target&& target, After&& after) {
@@ -189,11 +190,16 @@ class HostStaging {
   // (one thread's worth of work is done by the calling thread; after a failure nothing may still be on its way
   // through the blocks)
   template <typename Body, typename Meanwhile>
-  void run(int threads, size_t total, hipStream_t stream, Body&& body, Meanwhile&& meanwhile) {
+  void run(int threads, size_t total, hipStream_t stream, Body&& body, Meanwhile&& meanwhile, bool caller_too = false) {
     try {
       if (threads <= 1) {
         if (total > 0) body(0);
         meanwhile();
+      } else if (caller_too) {
+        run_on_threads(threads - 1, [&](int t) { body(t + 1); }, [&] {
+          body(0);
+          meanwhile();
+        });
       } else {
         run_on_threads(threads, body, meanwhile);
       }

@@ -618,7 +618,7 @@ def test_errors(tmp_path):
     e.build_graph()
 
 
-@pytest.mark.parametrize("nq,keep", [(3, 1), (700, 1), (60_000, 1), (700, 0)],
+@pytest.mark.parametrize("nq,keep", [(3, 1), (5000, 1), (60_000, 1), (5000, 0)],
                          ids=["read in place", "one thread", "several threads", "no pinned blocks"])
 def test_queries_may_be_reused_once_they_are_taken(tmp_path, nq, keep):
   """The caller's memory is overwritten the moment the engine says that it has read it; so is that of a second search,
