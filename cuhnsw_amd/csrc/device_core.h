@@ -1882,6 +1882,20 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
   // passes as it did there.
   int trail_at = 0;
   bool from_trail = false;
+  // 64 of its records at a time, lane by lane: a hop has two or three, and fetched for each hop anew they were a trip to
+  // memory and back twice per hop
+  uint4 win = make_uint4(0u, 0u, 0u, 0u);
+  int win_at = -64;
+  uint32_t win_last = 0u;  // the hop of the window's last record
+  auto window = [&](int hop) __attribute__((always_inline)) {  // from trail_at on, all of this hop's records at least
+    if (trail_at < trail_n && trail_at > win_at &&
+        (trail_at >= win_at + 64 || (win_at + 64 < trail_n && win_last <= (uint32_t)hop))) {
+      win_at = trail_at;
+      win = trail[win_at + lane < trail_n ? win_at + lane : trail_n - 1];
+      win_last = (uint32_t)__builtin_amdgcn_readlane((int)win.w, 63);
+    }
+    return trail_at - win_at;
+  };
   bool own_stretch = false;  // between two markers: hops this pass makes itself
   if (trail_hops > 0) st.n_dist += trail_n_dist;  // the evaluations that pass made up to the trail's end count as performed
   while (true) {
@@ -1947,10 +1961,11 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
     if (st.n_hops <= trail_hops) {
       // markers that take effect with this hop (a group may end and the next begin at the same one)
       while (true) {
-        const uint4 m = trail[trail_at < trail_n ? trail_at : 0];
-        const uint32_t kind = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.x);
-        const uint32_t at_hop = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.w);
-        if (trail_at >= trail_n || kind < kTrailBack || at_hop != (uint32_t)st.n_hops) break;
+        const int off = window(st.n_hops);
+        if (trail_at >= trail_n) break;
+        const uint32_t kind = (uint32_t)__builtin_amdgcn_readlane((int)win.x, off);
+        const uint32_t at_hop = (uint32_t)__builtin_amdgcn_readlane((int)win.w, off);
+        if (kind < kTrailBack || at_hop != (uint32_t)st.n_hops) break;
         own_stretch = kind == kTrailOwn;
         trail_at += 1;
       }
@@ -1962,29 +1977,24 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
       }
       if (!own_stretch) {
         // this hop's records: a run from trail_at on (at most one link row's worth: under 64)
-        const bool have = trail_at + lane < trail_n;
-        const uint4 r = trail[have ? trail_at + lane : 0];
-        const bool mine = have && r.x < kTrailBack && r.w == (uint32_t)st.n_hops;
+        const int off = window(st.n_hops);
+        const bool mine = lane >= off && win_at + lane < trail_n && win.x < kTrailBack && win.w == (uint32_t)st.n_hops;
         const unsigned long long run = __ballot(mine);
-        const bool wrong = mine && r.x != (uint32_t)cid;
-        if (__ballot(wrong) != 0ull) {
+        if (__ballot(mine && win.x != (uint32_t)cid) != 0ull) {
           trail_hops = 0;  // not the node that pass expanded here: nothing more is taken from the trail
         } else {
           n = __popcll(run);
-          if (mine) {
-            s.nbuf[lane] = r.y;
-            s.dbuf[lane] = __uint_as_float(r.z);
+          // the filter learns the nodes (a later hop this pass makes itself need not evaluate them again; where two of
+          // them fall into the same set of tags one is forgotten, as in visit_lossy)
+          if (__builtin_amdgcn_inverse_ballot_w64(run)) {
+            s.nbuf[lane - off] = win.y;
+            s.dbuf[lane - off] = __uint_as_float(win.z);
+            uint2* sets = reinterpret_cast<uint2*>(s.vcache);
+            const int set_bits = s.vc_bits - 1;
+            const uint32_t slot = win.y & ((1u << set_bits) - 1u);
+            sets[slot] = filter_push(sets[slot], win.y >> set_bits);
           }
-          // the filter learns the nodes (a later hop this pass makes itself need not evaluate them again), one
-          // lane after the other: two records of a hop may fall into the same set of tags
-          uint2* sets = reinterpret_cast<uint2*>(s.vcache);
-          const int set_bits = s.vc_bits - 1;
-          for (unsigned long long pend = run; pend != 0ull; pend &= pend - 1ull) {
-            if (lane == __builtin_ctzll(pend)) {
-              const uint32_t slot = r.y & ((1u << set_bits) - 1u);
-              sets[slot] = filter_push(sets[slot], r.y >> set_bits);
-            }
-          }
+          __builtin_amdgcn_wave_barrier();
           trail_at += n;
           from_trail = true;
         }

@@ -53,32 +53,35 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   a.report = nullptr;
   last_repeats = 0;
   last_trails = 0;
+  last_side_by_side = 0;
   if (use_static) {
     launch_search_static<DT, QR, NS>(ix, a, ms);
     return;
   }
   if (ms) HIP_CHECK(hipEventRecord(ev0, stream));
-  // the literal pass runs on the sorted set with ids and the LDS filter (no bitmap) unless the
-  // caller asked for literal queues only, which also means exact evaluation counters
-  // ...and unless the visited bitmaps of the wavefronts at work fit the L2 caches (32 MB) together:
-  // there the bitmap's atomics are cheap and the literal search with them is the faster one
-  const size_t bitmap_bytes = (size_t)std::min(num_cus * 24, a.nq) * ((host.N + 31) / 32) * 4;
-  const bool want_lean = lean_literal == 1 ? bitmap_bytes > ((size_t)32 << 20) : lean_literal > 1;
-  a.lean = (NS > 0 && fast_path != 0 && want_lean) ? auto_fc_bits(a.ef) : 0;
-  if (a.lean && filter_entries <= 0) {
-    // a batch of few queries leaves most of each CU's LDS unused: give the filter what is there
-    // (up to 32 KB), so that it forgets next to nothing
-    const int per_cu = (a.nq + num_cus - 1) / num_cus;
-    const size_t room = per_cu > 0 ? (size_t)(150 * 1024) / per_cu : 0;
-    const size_t other = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, 0, 0, 0).total + 256;
-    while (a.lean < 13 && other + ((size_t)4 << (a.lean + 1)) <= std::min<size_t>(room, 60 * 1024) &&
-           (((unsigned)host.N >> a.lean) < 0xFFFFu))
-      ++a.lean;
-  }
-  const LdsPlan lp = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean);
+  // The literal pass runs on the sorted set with ids and the LDS filter (no bitmap) where the first pass leaves it trails
+  // (which only that variant replays), and else unless the caller asked for literal queues only, which also means exact
+  // evaluation counters, or the visited bitmaps of the wavefronts at work fit the L2 caches (32 MB) together: there the
+  // bitmap's atomics are cheap and a search from the entry point with them is the faster one.
+  auto choose_variant = [&](bool with_trails) {
+    const size_t bitmap_bytes = (size_t)std::min(num_cus * 24, a.nq) * ((host.N + 31) / 32) * 4;
+    const bool want_lean = lean_literal == 1 ? with_trails || bitmap_bytes > ((size_t)32 << 20) : lean_literal > 1;
+    a.lean = (NS > 0 && fast_path != 0 && want_lean) ? auto_fc_bits(a.ef) : 0;
+    if (a.lean && filter_entries <= 0) {
+      // a batch of few queries leaves most of each CU's LDS unused: give the filter what is there
+      // (up to 32 KB), so that it forgets next to nothing
+      const int per_cu = (a.nq + num_cus - 1) / num_cus;
+      const size_t room = per_cu > 0 ? (size_t)(150 * 1024) / per_cu : 0;
+      const size_t other = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, 0, 0, 0).total + 256;
+      while (a.lean < 13 && other + ((size_t)4 << (a.lean + 1)) <= std::min<size_t>(room, 60 * 1024) &&
+             (((unsigned)host.N >> a.lean) < 0xFFFFu))
+        ++a.lean;
+    }
+  };
+  auto literal_lds = [&](int cand_lds) -> size_t {
+    return plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean).total;
+  };
   auto kernel = search_kernel<DT, QR, NS>;
-  int lit_slots = resident_slots(kernel, lp.total);
-  if (max_slots_override > 0) lit_slots = max_slots_override;
   int glob_cap = spill_cap > 0 ? spill_cap : std::max(4096, 8 * a.ef);
   int n_literal = a.nq;
   bool answered = false;
@@ -134,9 +137,12 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     // wavefront, link rows of one pass of 64 lanes, and batches of under three rounds of wavefronts: keeping
     // the trail costs the first pass 9 % (the kernel instance with the trail code 4 %, writing the records the
     // rest), which only a batch short enough to wait for its last hand-over gets back.  trails = 2: whatever
-    // the batch.
-    bool keep_trails = !alone && (QR == 1 || QR == 2) && trails && !a.reverse && a.lean && host.S0 <= 63 &&
+    // the batch.  (Nor where the batch runs alone: one query in a hundred or fewer is handed over there, and the records
+    // would cost every one of them 10 %, 0.383 -> 0.428 ms for a single query on 100 000 x 50 at ef 300.)
+    bool keep_trails = !alone && (QR == 1 || QR == 2) && trails && !a.reverse && host.S0 <= 63 &&
                        (trails > 1 || 4 * (long long)a.nq <= 11 * resident);
+    choose_variant(keep_trails);
+    keep_trails = keep_trails && a.lean;
     if (keep_trails) {
       // (normally there since the index became resident; a changed trail_cap / trail_spares asks again)
       if (d_trail.n < trail_records_wanted(slots)) {
@@ -187,13 +193,12 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       // one or two of these wavefronts per CU: LDS for a candidate queue that never spills costs the first
       // pass nothing (the queue of a long search outgrows 2 * ef entries)
       if (NS > 0) b.cand_lds = std::max(a.cand_lds, 1024);
-      const LdsPlan lp_side = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, b.cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean);
       // (the first pass starts after the batch's descents when its queries are put in order: 0.1 ms per
       // 10 000 queries of the 1.18 M x 50 set; allow ten times that on top of the usual 2 ms)
       b.start_ticks += (long long)wall_clock_khz * (a.nq / 10000 + 1);
       HIP_CHECK(hipEventRecord(ev_side0, stream));
       HIP_CHECK(hipStreamWaitEvent(stream2, ev_side0, 0));
-      hipLaunchKernelGGL(kernel, dim3(side_slots), dim3(64), lp_side.total, stream2, ix, b);
+      hipLaunchKernelGGL(kernel, dim3(side_slots), dim3(64), literal_lds(b.cand_lds), stream2, ix, b);
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipEventRecord(ev_side1, stream2));
     }
@@ -256,11 +261,15 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
         }
       }
     }
+  } else {
+    choose_variant(false);
   }
   if (n_literal > 0 && !answered) {
     timed = false;
     SearchArgs b = a;
     b.nq = n_literal;
+    const size_t lds = literal_lds(a.cand_lds);
+    const int lit_slots = max_slots_override > 0 ? max_slots_override : resident_slots(kernel, lds);
     int slots = std::max(1, std::min(lit_slots, b.nq));
     bool done = false;
     for (int attempt = 0; attempt < 8 && !done; ++attempt) {
@@ -269,7 +278,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       b.counter = d_ctl.p;
       b.status = d_ctl.p + 1;
       HIP_CHECK(hipMemsetAsync(d_ctl.p, 0, 3 * sizeof(int), stream));
-      hipLaunchKernelGGL(kernel, dim3(slots), dim3(64), lp.total, stream, ix, b);
+      hipLaunchKernelGGL(kernel, dim3(slots), dim3(64), lds, stream, ix, b);
       HIP_CHECK(hipGetLastError());
       int ctl[2];
       HIP_CHECK(hipMemcpyAsync(ctl, d_ctl.p, sizeof(ctl), hipMemcpyDeviceToHost, stream));

@@ -392,6 +392,24 @@ def test_handed_over_queries_start_from_the_first_pass_trail(oracle, tmp_path, d
     e.set_tunable(key, value)
 
 
+def test_small_indexes_keep_trails_too(oracle, tmp_path):
+  """With the default settings, on an index whose visited bitmaps would all fit the L2."""
+  n, d, nq = 5000, 16, 100
+  x, q = integer_vectors(n, d, seed=64, hi=30), integer_vectors(nq, d, seed=65, hi=30)
+  mult = 1 / np.log(8)
+  ix = oracle.OracleIndex("l2").build(x, _levels(n, mult, 66), 8, 16, 60, mult)
+  p = str(tmp_path / "t.idx")
+  ix.save(p)
+  e = _engine(tmp_path, dist_type="l2", max_m=8, max_m0=16)
+  e.load_index(p)
+  o_ids, o_d, o_f = ix.search(q, 10, 100)
+  for _ in range(2):   # (the first batch of an index is not expected to hand anything over and goes alone)
+    ids, dd, f = e.search_knn(q, 10, 100)
+    assert (ids == o_ids).all() and (dd == o_d).all() and (f == o_f).all()
+  assert e.last_search_side_by_side
+  assert e.last_search_trails == e.last_search_repeats > 0
+
+
 def test_overflowing_scratch_areas_are_retried(oracle, tmp_path):
   """Accept log and queue overflow area start far too small: the engine must notice, grow
   them and repeat the search with unchanged answers."""
