@@ -169,6 +169,12 @@ class Engine {
   int cand_lds_override = 0;
   int hnswlib_dist = 0;
   int spin_limit_override = -1;  // polls a waiting literal wavefront may spend (-1 = automatic)
+  static constexpr int kLiteralStreak = 15;  // batches that go to the literal queues alone before one asks the first pass again
+  int literal_streak = 0;
+  // the share of queries given up over the last few searches, cautiously: as if 750 more had been answered without (two of
+  // a thousand may be an accident)
+  double recent_queries = 0.0, recent_repeats = 0.0;
+  double cautious_share() const { return recent_repeats / (recent_queries + 750.0); }
   int side_per_cu = 0;         // its wavefronts per CU (0 = from the share of queries the last search gave up)
   bool share_known = false;               // repeat_share comes from searches of this index
   double repeat_share = 0.0;              // share of the last queries (256 or more, once there are so many) that were given up
@@ -432,6 +438,8 @@ class Engine {
     share_known = false;
     repeat_share = 0.0;
     share_queries = share_repeats = 0;
+    literal_streak = 0;
+    recent_queries = recent_repeats = 0.0;
     sequential_left = 0;
     literal_fallbacks = 0;
     last_side_by_side = 0;
@@ -442,6 +450,8 @@ class Engine {
   // than a third of 256 or more queries were given up the sorted set is tried no more.  Smaller batches are judged
   // together (not where the caller asked for the first pass whatever the batch).
   void learn_share(long long nq, long long given_up) {
+    recent_queries = 0.75 * recent_queries + (double)nq;
+    recent_repeats = 0.75 * recent_repeats + (double)given_up;
     if (nq < 256 && fast_path == 1) {
       nq = share_queries += nq;
       given_up = share_repeats += given_up;

@@ -86,11 +86,26 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   int n_literal = a.nq;
   bool answered = false;
   bool timed = false;  // ev1 has been recorded after the last kernel of this search
-  // The first pass takes every batch, however small: it needs half the literal search's time per expanded candidate, so
-  // that it is the faster way even for a query that has to be handed over now and then (100 000 x 50, ef 300: one query
-  // 0.81 -> 0.37 ms, 1 000 queries 1.69 -> 0.76; a 200 000 x 128 integer set, ef 128, 32 queries: 0.75 -> 0.61 on average,
-  // 1.06 where one of them is handed over).
-  if (NS > 0 && a.fast_path && a.fc_bits > 0) {  // (reverse_cand: fast_path is 2)
+  // The first pass takes every batch, however small: it needs half the literal search's time per expanded candidate
+  // (100 000 x 50, ef 300: one query 0.81 -> 0.33 ms, 1 000 queries 1.03 -> 0.55).  A query that is handed over ends
+  // later than it would have on the literal queues alone, though, replayed from its trail or not (1.23 ms there; 200 000
+  // x 128 integers, ef 300: 1.2 ms without a hand-over, 1.9 with one, literal queues alone 1.78).  So where 1.5 or more
+  // hand-overs are to be expected of a batch, three batches in four have one, and the batch is one round of literal
+  // wavefronts whose bitmaps fit the L2, it goes to the literal queues alone (there, 1 000 queries of which 12 are handed
+  // over: 2.27 -> 1.99 ms; 256 with 3: 1.89 -> 1.78; 32 with 0.4 stay, 1.46 against 1.60).  Not at ef <= 128, where a
+  // replay is short (1 000 queries with 2.7: 0.80 ms, 0.86 on the literal queues), and not on rows that are read from
+  // memory as long as the queues are busy (QR == 0).  One batch in sixteen takes the first pass all the same, so that the
+  // share is not taken for known forever.
+  bool literal_alone = false;
+  if (NS > 2 && QR > 0 && fast_path == 1 && a.fast_path == 1 && a.fc_bits > 0 && max_slots_override <= 0 &&
+      cautious_share() * a.nq >= 1.5) {
+    choose_variant(false);
+    if (!a.lean && a.nq <= resident_slots(kernel, literal_lds(a.cand_lds))) {
+      literal_alone = literal_streak < kLiteralStreak;
+      literal_streak = literal_alone ? literal_streak + 1 : 0;
+    }
+  }
+  if (NS > 0 && a.fast_path && a.fc_bits > 0 && !literal_alone) {  // (reverse_cand: fast_path is 2)
     d_redo.reserve((size_t)a.nq);
     a.redo = d_redo.p;
     auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;

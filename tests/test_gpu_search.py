@@ -410,6 +410,28 @@ def test_small_indexes_keep_trails_too(oracle, tmp_path):
   assert e.last_search_trails == e.last_search_repeats > 0
 
 
+def test_small_batches_with_many_hand_overs_take_the_literal_queues(oracle, tmp_path):
+  """Once an index is known to hand over several queries of such a batch: fifteen batches, then one that looks again.
+  The answers are the same either way."""
+  n, d, nq = 5000, 16, 60
+  x, q = integer_vectors(n, d, seed=64, hi=30), integer_vectors(nq, d, seed=65, hi=30)
+  mult = 1 / np.log(8)
+  ix = oracle.OracleIndex("l2").build(x, _levels(n, mult, 66), 8, 16, 60, mult)
+  p = str(tmp_path / "t.idx")
+  ix.save(p)
+  e = _engine(tmp_path, dist_type="l2", max_m=8, max_m0=16)
+  e.load_index(p)
+  o_ids, o_d, o_f = ix.search(q, 10, 200)
+  looked = []
+  for _ in range(18):
+    ids, dd, f = e.search_knn(q, 10, 200)
+    assert (ids == o_ids).all() and (dd == o_d).all() and (f == o_f).all()
+    looked.append(e.last_search_repeats > 0)
+  assert looked == [True] + [False] * 15 + [True, False]
+  e.search_knn(q, 10, 100)                 # a small set: the first pass, whatever it hands over
+  assert e.last_search_repeats > 0
+
+
 def test_overflowing_scratch_areas_are_retried(oracle, tmp_path):
   """Accept log and queue overflow area start far too small: the engine must notice, grow
   them and repeat the search with unchanged answers."""
