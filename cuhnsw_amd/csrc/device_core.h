@@ -186,9 +186,15 @@ __device__ __forceinline__ float4 load_chunk_f16(const void* base, uint64_t chun
 // node's.  The order is the same (only a key that is exactly the largest number is no longer told from an overflow), and
 // what a search returns is computed without the stop, or freed of it (answer_key).
 constexpr float kLargestKey = 3.402823466e+38f;
+// (written out: with both bounds in operands of its own the compiler keeps one of them in a vector register throughout)
+__device__ __forceinline__ float bounded_key(float x) {
+  float r;
+  asm("v_med3_f32 %0, %1, -%2, %2" : "=v"(r) : "v"(x), "s"(kLargestKey));
+  return r;
+}
 template <int DT, bool RAW>
 __device__ __forceinline__ float finish_sum(float s) {
-  if (DT == DIST_DOT) return RAW ? -s : __builtin_amdgcn_fmed3f(1.0f - s, -kLargestKey, kLargestKey);
+  if (DT == DIST_DOT) return RAW ? -s : bounded_key(1.0f - s);
   return RAW ? s : fminf(s, kLargestKey);
 }
 __device__ __forceinline__ float answer_key(float key) {

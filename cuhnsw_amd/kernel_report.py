@@ -37,6 +37,11 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_L2, 2, 5, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,5,trails>"),
     ("search_fast_kernel<DIST_DOT, 1, 2, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,2>"),
     ("search_fast_kernel<DIST_DOT, 2, 8, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,8>"),
+    ("search_fast_kernel<DIST_DOT, 2, 2, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,2>"),
+    ("search_fast_kernel<DIST_L2, 2, 2, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2>"),
+    ("search_fast_kernel<DIST_DOT, 1, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,5,few>"),
+    ("search_fast_kernel<DIST_L2, 2, 2, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2,few>"),
+    ("search_fast_kernel<DIST_L2, 0, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,5,few>"),
 ]
 OTHERS = [
     ("search_kernel<DIST_DOT, 1, 5>(DevIndex, SearchArgs)", "search_kernel<dot,1,5>"),
@@ -156,7 +161,8 @@ def loop_scratch_accesses(isa_text, mangled):
   # memory (the link row, the vectors).  The loop over the wavefront's queries and any loop that merely
   # alternates between two hop loops contain such a loop and are not counted themselves; the loop over a hop's
   # offers holds the insert but fetches nothing.
-  has_insert = [any(t.startswith("v_med3_f32") for t in ins) for _, ins in blocks]
+  # (the bound on a key is a v_med3_f32 as well, the one with a negated operand)
+  has_insert = [any(t.startswith("v_med3_f32") and "-" not in t for t in ins) for _, ins in blocks]
   has_fetch = [any(t.startswith("global_load") for t in ins) for _, ins in blocks]
   hot_blocks = set()
   def nest(nodes, edges):

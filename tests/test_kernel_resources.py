@@ -22,6 +22,12 @@ LIMITS = {
     "search_fast_kernel<l2,2,5,trails>": (7, 76),
     "search_fast_kernel<dot,1,2>": (7, 0),
     "search_fast_kernel<dot,2,8>": (5, 36),
+    "search_fast_kernel<dot,2,2>": (7, 20),
+    "search_fast_kernel<l2,2,2>": (7, 20),
+    # (a wavefront with a SIMD to itself: nothing spills, however wide the instance)
+    "search_fast_kernel<dot,1,5,few>": (1, 0),
+    "search_fast_kernel<l2,2,2,few>": (1, 0),
+    "search_fast_kernel<l2,0,5,few>": (1, 0),
 }
 
 
@@ -64,3 +70,11 @@ kern:
 .Lfunc_end0:
 """
   assert kernel_report.loop_scratch_accesses(isa, "kern") == (1, 3)
+  # a loop over rows inside the hop loop, which bounds their keys: not an insert, the hop loop is still the one around it
+  rows = """  s_cbranch_vccz .LBB0_4
+.LBB0_31:
+  global_load_dwordx4 v[8:11], v[6:7], off
+  v_med3_f32 v0, v1, -s2, s2
+  s_cbranch_scc1 .LBB0_31
+"""
+  assert kernel_report.loop_scratch_accesses(isa.replace("  s_cbranch_vccz .LBB0_4\n", rows), "kern") == (1, 3)
