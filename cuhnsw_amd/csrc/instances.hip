@@ -105,7 +105,9 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       literal_streak = literal_alone ? literal_streak + 1 : 0;
     }
   }
-  if (NS > 0 && a.fast_path && a.fc_bits > 0 && !literal_alone) {  // (reverse_cand: fast_path is 2)
+  const bool first_pass = NS > 0 && a.fast_path && a.fc_bits > 0 && !literal_alone;  // (reverse_cand: fast_path is 2)
+  if (!first_pass) choose_variant(false);
+  if constexpr (NS > 0) if (first_pass) {
     d_redo.reserve((size_t)a.nq);
     a.redo = d_redo.p;
     auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
@@ -276,8 +278,6 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
         }
       }
     }
-  } else {
-    choose_variant(false);
   }
   if (n_literal > 0 && !answered) {
     timed = false;
