@@ -1495,11 +1495,15 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
                                               SearchState& st, Frontier<NS>& fr, int& n, int& hop_cid, int& resume_at,
                                               unsigned long long& accepted, Trail& tr, const TieWatch& watch, int lane) {
   constexpr int N = NS > 0 ? NS : 1;
-  constexpr int kInsertAllFrom = 4;  // shorter lists go in one by one
+  // shorter lists go in one by one (2, 4 or 8 are the same within the runs' spread: 1.18 M x 50, ef 300, 10 000 queries
+  // 1.322 / 1.321 / 1.323 ms, one query on 100 000 x 50 0.279 each, 20 000 x 50 indexed 7.82 / 7.78 / 7.81 ms)
+  constexpr int kInsertAllFrom = 4;
   // more rows in flight: the search on long rows (dist_long), and small sets, which leave the registers for it (56 of 72;
   // 345 678 x 101 in fp16, ef 77, 5 003 queries: 0.85 -> 0.71 ms)
   constexpr int kWide = FEW ? 4 : (!BUILD && ((QR == 0 && NS <= 8) || (QR == 2 && NS == 2)) ? 2 : 1);
-  constexpr int K = FULL && (BUILD || FEW || NS > 2) ? (QR == 1 || FEW ? kAhead : 6) : 1;  // (longer rows: registers)
+  // candidates at a time at most, 8 / 6 / 4: 1.18 M x 50, ef 300, 10 000 queries 1.319 / 1.326 / 1.397 ms, one query on
+  // 100 000 x 50 0.280 / 0.287 / 0.295 ms; 1 M x 96, ef 256, 100 000 queries 9.74 / 9.83 / 9.90 ms (longer rows: registers)
+  constexpr int K = FULL && (BUILD || FEW || NS > 2) ? (QR == 1 || FEW ? kAhead : 6) : 1;
   // (said to be wavefront-uniform, so that they sit in scalar registers through the loop)
   const int w0 = WATCH ? uni(watch.id0) : -1, w1 = WATCH ? uni(watch.id1) : -1;
   const int w2 = WATCH ? uni(watch.id2) : -1, w3 = WATCH ? uni(watch.id3) : -1;

@@ -195,8 +195,8 @@ class Engine {
   int lean_literal = 1;  // literal pass: 0 = always the exact visited bitmap, 1 = automatic, 2 = always the LDS filter
   bool storage_half = false;  // vectors live in HBM as fp16 (set before set_data / load_index)
   bool tight_rows = false;    // rows padded to 16-byte chunks only, not to 128-byte lines (set before set_data / load_index)
-  int fast_path = 1;     // 0: search with the literal queues only; 1: sorted-set pass first when the batch is
-                         // larger than one round of literal wavefronts; 2: always
+  int fast_path = 1;     // 0: search with the literal queues only; 1: sorted-set pass first, unless the index is known
+                         // to hand over too many of such a batch's queries; 2: always
   int last_repeats = 0;  // queries of the last search that were repeated with the literal queues
   int last_trails = 0;   // how many of them came with the first pass's trail
   int count_build_work = 0;    // count the work of a build on the device (cuhnsw_last_build_counters)

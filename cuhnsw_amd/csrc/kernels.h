@@ -409,7 +409,8 @@ __device__ __forceinline__ const Args& fresh_args() {
 // A query in which two equal keys meet is not answered here: its index is appended to
 // a.redo (a.repeats counts them) and the literal search_kernel answers it afterwards.
 // (with at most five keys per lane and the query in at most two float4 registers the kernel is
-// held to 72 registers, seven wavefronts per SIMD, at the price of up to five spilled registers;
+// held to 72 registers, seven wavefronts per SIMD, at the price of up to eight spilled registers, none of them
+// touched inside a hop loop;
 // eight wavefronts are no faster; with eight keys per lane it fits 96 registers, five wavefronts
 // per SIMD, without spilling; the other shapes would spill heavily)
 // TRAILS: the pass leaves trails for the literal pass (a.trail set; 2 to 3 % more instructions: the host launches

@@ -198,9 +198,10 @@ int cuhnsw_trails_available(cuhnsw_engine* e);
  *   "spill_cap"     first size (entries) of the per-wavefront queue overflow area; the search
  *                   is repeated with four times the room when it proves too small (0 = automatic)
  *   "fast_path"     0 = search with literal hnswlib priority queues only (exact evaluation
- *                   counters in d_stats); 1 = first pass on the sorted set in registers when the
- *                   batch exceeds one round of resident wavefronts, literal queues for the queries
- *                   that met equal distances (default); 2 = first pass whatever the batch size
+ *                   counters in d_stats); 1 = first pass on the sorted set in registers, literal queues
+ *                   for the queries in which equal distances decide (default; literal queues for a whole batch
+ *                   where the index is known to hand over a third of its queries, or several of a small batch);
+ *                   2 = first pass whatever the index, with the literal pass beside it
  *   "filter_entries" entries of the first pass's LDS visited filter (0 = automatic)
  *   "query_order"   1 (default) = a search batch of 1.5 to 32 rounds of wavefronts (from one round on where the
  *                   first pass keeps trails) does its upper-level descents

@@ -120,7 +120,7 @@ def _full_size(oracle, tmp_path, name, shape, efs, recall_bars, n_oracle=500, n_
     e.set_tunable("fast_path", 1)
     assert (ids0 == ids[:n_literal]).all() and (d0 == dv[:n_literal]).all() and (f0 == found[:n_literal]).all()
     if min_repeats == 0:
-      # a batch of one round is answered by the literal queues by default: force the sorted-set pass as well
+      # a batch of one wavefront per SIMD takes the sorted-set pass alone: both passes side by side as well
       e.set_tunable("fast_path", 2)
       ids1, d1, f1 = e.search_knn(queries, k, ef)
       e.set_tunable("fast_path", 1)
@@ -139,7 +139,7 @@ def _full_size(oracle, tmp_path, name, shape, efs, recall_bars, n_oracle=500, n_
 
 
 def test_c1_full_size(oracle, tmp_path):
-  # 1 000 queries fit one round of wavefronts: the default path answers them with the literal queues alone
+  # 1 000 queries are one wavefront per SIMD: the default path is the sorted-set pass alone
   _full_size(oracle, tmp_path, "C1", (100_000, 50), [300], {300: 0.95}, n_oracle=1000, min_repeats=0)
 
 
