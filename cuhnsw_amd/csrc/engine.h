@@ -256,7 +256,7 @@ class Engine {
   //           3.9 MB 728 -> 633 us.
   // Beyond, the copies run at the bus's rate while a search's own reads and writes wait for it.
   static constexpr size_t kDirectQueries = (size_t)1 << 20, kDirectAnswers = (size_t)4 << 20;
-  static constexpr size_t kQueryBlock = (size_t)512 << 10;
+  static constexpr size_t kQueryBlock = (size_t)1 << 20;
   unsigned char* h_io = nullptr;
   size_t h_io_bytes = 0;
   void reserve_io(size_t bytes) {
@@ -678,7 +678,8 @@ class Engine {
       if (staging.block() > 0) {
         const unsigned char* src = reinterpret_cast<const unsigned char*>(q);
         unsigned char* dst = reinterpret_cast<unsigned char*>(d_q.p);
-        // (each copy is 15 us, whatever its size; threads pay from a megabyte each on.  10 000 x 128: 0.60 ms, 0.63 on one
+        // (each copy is 15 us, whatever its size; threads pay from a megabyte each on.  Up to 2 MB: 4 000 x 128 in blocks of
+        // 0.5 / 1 / 2 MB 303 / 303 / 320 us, 5 003 x 101 in fp16 682 / 669 / 667, out of the caller's memory 666.  10 000 x 128: 0.60 ms, 0.63 on one
         // thread, 0.61 to 0.67 in blocks of 1 or 0.5 MB; out of the caller's own memory in one copy that is waited for
         // 0.63; 100 000 x 128: 3.46, 3.89, 3.77 to 4.45 and 3.98 ms)
         const bool small = q_bytes <= staging.block();
