@@ -261,7 +261,8 @@ class Engine {
   size_t h_io_bytes = 0;
   void reserve_io(size_t bytes) {
     if (bytes <= h_io_bytes) return;
-    bytes = std::max(bytes, (size_t)64 << 10);
+    // (at least doubled: batches that grow by a query at a time do not allocate each time)
+    bytes = std::max({bytes, (size_t)64 << 10, std::min(2 * h_io_bytes, kDirectQueries + kDirectAnswers)});
     if (h_io) HIP_CHECK(hipHostFree(h_io));
     h_io = nullptr;
     h_io_bytes = 0;
