@@ -50,3 +50,24 @@ def test_workspace_is_given_back(tmp_path):
   e.close()
   assert _free() > bare
 
+
+
+def test_engines_together_keep_a_bounded_amount():
+  """Uploading rows that are padded on their way takes 32 MB of pinned blocks and as much on the device: the engines of
+  a process keep 256 MB of the former together, and those beyond that keep neither."""
+  x = gauss_mixture(2000, 50, seed=92)
+  before = _free()
+  engines = []
+  for _ in range(14):
+    e = capi.Engine()
+    e.set_tunable("trails", 0)
+    e.set_data(x)
+    engines.append(e)
+  assert before - _free() < 330 << 20      # (fourteen times 32 MB would be 448)
+  for e in engines[::5] + engines[-1:]:    # whether they keep the blocks or not
+    _index(e, x)
+    ids, _, _ = e.search_knn(x[:3], 1, 50)
+    assert list(ids[:, 0]) == [0, 1, 2]
+  for e in engines:
+    e.close()
+  assert before - _free() < 64 << 20
