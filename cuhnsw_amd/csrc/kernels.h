@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(64) entry_kernel(DevIndex ix, SearchArgs a) {
 // arithmetic, the same strict first minimum and the same counters as `descend`.
 template <int DT, int QR, bool HALF>
 __device__ __forceinline__ float entry4_key(const void* rows, uint32_t rowlen, uint32_t used, const QVec<QR>& qv,
-                                            uint32_t id, int sub) {
+                                            const float* neg, uint32_t id, int sub) {
   constexpr int R = QR > 0 ? QR : 1;
   const uint64_t first = (uint64_t)id * rowlen;
   float ax = 0.f, ay = 0.f, az = 0.f, aw = 0.f;
@@ -264,9 +264,9 @@ __device__ __forceinline__ float entry4_key(const void* rows, uint32_t rowlen, u
   for (int k = 0; k < R; ++k) {
     const uint32_t c = sub + 16 * k;
     const uint64_t at = first + (c < used ? c : 0);  // (as in dist_pass: one unconditional load, padding replaced)
-    const float4 t = HALF ? load_chunk_f16(rows, at) : load_chunk_f32(rows, at);
-    const float4 v = (DT == DIST_DOT || k < R / 2 || c < used) ? t : qv.q[k];
-    acc4<DT>(qv.q[k], v, ax, ay, az, aw);
+    const float4 v = HALF ? load_chunk_f16(rows, at) : load_chunk_f32(rows, at);
+    if (DT == DIST_DOT || k < R / 2) acc4<DT>(qv.q[k], v, ax, ay, az, aw);
+    else acc4_l2_if(qv.q[k], v, neg[k], ax, ay, az, aw);
   }
   return finish16<DT, false>(ax, ay, az, aw);
 }
@@ -275,13 +275,16 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
   const int lane = threadIdx.x, g = lane >> 4, sub = lane & 15;
   const uint32_t rowlen = (uint32_t)ix.Dp >> 2, used = (uint32_t)(ix.D + 3) >> 2;
   const void* rows = ix.vectors;
+  float neg[QR > 0 ? QR : 1];  // (as in dist_pass)
+#pragma unroll
+  for (int k = 0; k < (QR > 0 ? QR : 1); ++k) neg[k] = minus_one_if((uint32_t)(sub + 16 * k) < used);
   for (int q0 = blockIdx.x * 4; q0 < a.nq; q0 += gridDim.x * 4) {
     const int qi = q0 + g;
     const bool have = qi < a.nq;
     QVec<QR> qv;
     load_query<QR>(qv, nullptr, a.q + (size_t)(have ? qi : 0) * ix.D, ix.D, ix.Dp, lane);
     uint32_t cur = ix.enterpoint;
-    float dcur = entry4_key<DT, QR, HALF>(rows, rowlen, used, qv, cur, sub);
+    float dcur = entry4_key<DT, QR, HALF>(rows, rowlen, used, qv, neg, cur, sub);
     int level = ix.maxlevel;
     bool active = have && level > 0;
     int sweeps = 0, evals = 0;
@@ -305,7 +308,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
           for (int j = 0; j < B; ++j) ids[j] = (uint32_t)__shfl((int)id, 16 * g + p0 + j, 64);
 #pragma unroll
           for (int j = 0; j < B; ++j)
-            keys[j] = entry4_key<DT, QR, HALF>(rows, rowlen, used, qv, ids[j] != kEmpty ? ids[j] : cur, sub);
+            keys[j] = entry4_key<DT, QR, HALF>(rows, rowlen, used, qv, neg, ids[j] != kEmpty ? ids[j] : cur, sub);
 #pragma unroll
           for (int j = 0; j < B; ++j)
             if (ids[j] != kEmpty && keys[j] < best) {  // strictly closer: the first occurrence of the minimum wins
@@ -878,7 +881,6 @@ __device__ __forceinline__ void load_node_query_t(QVec<QR>& qv, float4* qlds, co
   const int rowlen = ix.Dp >> 2;
   const int used = (ix.D + 3) >> 2;  // chunks that hold data (the last one zero padded)
   const uint64_t first = (uint64_t)node * (uint32_t)rowlen;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   if (QR > 0) {
     const int sub = lane & 15;
 #pragma unroll
@@ -886,7 +888,7 @@ __device__ __forceinline__ void load_node_query_t(QVec<QR>& qv, float4* qlds, co
       const int c = sub + 16 * k;
       const uint64_t at = first + (c < used ? c : 0);  // unconditional load
       const float4 t = HALF ? load_chunk_f16(ix.vectors, at) : load_chunk_f32(ix.vectors, at);
-      qv.q[k] = c < used ? t : zero;
+      qv.q[k] = masked(t, mask_if(c < used));
     }
   } else {
     const int chunks = query_lds_chunks(ix.Dp);
@@ -894,7 +896,7 @@ __device__ __forceinline__ void load_node_query_t(QVec<QR>& qv, float4* qlds, co
     for (int c = lane; c < chunks; c += 64) {
       const uint64_t at = first + (c < used ? c : 0);
       const float4 t = HALF ? load_chunk_f16(ix.vectors, at) : load_chunk_f32(ix.vectors, at);
-      qlds[c] = c < used ? t : zero;
+      qlds[c] = masked(t, mask_if(c < used));
     }
     wave_sync();
   }
