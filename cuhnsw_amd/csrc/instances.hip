@@ -404,12 +404,6 @@ void Engine::build_levels() {
   workspace.begin();
   auto p_dists0 = workspace.part<float>((size_t)N * host.S0);
   auto p_distsU = workspace.part<float>(up_rows * host.SU);
-  auto p_sel0_ids = workspace.part<uint32_t>((size_t)bmax * host.max_m0);
-  auto p_sel0_keys = workspace.part<float>((size_t)bmax * host.max_m0);
-  auto p_sel0_cnt = workspace.part<int>((size_t)bmax);
-  auto p_selU_ids = workspace.part<uint32_t>(up_rows * host.max_m);
-  auto p_selU_keys = workspace.part<float>(up_rows * host.max_m);
-  auto p_selU_cnt = workspace.part<int>(up_rows);
   // a batch node posts at most max_m0 links on level 0 and max_m on each upper level
   auto p_dirty = workspace.part<unsigned long long>((size_t)bmax * ((size_t)host.max_m0 + (size_t)std::max(host.maxlevel, 1) * host.max_m));
   auto p_inbox0 = workspace.part<HeapEnt>((size_t)N * cap_in);
@@ -442,8 +436,6 @@ void Engine::build_levels() {
   a.save_remains = opt.save_remains ? 1 : 0;
   a.reverse = opt.reverse_cand ? 1 : 0;
   a.own_cap0 = own_links0 > 0 ? std::min(own_links0, host.max_m0) : host.max_m0;
-  a.sel0_ids = workspace.at(p_sel0_ids); a.sel0_keys = workspace.at(p_sel0_keys); a.sel0_cnt = workspace.at(p_sel0_cnt);
-  a.selU_ids = workspace.at(p_selU_ids); a.selU_keys = workspace.at(p_selU_keys); a.selU_cnt = workspace.at(p_selU_cnt);
   a.status = d_ctl.p + 1;
   a.inbox0 = workspace.at(p_inbox0); a.inbox0_cnt = workspace.at(p_inbox0_cnt);
   a.inboxU = workspace.at(p_inboxU); a.inboxU_cnt = workspace.at(p_inboxU_cnt);
@@ -523,8 +515,6 @@ void Engine::build_levels() {
     HIP_CHECK(hipGetLastError());
     if (cur_max >= 0) {
       long long work = (long long)b * m_max;
-      hipLaunchKernelGGL(apply_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream, ix, a);
-      HIP_CHECK(hipGetLastError());
       hipLaunchKernelGGL(k_reverse, dim3((unsigned)std::min<long long>(work, slots3)), dim3(64), lp3.total, stream, ix, a);
       HIP_CHECK(hipGetLastError());
     }

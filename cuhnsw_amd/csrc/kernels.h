@@ -4,7 +4,7 @@
 //                      (cpp/include/cuda_search_kernels.cuh:11-165 in the reference):
 //                      one launch does the descent through every upper level and the
 //                      level-0 ef-search for a whole query batch.
-// build_search_kernel, apply_kernel, reverse_kernel
+// build_search_kernel, reverse_kernel
 //                      replace BuildLevelGraphKernel + SearchHeuristic
 //                      (cpp/include/cuda_build_kernels.cuh:68-338) and the per-level host
 //                      orchestration (cpp/src/cuhnsw_build.cu:96-208).  The reference builds
@@ -12,14 +12,13 @@
 //                      per-node spin locks.  Here nodes are inserted in id order, each on all
 //                      of its levels at once (hnswlib's order: early nodes leave long-range
 //                      links on level 0, which is what keeps strongly clustered sets
-//                      navigable), in batches of three lock-free phases separated by kernel
-//                      boundaries:
+//                      navigable), in batches of two lock-free phases separated by a kernel
+//                      boundary:
 //                        1. every node of the batch descends from the current entry point,
-//                           searches each of its levels on the frozen graph and selects its
-//                           neighbours there (read-only on the graph),
-//                        2. the selections are written and each chosen neighbour y receives
-//                           the newcomer in y's inbox of that level,
-//                        3. one wavefront per touched (y, level) merges inbox and row (append
+//                           searches each of its levels on the frozen graph, selects its
+//                           neighbours there, writes its own rows (which nothing reaches yet)
+//                           and leaves itself in the inbox of each neighbour y it chose,
+//                        2. one wavefront per touched (y, level) merges inbox and row (append
 //                           while there is room, else the selection heuristic).
 //                      The result is deterministic for a given batch schedule.
 #pragma once
@@ -99,12 +98,6 @@ struct BuildArgs {
   int efc, nn_num0, nn_numU, save_remains;
   int reverse;   // expand the farthest waiting candidate (reverse_cand)
   int own_cap0;  // how many links a new node may choose for itself on level 0 (<= max_m0)
-  uint32_t* sel0_ids;  // count x max_m0: level-0 selections of the batch
-  float* sel0_keys;
-  int* sel0_cnt;
-  uint32_t* selU_ids;  // upper rows x max_m: upper-level selections, indexed like linksU rows
-  float* selU_keys;
-  int* selU_cnt;
   int* counter;
   int* status;
   SlotPool pool;
@@ -1008,7 +1001,63 @@ __device__ __forceinline__ int select_neighbors(const DevIndex& ix, const uint32
   return save_remains ? tail + 1 : head;
 }
 
-// Phase 1 of a build batch: search + select, read-only on the graph.
+__device__ __forceinline__ uint32_t* link_row_mut(const DevIndex& ix, uint32_t node, int level) {
+  return level == 0 ? ix.links0 + (size_t)node * ix.S0 : ix.linksU + (size_t)(ix.upper_off[node] + level - 1) * ix.SU;
+}
+__device__ __forceinline__ float* dist_row_mut(const DevIndex& ix, uint32_t node, int level) {
+  return level == 0 ? ix.dists0 + (size_t)node * ix.S0 : ix.distsU + (size_t)(ix.upper_off[node] + level - 1) * ix.SU;
+}
+
+// A new node's row of one level, chosen by the selection (LDS): written in its place, and the node left in the inbox of
+// each neighbour it chose, which goes on the list of touched rows with its first one.  Nothing reads either before the
+// batch's next phase.  (As a kernel of its own, a thread per slot of every row, this was 7 of the 104 ms that 1 183 514 x
+// 50 take to build: one counter for the touched rows, asked by every wavefront at once.  Here the searches of other nodes
+// run while the atomics are under way.)
+__device__ __forceinline__ void write_row_and_post(const DevIndex& ix, const BuildArgs& a, uint32_t x, int level, const uint32_t* oid,
+                                                   const float* okey, int deg, int lane) {
+  const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
+  uint32_t* row = link_row_mut(ix, x, level);
+  float* drow = dist_row_mut(ix, x, level);
+  for (int base = 0; base < m_cap; base += 64) {
+    const int j = base + lane;
+    const bool link = j < deg;
+    const uint32_t y = link ? oid[j] : kEmpty;
+    const float key = link ? okey[j] : 0.f;
+    if (j < m_cap) {
+      row[j] = y;
+      drow[j] = key;
+    }
+    bool first = false;
+    if (link) {
+      const size_t r = level == 0 ? (size_t)y : (size_t)(ix.upper_off[y] + level - 1);
+      const int slot = atomicAdd((level == 0 ? a.inbox0_cnt : a.inboxU_cnt) + r, 1);
+      first = slot == 0;
+      if (slot < a.cap_in) {
+        HeapEnt e;
+        e.key = key;
+        e.id = x;
+        (level == 0 ? a.inbox0 : a.inboxU)[r * a.cap_in + slot] = e;
+      }
+    }
+    const unsigned long long touched = __ballot(first);
+    if (touched != 0ull) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(a.dirty_cnt, __popcll(touched));
+      at = uni(at);
+      if (first) a.dirty[at + lanes_below(touched)] = (unsigned long long)y | ((unsigned long long)level << 32);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (lane == 0 && a.selected0) {
+    // (with free picks or the tail fill the row holds entries the rule's tests do not vouch for)
+    const unsigned char pure = (level == 0 ? a.nn_num0 : a.nn_numU) == 0 && !a.save_remains;
+    if (level == 0) a.selected0[x] = pure;
+    else a.selectedU[(size_t)(ix.upper_off[x] + level - 1)] = pure;
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Phase 1 of a build batch: search, select, write the new rows, post the reverse links.
 // (held to six / five wavefronts per SIMD where the query fits one / two float4 registers: a few
 // spilled registers, 3-4 % off the build time of the 1.18 M x 50 and 10 M x 96 sets)
 template <int DT, int QR, int NS>
@@ -1055,9 +1104,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
     const int lx = ix.levels[x];
     const int top_level = lx < a.cur_max ? lx : a.cur_max;  // levels x shares with the graph so far
     const bool here = listed || a.n_upper == 0 || lx <= 0;
-    if (lane == 0 && here) a.sel0_cnt[b] = 0;
-    // (the very first node has nothing to link to; a plain branch, not a `continue` after the
-    // one-lane store above, keeps the control flow simple for the compiler)
+    // (the very first node has nothing to link to)
     if (here && top_level >= 0) {
       QVec<QR> qv;
       load_node_query<QR>(qv, s.qlds, ix, x, lane);
@@ -1138,22 +1185,7 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
           level_work[4] += 1u;
         }
         if (QR == 0) load_node_query<QR>(qv, s.qlds, ix, x, lane);  // the LDS query copy was reused by the selection
-        uint32_t* out_ids;
-        float* out_keys;
-        if (level == 0) {
-          out_ids = a.sel0_ids + (size_t)b * ix.max_m0;
-          out_keys = a.sel0_keys + (size_t)b * ix.max_m0;
-          if (lane == 0) a.sel0_cnt[b] = deg;
-        } else {
-          const size_t r = (size_t)(ix.upper_off[x] + level - 1);
-          out_ids = a.selU_ids + r * ix.max_m;
-          out_keys = a.selU_keys + r * ix.max_m;
-          if (lane == 0) a.selU_cnt[r] = deg;
-        }
-        for (int j = lane; j < m_cap; j += 64) {
-          out_ids[j] = j < deg ? oid[j] : kEmpty;
-          out_keys[j] = j < deg ? okey[j] : 0.f;
-        }
+        write_row_and_post(ix, a, x, level, oid, okey, deg, lane);
         if (deg > 0) cur = oid[0];  // closest selected neighbour: entry for the level below
         wave_sync();
         if (!sorted_set) {
@@ -1172,77 +1204,11 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
   if (a.counters && lane < 10 && work[lane] != 0u) atomicAdd(a.counters + lane, (unsigned long long)work[lane]);
 }
 
-__device__ __forceinline__ uint32_t* link_row_mut(const DevIndex& ix, uint32_t node, int level) {
-  return level == 0 ? ix.links0 + (size_t)node * ix.S0 : ix.linksU + (size_t)(ix.upper_off[node] + level - 1) * ix.SU;
-}
-__device__ __forceinline__ float* dist_row_mut(const DevIndex& ix, uint32_t node, int level) {
-  return level == 0 ? ix.dists0 + (size_t)node * ix.S0 : ix.distsU + (size_t)(ix.upper_off[node] + level - 1) * ix.SU;
-}
-
-// Phase 2: write the selected rows and post the reverse links.  Thread (b, j) handles slot j
-// of node b on each of its levels.
-static __global__ void __launch_bounds__(256) apply_kernel(DevIndex ix, BuildArgs a) {
-  const int m_max = ix.max_m0 > ix.max_m ? ix.max_m0 : ix.max_m;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)a.count * m_max) return;
-  const int b = (int)(i / m_max), j = (int)(i % m_max);
-  const uint32_t x = (uint32_t)(a.begin + b);
-  const int lx = ix.levels[x];
-  const int top_level = lx < a.cur_max ? lx : a.cur_max;
-  for (int level = 0; level <= top_level; ++level) {
-    const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
-    if (j >= m_cap) continue;
-    const uint32_t* sel_ids;
-    const float* sel_keys;
-    int deg;
-    if (level == 0) {
-      sel_ids = a.sel0_ids + (size_t)b * ix.max_m0;
-      sel_keys = a.sel0_keys + (size_t)b * ix.max_m0;
-      deg = a.sel0_cnt[b];
-    } else {
-      const size_t r = (size_t)(ix.upper_off[x] + level - 1);
-      sel_ids = a.selU_ids + r * ix.max_m;
-      sel_keys = a.selU_keys + r * ix.max_m;
-      deg = a.selU_cnt[r];
-    }
-    const uint32_t y = j < deg ? sel_ids[j] : kEmpty;
-    const float key = sel_keys[j];
-    link_row_mut(ix, x, level)[j] = y;
-    dist_row_mut(ix, x, level)[j] = key;
-    if (j == 0 && a.selected0) {
-      // (with free picks or the tail fill the row holds entries the rule's tests do not vouch for)
-      const unsigned char pure = (level == 0 ? a.nn_num0 : a.nn_numU) == 0 && !a.save_remains;
-      if (level == 0) a.selected0[x] = pure;
-      else a.selectedU[(size_t)(ix.upper_off[x] + level - 1)] = pure;
-    }
-    if (j < deg) {
-      int* cnt;
-      HeapEnt* box;
-      if (level == 0) {
-        cnt = a.inbox0_cnt + y;
-        box = a.inbox0 + (size_t)y * a.cap_in;
-      } else {
-        const size_t ry = (size_t)(ix.upper_off[y] + level - 1);
-        cnt = a.inboxU_cnt + ry;
-        box = a.inboxU + ry * a.cap_in;
-      }
-      const int slot = atomicAdd(cnt, 1);
-      if (slot < a.cap_in) {
-        HeapEnt e;
-        e.key = key;
-        e.id = x;
-        box[slot] = e;
-      }
-      if (slot == 0) a.dirty[atomicAdd(a.dirty_cnt, 1)] = (unsigned long long)y | ((unsigned long long)level << 32);
-    }
-  }
-}
-
 // More newcomers chose node y on this level than its inbox holds (a hub of a clustered set, late in a
 // large batch).  Which of them reached the inbox depends on the order of the atomics, so the inbox is
-// not used: the batch's selections are scanned for y and the cap closest newcomers by (key, id) are
+// not used: the rows of the batch's nodes are scanned for y and the cap closest newcomers by (key, id) are
 // collected into obox (LDS, cap entries) — the same set in every run.  Returns how many newcomers chose
-// y in all.  Rare; one wavefront reads the whole batch's selection rows.
+// y in all.  Rare; one wavefront reads the rows of the whole batch.
 __device__ __forceinline__ int gather_overflowed_inbox(const DevIndex& ix, const BuildArgs& a, uint32_t y, int level,
                                                        HeapEnt* obox, int cap, int lane) {
   int size = 0, total = 0;
@@ -1256,20 +1222,10 @@ __device__ __forceinline__ int gather_overflowed_inbox(const DevIndex& ix, const
       const int lx = ix.levels[x];
       const int top_level = lx < a.cur_max ? lx : a.cur_max;
       if (level <= top_level) {
-        const uint32_t* ids;
-        const float* keys;
-        int deg;
-        if (level == 0) {
-          ids = a.sel0_ids + (size_t)b * ix.max_m0;
-          keys = a.sel0_keys + (size_t)b * ix.max_m0;
-          deg = a.sel0_cnt[b];
-        } else {
-          const size_t r = (size_t)(ix.upper_off[x] + level - 1);
-          ids = a.selU_ids + r * ix.max_m;
-          keys = a.selU_keys + r * ix.max_m;
-          deg = a.selU_cnt[r];
-        }
-        for (int j = 0; j < deg; ++j) {
+        const uint32_t* ids = link_row(ix, x, level);  // (no row of a batch's node is touched in its own batch)
+        const float* keys = dist_row_mut(ix, x, level);
+        const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
+        for (int j = 0; j < m_cap && ids[j] != kEmpty; ++j) {
           if (ids[j] == y) {
             hit = true;
             my_key = keys[j];
@@ -1315,7 +1271,7 @@ __device__ __forceinline__ int gather_overflowed_inbox(const DevIndex& ix, const
   return total;
 }
 
-// Phase 3: one wavefront per (node, level) that received reverse links.
+// Phase 2: one wavefront per (node, level) that received reverse links.
 template <int DT, int QR>
 __global__ void __launch_bounds__(64) reverse_kernel(DevIndex ix, BuildArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
