@@ -1295,100 +1295,118 @@ __global__ void __launch_bounds__(64) reverse_kernel(DevIndex ix, BuildArgs a) {
   if (lane < 16) work[lane] = 0u;
   wave_sync();
 
-  for (int di = blockIdx.x; di < n_dirty; di += gridDim.x) {
-    const unsigned long long entry = a.dirty[di];
-    const uint32_t y = (uint32_t)(entry & 0xffffffffull);
-    const int level = (int)(entry >> 32);
+  // What a touched row is made of, lane by lane: the row itself (its first 64 slots), its keys, its inbox and how many were
+  // posted there.  All of it is asked for at once (an inbox is read whole, whatever is in it), and for the next row before
+  // this one is dealt with: one after the other these are four trips to memory, which is what most rows' time was.
+  struct Touched {
+    uint32_t y, id;
+    int level, posted;
+    float key;
+    HeapEnt in;
+  };
+  auto fetch = [&](unsigned long long entry) __attribute__((always_inline)) {
+    Touched t;
+    t.y = (uint32_t)uni((int)(uint32_t)(entry & 0xffffffffull));
+    t.level = uni((int)(entry >> 32));
+    const size_t r = t.level == 0 ? (size_t)t.y : (size_t)(ix.upper_off[t.y] + t.level - 1);
+    const int S = row_stride(ix, t.level);
+    t.posted = (t.level == 0 ? a.inbox0_cnt : a.inboxU_cnt)[r];
+    t.id = link_row(ix, t.y, t.level)[lane < S ? lane : 0];
+    t.key = dist_row_mut(ix, t.y, t.level)[lane < S ? lane : 0];
+    t.in = ((t.level == 0 ? a.inbox0 : a.inboxU) + r * a.cap_in)[lane < a.cap_in ? lane : 0];
+    return t;
+  };
+  const int step = (int)gridDim.x;
+  Touched next;
+  unsigned long long entry_after = 0ull;
+  if ((int)blockIdx.x < n_dirty) {
+    next = fetch(a.dirty[blockIdx.x]);
+    entry_after = a.dirty[(int)blockIdx.x + step < n_dirty ? (int)blockIdx.x + step : 0];
+  }
+  for (int di = blockIdx.x; di < n_dirty; di += step) {
+    const Touched t = next;
+    if (di + step < n_dirty) {
+      next = fetch(entry_after);
+      entry_after = a.dirty[di + 2 * step < n_dirty ? di + 2 * step : 0];
+    }
+    const uint32_t y = t.y;
+    const int level = t.level;
     const int S = row_stride(ix, level);
     const int m_cap = level == 0 ? ix.max_m0 : ix.max_m;
-    int* cnt;
-    const HeapEnt* box;
-    if (level == 0) {
-      cnt = a.inbox0_cnt + y;
-      box = a.inbox0 + (size_t)y * a.cap_in;
-    } else {
-      const size_t ry = (size_t)(ix.upper_off[y] + level - 1);
-      cnt = a.inboxU_cnt + ry;
-      box = a.inboxU + ry * a.cap_in;
-    }
-    const int posted = *cnt;
-    int nin = posted < a.cap_in ? posted : a.cap_in;
+    int* cnt = level == 0 ? a.inbox0_cnt + y : a.inboxU_cnt + (size_t)(ix.upper_off[y] + level - 1);
+    const int posted = uni(t.posted);
+    const int n_new = posted < a.cap_in ? posted : a.cap_in;
+    HeapEnt in = t.in;
     if (posted > a.cap_in) {
       // (the overflow list takes the LDS of the selection's output rows, which are not in use yet; the
       // host sizes them for cap_in entries)
       HeapEnt* obox = reinterpret_cast<HeapEnt*>(smem + lp.out_id);
       const int total = gather_overflowed_inbox(ix, a, y, level, obox, a.cap_in, lane);
       if (lane == 0) atomicAdd(a.dropped, total - a.cap_in);
-      box = obox;
       wave_sync();
+      in = obox[lane < a.cap_in ? lane : 0];
     }
     uint32_t* row = link_row_mut(ix, y, level);
     float* drow = dist_row_mut(ix, y, level);
-    // existing links
+    // the links there are, in front of the candidate list (a newcomer cannot be among them: it was in no row before)
     int n0 = 0;
     for (int base = 0; base < S; base += 64) {
-      uint32_t id = (base + lane < S) ? row[base + lane] : kEmpty;
-      float key = (base + lane < S) ? drow[base + lane] : 0.f;
-      bool valid = id != kEmpty;
-      unsigned long long mask = __ballot(valid);
-      int pos = n0 + lanes_below(mask);
-      if (valid) { cbuf[pos].key = key; cbuf[pos].id = id; }
+      uint32_t id = t.id;
+      float key = t.key;
+      if (base > 0) {
+        id = row[base + lane < S ? base + lane : 0];
+        key = drow[base + lane < S ? base + lane : 0];
+      }
+      const unsigned long long mask = __ballot(base + lane < S && id != kEmpty);
+      if (__builtin_amdgcn_inverse_ballot_w64(mask)) {
+        HeapEnt e;
+        e.key = key;
+        e.id = id;
+        cbuf[n0 + lanes_below(mask)] = e;
+      }
+      __builtin_amdgcn_wave_barrier();
       n0 += __popcll(mask);
     }
-    wave_sync();
-    // newcomers that are not linked yet
-    int T = n0;
-    for (int base = 0; base < nin; base += 64) {
-      HeapEnt e;
-      e.key = 0.f; e.id = kEmpty;
-      bool keep = false;
-      if (base + lane < nin) {
-        e = box[base + lane];
-        keep = true;
-        for (int t = 0; t < n0; ++t) keep = keep && (cbuf[t].id != e.id);
+    const int T = n0 + n_new;
+    unsigned char* selected = !a.selected0 ? nullptr
+                              : (level == 0 ? a.selected0 + y : a.selectedU + (size_t)(ix.upper_off[y] + level - 1));
+    if (T <= m_cap) {
+      // room for all: the newcomers go behind the row, ordered by (key, id)
+      int before = 0;
+      for (int i = 0; i < n_new; ++i) {
+        const float key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, in.key), i));
+        const uint32_t id = (uint32_t)__builtin_amdgcn_readlane((int)in.id, i);
+        before += key < in.key || (key == in.key && id < in.id) ? 1 : 0;
       }
-      unsigned long long mask = __ballot(keep);
-      int pos = T + lanes_below(mask);
-      if (keep) cbuf[pos] = e;
-      T += __popcll(mask);
-    }
-    wave_sync();
-    const int n_new = T - n0;
-    if (n_new > 0) {
-      unsigned char* selected = !a.selected0 ? nullptr
-                                : (level == 0 ? a.selected0 + y : a.selectedU + (size_t)(ix.upper_off[y] + level - 1));
-      if (T <= m_cap) {
-        // room for all: append the newcomers, ordered by (key, id)
-        rank_sort(cbuf + n0, nullptr, n_new, sid, skey, lane);
-        wave_sync();
-        for (int t = lane; t < n_new; t += 64) {
-          row[n0 + t] = sid[t];
-          drow[n0 + t] = skey[t];
-        }
-        if (selected && lane == 0) *selected = 0;  // no longer what the selection rule alone would leave
-      } else {
-        rank_sort(cbuf, nullptr, T, sid, skey, lane);
-        wave_sync();
-        // A row that is an output of the rule is re-selected with the shortcut for newcomers: the nodes of this
-        // batch (ids from a.begin on; everything the row held before has a smaller id).
-        const int nn_num = level == 0 ? a.nn_num0 : a.nn_numU;
-        const bool pure = nn_num == 0 && !a.save_remains;
-        const bool shortcut = pure && selected && uni((int)*selected) != 0;
-        const int deg = select_neighbors<DT, QR>(ix, sid, skey, T, m_cap, nn_num, a.save_remains, oid, okey, s, lane,
-                                                 a.counters ? work + (level == 0 ? 0 : 5) : nullptr,
-                                                 shortcut ? (uint32_t)a.begin : 0u);
-        for (int j = lane; j < m_cap; j += 64) {
-          row[j] = j < deg ? oid[j] : kEmpty;
-          drow[j] = j < deg ? okey[j] : 0.f;
-        }
-        if (selected && lane == 0) *selected = pure ? 1 : 0;
+      if (lane < n_new) {
+        row[n0 + before] = in.id;
+        drow[n0 + before] = in.key;
       }
+      if (selected && lane == 0) *selected = 0;  // no longer what the selection rule alone would leave
+    } else {
+      if (lane < n_new) cbuf[n0 + lane] = in;
+      wave_sync();
+      rank_sort(cbuf, nullptr, T, sid, skey, lane);
+      wave_sync();
+      // A row that is an output of the rule is re-selected with the shortcut for newcomers: the nodes of this
+      // batch (ids from a.begin on; everything the row held before has a smaller id).
+      const int nn_num = level == 0 ? a.nn_num0 : a.nn_numU;
+      const bool pure = nn_num == 0 && !a.save_remains;
+      const bool shortcut = pure && selected && uni((int)*selected) != 0;
+      const int deg = select_neighbors<DT, QR>(ix, sid, skey, T, m_cap, nn_num, a.save_remains, oid, okey, s, lane,
+                                               a.counters ? work + (level == 0 ? 0 : 5) : nullptr,
+                                               shortcut ? (uint32_t)a.begin : 0u);
+      for (int j = lane; j < m_cap; j += 64) {
+        row[j] = j < deg ? oid[j] : kEmpty;
+        drow[j] = j < deg ? okey[j] : 0.f;
+      }
+      if (selected && lane == 0) *selected = pure ? 1 : 0;
     }
     if (lane == 0) *cnt = 0;
     if (a.counters && lane == 0) {
       unsigned int* level_work = work + (level == 0 ? 0 : 5);
       level_work[1] += 1u;
-      level_work[4] += n_new > 0 ? 1u : 0u;
+      level_work[4] += 1u;
     }
     wave_sync();
   }
