@@ -496,14 +496,15 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
     dist_long<DT, RAW, HALF, WIDE>(rows, rowlen, used, qlds, ids, n, out, g, sub);
   }
 }
-// (the element type of the stored vectors is a property of the index: one scalar branch per list; the code for fp16 goes
-// out of the way, which is 1 % of a search of one query)
+// (the element type of the stored vectors is a property of the index: one scalar branch per list.  In the wide instances the
+// code for fp16 goes out of the way, which is 1 % of a search of one query; elsewhere it costs spills.)
 // WIDE: how many rows are in flight; 1 = as many as registers allow beside a full machine's wavefronts, 4 = as a
 // wavefront with a SIMD to itself can have, 0 = four
 template <int DT, int QR, bool RAW, int WIDE = 1>
 __device__ __forceinline__ void dist_list(const DevIndex& ix, const QVec<QR>& qv, const float4* qlds,
                                           const uint32_t* ids, int n, float* out, int lane) {
-  if (__builtin_expect(uni(ix.half) != 0, 0)) dist_list_t<DT, QR, RAW, true, WIDE>(ix, qv, qlds, ids, n, out, lane);
+  const bool half = uni(ix.half) != 0;
+  if (WIDE >= 4 ? __builtin_expect(half, 0) : half) dist_list_t<DT, QR, RAW, true, WIDE>(ix, qv, qlds, ids, n, out, lane);
   else dist_list_t<DT, QR, RAW, false, WIDE>(ix, qv, qlds, ids, n, out, lane);
 }
 
