@@ -68,8 +68,9 @@ def build_lib():
   from cuhnsw_amd import kernel_report
   with tempfile.TemporaryDirectory(prefix="cuhnsw_build_") as tmp:
     # (the objects that take longest first)
-    jobs = [("instances.hip", ["-DCUHNSW_DT=" + dt, "-DCUHNSW_QR=%d" % qr], os.path.join(tmp, "%s_%d.o" % (dt, qr)))
-            for qr in (4, 2, 0, 1) for dt in ("DIST_DOT", "DIST_L2")]
+    jobs = [("instances.hip", ["-DCUHNSW_DT=" + dt, "-DCUHNSW_QR=%d" % qr, "-DCUHNSW_PART=%d" % part],
+             os.path.join(tmp, "%s_%d_%d.o" % (dt, qr, part)))
+            for part in (0, 1) for qr in (4, 2, 0, 1) for dt in ("DIST_DOT", "DIST_L2")]
     jobs += [(name, [], os.path.join(tmp, name + ".o")) for name in ("engine.hip", "index_file.cpp")]
     workers = max(1, min(len(jobs), len(os.sched_getaffinity(0)), int(os.environ.get("MAX_JOBS") or 8)))
     with concurrent.futures.ThreadPoolExecutor(workers) as pool:

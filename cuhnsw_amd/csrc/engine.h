@@ -521,9 +521,14 @@ class Engine {
     HIP_CHECK(hipMemsetAsync(d_bitmaps.p, 0, (size_t)pool_slots * pool.bitmap_words * 4, stream));
   }
 
-  // slots of sorted result keys per lane: the result set lives in registers while
-  // ef < 64 * NS; 0 selects the literal LDS heap for larger ef
-  static int key_slots(int ef) { return ef <= 128 ? 2 : (ef < 320 ? 5 : (ef <= 512 ? 8 : (ef < 1024 ? 16 : 0))); }
+  // slots of sorted result keys per lane: as few as hold the result set (an insert costs five instructions a slot), two at
+  // least (one for ef <= 64 is 0 to 2 % slower than two), eight for ef <= 512, sixteen beyond; 0 selects the literal LDS heap.
+  // (Against 2, 5 and 8 only: 300 000 x 50, 20 000 queries, ef 180 1.66 -> 1.52 ms, ef 250 1.74 -> 1.66, ef 350 3.13 -> 2.64,
+  // ef 430 2.87 -> 2.74; 300 000 x 96, 30 000 queries, ef 350 4.64 -> 3.91; 200 003 x 128 indexed at 200 66.6 -> 64.8 ms.)
+  static int key_slots(int ef) {
+    const int slots = (ef + 63) / 64;
+    return slots <= 8 ? std::max(slots, 2) : (ef < 1024 ? 16 : 0);
+  }
 
   // LDS entries of the candidate queue.  With the result keys in registers the queue is the
   // only large LDS user: 2*ef entries hold it in nearly every query (the rest spills to the
@@ -584,7 +589,7 @@ class Engine {
   }
 
   // ---- search ------------------------------------------------------------------------------
-  // (defined in instances.hip, one object per distance and row width)
+  // (defined in instances.hip, two objects per distance and row width)
   template <int DT, int QR, int NS>
   void launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_override, float* ms);
   template <int DT, int QR, int NS>

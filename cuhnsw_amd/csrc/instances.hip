@@ -1,5 +1,5 @@
-// Launches of the templated kernels, compiled once per distance and row width: the build passes CUHNSW_DT (DistType)
-// and CUHNSW_QR (kernels.h, query_regs), so that the objects compile side by side.
+// Launches of the templated kernels, compiled once per distance and row width: the build passes CUHNSW_DT (DistType),
+// CUHNSW_QR (kernels.h, query_regs) and CUHNSW_PART (0: searches, 1: index builds), so that the objects compile side by side.
 #include "engine.h"
 
 namespace cuhnsw_amd {
@@ -377,7 +377,11 @@ template <int DT, int QR>
 void Engine::launch_search_ns(int ns, const DevIndex& ix, SearchArgs& a, float* ms) {
   switch (ns) {
     case 2: launch_search<DT, QR, 2>(ix, a, search_slots, ms); break;
+    case 3: launch_search<DT, QR, 3>(ix, a, search_slots, ms); break;
+    case 4: launch_search<DT, QR, 4>(ix, a, search_slots, ms); break;
     case 5: launch_search<DT, QR, 5>(ix, a, search_slots, ms); break;
+    case 6: launch_search<DT, QR, 6>(ix, a, search_slots, ms); break;
+    case 7: launch_search<DT, QR, 7>(ix, a, search_slots, ms); break;
     case 8: launch_search<DT, QR, 8>(ix, a, search_slots, ms); break;
     case 16: launch_search<DT, QR, 16>(ix, a, search_slots, ms); break;
     default: launch_search<DT, QR, 0>(ix, a, search_slots, ms); break;
@@ -553,14 +557,21 @@ template <int DT, int QR>
 void Engine::build_ns(int ns) {
   switch (ns) {
     case 2: build_levels<DT, QR, 2>(); break;
+    case 3: build_levels<DT, QR, 3>(); break;
+    case 4: build_levels<DT, QR, 4>(); break;
     case 5: build_levels<DT, QR, 5>(); break;
+    case 6: build_levels<DT, QR, 6>(); break;
+    case 7: build_levels<DT, QR, 7>(); break;
     case 8: build_levels<DT, QR, 8>(); break;
     case 16: build_levels<DT, QR, 16>(); break;
     default: build_levels<DT, QR, 0>(); break;
   }
 }
 
+#if CUHNSW_PART == 0
 template void Engine::launch_search_ns<CUHNSW_DT, CUHNSW_QR>(int, const DevIndex&, SearchArgs&, float*);
+#else
 template void Engine::build_ns<CUHNSW_DT, CUHNSW_QR>(int);
+#endif
 
 }  // namespace cuhnsw_amd

@@ -401,14 +401,14 @@ __device__ __forceinline__ const Args& fresh_args() {
   return fresh_kernel_args<Args>((sizeof(DevIndex) + 7) / 8 * 8);
 }
 
-// First pass of a search batch: every query on the sorted set in registers (ef < 64*NS).
+// First pass of a search batch: every query on the sorted set in registers (ef <= 64*NS).
 // A query in which two equal keys meet is not answered here: its index is appended to
 // a.redo (a.repeats counts them) and the literal search_kernel answers it afterwards.
-// (with at most five keys per lane and the query in at most two float4 registers the kernel is
+// (with at most six keys per lane and the query in at most two float4 registers the kernel is
 // held to 72 registers, seven wavefronts per SIMD, at the price of up to eight spilled registers, none of them
-// touched inside a hop loop;
-// eight wavefronts are no faster; with eight keys per lane it fits 96 registers, five wavefronts
-// per SIMD, without spilling; the other shapes would spill heavily)
+// touched inside a hop loop, but for six keys; eight wavefronts are no faster, six are 0 to 3 % slower there (ef 350);
+// with seven and eight keys per lane it fits 96 registers, five wavefronts per SIMD: with six of them ef 430 is 2 % slower
+// to 5 % faster and ef 512 a fifth slower; the other shapes would spill heavily)
 // TRAILS: the pass leaves trails for the literal pass (a.trail set; 2 to 3 % more instructions: the host launches
 // this instance for batches of a round or two of wavefronts, where a query handed over late is a good part of the
 // batch's time, and the instance without the trail code otherwise).
@@ -416,7 +416,7 @@ __device__ __forceinline__ const Args& fresh_args() {
 // candidates at a time, with the registers that takes (100 000 x 50, ef 300, one query: 0.290 -> 0.278 ms; 100 000 x 960,
 // ef 300, 1 000 queries: 1.35 -> 1.29).
 template <int DT, int QR, int NS, bool TRAILS, bool FEW = false>
-__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : (NS == 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
+__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 6 ? 7 : (NS <= 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
   Scratch s;
@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
 
 // Search with literal hnswlib priority queues: the only pass for ef beyond the sorted set's
 // capacity, the second pass (over a.redo) otherwise.
-// NS > 0: result keys in registers (ef < 64*NS); NS == 0: literal result heap in LDS.
+// NS > 0: result keys in registers (ef <= 64*NS); NS == 0: literal result heap in LDS.
 // (held to 96 registers, five wavefronts per SIMD, where the query fits two float4 registers: a
 // batch answered by the literal queues alone runs 7-10 % faster for a dozen spilled registers)
 template <int DT, int QR, int NS>
