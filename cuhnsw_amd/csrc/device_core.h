@@ -947,82 +947,126 @@ __device__ __forceinline__ void frontier_insert_distinct(Frontier<NS>& f, float 
     f.v[j] = before_this ? (before_lower ? lo_v : id) : f.v[j];
   }
 }
-// All n offers of a list (lane i < n: the i-th; in the other lanes any key) into a set that has room for them.  Each set entry
-// counts the offers before it, each offer the entries and offers before it, and every entry goes to its new place through
-// LDS: the counting has no dependent steps (15 vector instructions per offer at ef 300, where an insert of its own is 39
-// and 0.25 us of latency), the rest is paid once.  `room`: 64 * NS words of LDS, whose contents are put back.  Returns
-// false, with nothing done, if two keys are equal (or the node is in the set already): those go in one by one, by the rules
-// for them.  last_key: the set's largest key afterwards.
-// (1.18 M x 50, ef 300, 10 000 queries: 1.51 -> 1.45 ms; 1 M x 96, ef 256, 100 000 queries: 10.28 -> 9.96; one query on
-// 100 000 x 50: 0.304 -> 0.288; 200 003 x 128 indexed: 73.6 -> 71.5 ms)
-template <int NS>
-__device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, int n, int size, int ef, float my_key, uint32_t my_id, uint32_t* room,
-                                                    float& last_key, int lane) {
+// Largest value of this lane and those below.
+__device__ __forceinline__ int max_so_far(int x) {
+  auto take = [&](int from) __attribute__((always_inline)) { x = from > x ? from : x; };
+  take(__builtin_amdgcn_update_dpp(x, x, 0x111, 0xF, 0xF, false));  // row_shr:1 (lanes without a source keep their own)
+  take(__builtin_amdgcn_update_dpp(x, x, 0x112, 0xF, 0xF, false));  // row_shr:2
+  take(__builtin_amdgcn_update_dpp(x, x, 0x114, 0xF, 0xF, false));  // row_shr:4
+  take(__builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xF, false));  // row_shr:8
+  take(__builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
+  take(__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+// Several offers of a list at once: those of the lanes in `offers` (fewer than 64; not SPARSE: the first lanes, and +inf in
+// the others), whose list lies in ids / keys (LDS), into a set of `size` entries; what does not fit behind ef entries falls off its end.  The offers are put
+// in order (in ids / keys), every entry finds by halving how many of them go before it, and entries and offers go to their
+// new places through LDS.  `room`: 64 * (NS + 1) words of LDS, whose contents are put back.  Returns false, with nothing
+// done, if two keys are equal (or the node is in the set already), or if the set's largest key would not stay above
+// `above`: those go in one by one, by the rules for them.  last_key: the set's largest key afterwards.
+// (An insert of its own is 39 instructions at ef 300 and 0.2 us of latency, this 200 for 14 offers.  Counting for each entry
+// and each offer what goes before it, offer by offer, was 45 instructions an offer: one query on 100 000 x 50 284 -> 272 us,
+// 1 000 queries there 636 -> 607, of which the full set's share below is half; 1 M x 96, ef 256, 100 000 queries 9.92 ->
+// 9.80 ms.)
+template <int NS, bool SPARSE>
+__device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned long long offers, int size, int ef, float my_key, uint32_t my_id,
+                                                    uint32_t* ids, float* keys, uint32_t* room, float above, float& last_key, int lane) {
   constexpr int N = NS > 0 ? NS : 1;
   lane = fresh(lane);
-  int before[N];  // offers that go before each of this lane's entries
+  const int n = __popcll(offers);
+  if (SPARSE) {  // the offers first, in their order
+    const int pos = lanes_below(offers);
+    wave_sync();
+    if (__builtin_amdgcn_inverse_ballot_w64(offers)) {
+      keys[pos] = my_key;
+      ids[pos] = my_id;
+    }
+    wave_sync();
+  }
+  const float listed_key = SPARSE ? (lane < n ? keys[lane] : INFINITY) : my_key;
+  const uint32_t listed_id = SPARSE ? ids[lane] : my_id;
+  int less = 0;  // offers before this lane's
+  for (int i = 0; i < n; i += 4) {
 #pragma unroll
-  for (int j = 0; j < N; ++j) before[j] = 0;
-  int place = 0, less = 0;  // this lane's offer: entries and offers before it
-  unsigned long long equal = 0ull;
-  for (int i = 0; i < n; ++i) {
-    const float key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_key), i));
-    int above = 0;
+    for (int u = 0; u < 4; ++u) {  // (past the last offer: +inf, which goes before nothing)
+      const float key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, listed_key), i + u));
+      less += key < listed_key ? 1 : 0;
+    }
+  }
+  uint32_t kept[N + 1];
+#pragma unroll
+  for (int j = 0; j <= N; ++j) kept[j] = room[64 * j + lane];
+  wave_sync();
+  keys[lane] = lane < n ? -INFINITY : INFINITY;
+  room[lane] = 0u;
+  wave_sync();
+  if (lane < n) {
+    keys[less] = listed_key;
+    ids[less] = listed_id;
+  }
+  wave_sync();
+  const float offer_key = keys[lane];  // in order from here on: lane r has the r-th
+  bool done = __ballot(offer_key == -INFINITY) == 0ull;  // (two equal offers went to one place and left another empty)
+  if (done) {
+    int before[N];  // offers that go before each of this lane's entries
+#pragma unroll
+    for (int j = 0; j < N; ++j) before[j] = 0;
+    for (int half = 1 << (31 - __builtin_clz(n)); half > 0; half >>= 1) {
+      float probe[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) probe[j] = keys[before[j] + half - 1];
+#pragma unroll
+      for (int j = 0; j < N; ++j) before[j] += probe[j] < f.k[j] ? half : 0;
+    }
+    // an offer's place: as many entries go before it as have no more offers before them than it has.  The last entry of
+    // each such number says how many there are up to it (the others write where nobody looks).
+    const int next_first = __builtin_amdgcn_update_dpp(-1, before[0], 0x130, 0xF, 0xF, false);  // wave_shl:1
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      above += __popcll(__ballot(key < f.k[j]));
-      before[j] += key < f.k[j] ? 1 : 0;
+      const int after = j + 1 < N ? before[j + 1 < N ? j + 1 : 0] : next_first;
+      room[after != before[j] ? before[j] : 64 + lane] = (uint32_t)(lane * N + j + 1);
     }
-    const unsigned long long self = 1ull << i;
-    place = __builtin_amdgcn_inverse_ballot_w64(self) ? 64 * N - above : place;
-    less += key < my_key ? 1 : 0;
-    equal |= __ballot(key == my_key) & ~self;
-  }
-  const unsigned long long offers = n < 64 ? (1ull << n) - 1ull : ~0ull;
-  if ((equal & offers) != 0ull) return false;
-  // (keys first, then ids: half the registers, of which the search has none to spare)
-  uint32_t kept[N];
-  const bool mine = __builtin_amdgcn_inverse_ballot_w64(offers);
-#pragma unroll
-  for (int j = 0; j < N; ++j) kept[j] = room[64 * j + lane];
-  wave_sync();
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int to = lane * N + j + before[j];
-    if (to < 64 * N) room[to] = __float_as_uint(f.k[j]);  // (what is pushed out is padding)
-  }
-  if (mine) room[place + less] = __float_as_uint(my_key);
-  wave_sync();
-  // an offer equal to an entry comes right after it (the padding on both sides is infinite)
-  unsigned long long twins = 0ull;
-  float key[N];
-#pragma unroll
-  for (int j = 0; j < N; ++j) key[j] = __uint_as_float(room[lane * N + j]);
-  const float last = __uint_as_float(room[64 * N - ef + size + n - 1]);
-  const float prev_last = __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, key[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-    twins |= __ballot(key[j] == (j > 0 ? key[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(key[j]) < INFINITY);
-  if (twins == 0ull) {
+    wave_sync();
+    const int place = max_so_far((int)room[lane]) + lane;
     wave_sync();
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int to = lane * N + j + before[j];
-      if (to < 64 * N) room[to] = f.v[j];
-      f.k[j] = key[j];
-    }
-    if (mine) room[place + less] = my_id;
+    for (int j = 0; j < N; ++j) room[lane * N + j + before[j]] = __float_as_uint(f.k[j]);
+    if (lane < n) room[place] = __float_as_uint(offer_key);
     wave_sync();
+    // an offer equal to an entry comes right beside it (the padding on both sides is infinite)
+    unsigned long long twins = 0ull;
 #pragma unroll
-    for (int j = 0; j < N; ++j) f.v[j] = room[lane * N + j];
-    last_key = uni(last);
+    for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j]);
+    const float last = uni(__uint_as_float(room[64 * N - ef + (size + n < ef ? size + n : ef) - 1]));
+    const float prev_last = __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, f.k[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      twins |= __ballot(f.k[j] == (j > 0 ? f.k[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(f.k[j]) < INFINITY);
+    done = twins == 0ull && last > above;
+    if (!done) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j + before[j]]);
+    } else {
+      wave_sync();
+#pragma unroll
+      for (int j = 0; j < N; ++j) room[lane * N + j + before[j]] = f.v[j];
+      if (lane < n) room[place] = ids[lane];
+      wave_sync();
+#pragma unroll
+      for (int j = 0; j < N; ++j) f.v[j] = room[lane * N + j];
+      last_key = last;
+    }
   }
   wave_sync();
 #pragma unroll
-  for (int j = 0; j < N; ++j) room[64 * j + lane] = kept[j];
+  for (int j = 0; j <= N; ++j) room[64 * j + lane] = kept[j];
+  if (!done) {  // (the list as it was)
+    keys[lane] = my_key;
+    ids[lane] = my_id;
+  }
   wave_sync();
-  return twins == 0ull;
+  return done;
 }
 template <int NS>
 __device__ __forceinline__ float frontier_max(const Frontier<NS>& f) {
@@ -1550,6 +1594,11 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   // shorter lists go in one by one (2, 4 or 8 are the same within the runs' spread: 1.18 M x 50, ef 300, 10 000 queries
   // 1.322 / 1.321 / 1.323 ms, one query on 100 000 x 50 0.279 each, 20 000 x 50 indexed 7.82 / 7.78 / 7.81 ms)
   constexpr int kInsertAllFrom = 4;
+  // On a full set most steps bring in nothing and the others a dozen offers: those of one evaluation enter it together from
+  // six on, in the instances that have the registers (a trail wants to know of each whether it was accepted when its turn
+  // came; sets of two registers take their offers one by one as fast).
+  constexpr bool kMerge = FEW && !TRAILS && NS > 2;
+  constexpr int kMergeFrom = 6;
   // more rows in flight: the search on long rows (dist_long), and small sets, which leave the registers for it (56 of 72;
   // 345 678 x 101 in fp16, ef 77, 5 003 queries: 0.85 -> 0.71 ms)
   constexpr int kWide = FEW ? 4 : (!BUILD && ((QR == 0 && NS <= 8) || (QR == 2 && NS == 2)) ? 2 : 1);
@@ -1564,6 +1613,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   HeapEnt* const cands = batch_candidates(s);
   unsigned long long ends = (uint32_t)n;   // end of each one's offers in s.nbuf / s.dbuf, eight bits each
   while (true) {
+    if (QR == 2 && NS > 2 && !BUILD && !FEW) lane = fresh(lane);  // (these are the instances short of registers)
     if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
     st.n_dist += n;
     wave_sync();
@@ -1586,13 +1636,33 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
     int row_end = K > 1 ? (int)(ends & 0xFFu) : n;
     int good = rows;                                        // candidates of the batch that are expanded for good
     const int acc_before = st.n_acc;
-    if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && st.n_acc + n <= ef && 64 * N <= (1 << s.vc_bits)) {
+    if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && n < 64 && st.n_acc + n <= ef && 64 * (N + 1) <= (1 << s.vc_bits)) {
       float last_key = 0.f;
-      if (frontier_insert_all<NS>(fr, n, st.n_acc, ef, my_key, my_id, reinterpret_cast<uint32_t*>(s.vcache), last_key, lane)) {
+      if (frontier_insert_all<NS, false>(fr, todo, st.n_acc, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), -INFINITY,
+                                  last_key, lane)) {
         if (TRAILS) accepted |= todo;
         st.n_acc = st.n_acc + n;
         st.maxkey = last_key;
         st.lower = last_key;
+        todo = 0ull;
+      }
+    }
+    if (FULL && kMerge && __popcll(todo) >= kMergeFrom && __popcll(todo) < 64 && 64 * (N + 1) <= (1 << s.vc_bits)) {
+      // the first candidate that an offer of those before it is closer than: its turn does not come now (tie_free_offers)
+      int upto = rows;
+      for (int c = rows - 1; c > 0; --c) {
+        const float next_key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cand.key), c));
+        const int end = (int)((ends >> (8 * (c - 1))) & 0xFFu);
+        if ((__ballot(my_key < next_key) & todo & (end < 64 ? (1ull << end) - 1ull : ~0ull)) != 0ull) upto = c;
+      }
+      const int end = (int)((ends >> (8 * (upto - 1))) & 0xFFu);
+      const unsigned long long now = todo & (end < 64 ? (1ull << end) - 1ull : ~0ull);
+      float last_key = 0.f;
+      if (__popcll(now) >= kMergeFrom &&
+          frontier_insert_all<NS, true>(fr, now, ef, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), w_hi, last_key, lane)) {
+        st.n_acc = st.n_acc + 1;  // (a full set only asks whether there were any)
+        st.lower = last_key;
+        good = upto;
         todo = 0ull;
       }
     }
