@@ -44,6 +44,9 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   a.nq_dev = nullptr;
   a.entry = nullptr;
   a.order_hist = nullptr;
+  a.regions = nullptr;
+  a.region_level = 0;
+  a.shares = nullptr;
   a.order = nullptr;
   a.trail = nullptr;
   a.redo_trail = nullptr;
@@ -172,10 +175,24 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     const bool in_order = query_order && (query_order > 1 ? a.nq > resident
                                                            : (keep_trails ? a.nq > resident : 2 * a.nq >= 3 * resident) &&
                                                                  a.nq <= 32 * resident);
+    // Three rounds and more: all but the longest of them by region (kernels.h).  The level whose nodes stand for the regions
+    // is the lowest that has four queries a node (of 1, 2, 3, 4: 2 is the best or next to it on 1 M x 96 with 100 000
+    // queries, 1.18 M x 50 with 40 000, 500 000 x 128 with 30 000 and 100 000 x 960 with 8 000, that is 25, 5, 15 and 20).
+    // Not on an index of which every chiplet's 4 MB of L2 holds a good part anyway: 20 000 x 30 (5 MB) 1.68 -> 1.75 ms,
+    // 40 000 x 50 (15 MB) 1.98 -> 2.00 and 2.70 -> 2.61, 40 000 x 128 (26 MB) 2.56 -> 2.33.
+    const size_t index_bytes = (size_t)host.N * ((size_t)Dp * (storage_half ? 2 : 4) + (size_t)host.S0 * 4);
+    int region_level = 0;
+    if (in_order && !keep_trails && a.nq >= 3 * resident && (query_order > 1 || index_bytes > (size_t)12 << 20)) {
+      double nodes = host.N;
+      for (int level = 1; level <= host.maxlevel && region_level == 0; ++level) {
+        nodes /= std::max(host.max_m, 2);
+        if (a.nq >= 4.0 * nodes) region_level = level;
+      }
+    }
     if (in_order) {
       d_entry.reserve((size_t)a.nq);
-      d_order.reserve((size_t)a.nq);
-      d_order_hist.reserve((size_t)kOrderBuckets);
+      d_order.reserve((size_t)a.nq * (region_level > 0 ? 2 : 1));
+      d_order_hist.reserve(kOrderWords);
     }
     if (keep_trails) {
       d_redo_trail.reserve((size_t)a.nq);
@@ -195,7 +212,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       a.repeats = ctl + 32;
       a.done = ctl + 64;
     } else {
-      const int n_hist = in_order ? kOrderBuckets : 0;
+      const int n_hist = in_order ? kOrderWords : 0;
       const int n_fill = std::max(std::max(a.nq, n_hist), 128);
       hipLaunchKernelGGL(prepare_search_kernel, dim3((unsigned)((n_fill + 255) / 256)), dim3(256), 0, stream, d_ctl.p, 128,
                          d_redo.p, a.nq, in_order ? d_order_hist.p : nullptr, n_hist);
@@ -226,6 +243,12 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       a.entry = d_entry.p;
       a.order = d_order.p;
       a.order_hist = d_order_hist.p;
+      int* const cut = d_order_hist.p + 2 * kOrderBuckets + 32 * (kShares + 1);
+      if (region_level > 0) {
+        a.regions = d_order.p + a.nq;
+        a.region_level = region_level;
+        a.shares = d_order_hist.p + 2 * kOrderBuckets;
+      }
       if constexpr (QR == 1 || QR == 2) {
         // four queries per wavefront, one per group of 16 lanes
         auto k_entry = entry4_kernel<DT, QR>;
@@ -238,10 +261,19 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
         hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), entry_lds, stream, ix, a);
       }
       HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(order_prefix_kernel, dim3(1), dim3(1024), 0, stream, d_order_hist.p);
+      const dim3 per_query((unsigned)((a.nq + 1023) / 1024));
+      int* const region_hist = d_order_hist.p + kOrderBuckets;
+      hipLaunchKernelGGL(order_prefix_kernel, dim3(1), dim3(1024), 0, stream, d_order_hist.p, std::max(1, a.nq / kLongestOf),
+                         a.regions ? cut : nullptr);
       HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(order_scatter_kernel, dim3((unsigned)((a.nq + 1023) / 1024)), dim3(1024), 0, stream, d_entry.p,
-                         a.nq, d_order_hist.p, d_order.p);
+      if (a.regions) {
+        hipLaunchKernelGGL(region_count_kernel, per_query, dim3(1024), 0, stream, d_entry.p, a.regions, a.nq, cut, region_hist);
+        HIP_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(region_prefix_kernel, dim3(1), dim3(1024), 0, stream, region_hist, cut);
+        HIP_CHECK(hipGetLastError());
+      }
+      hipLaunchKernelGGL(order_scatter_kernel, per_query, dim3(1024), 0, stream, d_entry.p, a.regions, cut, a.nq, d_order_hist.p, region_hist,
+                         d_order.p);
       HIP_CHECK(hipGetLastError());
     }
     if (alone) {

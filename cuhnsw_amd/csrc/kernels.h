@@ -28,6 +28,8 @@ namespace cuhnsw_amd {
 
 // what the entries of the list of given-up queries hold that never come: the first pass is through
 constexpr int kListEnds = -2;
+// chiplets with an L2 each
+constexpr int kShares = 8;
 
 struct SlotPool {
   uint32_t* bitmaps;
@@ -79,7 +81,12 @@ struct SearchArgs {
   // null = queries in the caller's order, each descending from the top level itself.
   uint4* entry;     // per query: level-0 entry point, its key (bits), evaluations and sweeps of the descent
   int* order_hist;  // kOrderBuckets counters, then cursors
-  int* order;       // nq query indices, largest entry key first
+  int* order;       // nq query indices, in the order they are taken
+  // Large batches besides: all but the longest queries by region (see below); null / 0 = largest entry key first throughout
+  int* regions;      // the region each query falls into
+  int region_level;  // the level at which the node its descent leaves says so
+  int* shares;       // kShares + 1 work queue heads, 32 words apart: one over the longest queries, then one over each share of
+                     // the others; behind them, how many the longest are
   // Trails of the sorted-set pass (device_core.h, struct Trail), all null / 0 = none are kept.  Buffer b holds
   // trail_cap records from trail + b * trail_cap on; wavefront w of the sorted-set pass starts on buffer w and,
   // each time it hands over a query whose trail the literal pass is to read, goes on with the next unused one
@@ -207,13 +214,27 @@ __host__ __device__ inline FastLdsPlan plan_fast_lds(int qr, int Dp, int lcap, i
 // query would do anyway), the queries are put in descending order of their entry key (a counting sort on the
 // key's leading bits: order_prefix_kernel, order_scatter_kernel) and the first pass takes them in that order.
 // The answers do not depend on the order in which queries are taken.
+//
+// Neighbours together: a batch of three rounds and more is bound by the rows its searches fetch (1 M x 96, 100 000
+// queries: 48 GB in 9.7 ms, next to none of it from the L2 caches), and queries next to each other search among the same
+// rows.  So only the fifth with the largest entry keys goes first and longest first; the others go by region -- the node at
+// which their descent leaves an upper level -- and every chiplet, which has an L2 of its own, takes them from an eighth of
+// its own, then helps the others.  (In turn with longest first throughout: 1 M x 96, ef 256, 100 000 queries 9.76 -> 9.37
+// ms; 1.18 M x 50, ef 300, 40 000 queries 3.96 -> 3.69; 500 000 x 128, ef 300, 30 000 queries 5.70 -> 5.58; 100 000 x 960,
+// 8 000 queries 4.83 -> 4.63.  A twentieth or a tenth first: 4 to 12 % better on some of these, 8 % worse on 500 000 x 128,
+// whose last round then has long queries in it.  1.18 M x 50, 10 000 queries, 1.4 rounds: 1.32 -> 1.48.)
+constexpr int kLongestOf = 5;
 constexpr int kOrderBits = 14;
 constexpr int kOrderBuckets = 1 << kOrderBits;
+// counters of the keys and of the regions, the work queue heads, and where the longest queries end (bucket, number)
+constexpr int kOrderWords = 2 * kOrderBuckets + 32 * (kShares + 1) + 32;
 // bucket 0 holds the largest keys (the float's bits made monotone, leading bits, reversed)
 __device__ __forceinline__ int order_bucket(uint32_t key_bits) {
   const uint32_t u = key_bits ^ ((key_bits >> 31) ? 0xFFFFFFFFu : 0x80000000u);
   return (kOrderBuckets - 1) - (int)(u >> (32 - kOrderBits));
 }
+// neighbouring queries in neighbouring places: any order of the regions will do
+__device__ __forceinline__ int region_bucket(uint32_t node) { return (int)((node * 2654435761u) >> (32 - kOrderBits)); }
 template <int DT, int QR>
 __global__ void __launch_bounds__(64) entry_kernel(DevIndex ix, SearchArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -232,10 +253,14 @@ __global__ void __launch_bounds__(64) entry_kernel(DevIndex ix, SearchArgs a) {
     st.n_dist_upper = 0; st.n_sweeps = 0;
     uint32_t cur = ix.enterpoint;
     float dcur = dist_single<DT, QR>(ix, qv, cur, s, lane);
-    descend<DT, QR>(ix, qv, ix.maxlevel, 0, cur, dcur, s, st, lane);
+    const int region_level = a.region_level < ix.maxlevel ? a.region_level : ix.maxlevel;
+    descend<DT, QR>(ix, qv, ix.maxlevel, region_level > 0 ? region_level - 1 : 0, cur, dcur, s, st, lane);
+    const uint32_t region = cur;
+    if (region_level > 1) descend<DT, QR>(ix, qv, region_level - 1, 0, cur, dcur, s, st, lane);
     if (lane == 0) {
       const uint32_t bits = __float_as_uint(dcur);
       a.entry[qi] = make_uint4(cur, bits, (uint32_t)st.n_dist_upper, (uint32_t)st.n_sweeps);
+      if (a.regions) a.regions[qi] = region_bucket(region);
       atomicAdd(a.order_hist + order_bucket(bits), 1);
     }
     wave_sync();
@@ -281,6 +306,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
     int level = ix.maxlevel;
     bool active = have && level > 0;
     int sweeps = 0, evals = 0;
+    uint32_t region = cur;
     while (__ballot(active) != 0ull) {
       const uint32_t* row = ix.linksU + (size_t)(ix.upper_off[active ? cur : ix.enterpoint] + (active ? level : 1) - 1) * ix.SU;
       float best = INFINITY;
@@ -317,6 +343,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
           dcur = best;
           cur = best_id;  // and sweep again on this level
         } else {
+          if (level == a.region_level) region = cur;
           level -= 1;
           active = level > 0;
         }
@@ -325,6 +352,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
     if (have && sub == 0) {
       const uint32_t bits = __float_as_uint(dcur);
       a.entry[qi] = make_uint4(cur, bits, (uint32_t)evals, (uint32_t)sweeps);
+      if (a.regions) a.regions[qi] = region_bucket(region);
       atomicAdd(a.order_hist + order_bucket(bits), 1);
     }
   }
@@ -334,8 +362,10 @@ __global__ void __launch_bounds__(64) entry4_kernel(DevIndex ix, SearchArgs a) {
   if (uni(ix.half) != 0) entry4_body<DT, QR, true>(ix, a);
   else entry4_body<DT, QR, false>(ix, a);
 }
-// counters -> first position of every bucket (exclusive prefix sum; one workgroup of 1024)
-static __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist) {
+// counters -> first position of every bucket (exclusive prefix sum over `from` and what lies before; one workgroup of 1024).
+// cut: the longest queries end with the first bucket at which there are `most` of them or more; set to that bucket and to
+// their number.
+__device__ __forceinline__ void order_prefix(int* hist, int from, int most, int* cut) {
   __shared__ int part[1024];
   constexpr int per = kOrderBuckets / 1024;
   const int t = threadIdx.x;
@@ -354,33 +384,54 @@ static __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist) {
     part[t] += add;
     __syncthreads();
   }
-  int run = part[t] - sum;
+  int run = part[t] - sum + from;
 #pragma unroll
   for (int i = 0; i < per; ++i) {
     hist[t * per + i] = run;
+    if (cut && run < most && run + local[i] >= most) {
+      cut[0] = t * per + i;
+      cut[1] = run + local[i];
+    }
     run += local[i];
   }
 }
-static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4* entry, int nq, int* cursor, int* order) {
+static __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist, int most, int* cut) { order_prefix(hist, 0, most, cut); }
+static __global__ void __launch_bounds__(1024) region_prefix_kernel(int* hist, const int* cut) { order_prefix(hist, cut[1], 0, nullptr); }
+// how many queries that are not among the longest each region has
+static __global__ void __launch_bounds__(1024) region_count_kernel(const uint4* entry, const int* regions, int nq, const int* cut, int* hist) {
+  const int qi = blockIdx.x * 1024 + threadIdx.x;
+  if (qi < nq && order_bucket(entry[qi].y) > cut[0]) atomicAdd(hist + regions[qi], 1);
+}
+// Queries to their places: by entry key, or (regions) only the longest of them and the others by region.
+static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4* entry, const int* regions, const int* cut, int nq, int* cursor,
+                                                                    int* region_cursor, int* order) {
   // The keys of a batch fall into a few dozen buckets: a workgroup ranks its 1024 queries in LDS and takes one
   // range per bucket it met from the global cursors (the order inside a bucket is free).
   __shared__ int cnt[kOrderBuckets];
   const int t = threadIdx.x;
-  for (int i = t; i < kOrderBuckets; i += 1024) cnt[i] = 0;
-  __syncthreads();
   const int qi = blockIdx.x * 1024 + t;
-  int bucket = 0, rank = 0;
-  if (qi < nq) {
-    bucket = order_bucket(entry[qi].y);
-    rank = atomicAdd(&cnt[bucket], 1);
+  const int last = regions ? cut[0] : kOrderBuckets;
+  for (int part = 0; part < (regions ? 2 : 1); ++part) {
+    int* from = part == 0 ? cursor : region_cursor;
+    for (int i = t; i < kOrderBuckets; i += 1024) cnt[i] = 0;
+    __syncthreads();
+    int bucket = 0, rank = 0;
+    bool mine = false;
+    if (qi < nq) {
+      bucket = order_bucket(entry[qi].y);
+      mine = (bucket <= last) == (part == 0);
+      if (part == 1) bucket = regions[qi];
+      if (mine) rank = atomicAdd(&cnt[bucket], 1);
+    }
+    __syncthreads();
+    for (int i = t; i < kOrderBuckets; i += 1024) {
+      const int c = cnt[i];
+      if (c > 0) cnt[i] = atomicAdd(from + i, c);
+    }
+    __syncthreads();
+    if (mine) order[cnt[bucket] + rank] = qi;
+    __syncthreads();
   }
-  __syncthreads();
-  for (int i = t; i < kOrderBuckets; i += 1024) {
-    const int c = cnt[i];
-    if (c > 0) cnt[i] = atomicAdd(cursor + i, c);
-  }
-  __syncthreads();
-  if (qi < nq) order[cnt[bucket] + rank] = qi;
 }
 
 // A kernel's arguments read afresh from where the launch put them.  The compiler loads every argument once, when the
@@ -428,13 +479,32 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 6 
   // tells a literal pass waiting beside this one that the two kernels do run at the same time
   if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(a0.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int trail_buf = (TRAILS && a0.trail) ? (int)blockIdx.x : -1;  // the buffer this wavefront's trails go to
+  int share_at = 0;  // the queue this wavefront is at (a.shares)
 
   for (;;) {
     int lane = fresh((int)threadIdx.x);
     const SearchArgs& in = fresh_args<SearchArgs>();
     const DevIndex& from = fresh_index();
     int qi = 0;
-    if (lane == 0) {
+    if (!FEW && !TRAILS && in.shares) {
+      // the longest queries, then this chiplet's share of the others, then what is left of the other chiplets'
+      const int longest = in.shares[32 * (kShares + 1) + 1];
+      qi = in.nq;
+      while (share_at <= kShares) {
+        const int share = (int)(__builtin_amdgcn_s_getreg(20 | (31 << 11)) + share_at) & (kShares - 1);  // (XCC_ID, all 32 bits)
+        const long long others = in.nq - longest;
+        const int begin = share_at == 0 ? 0 : longest + (int)(others * share / kShares);
+        const int end = share_at == 0 ? longest : longest + (int)(others * (share + 1) / kShares);
+        int at = 0;
+        if (lane == 0) at = begin + atomicAdd(in.shares + 32 * (share_at == 0 ? 0 : share + 1), 1);
+        at = uni(at);
+        if (at < end) {
+          qi = in.order[at];
+          break;
+        }
+        share_at += 1;
+      }
+    } else if (lane == 0) {
       qi = atomicAdd(in.counter, 1);
       if (qi < in.nq && in.order) qi = in.order[qi];
     }
