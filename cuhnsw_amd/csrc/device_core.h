@@ -962,8 +962,9 @@ __device__ __forceinline__ int max_so_far(int x) {
 // the others), whose list lies in ids / keys (LDS), into a set of `size` entries; what does not fit behind ef entries falls off its end.  The offers are put
 // in order (in ids / keys), every entry finds by halving how many of them go before it, and entries and offers go to their
 // new places through LDS.  `room`: 64 * (NS + 1) words of LDS, whose contents are put back.  Returns false, with nothing
-// done, if two keys are equal (or the node is in the set already), or if the set's largest key would not stay above
-// `above`: those go in one by one, by the rules for them.  last_key: the set's largest key afterwards.
+// done, if two keys are equal (or the node is in the set already), also if one of them is the set's last then and the other
+// the first to fall off (hnswlib expands both, and its heap says which one leaves), or if the set's largest key would not
+// stay above `above`: those go in one by one, by the rules for them.  last_key: the set's largest key afterwards.
 // (An insert of its own is 39 instructions at ef 300 and 0.2 us of latency, this 200 for 14 offers.  Counting for each entry
 // and each offer what goes before it, offer by offer, was 45 instructions an offer: one query on 100 000 x 50 284 -> 272 us,
 // 1 000 queries there 636 -> 607, of which the full set's share below is half; 1 M x 96, ef 256, 100 000 queries 9.92 ->
@@ -1038,12 +1039,13 @@ __device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned lo
 #pragma unroll
     for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j]);
     const float last = uni(__uint_as_float(room[64 * N - ef + (size + n < ef ? size + n : ef) - 1]));
+    const float fallen = uni(__uint_as_float(room[64 * N]));  // the first to fall off (padding where all of them fit)
     const float prev_last = __builtin_bit_cast(
         float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, f.k[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
 #pragma unroll
     for (int j = 0; j < N; ++j)
       twins |= __ballot(f.k[j] == (j > 0 ? f.k[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(f.k[j]) < INFINITY);
-    done = twins == 0ull && last > above;
+    done = twins == 0ull && last > above && last != fallen;
     if (!done) {
 #pragma unroll
       for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j + before[j]]);

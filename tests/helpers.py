@@ -34,6 +34,42 @@ def ring_graph(n, max_m0, hops=(1, 2)):
   return links0
 
 
+def graph_cut_between_equals(rng, ef, width):
+  """(coordinates on a line, level-0 links) of a graph on which the search for the origin from node 0 fills its set of ef
+  entries and then expands a node that offers as many closer entries as there are beyond one of the set, E, and among them
+  O, as far from the origin as E.  E is the set's last entry then and O the first outside it, or the other way round; only O
+  leads to the last node, the nearest of all.  At most `width` links a node; squared distances are exact."""
+  chain = -(-(ef - 1) // width)                  # nodes that bring the set's entries in, the next one and in the end the offers
+  m = int(rng.integers(2, min(width, ef - chain) - 1))      # offers beside O, and entries beyond E (node 0 the farthest)
+  lows = ef - chain - m - 1                      # entries closer than E
+  places = np.sort(2 * rng.choice(np.arange(50, 50 + 3 * (lows + 2 * m + 1)), lows + 2 * m + 1, replace=False))
+  closer, e, beyond = rng.permutation(places[:lows + m]), places[lows + m], places[lows + m + 1:]
+  coordinates, rows = [], []
+
+  def add(distance, side=None):
+    coordinates.append(int(distance) * (side or int(rng.choice([-1, 1]))))
+    rows.append([0])                             # (back to where the search began: nothing new)
+    return len(rows) - 1
+
+  add(beyond[-1])
+  entries = [(v, None) for v in np.concatenate([closer[:lows], beyond[:-1]])] + [(e, 1)]
+  entries = [entries[i] for i in rng.permutation(len(entries))]
+  at = 0
+  for step in range(chain):
+    nb = [add(*v) for v in entries[:width - 1]]
+    entries = entries[width - 1:]
+    nb.insert(int(rng.integers(0, len(nb) + 1)), add(3 + 2 * (chain - step)))
+    rows[at], at = nb, max(nb, key=lambda i: -abs(coordinates[i]))
+  assert not entries and len(rows) == ef
+  nb = [add(v) for v in closer[lows:]]
+  o = add(e, -1)
+  nb.insert(int(rng.integers(0, m)), o)          # (not the last, when the bound has come down to E)
+  rows[at] = nb
+  rows[o] = [0, len(rows)]
+  add(1)
+  return coordinates, rows
+
+
 def recall(found_ids, truth_ids):
   k = truth_ids.shape[1]
   return float(np.mean([len(set(a) & set(b)) / k for a, b in zip(found_ids, truth_ids)]))

@@ -1,17 +1,21 @@
 """A model of how a list of offers enters the sorted set in one go (frontier_insert_all of device_core.h), step by step as the
 lanes do it: the offers put in order, each entry's count of offers before it found by halving, each offer's place from the
-last entry of every count, everything moved through 64 * (NS + 1) words."""
+last entry of every count, everything moved through 64 * (NS + 1) words.  Equal keys send the offers the other way, also
+where the set's end comes between the two; below that the dropped ones are no candidates any more."""
 import numpy as np
 import pytest
 
 
-def insert_all(ns, ef, size, held, offers):
-  """(the set afterwards, or None where equal keys send the offers the other way; every index that was written or read)"""
+def insert_all(ns, ef, size, held, ids, offers, offer_ids):
+  """(keys and ids of the set afterwards, or None where equal keys send the offers the other way; every index of the
+  offers' list that was read)"""
   total, n = 64 * ns, len(offers)
   touched = []
   less = np.array([np.count_nonzero(offers < k) for k in offers])
   keys = np.where(np.arange(64) < n, -np.inf, np.inf).astype(np.float32)
   keys[less] = offers
+  listed = np.zeros(64, int)
+  listed[less] = offer_ids
   if np.isneginf(keys).any():
     return None, touched
   before = np.zeros(total, int)
@@ -21,20 +25,28 @@ def insert_all(ns, ef, size, held, offers):
     before += np.where(keys[before + half - 1] < held, half, 0)
     half >>= 1
   assert max(touched) < 64
-  room = np.zeros(total + 64, np.float64)
+  room, room_ids = np.full(total + 64, np.nan, np.float32), np.zeros(total + 64, int)
   counts = np.zeros(64, int)
   last_of_its_count = np.append(before[1:] != before[:-1], True)
   counts[before[last_of_its_count]] = np.flatnonzero(last_of_its_count) + 1
   place = np.maximum.accumulate(counts)[:n] + np.arange(n)
   to = np.arange(total) + before
   assert len(set(to) | set(place)) == total + n and max(to.max(), place.max()) < total + 64
-  room[to] = held
-  room[place] = keys[:n]
+  room[to], room_ids[to] = held, ids
+  room[place], room_ids[place] = keys[:n], listed[:n]
   after = room[:total]
   finite = np.isfinite(after)
-  if (after[1:] == after[:-1])[finite[1:]].any():
+  last = room[total - ef + min(size + n, ef) - 1]
+  if (after[1:] == after[:-1])[finite[1:]].any() or room[total] == last:
     return None, touched
-  return after.astype(np.float32), touched
+  return (after, room_ids[:total]), touched
+
+
+def in_the_set(ns, ef, entries):
+  held = np.full(64 * ns, np.inf, np.float32)
+  held[:64 * ns - ef] = -np.inf
+  held[64 * ns - ef:64 * ns - ef + len(entries)] = entries
+  return held
 
 
 @pytest.mark.parametrize("ns,ef", [(2, 65), (2, 128), (3, 150), (4, 256), (5, 300), (8, 512)])
@@ -52,18 +64,32 @@ def test_merged_lists_are_the_smallest_of_both(ns, ef):
     entries = np.sort(entries)
     size = len(entries)
     offers = draw(n) - (np.float32(9) if case % 5 == 0 else np.float32(0))
-    held = np.full(64 * ns, np.inf, np.float32)
-    held[:64 * ns - ef] = -np.inf
-    held[64 * ns - ef:64 * ns - ef + size] = entries
-    after, _ = insert_all(ns, ef, size, held, offers)
-    both = np.sort(np.concatenate([entries, offers]))
-    if len(set(both)) < len(both):
-      # (equal keys: refused, unless all but one of them fell off the end)
-      if after is None:
-        continue
-      both = np.sort(np.unique(both))
-    assert after is not None
-    want = both[:ef]
+    held = in_the_set(ns, ef, entries)
+    ids = np.full(64 * ns, -1)
     first = 64 * ns - ef
-    assert (after[first:first + len(want)] == want).all() and (after[:first] == -np.inf).all()
-    assert (after[first + len(want):] == np.inf).all()
+    ids[first:first + size] = np.arange(size)
+    after, _ = insert_all(ns, ef, size, held, ids, offers, 1000 + np.arange(n))
+    both = np.concatenate([entries, offers])
+    order = np.argsort(both, kind="stable")
+    inside = both[order][:ef]
+    bound = inside[-1]
+    within = both[both <= bound]
+    if len(set(within)) < len(within) or len(set(offers)) < n:
+      assert after is None, "equal keys within the bound, or of two offers"
+      continue
+    assert after is not None
+    assert (after[0][first:first + len(inside)] == inside).all() and (after[0][:first] == -np.inf).all()
+    assert (after[0][first + len(inside):] == np.inf).all()
+    assert (after[1][first:first + len(inside)] == np.concatenate([np.arange(size), 1000 + np.arange(n)])[order][:ef]).all()
+
+
+@pytest.mark.parametrize("at", range(7))
+def test_equal_keys_on_both_sides_of_the_sets_end_are_refused(at):
+  """The dropped one is as close as the bound: a candidate still, which the offer would be lost as."""
+  ns, ef = 3, 150
+  entries = np.arange(10, 1510, 10).astype(np.float32)
+  offers = np.insert(np.arange(5, 65, 10).astype(np.float32), at, np.float32(1440))
+  held = in_the_set(ns, ef, entries)
+  assert insert_all(ns, ef, ef, held, np.arange(64 * ns), offers, np.arange(7))[0] is None
+  offers[at] = 1450  # (pushed out together with its equal: beyond the bound, both dead)
+  assert insert_all(ns, ef, ef, held, np.arange(64 * ns), offers, np.arange(7))[0] is not None

@@ -16,12 +16,16 @@ on the order in which a followed-through group was expanded, which is what the r
 import numpy as np
 import pytest
 
+from helpers import graph_cut_between_equals
+
 INF = float("inf")
 
 
-def sorted_set_search(keys_of, rows, ep, k, ef, trail=None):
+def sorted_set_search(keys_of, rows, ep, k, ef, trail=None, together=None, cut_rule=True):
   """Returns None when given up, else (ids, keys, hops, evaluations, met equal keys).  trail: a dict that receives
-  "rec" (the records and markers) and "hops" (the expansions they cover)."""
+  "rec" (the records and markers) and "hops" (the expansions they cover).  together: so many offers of one hop or more
+  enter a full set in one go (frontier_insert_all), unless equal keys forbid it; cut_rule: also those of which one is
+  the set's last entry afterwards and the other the first that was pushed out."""
   tr = {"rec": [], "on": True, "own": False, "hops": 0}
 
   def stop(h):                            # the trail ends: h expansions are complete
@@ -47,6 +51,16 @@ def sorted_set_search(keys_of, rows, ep, k, ef, trail=None):
   offers = []
   while True:
     accepted = []
+    passing = [o for o in offers if S[-1][0] > o[0]]
+    if together is not None and calm and len(S) >= ef and len(passing) >= together:
+      merged = sorted(S + [[key, node, False] for key, node in passing], key=lambda e: e[0])
+      equal = any(a[0] == b[0] for a, b in zip(merged[:ef], merged[1:ef]))
+      equal = equal or len({key for key, _ in passing}) < len(passing)
+      equal = equal or (cut_rule and merged[ef - 1][0] == merged[ef][0])
+      if not equal and not (watch and merged[ef - 1][0] <= max(w[0] for w in watch)):
+        S = merged[:ef]
+        offers = []
+        sorted_set_search.entered_together += 1
     for key, node in offers:
       full = len(S) >= ef
       if full and not (S[-1][0] > key):
@@ -168,6 +182,7 @@ sorted_set_search.answered_after_twins = 0    # (statistics for the test below: 
 sorted_set_search.calmed_down = 0             # (and so has the return to the tie-free loop,
 sorted_set_search.calmed_down_watching = 0    # with and without entries to watch,
 sorted_set_search.calmed_down_past_a_ghost = 0  # and after an eviction out of equal largest keys)
+sorted_set_search.entered_together = 0        # (and offers that entered a full set in one go)
 
 
 def _push_heap(h, value):
@@ -345,21 +360,53 @@ def test_rules_never_let_an_order_dependent_case_through(oracle, seed):
       ids, dists, found, cnt = ix.search(q, k, ef, convention="hnswlib", counters=True)
       for r in range(q.shape[0]):
         keys_of = lambda node, qq=q[r]: float(np.float32(((qq - x[node]) ** 2).sum()))
-        got = sorted_set_search(keys_of, rows, 0, k, ef)
-        if got is None:
-          given_up += 1
-          continue
-        answered += 1
-        m_ids, m_keys, hops, evals, tied = got
-        answered_with_ties += bool(tied)
-        f = found[r]
-        assert f == len(m_ids)
-        assert list(ids[r, :f]) == m_ids, (seed, graph, r, k, ef)
-        assert list(dists[r, :f]) == m_keys
-        assert cnt[r, 1] == hops and cnt[r, 0] == evals, (seed, graph, r, k, ef)
+        for together in (None, 1, 3):
+          got = sorted_set_search(keys_of, rows, 0, k, ef, together=together)
+          if got is None:
+            given_up += together is None
+            continue
+          m_ids, m_keys, hops, evals, tied = got
+          if together is None:
+            answered += 1
+            answered_with_ties += bool(tied)
+          f = found[r]
+          assert f == len(m_ids)
+          assert list(ids[r, :f]) == m_ids, (seed, graph, r, k, ef, together)
+          assert list(dists[r, :f]) == m_keys
+          assert cnt[r, 1] == hops and cnt[r, 0] == evals, (seed, graph, r, k, ef, together)
   # both outcomes are exercised, and so are searches that met equal keys and were still answered, some of them
   # by following the twins of an eviction through
   assert answered > 1000 and given_up > 100 and answered_with_ties > 300, (answered, given_up, answered_with_ties)
   assert sorted_set_search.answered_after_twins > 0
   assert sorted_set_search.calmed_down > 100 and sorted_set_search.calmed_down_watching > 100
   assert sorted_set_search.calmed_down_past_a_ghost > 20
+  assert sorted_set_search.entered_together > 100
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_a_cut_between_two_equal_keys_is_noticed(oracle, seed):
+  """Offers that push a full set's entries out up to one whose equal is among them: hnswlib expands both, and what the
+  equal that was dropped leads to is in the answer.  (Without the rule for the cut nearly every such search is answered
+  wrongly, and none given up.)"""
+  rng = np.random.default_rng(7000 + seed)
+  wrong = {True: 0, False: 0}
+  for _ in range(100):
+    ef = int(rng.integers(10, 30))
+    coordinates, rows = graph_cut_between_equals(rng, ef, width=64)
+    x = np.array(coordinates, np.float32)[:, None]
+    links0 = np.zeros((len(rows), 1 + 64), np.uint32)
+    for i, nb in enumerate(rows):
+      links0[i, 0] = len(nb)
+      links0[i, 1:1 + len(nb)] = nb
+    ix = oracle.OracleIndex("l2").from_arrays(x, np.zeros(len(rows), np.int32), links0, np.zeros(0, np.uint32),
+                                              max_m=32, max_m0=64, maxlevel=0, enterpoint=0)
+    k = int(rng.integers(1, 8))
+    ids, dists, found, cnt = ix.search(np.zeros((1, 1), np.float32), k, ef, convention="hnswlib", counters=True)
+    f = found[0]
+    assert ids[0, 0] == len(rows) - 1          # the nearest is where only the dropped equal leads
+    for cut_rule in (True, False):
+      got = sorted_set_search(lambda node: float(x[node, 0] ** 2), rows, 0, k, ef, together=3, cut_rule=cut_rule)
+      if got is None:
+        continue
+      wrong[cut_rule] += not (got[0] == list(ids[0, :f]) and got[1] == list(dists[0, :f]) and got[2] == cnt[0, 1])
+  assert wrong[True] == 0 and wrong[False] > 60, wrong
