@@ -190,7 +190,8 @@ class Engine {
   bool trails_unavailable = false;  // the trail buffers could not be allocated: searches go on without trails
   int filter_entries = 0;  // entries of the sorted-set search's visited filter (0 = automatic)
   int first_pass_waves = 0;  // wavefronts per CU of the first pass (0 = as many as fit)
-  int query_order = 1;     // first pass of 1.5 to 32 rounds of wavefronts: longest queries first (0: caller's order)
+  int query_order = 1;     // first pass of 1.5 to 32 rounds of wavefronts: longest queries first, those of large batches by
+                           // region (3: not those; 2: both whatever the sizes; 0: caller's order)
   bool fast_suspended = false;  // this index ties too often for the sorted-set search to pay (integer data)
   int lean_literal = 1;  // literal pass: 0 = always the exact visited bitmap, 1 = automatic, 2 = always the LDS filter
   bool storage_half = false;  // vectors live in HBM as fp16 (set before set_data / load_index)

@@ -216,13 +216,13 @@ __host__ __device__ inline FastLdsPlan plan_fast_lds(int qr, int Dp, int lcap, i
 // The answers do not depend on the order in which queries are taken.
 //
 // Neighbours together: a batch of three rounds and more is bound by the rows its searches fetch (1 M x 96, 100 000
-// queries: 48 GB in 9.7 ms, next to none of it from the L2 caches), and queries next to each other search among the same
-// rows.  So only the fifth with the largest entry keys goes first and longest first; the others go by region -- the node at
-// which their descent leaves an upper level -- and every chiplet, which has an L2 of its own, takes them from an eighth of
-// its own, then helps the others.  (In turn with longest first throughout: 1 M x 96, ef 256, 100 000 queries 9.76 -> 9.37
-// ms; 1.18 M x 50, ef 300, 40 000 queries 3.96 -> 3.69; 500 000 x 128, ef 300, 30 000 queries 5.70 -> 5.58; 100 000 x 960,
-// 8 000 queries 4.83 -> 4.63.  A twentieth or a tenth first: 4 to 12 % better on some of these, 8 % worse on 500 000 x 128,
-// whose last round then has long queries in it.  1.18 M x 50, 10 000 queries, 1.4 rounds: 1.32 -> 1.48.)
+// queries, longest first: 60 GB in 9.6 ms, two L2 requests in a hundred hits), and queries next to each other search among
+// the same rows (by region: 51 GB in 9.0 ms, 17 in a hundred).  So only the fifth with the largest entry keys goes first and
+// longest first; the others go by region -- the node at which their descent leaves an upper level -- and every chiplet,
+// which has an L2 of its own, takes them from an eighth of its own, then helps the others.  (Which batches: launch_search,
+// with both sides.  A tenth first instead of a fifth: 1.18 M x 50, 40 000 queries 3.92 -> 4.11 ms, 10 M x 96, ef 256, 100 000 13.56 ->
+// 13.80, 500 000 x 128, 30 000 5.46 -> 5.70; a third: 300 000 x 128, ef 200, 50 000 5.14 -> 5.29, 100 000 x 960, 8 000 4.62 ->
+// 4.79, but 1.18 M x 80, 60 000 6.69 -> 6.51.  1.18 M x 50, 10 000 queries, 1.4 rounds, by region: 1.32 -> 1.48.)
 constexpr int kLongestOf = 5;
 constexpr int kOrderBits = 14;
 constexpr int kOrderBuckets = 1 << kOrderBits;

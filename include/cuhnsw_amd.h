@@ -206,8 +206,13 @@ int cuhnsw_trails_available(cuhnsw_engine* e);
  *   "query_order"   1 (default) = a search batch of 1.5 to 32 rounds of wavefronts (from one round on where the
  *                   first pass keeps trails) does its upper-level descents
  *                   first and takes its queries by descending distance of their level-0 entry point (the longest
- *                   searches first: a launch ends when its last query does); 2 = from more than one round on;
- *                   0 = in the caller's order.  Same answers and counters either way.
+ *                   searches first: a launch ends when its last query does).  In batches of three rounds and more
+ *                   only a fifth of them goes so, and the others by region of the index, where that brings their rows
+ *                   together in the L2 caches: an index of more than 12 MB, of which the queries at work on a chiplet
+ *                   have 8 MB to themselves or less (16 MB for ef_search <= 128; rows of more than 128 elements: any).
+ *                   2 = from more than one round on, by region from three on; 3 = as 1, but longest first throughout;
+ *                   0 = in the caller's order.
+ *                   Same answers and counters either way.
  *   "first_pass_waves" wavefronts per CU of the first pass (0 = as many as fit, the default)
  *   "concurrent_literal" 1 = the literal pass runs beside the first pass on a second stream
  *                   (default), 0 = after it

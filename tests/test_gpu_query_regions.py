@@ -32,3 +32,23 @@ def test_queries_by_region(oracle, tmp_path, d, dist, max_m):
         g_ids, g_d, g_f, stats = _device_search(e, q, k, ef)
         assert (g_f == o_f).all() and (g_ids == o_ids).all() and (g_d == o_d).all()
         assert (stats[:, 1:] == o_cnt[:, 1:4]).all()
+
+
+@pytest.mark.parametrize("mult", [1 / np.log(24), 1 / np.log(3), 0.0])
+def test_levels_of_another_thickness(oracle, tmp_path, mult):
+  """The level that stands for the regions is found by the nodes it has, not by max_m: many levels, few, none above 0."""
+  n, d, k, ef = 3000, 24, 10, 80
+  x = gauss_mixture(n, d, seed=31)
+  ix = oracle.OracleIndex("dot").build(x, _levels(n, mult, 32), 12, 24, 60, max(mult, 0.1))
+  p = str(tmp_path / "i.idx")
+  ix.save(p)
+  e = _engine(tmp_path, dist_type="dot", max_m=12, max_m0=24)
+  e.load_index(p)
+  q = gauss_mixture(2000, d, seed=33)
+  o_ids, o_d, o_f, o_cnt = ix.search(q, k, ef, counters=True)
+  e.set_tunable("search_slots", 64)
+  for order in (1, 2, 3):
+    e.set_tunable("query_order", order)
+    g_ids, g_d, g_f, stats = _device_search(e, q, k, ef)
+    assert (g_f == o_f).all() and (g_ids == o_ids).all() and (g_d == o_d).all()
+    assert (stats[:, 1:] == o_cnt[:, 1:4]).all()
