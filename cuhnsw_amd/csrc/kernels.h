@@ -459,7 +459,9 @@ __device__ __forceinline__ const Args& fresh_args() {
 // held to 72 registers, seven wavefronts per SIMD, at the price of up to eight spilled registers, none of them
 // touched inside a hop loop, but for six keys; eight wavefronts are no faster, six are 0 to 3 % slower there (ef 350);
 // with seven and eight keys per lane it fits 96 registers, five wavefronts per SIMD: with six of them ef 430 is 2 % slower
-// to 5 % faster and ef 512 a fifth slower; the other shapes would spill heavily)
+// to 5 % faster and ef 512 a fifth slower; the other shapes would spill heavily.  129 to 256 elements in L2 with five keys
+// per lane would take one register too many for five wavefronts: 100 000 x 180 in fp16, ef 300, 40 000 queries 5.43 -> 4.87
+// ms, in fp32 5.33 -> 4.94, 150 000 x 250 6.26 -> 6.34.  Not with two keys, six wavefronts or seven: 4.73 and 4.77 at ef 128.)
 // TRAILS: the pass leaves trails for the literal pass (a.trail set; 2 to 3 % more instructions: the host launches
 // this instance for batches of a round or two of wavefronts, where a query handed over late is a good part of the
 // batch's time, and the instance without the trail code otherwise).
@@ -467,7 +469,7 @@ __device__ __forceinline__ const Args& fresh_args() {
 // candidates at a time, with the registers that takes (100 000 x 50, ef 300, one query: 0.290 -> 0.278 ms; 100 000 x 960,
 // ef 300, 1 000 queries: 1.35 -> 1.29).
 template <int DT, int QR, int NS, bool TRAILS, bool FEW = false>
-__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 6 ? 7 : (NS <= 8 ? 5 : 1)) : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
+__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 6 ? 7 : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
   Scratch s;

@@ -42,6 +42,7 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_DOT, 1, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,5,few>"),
     ("search_fast_kernel<DIST_L2, 2, 2, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2,few>"),
     ("search_fast_kernel<DIST_L2, 0, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,5,few>"),
+    ("search_fast_kernel<DIST_L2, 4, 5, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,4,5>"),
 ]
 OTHERS = [
     ("search_kernel<DIST_DOT, 1, 5>(DevIndex, SearchArgs)", "search_kernel<dot,1,5>"),

@@ -28,6 +28,7 @@ LIMITS = {
     "search_fast_kernel<dot,1,5,few>": (1, 0),
     "search_fast_kernel<l2,2,2,few>": (1, 0),
     "search_fast_kernel<l2,0,5,few>": (1, 0),
+    "search_fast_kernel<l2,4,5>": (5, 20),
 }
 
 
