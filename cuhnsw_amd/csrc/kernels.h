@@ -456,9 +456,13 @@ __device__ __forceinline__ const Args& fresh_args() {
 // A query in which two equal keys meet is not answered here: its index is appended to
 // a.redo (a.repeats counts them) and the literal search_kernel answers it afterwards.
 // (with at most six keys per lane and the query in at most two float4 registers the kernel is
-// held to 72 registers, seven wavefronts per SIMD, at the price of up to eight spilled registers, none of them
-// touched inside a hop loop, but for six keys; eight wavefronts are no faster, six are 0 to 3 % slower there (ef 350);
-// with seven and eight keys per lane it fits 96 registers, five wavefronts per SIMD: with six of them ef 430 is 2 % slower
+// held to 72 registers, seven wavefronts per SIMD, at the price of up to nine spilled registers, none of them
+// touched inside a hop loop; eight wavefronts are no faster.  Six keys per lane spill up to 19, and where their reloads are
+// in the loop six wavefronts are the better ones, fast_waves_of_six: 400 000 x 50, ef 330, 40 000 queries 4.05 -> 3.92 ms,
+// 10 000 with trails 1.66 -> 1.63, 300 000 x 60 L2 1.59 -> 1.44, x 100 1.92 -> 1.86; seven stay where they are not, 300 000 x
+// 60 L2, 40 000 3.33 against 3.50, 200 000 x 128 L2 7.51 against 8.05, or are few, 400 000 x 96 4.64 against 4.69 and, with
+// trails, 1.67 against 1.72.
+// With seven and eight keys per lane it fits 96 registers, five wavefronts per SIMD: with six of them ef 430 is 2 % slower
 // to 5 % faster and ef 512 a fifth slower; the other shapes would spill heavily.  129 to 256 elements in L2 with five keys
 // per lane would take one register too many for five wavefronts: 100 000 x 180 in fp16, ef 300, 40 000 queries 5.43 -> 4.87
 // ms, in fp32 5.33 -> 4.94, 150 000 x 250 6.26 -> 6.34.  Not with two keys, six wavefronts or seven: 4.73 and 4.77 at ef 128.)
@@ -468,8 +472,9 @@ __device__ __forceinline__ const Args& fresh_args() {
 // FEW: for batches that leave the machine idle, at most a wavefront per SIMD: twice the rows in flight and more
 // candidates at a time, with the registers that takes (100 000 x 50, ef 300, one query: 0.290 -> 0.278 ms; 100 000 x 960,
 // ef 300, 1 000 queries: 1.35 -> 1.29).
+constexpr int fast_waves_of_six(int dt, int qr, bool trails) { return (dt == DIST_DOT ? qr == 1 : trails) ? 6 : 7; }
 template <int DT, int QR, int NS, bool TRAILS, bool FEW = false>
-__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 6 ? 7 : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
+__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : NS == 6 ? fast_waves_of_six(DT, QR, TRAILS) : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
   Scratch s;

@@ -14,6 +14,7 @@ cuhnsw_amd/build.py records the remarks of the library's own build, for every ke
 profiles/kernel_resources.json; tests/test_kernel_resources.py compiles the first-pass kernels with this module
 and fails when one of them loses a wavefront per SIMD, spills more, or gains a scratch access inside its hop loop.
 """
+import concurrent.futures
 import os
 import re
 import subprocess
@@ -43,6 +44,21 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_L2, 2, 2, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2,few>"),
     ("search_fast_kernel<DIST_L2, 0, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,5,few>"),
     ("search_fast_kernel<DIST_L2, 4, 5, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,4,5>"),
+    ("search_fast_kernel<DIST_DOT, 1, 3, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,3>"),
+    ("search_fast_kernel<DIST_DOT, 1, 4, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,4>"),
+    ("search_fast_kernel<DIST_DOT, 2, 4, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,4>"),
+    ("search_fast_kernel<DIST_L2, 2, 3, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,3>"),
+    ("search_fast_kernel<DIST_L2, 2, 4, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,4>"),
+    ("search_fast_kernel<DIST_L2, 2, 4, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,4,trails>"),
+    ("search_fast_kernel<DIST_DOT, 1, 6, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,6>"),
+    ("search_fast_kernel<DIST_L2, 1, 6, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,1,6>"),
+    ("search_fast_kernel<DIST_DOT, 2, 6, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,6>"),
+    ("search_fast_kernel<DIST_L2, 2, 6, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,6>"),
+    ("search_fast_kernel<DIST_L2, 2, 6, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,6,trails>"),
+    ("search_fast_kernel<DIST_DOT, 1, 7, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,7>"),
+    ("search_fast_kernel<DIST_L2, 2, 7, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,7>"),
+    ("search_fast_kernel<DIST_DOT, 2, 4, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,4,few>"),
+    ("search_fast_kernel<DIST_L2, 0, 6, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,6,few>"),
 ]
 OTHERS = [
     ("search_kernel<DIST_DOT, 1, 5>(DevIndex, SearchArgs)", "search_kernel<dot,1,5>"),
@@ -191,31 +207,34 @@ def loop_scratch_accesses(isa_text, mangled):
   return in_loops, total
 
 
-def compile_kernels(instances):
-  """Compiles each kernel instance on its own; returns {short name: resource dict}."""
-  out = {}
+def _compile_kernel(text, short):
   with tempfile.TemporaryDirectory(prefix="cuhnsw_kr_") as tmp:
-    for text, short in instances:
-      src = os.path.join(tmp, "k.hip")
-      asm = os.path.join(tmp, "k.s")
-      with open(src, "w") as f:
-        f.write('#include "kernels.h"\nusing namespace cuhnsw_amd;\ntemplate __global__ void cuhnsw_amd::%s;\n' % text)
-      r = subprocess.run([HIPCC] + DEVICE_FLAGS + ["-I" + CSRC, "--cuda-device-only", "-S", "-x", "hip", src, "-o", asm,
-                                                   "-Rpass-analysis=kernel-resource-usage"],
-                         capture_output=True, text=True)
-      if r.returncode != 0:
-        raise RuntimeError("hipcc failed on %s:\n%s" % (short, r.stderr[-2000:]))
-      base = text.split("<")[0]
-      mangled = [k for k in parse_remarks(r.stderr) if base in k]
-      if len(mangled) != 1:
-        raise RuntimeError("%s: expected one kernel named %s, found %r" % (short, base, mangled))
-      info = dict(parse_remarks(r.stderr)[mangled[0]])
-      with open(asm) as f:
-        in_loops, total = loop_scratch_accesses(f.read(), mangled[0])
-      info["scratch_instructions"] = total
-      info["scratch_instructions_in_hop_loops"] = in_loops
-      out[short] = info
-  return out
+    src = os.path.join(tmp, "k.hip")
+    asm = os.path.join(tmp, "k.s")
+    with open(src, "w") as f:
+      f.write('#include "kernels.h"\nusing namespace cuhnsw_amd;\ntemplate __global__ void cuhnsw_amd::%s;\n' % text)
+    r = subprocess.run([HIPCC] + DEVICE_FLAGS + ["-I" + CSRC, "--cuda-device-only", "-S", "-x", "hip", src, "-o", asm,
+                                                 "-Rpass-analysis=kernel-resource-usage"],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+      raise RuntimeError("hipcc failed on %s:\n%s" % (short, r.stderr[-2000:]))
+    base = text.split("<")[0]
+    mangled = [k for k in parse_remarks(r.stderr) if base in k]
+    if len(mangled) != 1:
+      raise RuntimeError("%s: expected one kernel named %s, found %r" % (short, base, mangled))
+    info = dict(parse_remarks(r.stderr)[mangled[0]])
+    with open(asm) as f:
+      in_loops, total = loop_scratch_accesses(f.read(), mangled[0])
+  info["scratch_instructions"] = total
+  info["scratch_instructions_in_hop_loops"] = in_loops
+  return info
+
+
+def compile_kernels(instances):
+  """Compiles each kernel instance on its own, side by side; returns {short name: resource dict}."""
+  workers = max(1, min(len(instances), len(os.sched_getaffinity(0)), int(os.environ.get("MAX_JOBS") or 8)))
+  with concurrent.futures.ThreadPoolExecutor(workers) as pool:
+    return dict(zip([short for _, short in instances], pool.map(lambda i: _compile_kernel(*i), instances)))
 
 
 def main():
