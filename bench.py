@@ -239,7 +239,8 @@ def main():
   ap.add_argument("--fast-path", type=int, default=1, choices=[0, 1, 2],
                   help="0 = literal priority queues only, 1 = default, 2 = sorted-set first pass whatever the batch size")
   ap.add_argument("--query-order", type=int, default=1, choices=[0, 1, 2, 3],
-                  help="0 = queries in the caller's order, 1 = longest first from one to one and a half rounds of wavefronts on, 2 = from one")
+                  help="0 = queries in the caller's order, 1 = longest first from one to one and a half rounds of wavefronts on, large "
+                       "batches by region, 2 = both whatever the sizes, 3 = longest first throughout")
   ap.add_argument("--trails", type=int, default=1, choices=[0, 1, 2],
                   help="0 = the literal pass searches handed-over queries from the entry point, 1 = from the first pass's "
                        "trail in batches of up to two rounds of wavefronts (default), 2 = in every batch")

@@ -25,15 +25,11 @@ void HostIndex::layout_upper() {
   SU = strideU(max_m);
   upper_off.resize(N);
   int64_t rows = 0;
-  std::fill(nodes_at, nodes_at + kCountedLevels, 0);
   for (int i = 0; i < N; ++i) {
     upper_off[i] = levels[i] > 0 ? rows : -1;
     rows += levels[i];
-    if (levels[i] > 0) ++nodes_at[std::min(levels[i], kCountedLevels - 1)];
   }
   upper_rows = rows;
-  for (int l = kCountedLevels - 2; l > 0; --l) nodes_at[l] += nodes_at[l + 1];
-  nodes_at[0] = N;
 }
 
 void HostIndex::layout_links() {

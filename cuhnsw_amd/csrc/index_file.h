@@ -27,8 +27,6 @@ struct HostIndex {
   std::vector<int64_t> upper_off;      // N: index of the node's level-1 row in linksU, -1 if none
   std::vector<uint32_t> linksU;        // (sum of levels) x SU; row of (node, level) = upper_off[node] + level - 1
   int64_t upper_rows = 0;
-  static constexpr int kCountedLevels = 32;
-  int64_t nodes_at[kCountedLevels] = {};  // nodes that reach a level (beyond the last: counted there)
   // hnswlib's delete marks (markDelete: bit 0 of the third byte of an element's level-0 count word), one
   // byte per element, or empty when nothing is marked.  A marked element is searched through like any
   // other and never returned.  The reference keeps no such mark: it reads the count word as a plain count
@@ -38,7 +36,7 @@ struct HostIndex {
 
   static int stride0(int max_m0) { return (max_m0 + 31) / 32 * 32; }
   static int strideU(int max_m) { return (max_m + 15) / 16 * 16; }
-  // strides, offsets and numbers of upper rows and nodes from N, levels, max_m, max_m0
+  // strides, offsets and number of upper rows from N, levels, max_m, max_m0
   void layout_upper();
   // the same, and empty link tables on the host (an engine with a GPU keeps its links there)
   void layout_links();

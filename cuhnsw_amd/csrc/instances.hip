@@ -196,8 +196,13 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     const bool by_region = query_order == 2 || (query_order == 1 && index_bytes > kRegionIndexFrom && near_by);
     int region_level = 0;
     if (in_order && !keep_trails && a.nq >= 3 * resident && by_region) {
-      for (int level = 1; level <= std::min(host.maxlevel, HostIndex::kCountedLevels - 1) && region_level == 0; ++level)
-        if (a.nq >= 4 * host.nodes_at[level]) region_level = level;
+      // (a level has this share of the nodes of the one below it: so many upper rows are there for so many nodes)
+      const double share = (double)host.upper_rows / ((double)host.upper_rows + host.N);
+      double nodes = host.N;
+      for (int level = 1; level <= host.maxlevel && region_level == 0; ++level) {
+        nodes *= share;
+        if (a.nq >= 4.0 * nodes) region_level = level;
+      }
     }
     if (in_order) {
       d_entry.reserve((size_t)a.nq);

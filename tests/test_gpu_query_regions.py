@@ -36,7 +36,7 @@ def test_queries_by_region(oracle, tmp_path, d, dist, max_m):
 
 @pytest.mark.parametrize("mult", [1 / np.log(24), 1 / np.log(3), 0.0])
 def test_levels_of_another_thickness(oracle, tmp_path, mult):
-  """The level that stands for the regions is found by the nodes it has, not by max_m: many levels, few, none above 0."""
+  """The level that stands for the regions goes by the levels the nodes have, not by max_m: many, few, none above 0."""
   n, d, k, ef = 3000, 24, 10, 80
   x = gauss_mixture(n, d, seed=31)
   ix = oracle.OracleIndex("dot").build(x, _levels(n, mult, 32), 12, 24, 60, max(mult, 0.1))
