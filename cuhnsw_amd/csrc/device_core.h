@@ -1039,7 +1039,7 @@ __device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned lo
 #pragma unroll
     for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j]);
     const float last = uni(__uint_as_float(room[64 * N - ef + (size + n < ef ? size + n : ef) - 1]));
-    const float fallen = uni(__uint_as_float(room[64 * N]));  // the first to fall off (not SPARSE: none does)
+    const bool cut = SPARSE && uni(__uint_as_float(room[64 * N])) == last;  // with the first to fall off (not SPARSE: none does)
     const float prev_last = __builtin_bit_cast(
         float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, f.k[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
 #pragma unroll
@@ -1047,7 +1047,7 @@ __device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned lo
       twins |= __ballot(f.k[j] == (j > 0 ? f.k[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(f.k[j]) < INFINITY);
     // (the comparison with -inf always holds; without it the instances for six keys a lane and rows of 65 to 128 elements
     // spill five registers more and reload some in the hop loop: 200 000 x 128, ef 330, 40 000 queries 7.51 -> 7.85 ms)
-    done = twins == 0ull && last > -INFINITY && last < fallen;
+    done = twins == 0ull && last > -INFINITY && !cut;
     if (!done) {
 #pragma unroll
       for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j + before[j]]);

@@ -38,7 +38,7 @@ LIMITS = {
     "search_fast_kernel<l2,2,4,trails>": (7, 24),
     "search_fast_kernel<dot,1,6>": (6, 36),
     "search_fast_kernel<l2,1,6>": (7, 48),
-    "search_fast_kernel<dot,2,6>": (7, 56, 3),  # (a few reloads in the loop, and still faster than six wavefronts)
+    "search_fast_kernel<dot,2,6>": (7, 60, 7),  # (a few reloads in the loop, and still faster than six wavefronts)
     "search_fast_kernel<l2,2,6>": (7, 44),
     "search_fast_kernel<l2,2,6,trails>": (6, 20),
     "search_fast_kernel<dot,1,7>": (5, 0),
