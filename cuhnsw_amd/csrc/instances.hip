@@ -182,15 +182,16 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     // 40 000 x 50 (15 MB) 1.98 -> 2.00 and 2.70 -> 2.61, 40 000 x 128 (26 MB) 2.56 -> 2.33.
     // Nor, on rows of up to 128 elements, where the queries that a chiplet has at work lie so far apart that its L2 holds
     // little of what they search: their share of the index is the measure, twice the L2, and four times for the short
-    // searches of ef <= 128, whose hand-overs late in a batch (the price of not going longest first) are short as well.
+    // searches (ef <= 128) of rows of more than 64 elements: hand-overs late in a batch, the price of not going longest
+    // first, are short there as well.
     // Longest first throughout / by region, means over 5 to 40 draws: 1 M x 96, 100 000 queries, ef 256 (4.6 MB) 9.64 /
     // 9.03 ms; 500 000 x 128, 60 000, ef 100 (4.8 MB) 5.56 / 4.87; 1.18 M x 50, ef 300, 100 000 (4 MB) 8.27 / 8.29, 40 000
     // (10 MB) 3.93 / 3.90, 4.04 / 4.16 and 4.11 / 4.00; 1.18 M x 80, ef 300, 25 000 (22 MB) 3.42 / 3.56; 2 M x 96, 22 000, ef 256
     // (41 MB) 3.42 / 3.72; 10 M x 96, ef 256, 100 000 (46 MB) 13.6 / 14.9, 30 000 (153 MB) 5.21 / 5.83; at ef 128 50 000 on
-    // 1 M x 96 (9 MB) 4.47 / 4.15, 40 000 on 1.18 M x 50 (10 MB) 2.56 / 2.44, 100 000 on 3 M x 96 (14 MB) 8.89 / 8.50, but
-    // 30 000 there (46 MB) 3.36 / 3.42.  Longer rows gain however far apart: 1 M x 960, 8 000, ef 300 (135 MB) 11.2 / 10.6.
+    // 1 M x 96 (9 MB) 4.47 / 4.15, 100 000 on 3 M x 96 (14 MB) 8.89 / 8.50, but 30 000 there (46 MB) 3.36 / 3.42, and 40 000 on
+    // 1.18 M x 50 (11 MB) 2.48 / 2.49, at ef 64 1.62 / 1.64.  Longer rows gain however far apart: 1 M x 960, 8 000, ef 300 (135 MB) 11.2 / 10.6.
     constexpr size_t kRegionIndexFrom = (size_t)12 << 20;
-    constexpr size_t kRegionAtWork = (size_t)(NS > 2 ? 8 : 16) << 20;
+    constexpr size_t kRegionAtWork = (size_t)(NS == 2 && QR == 2 ? 16 : 8) << 20;
     const size_t index_bytes = (size_t)host.N * ((size_t)Dp * (storage_half ? 2 : 4) + (size_t)host.S0 * 4);
     const bool near_by = !(QR == 1 || QR == 2) || (double)index_bytes * resident <= (double)kRegionAtWork * kShares * a.nq;
     const bool by_region = query_order == 2 || (query_order == 1 && index_bytes > kRegionIndexFrom && near_by);

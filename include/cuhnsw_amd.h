@@ -209,7 +209,8 @@ int cuhnsw_trails_available(cuhnsw_engine* e);
  *                   searches first: a launch ends when its last query does).  In batches of three rounds and more
  *                   only a fifth of them goes so, and the others by region of the index, where that brings their rows
  *                   together in the L2 caches: an index of more than 12 MB, of which the queries at work on a chiplet
- *                   have 8 MB to themselves or less (16 MB for ef_search <= 128; rows of more than 128 elements: any).
+ *                   have 8 MB to themselves or less (16 MB for ef_search <= 128 on rows of more than 64 elements; rows of
+ *                   more than 128 elements: any).
  *                   2 = from more than one round on, by region from three on; 3 = as 1, but longest first throughout;
  *                   0 = in the caller's order.
  *                   Same answers and counters either way.
