@@ -384,15 +384,24 @@ __device__ __forceinline__ void order_prefix(int* hist, int from, int most, int*
     part[t] += add;
     __syncthreads();
   }
-  int run = part[t] - sum + from;
+  const int first = part[t] - sum + from;
+  int run = first;
 #pragma unroll
   for (int i = 0; i < per; ++i) {
     hist[t * per + i] = run;
-    if (cut && run < most && run + local[i] >= most) {
-      cut[0] = t * per + i;
-      cut[1] = run + local[i];
-    }
     run += local[i];
+  }
+  // (one thread's business, and apart from the loop above, whose stores it would take apart: 6 us in it, 11 there)
+  if (cut && first < most && run >= most) {
+    run = first;
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+      if (run < most && run + local[i] >= most) {
+        cut[0] = t * per + i;
+        cut[1] = run + local[i];
+      }
+      run += local[i];
+    }
   }
 }
 static __global__ void __launch_bounds__(1024) order_prefix_kernel(int* hist, int most, int* cut) { order_prefix(hist, 0, most, cut); }
