@@ -44,6 +44,8 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_L2, 2, 2, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2,few>"),
     ("search_fast_kernel<DIST_L2, 0, 5, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,5,few>"),
     ("search_fast_kernel<DIST_L2, 4, 5, false>(DevIndex, SearchArgs)", "search_fast_kernel<l2,4,5>"),
+    ("search_fast_kernel<DIST_L2, 0, 7, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,7,few>"),
+    ("search_fast_kernel<DIST_DOT, 0, 8, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,0,8,few>"),
     ("search_fast_kernel<DIST_DOT, 1, 3, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,3>"),
     ("search_fast_kernel<DIST_DOT, 1, 4, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,4>"),
     ("search_fast_kernel<DIST_DOT, 2, 4, false>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,4>"),
@@ -207,6 +209,19 @@ def loop_scratch_accesses(isa_text, mangled):
   return in_loops, total
 
 
+def loads_in_turn(isa_text, mangled):
+  """How often, at most, a block with eight or more wide fetches (the rows of a distance pass) waits for all of them before
+  it issues another one: 0 where they are in flight together, seven where each is waited for in turn."""
+  start = isa_text.index("\n" + mangled + ":")
+  worst = 0
+  for _, ins in _blocks(isa_text[start:isa_text.index(".Lfunc_end", start)]):
+    marks = ["load" if re.match(r"global_load_dwordx[24]", t) else "wait" for t in ins
+             if re.match(r"global_load_dwordx[24]", t) or (t.startswith("s_waitcnt") and "vmcnt(0)" in t)]
+    if marks.count("load") >= 8:
+      worst = max(worst, sum(1 for a, b in zip(marks, marks[1:]) if (a, b) == ("wait", "load")))
+  return worst
+
+
 def _compile_kernel(text, short):
   with tempfile.TemporaryDirectory(prefix="cuhnsw_kr_") as tmp:
     src = os.path.join(tmp, "k.hip")
@@ -224,7 +239,9 @@ def _compile_kernel(text, short):
       raise RuntimeError("%s: expected one kernel named %s, found %r" % (short, base, mangled))
     info = dict(parse_remarks(r.stderr)[mangled[0]])
     with open(asm) as f:
-      in_loops, total = loop_scratch_accesses(f.read(), mangled[0])
+      isa = f.read()
+  in_loops, total = loop_scratch_accesses(isa, mangled[0])
+  info["loads_in_turn"] = loads_in_turn(isa, mangled[0])
   info["scratch_instructions"] = total
   info["scratch_instructions_in_hop_loops"] = in_loops
   return info

@@ -29,6 +29,8 @@ LIMITS = {
     "search_fast_kernel<l2,2,2,few>": (1, 0),
     "search_fast_kernel<l2,0,5,few>": (1, 0),
     "search_fast_kernel<l2,4,5>": (5, 20),
+    "search_fast_kernel<l2,0,7,few>": (1, 0),
+    "search_fast_kernel<dot,0,8,few>": (1, 0),
     # the other sizes of the set
     "search_fast_kernel<dot,1,3>": (7, 0),
     "search_fast_kernel<dot,1,4>": (7, 36),
@@ -60,6 +62,13 @@ def test_first_pass_kernel_keeps_its_register_budget(report, name):
   assert r["waves_per_simd"] >= waves, r
   assert r["scratch_bytes_per_lane"] <= scratch, r
   assert r["scratch_instructions_in_hop_loops"] <= in_loops, r
+
+
+@pytest.mark.parametrize("name", sorted(n for n in LIMITS if "few" in n))
+def test_rows_are_in_flight_together(report, name):
+  """A wavefront with a SIMD to itself has nobody to wait for its loads beside: the rows of a distance pass, fp16 included,
+  are asked for before the first of them is waited for (each in turn, and a search takes twice its time)."""
+  assert report[name]["loads_in_turn"] <= 2, report[name]
 
 
 def test_loop_analysis_sees_a_spill_inside_a_loop():
