@@ -466,7 +466,11 @@ void Engine::build_levels() {
   auto p_inbox0_cnt = workspace.part<int>((size_t)N);
   auto p_inboxU_cnt = workspace.part<int>(up_rows);
   auto p_selected = workspace.part<unsigned char>((size_t)N + up_rows);  // per link row: the row is an output of the selection rule (kernels.h, BuildArgs)
-  auto p_batch_ctl = workspace.part<int>((size_t)n_batches * 2);         // work counter and dirty count of each batch
+  // work counter and number of touched rows of each batch, which all wavefronts of its search ask for all the time: in one
+  // memory line they wait for each other (300 000 x 8 indexed 17.4 -> 19.6 ms, x 30 22.3 -> 23.8, 1 183 514 x 50 from array
+  // to file 125.6 -> 128.1)
+  auto p_batch_ctl = workspace.part<int>((size_t)n_batches);
+  auto p_dirty_cnt = workspace.part<int>((size_t)n_batches);
   workspace.reserve();
   HIP_CHECK(hipMemsetAsync(workspace.at(p_inbox0_cnt), 0, workspace.bytes_from(p_inbox0_cnt), stream));
   HIP_CHECK(hipMemsetAsync(workspace.at(p_work), 0, 10 * sizeof(unsigned long long), stream));
@@ -555,8 +559,8 @@ void Engine::build_levels() {
     a.count = b;
     a.cur_ep = cur_ep;
     a.cur_max = cur_max;
-    a.counter = workspace.at(p_batch_ctl) + 2 * batch;
-    a.dirty_cnt = a.counter + 1;
+    a.counter = workspace.at(p_batch_ctl) + batch;
+    a.dirty_cnt = workspace.at(p_dirty_cnt) + batch;
     if (level_first) {
       const int from = batch > 0 ? upper_end[batch - 1] : 0;
       a.upper = workspace.at(p_upper) + from;
