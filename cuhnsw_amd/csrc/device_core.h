@@ -331,8 +331,9 @@ __device__ __forceinline__ void load_query(QVec<QR>& qv, float4* qlds, const flo
   }
 }
 
-// one pass over 4*U rows starting at ids[r]: loads first, arithmetic after
-template <int DT, int R, int U, bool RAW, bool HALF>
+// one pass over 4*U rows starting at ids[r]: loads first, arithmetic after.  SELECT: chunks past the data are left out by a
+// select after all (literal_select)
+template <int DT, int R, int U, bool RAW, bool HALF, bool SELECT = false>
 __device__ __forceinline__ void dist_pass(const void* rows, uint32_t rowlen, uint32_t used, const float4* q,
                                           const uint32_t* ids, int r, int n, float* out, int g, int sub) {
   float4 v[U][R];
@@ -350,7 +351,8 @@ __device__ __forceinline__ void dist_pass(const void* rows, uint32_t rowlen, uin
       // 16 * (R / 2) chunks, so only the upper half of k can be past its end.
       const uint32_t c = sub + 16 * k;
       const uint64_t at = first + (c < used ? c : 0);
-      v[u][k] = HALF ? load_chunk_f16(rows, at) : load_chunk_f32(rows, at);
+      const float4 t = HALF ? load_chunk_f16(rows, at) : load_chunk_f32(rows, at);
+      v[u][k] = SELECT && DT != DIST_DOT && k >= R / 2 && !(c < used) ? q[k] : t;
     }
   }
   float neg[R];
@@ -366,7 +368,7 @@ __device__ __forceinline__ void dist_pass(const void* rows, uint32_t rowlen, uin
     float ax = 0.f, ay = 0.f, az = 0.f, aw = 0.f;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      if (DT == DIST_DOT || k < R / 2) acc4<DT>(q[k], v[u][k], ax, ay, az, aw);
+      if (DT == DIST_DOT || k < R / 2 || SELECT) acc4<DT>(q[k], v[u][k], ax, ay, az, aw);
       else if (RAW) acc4<DT>(q[k], masked(v[u][k], keep[k]), ax, ay, az, aw);
       else acc4_l2_if(q[k], v[u][k], neg[k], ax, ay, az, aw);
     }
@@ -478,7 +480,7 @@ __device__ __forceinline__ void dist_long(const void* rows, int rowlen, int used
 }
 
 // keys of ids[0..n) (LDS) against the query -> out[0..n) (LDS).  n is wavefront-uniform.
-template <int DT, int QR, bool RAW, bool HALF, int WIDE = 1>
+template <int DT, int QR, bool RAW, bool HALF, int WIDE = 1, bool SELECT = false>
 __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& qv, const float4* qlds, const uint32_t* ids,
                                             int n, float* out, int lane) {
   const int g = lane >> 4, sub = lane & 15;
@@ -493,16 +495,16 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
     while (r < n) {
       const int rem = n - r;
       if (UMAX >= 8 && rem > 16) {
-        dist_pass<DT, R, (UMAX >= 8 ? 8 : 1), RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
+        dist_pass<DT, R, (UMAX >= 8 ? 8 : 1), RAW, HALF, SELECT>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
         r += 32;
       } else if (UMAX >= 4 && rem > 8) {
-        dist_pass<DT, R, (UMAX >= 4 ? 4 : 1), RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
+        dist_pass<DT, R, (UMAX >= 4 ? 4 : 1), RAW, HALF, SELECT>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
         r += 16;
       } else if (UMAX >= 2 && rem > 4) {
-        dist_pass<DT, R, (UMAX >= 2 ? 2 : 1), RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
+        dist_pass<DT, R, (UMAX >= 2 ? 2 : 1), RAW, HALF, SELECT>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
         r += 8;
       } else {
-        dist_pass<DT, R, 1, RAW, HALF>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
+        dist_pass<DT, R, 1, RAW, HALF, SELECT>(rows, rowlen, used, qv.q, ids, r, n, out, g, sub);
         r += 4;
       }
     }
@@ -514,12 +516,12 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
 // code for fp16 goes out of the way, which is 1 % of a search of one query; elsewhere it costs spills.)
 // WIDE: how many rows are in flight; 1 = as many as registers allow beside a full machine's wavefronts, 4 = as a
 // wavefront with a SIMD to itself can have, 0 = four
-template <int DT, int QR, bool RAW, int WIDE = 1>
+template <int DT, int QR, bool RAW, int WIDE = 1, bool SELECT = false>
 __device__ __forceinline__ void dist_list(const DevIndex& ix, const QVec<QR>& qv, const float4* qlds,
                                           const uint32_t* ids, int n, float* out, int lane) {
   const bool half = uni(ix.half) != 0;
-  if (WIDE >= 4 ? __builtin_expect(half, 0) : half) dist_list_t<DT, QR, RAW, true, WIDE>(ix, qv, qlds, ids, n, out, lane);
-  else dist_list_t<DT, QR, RAW, false, WIDE>(ix, qv, qlds, ids, n, out, lane);
+  if (WIDE >= 4 ? __builtin_expect(half, 0) : half) dist_list_t<DT, QR, RAW, true, WIDE, SELECT>(ix, qv, qlds, ids, n, out, lane);
+  else dist_list_t<DT, QR, RAW, false, WIDE, SELECT>(ix, qv, qlds, ids, n, out, lane);
 }
 
 // The same for the searches on the literal queues: long rows eight at a time (dist_long), L2 rows of two chunks per lane
@@ -528,6 +530,13 @@ __device__ __forceinline__ void dist_list(const DevIndex& ix, const QVec<QR>& qv
 template <int DT, int QR, int NS>
 constexpr int literal_wide() {
   return QR == 0 && NS <= 8 ? 2 : (DT == DIST_L2 && QR == 2 ? 0 : 1);
+}
+// And there L2 rows of up to 64 elements leave chunks past the data out by a select, where the result set is larger than five
+// keys per lane or a heap in LDS (60 000 x 40 integers: 100 queries at ef 600 1.87 -> 1.78 ms, 2 000 at 1 100 6.11 -> 5.84; at
+// ef 300 no difference, at 128 0.87 against 0.88).
+template <int DT, int QR, int NS>
+constexpr bool literal_select() {
+  return DT == DIST_L2 && QR == 1 && (NS == 0 || NS > 5);
 }
 
 __device__ __forceinline__ const uint32_t* link_row(const DevIndex& ix, uint32_t node, int level) {
@@ -823,9 +832,10 @@ __device__ __forceinline__ void search_level(const DevIndex& ix, const QVec<QR>&
   SplitHeap cand{s.cand, s.cand_glob, s.cand_lds};
   const int S = row_stride(ix, level);
   constexpr int kWide = BUILD ? 1 : literal_wide<DT, QR, NS>();
+  constexpr bool kSelect = !BUILD && literal_select<DT, QR, NS>();
   int n = n_seed;
   if (n > 0) {
-    dist_list<DT, QR, false>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+    dist_list<DT, QR, false, 1, kSelect>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
     st.n_dist += n;
   }
   while (true) {
@@ -854,13 +864,13 @@ __device__ __forceinline__ void search_level(const DevIndex& ix, const QVec<QR>&
       const VisitPending vp = visit_issue(row, S, s, lane);
       wave_sync();
       n = vp.n_ask;
-      if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+      if (n > 0) dist_list<DT, QR, false, kWide, kSelect>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
       wave_sync();
       st.n_dist += visit_commit(vp, s, st, lane);
     } else {
       n = visit_row(row, S, s, st, lane);
       wave_sync();
-      if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+      if (n > 0) dist_list<DT, QR, false, kWide, kSelect>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
       st.n_dist += n;
     }
   }
@@ -2051,7 +2061,7 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
   bool own_stretch = false;  // between two markers: hops this pass makes itself
   if (trail_hops > 0) st.n_dist += trail_n_dist;  // the evaluations that pass made up to the trail's end count as performed
   while (true) {
-    if (n > 0 && !from_trail) dist_list<DT, QR, false, literal_wide<DT, QR, NS>()>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+    if (n > 0 && !from_trail) dist_list<DT, QR, false, literal_wide<DT, QR, NS>(), literal_select<DT, QR, NS>()>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
     st.n_dist += from_trail ? 0 : n;
     wave_sync();
     for (int base = 0; base < n; base += 64) {
