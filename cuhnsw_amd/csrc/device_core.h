@@ -986,16 +986,17 @@ __device__ __forceinline__ int max_so_far(int x) {
 // the others), whose list lies in ids / keys (LDS), into a set of `size` entries; what does not fit behind ef entries falls off its end.  The offers are put
 // in order (in ids / keys), every entry finds by halving how many of them go before it, and entries and offers go to their
 // new places through LDS.  `room`: 64 * (NS + 1) words of LDS, whose contents are put back.  Returns false, with nothing
-// done, if two keys are equal (or the node is in the set already), also if one of them is the set's last then and the other
-// the first to fall off (hnswlib expands both, and its heap says which one leaves): those go in one by one, by the rules for
-// them.  last_key: the set's largest key afterwards.
+// done, if an offer has the key of another or of an entry (or its node is in the set already), also if one of the two is the
+// set's last then and the other the first to fall off (hnswlib expands both, and its heap says which one leaves), or if the
+// set's largest key would not stay above `above`: those go in one by one, by the rules for them.  last_key: the set's largest
+// key afterwards.
 // (An insert of its own is 39 instructions at ef 300 and 0.2 us of latency, this 200 for 14 offers.  Counting for each entry
 // and each offer what goes before it, offer by offer, was 45 instructions an offer: one query on 100 000 x 50 284 -> 272 us,
 // 1 000 queries there 636 -> 607, of which the full set's share below is half; 1 M x 96, ef 256, 100 000 queries 9.92 ->
 // 9.80 ms.)
 template <int NS, bool SPARSE>
 __device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned long long offers, int size, int ef, float my_key, uint32_t my_id,
-                                                    uint32_t* ids, float* keys, uint32_t* room, float& last_key, int lane) {
+                                                    uint32_t* ids, float* keys, uint32_t* room, float above, float& last_key, int lane) {
   constexpr int N = NS > 0 ? NS : 1;
   lane = fresh(lane);
   const int n = __popcll(offers);
@@ -1063,15 +1064,20 @@ __device__ __forceinline__ bool frontier_insert_all(Frontier<NS>& f, unsigned lo
 #pragma unroll
     for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j]);
     const float last = uni(__uint_as_float(room[64 * N - ef + (size + n < ef ? size + n : ef) - 1]));
-    const bool cut = SPARSE && uni(__uint_as_float(room[64 * N])) == last;  // with the first to fall off (not SPARSE: none does)
-    const float prev_last = __builtin_bit_cast(
-        float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, f.k[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
+    if (SPARSE) {
+      // (those that fall off included, as far as they are no farther than the set's last: candidates all the same.  Equal
+      // entries that were there before are none of its business.)
+      twins = __ballot(lane < n && offer_key <= last && place > 0 && __uint_as_float(room[place > 0 ? place - 1 : 0]) == offer_key);
+    } else {
+      const float prev_last = __builtin_bit_cast(
+          float, __builtin_amdgcn_update_dpp((int)0xFF800000u, __builtin_bit_cast(int, f.k[N - 1]), 0x138, 0xF, 0xF, false));  // wave_shr:1
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      twins |= __ballot(f.k[j] == (j > 0 ? f.k[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(f.k[j]) < INFINITY);
-    // (the comparison with -inf always holds; without it the instances for six keys a lane and rows of 65 to 128 elements
-    // spill five registers more and reload some in the hop loop: 200 000 x 128, ef 330, 40 000 queries 7.51 -> 7.85 ms)
-    done = twins == 0ull && last > -INFINITY && !cut;
+      for (int j = 0; j < N; ++j)
+        twins |= __ballot(f.k[j] == (j > 0 ? f.k[j > 0 ? j - 1 : 0] : prev_last)) & __ballot(__builtin_fabsf(f.k[j]) < INFINITY);
+    }
+    // (the comparison holds wherever `above` is -inf; without it the instances for six keys a lane and rows of 65 to 128
+    // elements spill five registers more and reload some in the hop loop: 200 000 x 128, ef 330, 40 000 queries 7.51 -> 7.85 ms)
+    done = twins == 0ull && last > above;
     if (!done) {
 #pragma unroll
       for (int j = 0; j < N; ++j) f.k[j] = __uint_as_float(room[lane * N + j + before[j]]);
@@ -1624,10 +1630,10 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   constexpr int kInsertAllFrom = 4;
   // On a full set most steps bring in nothing and the others a dozen offers: those of one evaluation enter it together from
   // six on, in the instances that have the registers (a trail wants to know of each whether it was accepted when its turn
-  // came; sets of two registers take their offers one by one as fast).  Not where equal keys have met: most of them are in
-  // the set still, and it would be refused after all its work (one query on 200 000 x 128 integers, ef 300: 0.506 ms with it
-  // there, 0.495 without; 32 queries 1.103 and 1.096).
-  constexpr bool kMerge = FEW && !TRAILS && !WATCH && NS > 2;
+  // came; sets of two registers take their offers one by one as fast).  Also beside equal keys, as long as none of the offers
+  // has one (one query on 200 000 x 128 integers, ef 300: 0.493 ms, refused for any equal keys in the set 0.504; not tried
+  // beside them 0.495, but 1 000 queries on 100 000 x 50, one in eight of which meets two by accident, 0.539 instead of 0.528).
+  constexpr bool kMerge = FEW && !TRAILS && NS > 2;
   constexpr int kMergeFrom = 6;
   // more rows in flight: the search on long rows (dist_long), and small sets, which leave the registers for it (56 of 72;
   // 345 678 x 101 in fp16, ef 77, 5 003 queries: 0.85 -> 0.71 ms)
@@ -1668,8 +1674,8 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
     const int acc_before = st.n_acc;
     if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && n < 64 && st.n_acc + n <= ef && 64 * (N + 1) <= (1 << s.vc_bits)) {
       float last_key = 0.f;
-      if (frontier_insert_all<NS, false>(fr, todo, st.n_acc, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), last_key,
-                                         lane)) {
+      if (frontier_insert_all<NS, false>(fr, todo, st.n_acc, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), -INFINITY,
+                                         last_key, lane)) {
         if (TRAILS) accepted |= todo;
         st.n_acc = st.n_acc + n;
         st.maxkey = last_key;
@@ -1689,7 +1695,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
       const unsigned long long now = todo & (end < 64 ? (1ull << end) - 1ull : ~0ull);
       float last_key = 0.f;
       if (__popcll(now) >= kMergeFrom &&
-          frontier_insert_all<NS, true>(fr, now, ef, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), last_key, lane)) {
+          frontier_insert_all<NS, true>(fr, now, ef, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), w_hi, last_key, lane)) {
         st.n_acc = st.n_acc + 1;  // (a full set only asks whether there were any)
         st.lower = last_key;
         good = upto;

@@ -34,7 +34,8 @@ def test_overflowed_distances_find_their_place(ns, ef, extreme):
 
 
 def test_an_infinite_key_would_be_written_behind_the_set():
-  """Why the keys stop short of it: nothing in the set compares above an infinity, the padding included.  The list would be
-  refused, as where the set's last entry and the first that falls off are equal."""
-  held = in_the_set(5, 300, np.array([1.0], np.float32))
-  assert insert_all(5, 300, 1, held, np.zeros(320, int), np.array([0.5, np.inf], np.float32), np.zeros(2, int))[0] is None
+  """Why the keys stop short of it: nothing in the set compares above an infinity, the padding included."""
+  held, ids = in_the_set(5, 300, np.array([1.0], np.float32)), np.zeros(320, int)
+  after, _ = insert_all(5, 300, 1, held, ids, np.array([0.5, np.inf], np.float32), np.array([7, 8]))
+  first = 64 * 5 - 300
+  assert (after[0][first:first + 2] == [0.5, 1.0]).all() and after[1][first] == 7 and not (after[1] == 8).any()

@@ -1,7 +1,8 @@
 """A model of how a list of offers enters the sorted set in one go (frontier_insert_all of device_core.h), step by step as the
 lanes do it: the offers put in order, each entry's count of offers before it found by halving, each offer's place from the
-last entry of every count, everything moved through 64 * (NS + 1) words.  Equal keys send the offers the other way, also
-where the set's end comes between the two; below that the dropped ones are no candidates any more."""
+last entry of every count, everything moved through 64 * (NS + 1) words.  An offer's equal sends them the other way, also
+where the set's end comes between the two; farther out the dropped ones are no candidates any more.  Into a full set equal
+entries that were there before are no reason."""
 import numpy as np
 import pytest
 
@@ -37,7 +38,11 @@ def insert_all(ns, ef, size, held, ids, offers, offer_ids):
   after = room[:total]
   finite = np.isfinite(after)
   last = room[total - ef + min(size + n, ef) - 1]
-  if (after[1:] == after[:-1])[finite[1:]].any() or room[total] == last:
+  if size < ef:
+    refused = (after[1:] == after[:-1])[finite[1:]].any()
+  else:
+    refused = any(key <= last and at > 0 and room[at - 1] == key for at, key in zip(place, keys))
+  if refused:
     return None, touched
   return (after, room_ids[:total]), touched
 
@@ -91,5 +96,9 @@ def test_equal_keys_on_both_sides_of_the_sets_end_are_refused(at):
   offers = np.insert(np.arange(5, 65, 10).astype(np.float32), at, np.float32(1440))
   held = in_the_set(ns, ef, entries)
   assert insert_all(ns, ef, ef, held, np.arange(64 * ns), offers, np.arange(7))[0] is None
+  held[-9] = held[-8]  # (1 430 twice, a pair that was there before: the offers below it enter all the same)
+  after = insert_all(ns, ef, ef, held, np.arange(64 * ns), np.delete(offers, at), np.arange(6))[0]
+  assert after is not None and np.count_nonzero(after[0] == held[-8]) == 2
+  held[-9] = 1420
   offers[at] = 1450  # (pushed out together with its equal: beyond the bound, both dead)
   assert insert_all(ns, ef, ef, held, np.arange(64 * ns), offers, np.arange(7))[0] is not None

@@ -24,8 +24,8 @@ INF = float("inf")
 def sorted_set_search(keys_of, rows, ep, k, ef, trail=None, together=None, cut_rule=True):
   """Returns None when given up, else (ids, keys, hops, evaluations, met equal keys).  trail: a dict that receives
   "rec" (the records and markers) and "hops" (the expansions they cover).  together: so many offers of one hop or more
-  enter a full set in one go (frontier_insert_all), unless equal keys forbid it; cut_rule: also those of which one is
-  the set's last entry afterwards and the other the first that was pushed out."""
+  enter a full set in one go (frontier_insert_all), unless one of them has the key of another or of an entry; cut_rule:
+  also where one of the two is the set's last entry afterwards and the other the first that was pushed out."""
   tr = {"rec": [], "on": True, "own": False, "hops": 0}
 
   def stop(h):                            # the trail ends: h expansions are complete
@@ -53,14 +53,16 @@ def sorted_set_search(keys_of, rows, ep, k, ef, trail=None, together=None, cut_r
     accepted = []
     passing = [o for o in offers if S[-1][0] > o[0]]
     if together is not None and calm and len(S) >= ef and len(passing) >= together:
-      merged = sorted(S + [[key, node, False] for key, node in passing], key=lambda e: e[0])
-      equal = any(a[0] == b[0] for a, b in zip(merged[:ef], merged[1:ef]))
+      new = {node for _, node in passing}
+      merged = sorted(S + [[key, node, False] for key, node in passing], key=lambda e: e[0])  # (an offer behind its equal)
+      reach = len(merged) if cut_rule else ef
+      equal = any(a[0] == b[0] <= merged[ef - 1][0] and b[1] in new for a, b in zip(merged[:reach], merged[1:reach]))
       equal = equal or len({key for key, _ in passing}) < len(passing)
-      equal = equal or (cut_rule and merged[ef - 1][0] == merged[ef][0])
       if not equal and not (watch and merged[ef - 1][0] <= max(w[0] for w in watch)):
         S = merged[:ef]
         offers = []
         sorted_set_search.entered_together += 1
+        sorted_set_search.entered_beside_equal_keys += have_tie
     for key, node in offers:
       full = len(S) >= ef
       if full and not (S[-1][0] > key):
@@ -182,7 +184,8 @@ sorted_set_search.answered_after_twins = 0    # (statistics for the test below: 
 sorted_set_search.calmed_down = 0             # (and so has the return to the tie-free loop,
 sorted_set_search.calmed_down_watching = 0    # with and without entries to watch,
 sorted_set_search.calmed_down_past_a_ghost = 0  # and after an eviction out of equal largest keys)
-sorted_set_search.entered_together = 0        # (and offers that entered a full set in one go)
+sorted_set_search.entered_together = 0        # (and offers that entered a full set in one go,
+sorted_set_search.entered_beside_equal_keys = 0  # also once equal keys have met)
 
 
 def _push_heap(h, value):
@@ -380,7 +383,7 @@ def test_rules_never_let_an_order_dependent_case_through(oracle, seed):
   assert sorted_set_search.answered_after_twins > 0
   assert sorted_set_search.calmed_down > 100 and sorted_set_search.calmed_down_watching > 100
   assert sorted_set_search.calmed_down_past_a_ghost > 20
-  assert sorted_set_search.entered_together > 100
+  assert sorted_set_search.entered_together > 100 and sorted_set_search.entered_beside_equal_keys > 20
 
 
 @pytest.mark.parametrize("seed", range(3))
