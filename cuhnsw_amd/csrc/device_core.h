@@ -33,6 +33,7 @@
 #include "heap_coop.h"
 #include "index_file.h"
 #include "options.h"
+#include "visited_filter.h"
 
 namespace cuhnsw_amd {
 
@@ -61,6 +62,7 @@ struct Scratch {
   float4* qlds;        // LDS copy of the query (only when the query is not kept in registers)
   uint16_t* vcache;    // LDS, direct-mapped cache of ids known to be visited (null = none)
   int vc_bits;         // log2 of its size: slot = id & (size-1), tag = id >> vc_bits
+  FilterShape filter;  // where vcache is the sorted-set search's filter instead (visit_lossy)
   uint32_t* bitmap;    // global, one bit per node
   uint32_t* undo;      // global, ids whose bit is set
   int undo_cap;
@@ -336,6 +338,7 @@ __device__ __forceinline__ void load_query(QVec<QR>& qv, float4* qlds, const flo
 template <int DT, int R, int U, bool RAW, bool HALF, bool SELECT = false>
 __device__ __forceinline__ void dist_pass(const void* rows, uint32_t rowlen, uint32_t used, const float4* q,
                                           const uint32_t* ids, int r, int n, float* out, int g, int sub) {
+  if (DT != DIST_DOT && R == 2) sub = fresh(sub);  // (these are short of registers where the set is large)
   float4 v[U][R];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -1351,53 +1354,66 @@ __device__ __forceinline__ void search_level_far_lds(const DevIndex& ix, const Q
 // before"), a miss may be a node whose tag has been pushed out since: it is then evaluated
 // again, which changes nothing — if it is still in the set the insert finds it, and if it was
 // rejected or evicted its key is still not below the bound.  No atomics, no global memory,
-// nothing to undo.  s.vcache / s.vc_bits hold the table and log2 of its size in 32-bit words.
+// nothing to undo.  s.vcache / s.filter hold the table and its shape.
 // (Four ways rather than two at the same size: on the 1.18 M-point set the neighbourhoods
 // overlap so much that most forgotten nodes were victims of set conflicts, not of capacity —
 // repeated evaluations fell from 31 % to 12 % of the distinct ones.)
 __device__ __forceinline__ void filter_reset(Scratch& s, int lane) {
   uint4* c4 = reinterpret_cast<uint4*>(s.vcache);
-  const int n4 = (1 << s.vc_bits) >> 2;  // 2 sets per 16 bytes
-  for (int i = lane; i < n4; i += 64) c4[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  const int n4 = (s.filter.sets() + 1) >> 1;  // 2 sets per 16 bytes
+  for (int i = lane; i < n4; i += 64) {
+    const uint32_t a = filter_empty_tag(s.filter, 2u * (uint32_t)i) * 0x10001u, b = filter_empty_tag(s.filter, 2u * (uint32_t)i + 1u) * 0x10001u;
+    c4[i] = make_uint4(a, a, b, b);
+  }
   wave_sync();
 }
-__device__ __forceinline__ uint2 filter_push(uint2 w, uint32_t tag) {
-  return make_uint2((w.x << 16) | tag, (w.y << 16) | (w.x >> 16));
+__device__ __forceinline__ uint2 filter_push(uint2 w, uint32_t place) {
+  return make_uint2(__builtin_amdgcn_alignbit(w.x, place << 16, 16), (w.y << 16) | (w.x >> 16));
 }
 // the lanes whose tag is not among the four of their set
-__device__ __forceinline__ unsigned long long filter_misses(uint2 w, uint32_t tag) {
-  return __ballot((w.x & 0xFFFFu) != tag) & __ballot((w.x >> 16) != tag) & __ballot((w.y & 0xFFFFu) != tag) &
-         __ballot((w.y >> 16) != tag);
+__device__ __forceinline__ unsigned long long filter_misses(uint2 w, uint32_t place) {
+  const uint16_t tag = (uint16_t)place;
+  return __ballot((uint16_t)w.x != tag) & __ballot((uint16_t)(w.x >> 16) != tag) & __ballot((uint16_t)w.y != tag) &
+         __ballot((uint16_t)(w.y >> 16) != tag);
 }
 // Compacts the ids of a link row that the filter does not know into s.nbuf; returns how many.
-__device__ __forceinline__ int visit_lossy(const uint32_t* row, int S, Scratch& s, int lane) {
+template <bool WIDE>
+__device__ __forceinline__ int visit_lossy_t(const uint32_t* row, int S, Scratch& s, int lane) {
   int n = 0;
   uint2* sets = reinterpret_cast<uint2*>(s.vcache);
-  const int set_bits = s.vc_bits - 1;
-  const uint32_t mask_bits = (1u << set_bits) - 1u;
   for (int base = 0; base < S; base += 64) {
     const uint32_t got = row[base + lane < S ? base + lane : 0];  // unconditional load, then a select
     const uint32_t id = (base + lane < S) ? got : kEmpty;
-    // (every lane looks its set up — an empty slot's id maps to some set and to a tag no set can hold — so that
-    // the only predicated part is the two LDS writes at the end)
-    const uint32_t slot = id & mask_bits;
-    const uint32_t tag = id >> set_bits;
+    // (every lane looks its set up — an empty slot's "id" has some set too — so that the only predicated part is the two
+    // LDS writes at the end)
+    const uint32_t place = filter_place<WIDE>(id);
+    const uint32_t slot = filter_set<WIDE>(s.filter, place);
     const uint2 w = sets[slot];
-    const unsigned long long mask = __ballot(id != kEmpty) & filter_misses(w, tag);
+    const unsigned long long mask = __ballot(id != kEmpty) & filter_misses(w, place);
     if (__builtin_amdgcn_inverse_ballot_w64(mask)) {
-      sets[slot] = filter_push(w, tag);
+      sets[slot] = filter_push(w, place);
       s.nbuf[n + lanes_below(mask)] = id;
     }
     n += __popcll(mask);
   }
   return n;
 }
+__device__ __forceinline__ int visit_lossy(const uint32_t* row, int S, Scratch& s, int lane) {
+  if (__builtin_expect(s.filter.more_bits() != 0, 0)) return visit_lossy_t<true>(row, S, s, lane);
+  return visit_lossy_t<false>(row, S, s, lane);
+}
+// an id's place and its set
+__device__ __forceinline__ uint32_t filter_find(FilterShape f, uint32_t id, uint32_t& slot) {
+  const uint32_t place = f.more_bits() != 0 ? filter_place<true>(id) : filter_place<false>(id);
+  slot = filter_set<true>(f, place);
+  return place;
+}
 __device__ __forceinline__ void visit_lossy_single(Scratch& s, uint32_t id, int lane) {
   if (lane == 0) {
     uint2* sets = reinterpret_cast<uint2*>(s.vcache);
-    const int set_bits = s.vc_bits - 1;
-    const uint32_t slot = id & ((1u << set_bits) - 1u);
-    sets[slot] = filter_push(sets[slot], id >> set_bits);
+    uint32_t slot;
+    const uint32_t place = filter_find(s.filter, id, slot);
+    sets[slot] = filter_push(sets[slot], place);
   }
 }
 
@@ -1405,13 +1421,11 @@ __device__ __forceinline__ void visit_lossy_single(Scratch& s, uint32_t id, int 
 // the filter one after the other -- so that a node two of them link to is in the first one's list only -- with all of
 // their fetches in flight at once.  Compacts like visit_lossy; ends gets the end of each row's list, eight bits each.  At
 // most 64 ids in all: the rows that do not fit are left out (returns how many are in).  S <= 64.
-template <int K>
-__device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t cands, int rows, int level, int S, Scratch& s,
-                                                int& n_ids, unsigned long long& ends, int lane) {
+template <int K, bool WIDE>
+__device__ __forceinline__ int visit_lossy_rows_t(const DevIndex& ix, uint32_t cands, int rows, int level, int S, Scratch& s,
+                                                  int& n_ids, unsigned long long& ends, int lane) {
   static_assert(K <= 8, "eight ends in 64 bits");
   uint2* sets = reinterpret_cast<uint2*>(s.vcache);
-  const int set_bits = s.vc_bits - 1;
-  const uint32_t mask_bits = (1u << set_bits) - 1u;
   uint32_t got[K];
 #pragma unroll
   for (int r = 0; r < K; ++r) {
@@ -1424,16 +1438,16 @@ __device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t can
   for (int r = 0; r < K; ++r) {
     if (r < in) {
       const uint32_t id = lane < S ? got[r] : kEmpty;
-      const uint32_t slot = id & mask_bits;
-      const uint32_t tag = id >> set_bits;
+      const uint32_t place = filter_place<WIDE>(id);
+      const uint32_t slot = filter_set<WIDE>(s.filter, place);
       const uint2 w = sets[slot];
-      const unsigned long long mask = __ballot(id != kEmpty) & filter_misses(w, tag);
+      const unsigned long long mask = __ballot(id != kEmpty) & filter_misses(w, place);
       const int more = __popcll(mask);
       if (r > 0 && n + more > 64) {
         in = r;
       } else {
         if (__builtin_amdgcn_inverse_ballot_w64(mask)) {
-          sets[slot] = filter_push(w, tag);
+          sets[slot] = filter_push(w, place);
           s.nbuf[n + lanes_below(mask)] = id;
         }
         __builtin_amdgcn_wave_barrier();
@@ -1445,19 +1459,30 @@ __device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t can
   n_ids = n;
   return in;
 }
-// Takes the ids of the lanes that say so out of the filter again: an empty tag is all ones.  (Two of them may share a
-// word: each sets its own half with an atomic.)
+template <int K>
+__device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t cands, int rows, int level, int S, Scratch& s,
+                                                int& n_ids, unsigned long long& ends, int lane) {
+  if (__builtin_expect(s.filter.more_bits() != 0, 0)) return visit_lossy_rows_t<K, true>(ix, cands, rows, level, S, s, n_ids, ends, lane);
+  return visit_lossy_rows_t<K, false>(ix, cands, rows, level, S, s, n_ids, ends, lane);
+}
+// Takes the ids of the lanes that say so out of the filter again.  (Two of them may share a word: each makes its own half the
+// set's empty tag with two atomics -- which may come twice for one id, listed twice where the filter lost it in between.)
 __device__ __forceinline__ void filter_forget(Scratch& s, uint32_t id, bool mine) {
-  const int set_bits = s.vc_bits - 1;
-  const uint32_t slot = id & ((1u << set_bits) - 1u);
-  const uint32_t tag = id >> set_bits;
   uint2* sets = reinterpret_cast<uint2*>(s.vcache);
   if (mine) {
+    uint32_t slot;
+    const uint32_t tag = filter_find(s.filter, id, slot) & 0xFFFFu, empty = filter_empty_tag(s.filter, slot) * 0x10001u;
     const uint2 w = sets[slot];
     const uint32_t x = ((w.x & 0xFFFFu) == tag ? 0xFFFFu : 0u) | ((w.x >> 16) == tag ? 0xFFFF0000u : 0u);
     const uint32_t y = ((w.y & 0xFFFFu) == tag ? 0xFFFFu : 0u) | ((w.y >> 16) == tag ? 0xFFFF0000u : 0u);
-    if (x) __hip_atomic_fetch_or(&sets[slot].x, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-    if (y) __hip_atomic_fetch_or(&sets[slot].y, y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (x) {
+      __hip_atomic_fetch_and(&sets[slot].x, ~x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      __hip_atomic_fetch_or(&sets[slot].x, empty & x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    if (y) {
+      __hip_atomic_fetch_and(&sets[slot].y, ~y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      __hip_atomic_fetch_or(&sets[slot].y, empty & y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -1649,7 +1674,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   HeapEnt* const cands = batch_candidates(s);
   unsigned long long ends = (uint32_t)n;   // end of each one's offers in s.nbuf / s.dbuf, eight bits each
   while (true) {
-    if (QR == 2 && NS > 2 && !BUILD && !FEW) lane = fresh(lane);  // (these are the instances short of registers)
+    if ((QR == 2 || (QR == 1 && (TRAILS || NS == 6) )) && NS > 2 && !BUILD && !FEW) lane = fresh(lane);  // (these are the instances short of registers)
     if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
     st.n_dist += n;
     wave_sync();
@@ -1672,7 +1697,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
     int row_end = K > 1 ? (int)(ends & 0xFFu) : n;
     int good = rows;                                        // candidates of the batch that are expanded for good
     const int acc_before = st.n_acc;
-    if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && n < 64 && st.n_acc + n <= ef && 64 * (N + 1) <= (1 << s.vc_bits)) {
+    if (!FULL && (BUILD || FEW || NS > 2) && n >= kInsertAllFrom && n < 64 && st.n_acc + n <= ef && 32 * (N + 1) <= s.filter.sets()) {
       float last_key = 0.f;
       if (frontier_insert_all<NS, false>(fr, todo, st.n_acc, ef, my_key, my_id, s.nbuf, s.dbuf, reinterpret_cast<uint32_t*>(s.vcache), -INFINITY,
                                          last_key, lane)) {
@@ -1683,7 +1708,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
         todo = 0ull;
       }
     }
-    if (FULL && kMerge && __popcll(todo) >= kMergeFrom && __popcll(todo) < 64 && 64 * (N + 1) <= (1 << s.vc_bits)) {
+    if (FULL && kMerge && __popcll(todo) >= kMergeFrom && __popcll(todo) < 64 && 32 * (N + 1) <= s.filter.sets()) {
       // the first candidate that an offer of those before it is closer than: its turn does not come now (tie_free_offers)
       int upto = rows;
       for (int c = rows - 1; c > 0; --c) {
@@ -1882,6 +1907,7 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
       gave_up = false;
     }
     while (true) {
+      if ((QR == 1 || (QR == 2 && DT == DIST_DOT)) && NS == 6 && !BUILD && !FEW) lane = fresh(lane);
       if (resume_at < 0) {
         if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
         st.n_dist += n;
@@ -2158,9 +2184,9 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
             s.nbuf[lane - off] = win.y;
             s.dbuf[lane - off] = __uint_as_float(win.z);
             uint2* sets = reinterpret_cast<uint2*>(s.vcache);
-            const int set_bits = s.vc_bits - 1;
-            const uint32_t slot = win.y & ((1u << set_bits) - 1u);
-            sets[slot] = filter_push(sets[slot], win.y >> set_bits);
+            uint32_t slot;
+            const uint32_t place = filter_find(s.filter, win.y, slot);
+            sets[slot] = filter_push(sets[slot], place);
           }
           __builtin_amdgcn_wave_barrier();
           trail_at += n;

@@ -554,23 +554,59 @@ class Engine {
     return bits;
   }
 
-  // log2 of the size in 32-bit words (two 16-bit tags each; a set is two words, four ways) of
-  // the LDS visited filter of the sorted-set search.  A search at ef = 300 evaluates 1 100 to
-  // 1 300 distinct nodes on the million-point sets (max_m0 24 and 32 alike), about 800 at
-  // ef = 100; the filter gets 4 * ef + 512 entries rounded up to a power of two (1 024 up to
-  // ef = 128, 2 048 = 4 KB up to ef = 384), and twice as much when a repeated evaluation is
-  // expensive (rows of 2 KB and more).  More costs occupancy and is slower, less repeats more.
-  // 0 when ids do not fit the tags.
-  int auto_fc_bits(int ef) const {
+  // The visited filter (visited_filter.h) a search on the sorted set should have at least.  A search at ef = 300 evaluates
+  // 1 100 to 1 300 distinct nodes on the million-point sets (max_m0 24 and 32 alike), about 800 at ef = 100; the filter gets
+  // 4 * ef + 512 entries, and twice as many when a repeated evaluation is expensive (rows of 2 KB and more).  Without sets
+  // when ids do not fit the tags of a filter of that many entries, rounded up to a power of two.
+  FilterShape least_filter(int ef) const {
     long long want = filter_entries > 0 ? filter_entries : 4ll * ef + 512;
     if (filter_entries <= 0 && Dp >= 512) want *= 2;
     int bits = 8;
     while ((2ll << bits) < want && bits < 13) ++bits;
-    if (((unsigned)host.N >> (bits - 1)) >= 0xFFFFu) return 0;  // tags are 16 bits wide, sets 64
-    return bits;
+    if (((unsigned)host.N >> (bits - 1)) >= 0xFFFFu) return FilterShape();  // tags are 16 bits wide, sets 64
+    return filter_shape((int)std::min<long long>((want + 3) / 4, 1 << (bits - 1)), host.N);
+  }
+  // ... and the one it gets: what the wavefronts that the kernel's registers allow leave of LDS is the filter's, as far as it
+  // needs it (four times the least: next to nothing is forgotten then).  Nor must it be what limits the wavefronts: half the
+  // filter repeats more evaluations, but is the faster choice wherever it buys 15 % more of them.
+  // (Against the next power of two above the least: 500 000 x 128 at ef 128, 256 -> 568 sets, 10 000 queries 1.93 -> 1.81 ms; 1 M x
+  // 96, ef 256, topk 100, 512 -> 568 sets, 100 000 queries 9.28 -> 9.14; 1 183 514 x 50 indexed and saved, 256 -> 425, 124.7 ->
+  // 123.0.)
+  struct Fitted {
+    const void* kernel;
+    size_t lds;
+    int sets;
+  };
+  std::vector<Fitted> filters_known;
+  template <typename K, typename Lds>
+  FilterShape fit_filter(K kernel, FilterShape f, Lds&& lds_of) {
+    if (filter_entries > 0 || f.sets() == 0) return f;
+    const void* const id = reinterpret_cast<const void*>(kernel);
+    const size_t least_lds = lds_of(f);
+    for (const Fitted& k : filters_known)
+      if (k.kernel == id && k.lds == least_lds) return filter_shape(k.sets, host.N);
+    const int most = std::min(4 * f.sets(), kMostFilterSets);
+    while (true) {
+      const FilterShape half = filter_shape(f.sets() / 2, host.N);
+      if (half.sets() >= f.sets() || resident_slots(kernel, lds_of(half)) * 20 < resident_slots(kernel, lds_of(f)) * 23) break;
+      f = half;
+    }
+    const int waves = resident_slots(kernel, lds_of(f));
+    for (int low = f.sets(), high = most; high - low >= 8;) {
+      const FilterShape mid = filter_shape((low + high) / 2, host.N);
+      if (mid.sets() > low && mid.sets() < high && resident_slots(kernel, lds_of(mid)) >= waves) low = (f = mid).sets();
+      else high = (low + high) / 2;
+    }
+    if (filters_known.size() >= 64) filters_known.clear();
+    filters_known.push_back({id, least_lds, f.sets()});
+    return f;
   }
 
-  // (asked of the runtime once per kernel and LDS size: a search wants to know half a dozen of them)
+  // How many wavefronts (workgroups of one) of a kernel the GPU holds.  A workgroup's LDS is handed out in whole steps of
+  // kLdsStep bytes, which the runtime's answer leaves out (measured with workgroups that count each other, 160 KB per CU:
+  // 5 120 bytes 32 on a CU, 5 184 25, 6 464 21, 7 744 18; the runtime says 32, 31, 25 and 21).  (Asked once per kernel and LDS
+  // size: a search wants to know half a dozen of them.)
+  static constexpr size_t kLdsStep = 1280;
   struct Resident {
     const void* kernel;
     size_t lds;
@@ -579,13 +615,17 @@ class Engine {
   std::vector<Resident> resident_known;
   template <typename K>
   int resident_slots(K kernel, size_t lds) {
+    const void* const id = reinterpret_cast<const void*>(kernel);
     for (const Resident& r : resident_known)
-      if (r.kernel == reinterpret_cast<const void*>(kernel) && r.lds == lds) return r.slots;
+      if (r.kernel == id && r.lds == lds) return r.slots;
+    hipFuncAttributes attr;
+    HIP_CHECK(hipFuncGetAttributes(&attr, id));
+    const size_t fixed = attr.sharedSizeBytes, whole = (fixed + lds + kLdsStep - 1) / kLdsStep * kLdsStep;
     int per_cu = 0;
-    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, lds));
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, std::max(whole, fixed) - fixed));
     per_cu = std::max(1, std::min(per_cu, 32));
-    if (resident_known.size() >= 64) resident_known.clear();
-    resident_known.push_back({reinterpret_cast<const void*>(kernel), lds, per_cu * num_cus});
+    if (resident_known.size() >= 256) resident_known.clear();
+    resident_known.push_back({id, lds, per_cu * num_cus});
     return per_cu * num_cus;
   }
 
@@ -622,7 +662,7 @@ class Engine {
         throw std::runtime_error("search_knn (no allocation): at most " + std::to_string(kStaticMaxQueries) + " queries per call");
       if (ef > kStaticMaxEf)
         throw std::runtime_error("search_knn (no allocation): max(topk, ef_search) must not exceed " + std::to_string(kStaticMaxEf));
-      if (auto_fc_bits(ef) == 0)
+      if (least_filter(ef).sets() == 0)
         throw std::runtime_error("search_knn (no allocation): the index has too many points for the LDS visited filter");
     }
     DevIndex ix = dev_index();
@@ -630,7 +670,8 @@ class Engine {
     a.q = d_qdata; a.nq = nq; a.k = k; a.ef = ef;
     a.nns = d_nns_out; a.dists = d_dist_out; a.found = d_found_out; a.stats = d_stats;
     a.hnswlib_dist = hnswlib_dist;
-    a.lcap = (std::max(std::max(host.S0, host.SU), std::max(k, 64)) + 63) / 64 * 64;
+    a.rcap = (std::max(std::max(host.S0, host.SU), 64) + 63) / 64 * 64;
+    a.lcap = std::max(a.rcap, (k + 63) / 64 * 64);
     const int q = qr();
     size_t fixed = (size_t)a.lcap * 8 + (q == 0 ? (size_t)query_lds_chunks(Dp) * 16 : 0);
     int ns = key_slots(ef);
@@ -651,8 +692,8 @@ class Engine {
     // literal pass does, on a sorted list in LDS
     if (a.reverse) a.fast_path = ns > 0 ? 2 : 0;
     if (a.reverse && no_alloc && ns == 0) throw std::runtime_error("search_knn (no allocation): reverse_cand needs ef_search below 1024");
-    a.fc_bits = (ns > 0 && a.fast_path) ? auto_fc_bits(ef) : 0;
-    if (a.reverse && ns > 0 && a.fc_bits == 0)
+    a.fc = (ns > 0 && a.fast_path) ? least_filter(ef) : FilterShape();
+    if (a.reverse && ns > 0 && a.fc.sets() == 0)
       throw std::runtime_error("search_knn: reverse_cand needs fewer than 2^28 points");
     // with the keys in registers the queue's LDS share doubles as result buffer (lcap entries,
     // then lcap label slots) and as the replay heap (ef + 1 entries)

@@ -69,20 +69,22 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   auto choose_variant = [&](bool with_trails) {
     const size_t bitmap_bytes = (size_t)std::min(num_cus * 24, a.nq) * ((host.N + 31) / 32) * 4;
     const bool want_lean = lean_literal == 1 ? with_trails || bitmap_bytes > ((size_t)32 << 20) : lean_literal > 1;
-    a.lean = (NS > 0 && fast_path != 0 && want_lean) ? auto_fc_bits(a.ef) : 0;
-    if (a.lean && filter_entries <= 0) {
+    a.lean = (NS > 0 && fast_path != 0 && want_lean) ? least_filter(a.ef) : FilterShape();
+    if (a.lean.sets() && filter_entries <= 0) {
+      int sets = 256;
+      while (sets < a.lean.sets()) sets *= 2;
+      a.lean = filter_shape(std::min(sets, 4096), host.N);
       // a batch of few queries leaves most of each CU's LDS unused: give the filter what is there
       // (up to 32 KB), so that it forgets next to nothing
       const int per_cu = (a.nq + num_cus - 1) / num_cus;
       const size_t room = per_cu > 0 ? (size_t)(150 * 1024) / per_cu : 0;
-      const size_t other = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, 0, 0, 0).total + 256;
-      while (a.lean < 13 && other + ((size_t)4 << (a.lean + 1)) <= std::min<size_t>(room, 60 * 1024) &&
-             (((unsigned)host.N >> a.lean) < 0xFFFFu))
-        ++a.lean;
+      const size_t other = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0).total + 256;
+      while (a.lean.sets() < 4096 && other + 2 * a.lean.bytes() <= std::min<size_t>(room, 60 * 1024))
+        a.lean = filter_shape(std::min(2 * a.lean.sets(), 4096), host.N);
     }
   };
   auto literal_lds = [&](int cand_lds) -> size_t {
-    return plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, cand_lds, a.lcap, 0, 0, a.lean ? 0 : a.vc_bits, 0, a.lean).total;
+    return plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, cand_lds, a.lcap, 0, 0, a.lean.sets() ? 0 : a.vc_bits, FilterShape(), a.lean).total;
   };
   auto kernel = search_kernel<DT, QR, NS>;
   int glob_cap = spill_cap > 0 ? spill_cap : std::max(4096, 8 * a.ef);
@@ -100,32 +102,24 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   // memory as long as the queues are busy (QR == 0).  One batch in sixteen takes the first pass all the same, so that the
   // share is not taken for known forever.
   bool literal_alone = false;
-  if (NS > 2 && QR > 0 && fast_path == 1 && a.fast_path == 1 && a.fc_bits > 0 && max_slots_override <= 0 &&
+  if (NS > 2 && QR > 0 && fast_path == 1 && a.fast_path == 1 && a.fc.sets() > 0 && max_slots_override <= 0 &&
       cautious_share() * a.nq >= 1.5) {
     choose_variant(false);
-    if (!a.lean && a.nq <= resident_slots(kernel, literal_lds(a.cand_lds))) {
+    if (!a.lean.sets() && a.nq <= resident_slots(kernel, literal_lds(a.cand_lds))) {
       literal_alone = literal_streak < kLiteralStreak;
       literal_streak = literal_alone ? literal_streak + 1 : 0;
     }
   }
-  const bool first_pass = NS > 0 && a.fast_path && a.fc_bits > 0 && !literal_alone;  // (reverse_cand: fast_path is 2)
+  const bool first_pass = NS > 0 && a.fast_path && a.fc.sets() > 0 && !literal_alone;  // (reverse_cand: fast_path is 2)
   if (!first_pass) choose_variant(false);
   if constexpr (NS > 0) if (first_pass) {
     d_redo.reserve((size_t)a.nq);
     a.redo = d_redo.p;
     auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
-    auto fast_lds = [&](int bits) -> size_t { return plan_fast_lds(QR, ix.Dp, a.lcap, bits).total; };
-    auto fast_slots = [&](int bits) -> int { return resident_slots(fast_kernel, fast_lds(bits)); };
-    // the filter must not be what limits the wavefronts per CU: half the filter repeats more
-    // evaluations but is the faster choice wherever it buys 15 % more wavefronts
-    while (filter_entries <= 0 && a.fc_bits > 9) {
-      const int now = fast_slots(a.fc_bits);
-      const int with_half = fast_slots(a.fc_bits - 1);
-      if (with_half * 20 < now * 23) break;  // less than 15 % more
-      --a.fc_bits;
-    }
-    const size_t fast_lds_bytes = fast_lds(a.fc_bits);
-    int slots = fast_slots(a.fc_bits);
+    auto fast_lds = [&](FilterShape f) -> size_t { return plan_fast_lds(QR, ix.Dp, a.rcap, f, a.k).total; };
+    a.fc = fit_filter(fast_kernel, a.fc, fast_lds);
+    const size_t fast_lds_bytes = fast_lds(a.fc);
+    int slots = resident_slots(fast_kernel, fast_lds_bytes);
     // A batch of at most one wavefront per SIMD that is not expected to hand anything over does without the second
     // stream: its events and the wait for the waiting wavefronts are 60 us of a search of a few hundred.
     const bool alone = fast_path == 1 && !a.reverse && a.nq <= std::min(4 * num_cus, slots) && first_pass_waves == 0 &&
@@ -162,7 +156,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
     bool keep_trails = !alone && (QR == 1 || QR == 2) && trails && !a.reverse && host.S0 <= 63 &&
                        (trails > 1 || 4 * (long long)a.nq <= 11 * resident);
     choose_variant(keep_trails);
-    keep_trails = keep_trails && a.lean;
+    keep_trails = keep_trails && a.lean.sets() > 0;
     if (keep_trails) {
       // (normally there since the index became resident; a changed trail_cap / trail_spares asks again)
       if (d_trail.n < trail_records_wanted(slots)) {
@@ -272,7 +266,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
         hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), 0, stream, ix, a);
       } else {
         auto k_entry = entry_kernel<DT, QR>;
-        const size_t entry_lds = plan_fast_lds(QR, ix.Dp, a.lcap, 0).total;
+        const size_t entry_lds = plan_fast_lds(QR, ix.Dp, a.rcap, FilterShape(), 0).total;
         const int entry_grid = std::max(1, std::min(a.nq, resident_slots(k_entry, entry_lds)));
         hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), entry_lds, stream, ix, a);
       }
@@ -378,17 +372,12 @@ void Engine::launch_search_static(const DevIndex& ix, SearchArgs& a, float* ms) 
     a.done = sc->ctl + 64;
     a.redo = sc->redo;
     a.fast_path = 2;
-    a.lean = a.fc_bits;  // literal searches keep the LDS filter and the sorted set with ids: no bitmap in HBM
+    a.lean = a.fc;  // literal searches keep the LDS filter and the sorted set with ids: no bitmap in HBM
     auto kernel = search_kernel<DT, QR, NS>;
     auto fast_kernel = search_fast_kernel<DT, QR, NS, false>;
-    while (filter_entries <= 0 && a.fc_bits > 9) {  // (as in the allocating search: the filter must not cost occupancy)
-      const int now = resident_slots(fast_kernel, plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits).total);
-      const int with_half = resident_slots(fast_kernel, plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits - 1).total);
-      if (with_half * 20 < now * 23) break;
-      --a.fc_bits;
-    }
-    const FastLdsPlan fp = plan_fast_lds(QR, ix.Dp, a.lcap, a.fc_bits);
-    const LdsPlan lp = plan_lds(QR, ix.Dp, -1, a.cand_lds, a.lcap, 0, 0, 0, 0, a.lean);
+    a.fc = fit_filter(fast_kernel, a.fc, [&](FilterShape f) { return plan_fast_lds(QR, ix.Dp, a.rcap, f, a.k).total; });
+    const FastLdsPlan fp = plan_fast_lds(QR, ix.Dp, a.rcap, a.fc, a.k);
+    const LdsPlan lp = plan_lds(QR, ix.Dp, -1, a.cand_lds, a.lcap, 0, 0, 0, FilterShape(), a.lean);
     const int slots = std::max(1, std::min(resident_slots(fast_kernel, fp.total), a.nq));
     const int lit_slots = std::max(1, std::min(std::min(resident_slots(kernel, lp.total), kStaticSlots), a.nq));
     if (ms) HIP_CHECK(hipEventRecord(ev0, stream));
@@ -505,14 +494,16 @@ void Engine::build_levels() {
   a.lcap = (std::max(s_max, 64) + 63) / 64 * 64;
   size_t fixed = (size_t)a.lcap * 8 + (size_t)efc * 8 + (size_t)m_max * 8 + 64 +
                  (QR == 0 ? (size_t)query_lds_chunks(Dp) * 16 : 0);
-  a.fc_bits = NS > 0 ? auto_fc_bits(efc) : 0;
-  const bool sorted_set = NS > 0 && a.fc_bits > 0;  // then neither queue nor literal cache is needed
+  a.fc = NS > 0 ? least_filter(efc) : FilterShape();
+  const bool sorted_set = NS > 0 && a.fc.sets() > 0;  // then neither queue nor literal cache is needed
   if (a.reverse && NS > 0 && !sorted_set) throw std::runtime_error("build_graph: reverse_cand needs fewer than 2^28 points");
   a.cand_lds = sorted_set ? 0 : auto_cand_lds(efc, NS, 64, fixed);
   a.vc_bits = sorted_set ? 0 : auto_vc_bits();
-  const LdsPlan lp1 = plan_lds(QR, Dp, sorted_set ? -1 : efc, a.cand_lds, a.lcap, efc, m_max, a.vc_bits, a.fc_bits);
+  auto search_lds = [&](FilterShape f) { return plan_lds(QR, Dp, sorted_set ? -1 : efc, a.cand_lds, a.lcap, efc, m_max, a.vc_bits, f).total; };
+  a.fc = fit_filter(k_search, a.fc, search_lds);
+  const size_t lds1 = search_lds(a.fc);
   const LdsPlan lp3 = plan_lds(QR, Dp, s_max + cap_in, 0, a.lcap, s_max + cap_in, std::max(m_max, cap_in));
-  const int slots1 = resident_slots(k_search, lp1.total);
+  const int slots1 = resident_slots(k_search, lds1);
   const int slots3 = resident_slots(k_reverse, lp3.total);
   // the sorted-set search needs no per-wavefront global memory (no bitmap, no undo list, no log)
   if (!sorted_set) ensure_pool(slots1, glob_cap, 2 * glob_cap);
@@ -567,7 +558,7 @@ void Engine::build_levels() {
       a.n_upper = upper_end[batch] - from;
     }
     ++batch;
-    hipLaunchKernelGGL(k_search, dim3(std::min(b, slots1)), dim3(64), lp1.total, stream, ix, a);
+    hipLaunchKernelGGL(k_search, dim3(std::min(b, slots1)), dim3(64), lds1, stream, ix, a);
     HIP_CHECK(hipGetLastError());
     if (cur_max >= 0) {
       long long work = (long long)b * m_max;

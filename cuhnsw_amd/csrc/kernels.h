@@ -69,14 +69,15 @@ struct SearchArgs {
                           // device (the count the first pass left) instead of taken from nq
   int slot_base;   // first slot of the pool this launch may use (two literal launches can be in flight)
   SlotPool pool;
-  int cand_lds, lcap, hnswlib_dist;
+  int cand_lds, hnswlib_dist;
+  int rcap, lcap;  // ids and keys a row buffer holds: those of a link row; literal pass: those of the answer too
   int vc_bits;  // log2 entries of the LDS visited cache of the literal search, 0 = none
-  int fc_bits;  // log2 sets (two tags each) of the LDS visited filter of the sorted-set search, 0 = that search is off
+  FilterShape fc;  // the LDS visited filter of the sorted-set search (no sets: that search is off)
   int fast_path;  // 0 = literal queues only (exact evaluation counters)
   int reverse;    // expand the farthest waiting candidate (reverse_cand); sorted-set pass only
   const uint32_t* deleted;  // one bit per element (hnswlib's delete marks) or null; literal queues in LDS only (NS == 0)
-  int lean;       // literal pass: result set = sorted set with ids, visited = LDS filter of 2^lean sets
-                  // (no bitmap, evaluation counters include repeats); 0 = exact bitmap
+  FilterShape lean;  // literal pass: result set = sorted set with ids, visited = an LDS filter of this shape
+                     // (no bitmap, evaluation counters include repeats); no sets = exact bitmap
   // Sorted-set pass with its queries taken longest first (entry_kernel and the two order kernels below); all
   // null = queries in the caller's order, each descending from the top level itself.
   uint4* entry;     // per query: level-0 entry point, its key (bits), evaluations and sweeps of the descent
@@ -109,7 +110,8 @@ struct BuildArgs {
   int* status;
   SlotPool pool;
   int cand_lds, lcap;
-  int vc_bits, fc_bits;
+  int vc_bits;
+  FilterShape fc;
   HeapEnt* inbox0;  // N x cap_in
   int* inbox0_cnt;  // N
   HeapEnt* inboxU;  // upper rows x cap_in
@@ -152,10 +154,10 @@ inline int query_regs(int Dp) {
 struct LdsPlan {
   size_t qlds, top, cand, sorted_id, sorted_key, out_id, out_key, nbuf, dbuf, vcache, fcache, lfilter, total;
 };
-// fc_bits: filter lying over the queue (build); lf_bits: filter of its own beside the queue (the
+// fc: filter lying over the queue (build); lf: filter of its own beside the queue (the
 // literal search on the sorted set)
 __host__ __device__ inline LdsPlan plan_lds(int qr, int Dp, int ef, int cand_lds, int lcap, int n_sorted, int n_out,
-                                            int vc_bits = 0, int fc_bits = 0, int lf_bits = 0) {
+                                            int vc_bits = 0, FilterShape fc = FilterShape(), FilterShape lf = FilterShape()) {
   LdsPlan p;
   size_t o = 0;
   p.qlds = o;
@@ -164,7 +166,7 @@ __host__ __device__ inline LdsPlan plan_lds(int qr, int Dp, int ef, int cand_lds
   p.cand = o; o = align16(o + (size_t)cand_lds * 8);
   p.vcache = o; o = align16(o + (vc_bits > 0 ? ((size_t)2 << vc_bits) : 0));
   p.fcache = p.cand;
-  const size_t fend = p.fcache + (fc_bits > 0 ? ((size_t)4 << fc_bits) : 0);
+  const size_t fend = p.fcache + fc.bytes();
   if (fend > o) o = align16(fend);
   p.sorted_id = o; o = align16(o + (size_t)n_sorted * 4);
   p.sorted_key = o; o = align16(o + (size_t)n_sorted * 4);
@@ -172,7 +174,7 @@ __host__ __device__ inline LdsPlan plan_lds(int qr, int Dp, int ef, int cand_lds
   p.out_key = o; o = align16(o + (size_t)n_out * 4);
   p.nbuf = o; o = align16(o + (size_t)nbuf_words(lcap) * 4);
   p.dbuf = o; o = align16(o + (size_t)lcap * 4);
-  p.lfilter = o; o = align16(o + (lf_bits > 0 ? ((size_t)4 << lf_bits) : 0));
+  p.lfilter = o; o = align16(o + lf.bytes());
   p.total = o;
   return p;
 }
@@ -188,18 +190,20 @@ __device__ __forceinline__ void bind_slot(Scratch& s, const SlotPool& pool, int 
   s.log_cap = pool.log_cap;
 }
 
-// LDS of the sorted-set search: query copy (long rows only), visited filter, row buffers
+// LDS of the sorted-set search: query copy (long rows only), visited filter, row buffers.  The answer (ids, keys, and a copy of
+// the ids where equal keys are put in order) lies over the filter, which is done with by then: a wavefront's LDS is handed out
+// in steps of 1 280 bytes, and with topk 100 in buffers of its own the filter of 28 wavefronts on a CU is a tenth smaller.
 struct FastLdsPlan {
   size_t qlds, fcache, nbuf, dbuf, total;
 };
-__host__ __device__ inline FastLdsPlan plan_fast_lds(int qr, int Dp, int lcap, int fc_bits) {
+__host__ __device__ inline FastLdsPlan plan_fast_lds(int qr, int Dp, int rcap, FilterShape fc, int k) {
   FastLdsPlan p;
   size_t o = 0;
   p.qlds = o;
   if (qr == 0) o += (size_t)query_lds_chunks(Dp) * 16;
-  p.fcache = o; o = align16(o + ((size_t)4 << fc_bits));
-  p.nbuf = o; o = align16(o + (size_t)nbuf_words(lcap) * 4);
-  p.dbuf = o; o = align16(o + (size_t)lcap * 4);
+  p.fcache = o; o = align16(o + (fc.bytes() > 12u * (uint32_t)k ? (size_t)fc.bytes() : (size_t)12 * (size_t)k));
+  p.nbuf = o; o = align16(o + (size_t)nbuf_words(rcap) * 4);
+  p.dbuf = o; o = align16(o + (size_t)rcap * 4);
   p.total = o;
   return p;
 }
@@ -239,7 +243,7 @@ template <int DT, int QR>
 __global__ void __launch_bounds__(64) entry_kernel(DevIndex ix, SearchArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x;
-  const FastLdsPlan lp = plan_fast_lds(QR, ix.Dp, a.lcap, 0);
+  const FastLdsPlan lp = plan_fast_lds(QR, ix.Dp, a.rcap, FilterShape(), 0);
   Scratch s;
   s.vcache = nullptr;
   s.vc_bits = 0;
@@ -485,10 +489,10 @@ constexpr int fast_waves_of_six(int dt, int qr, bool trails) { return (dt == DIS
 template <int DT, int QR, int NS, bool TRAILS, bool FEW = false>
 __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : NS == 6 ? fast_waves_of_six(DT, QR, TRAILS) : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.lcap, a0.fc_bits);
+  const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.rcap, a0.fc, a0.k);
   Scratch s;
   s.vcache = reinterpret_cast<uint16_t*>(smem + lp.fcache);
-  s.vc_bits = a0.fc_bits;
+  s.filter = a0.fc;
   s.qlds = reinterpret_cast<float4*>(smem + lp.qlds);
   s.nbuf = reinterpret_cast<uint32_t*>(smem + lp.nbuf);
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
@@ -568,7 +572,7 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
     const bool cut_tie = how == 2 && !a.reverse && frontier_tie_within<NS>(fr, a.ef, T0, st.top_size, lane, T0 - 1);
     const int inner_tie = __builtin_amdgcn_readfirstlane(
         (how == 2 && !a.reverse && frontier_tie_within<NS>(fr, a.ef, T0 - 1, st.top_size, lane)) ? 1 : 0);
-    const bool gave_up = how == 1 || cut_tie || (inner_tie && T0 > (1 << a.fc_bits));  // (the filter's LDS is the sort's buffer)
+    const bool gave_up = how == 1 || cut_tie;
     if (gave_up) {
       // (the trail's records are written by many lanes: all of them out before lane 0 publishes the entry)
       const bool with_trail = TRAILS && a.redo_trail && trail_buf >= 0 && tr.n > 0 && tr.hops > 0;
@@ -593,21 +597,23 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
       }
     } else {
       const int T = __builtin_amdgcn_readfirstlane(st.top_size < a.k ? st.top_size : a.k);
+      uint32_t* const ids = reinterpret_cast<uint32_t*>(s.vcache);
+      float* const keys = reinterpret_cast<float*>(ids + a.k);
       wave_sync();
-      frontier_dump<NS>(fr, a.ef, T, s.nbuf, s.dbuf, lane);
+      frontier_dump<NS>(fr, a.ef, T, ids, keys, lane);
       wave_sync();
-      if (inner_tie) order_equal_keys(ix, s.nbuf, s.dbuf, T, reinterpret_cast<uint32_t*>(s.vcache), lane);
+      if (inner_tie) order_equal_keys(ix, ids, keys, T, ids + 2 * a.k, lane);
       if (!a.hnswlib_dist && T > 0) {
-        dist_list<DT, QR, true>(ix, qv, s.qlds, s.nbuf, T, s.dbuf, lane);
+        dist_list<DT, QR, true>(ix, qv, s.qlds, ids, T, keys, lane);
         wave_sync();
       }
       for (int r = lane; r < a.k; r += 64) {
         int out_id = -1;
         float out_d = INFINITY;
         if (r < T) {
-          const uint32_t id = s.nbuf[r];
+          const uint32_t id = ids[r];
           out_id = ix.labels ? (int)ix.labels[id] : (int)id;
-          out_d = a.hnswlib_dist ? answer_key(s.dbuf[r]) : s.dbuf[r];
+          out_d = a.hnswlib_dist ? answer_key(keys[r]) : keys[r];
         }
         a.nns[(size_t)qi * a.k + r] = out_id;
         a.dists[(size_t)qi * a.k + r] = out_d;
@@ -654,12 +660,12 @@ template <int DT, int QR, int NS>
 __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) ? 5 : 1) search_kernel(DevIndex ix, SearchArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x;
-  const bool lean = NS > 0 && a.lean > 0;
-  const LdsPlan lp = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, lean ? 0 : a.vc_bits, 0, a.lean);
+  const bool lean = NS > 0 && a.lean.sets() > 0;
+  const LdsPlan lp = plan_lds(QR, ix.Dp, NS > 0 ? -1 : a.ef, a.cand_lds, a.lcap, 0, 0, lean ? 0 : a.vc_bits, FilterShape(), a.lean);
   Scratch s;
   if (lean) {
     s.vcache = reinterpret_cast<uint16_t*>(smem + lp.lfilter);
-    s.vc_bits = a.lean;
+    s.filter = a.lean;
   } else {
     s.vcache = a.vc_bits > 0 ? reinterpret_cast<uint16_t*>(smem + lp.vcache) : nullptr;
     s.vc_bits = a.vc_bits;
@@ -842,7 +848,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
       // eviction had twins to choose from; then the result heap is replayed from the log, as below.
       const bool inner_tie = !st.fail && frontier_tie_within<NS>(fr, a.ef, T - 1, st.top_size, lane);
       const bool replay = !st.fail && (frontier_tie_within<NS>(fr, a.ef, T, st.top_size, lane, T - 1) ||
-                                       (ambiguous && T == st.top_size) || (inner_tie && T > (1 << a.lean)));
+                                       (ambiguous && T == st.top_size) || (inner_tie && T > 2 * a.lean.sets()));
       if (!st.fail && !replay) {
         wave_sync();
         frontier_dump<NS>(fr, a.ef, T, s.nbuf, s.dbuf, lane);
@@ -1151,12 +1157,13 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
   extern __shared__ __align__(16) unsigned char smem[];
   int lane = threadIdx.x;
   const int m_max = ix.max_m0 > ix.max_m ? ix.max_m0 : ix.max_m;
-  const bool sorted_set = NS > 0 && a.fc_bits > 0;
-  const LdsPlan lp = plan_lds(QR, ix.Dp, sorted_set ? -1 : a.efc, a.cand_lds, a.lcap, a.efc, m_max, a.vc_bits, a.fc_bits);
+  const bool sorted_set = NS > 0 && a.fc.sets() > 0;
+  const LdsPlan lp = plan_lds(QR, ix.Dp, sorted_set ? -1 : a.efc, a.cand_lds, a.lcap, a.efc, m_max, a.vc_bits, a.fc);
   Scratch s;
   s.vcache = sorted_set ? reinterpret_cast<uint16_t*>(smem + lp.fcache)
                         : (a.vc_bits > 0 ? reinterpret_cast<uint16_t*>(smem + lp.vcache) : nullptr);
-  s.vc_bits = sorted_set ? a.fc_bits : a.vc_bits;
+  s.vc_bits = a.vc_bits;
+  s.filter = a.fc;
   s.qlds = reinterpret_cast<float4*>(smem + lp.qlds);
   s.top = reinterpret_cast<HeapEnt*>(smem + lp.top);
   s.cand = reinterpret_cast<HeapEnt*>(smem + lp.cand);
