@@ -51,6 +51,28 @@ struct DevIndex {
   int half;                  // vectors are stored as fp16 (all arithmetic stays fp32 on the stored values)
 };
 
+// What the wavefronts of a team share in LDS beside the visited filter (team_help): whose list is in which slot, four slots to a bucket;
+// the candidates that come next; whether the search is over; room to work in for the wavefront that searches; the lists.
+constexpr int kTeamSlots = 128;  // at most
+struct Team {
+  uint32_t* base = nullptr;
+  int bucket_bits = 0;  // log2 of the buckets
+  int stride = 0;       // ids (and keys) a list holds
+  int lists = 0;        // where they begin
+  static constexpr int kInLine = 32;
+  static constexpr int kLine = kTeamSlots, kOver = kLine + 2 * (kInLine + 1), kRoom = kOver + 2;
+  __host__ __device__ static int lists_at(int ns) { return kRoom + 128 * (ns + 1); }
+  __host__ __device__ static int words(int ns, int bucket_bits, int stride) { return lists_at(ns) + (8 << bucket_bits) * stride; }
+  __device__ __forceinline__ uint32_t* owner() const { return base; }
+  // the closest candidates; behind them a place that nobody reads
+  __device__ __forceinline__ HeapEnt* line() const { return reinterpret_cast<HeapEnt*>(base + kLine); }
+  __device__ __forceinline__ uint32_t* over() const { return base + kOver; }
+  __device__ __forceinline__ uint32_t* room() const { return base + kRoom; }
+  __device__ __forceinline__ uint32_t bucket(uint32_t id) const { return (id * 2654435761u) >> (32 - bucket_bits); }
+  __device__ __forceinline__ uint32_t* ids(int slot) const { return base + lists + 2 * slot * stride; }
+  __device__ __forceinline__ float* keys(int slot) const { return reinterpret_cast<float*>(ids(slot) + stride); }
+};
+
 // per resident wavefront scratch: LDS pointers + this wavefront's global slot
 struct Scratch {
   HeapEnt* top;        // LDS, ef + 1 entries
@@ -70,6 +92,7 @@ struct Scratch {
   HeapEnt* log;        // global, every accepted (key, id) in acceptance order
   int log_cap;
   StageTree tree;      // per-lane constants of the cooperative heap pop
+  Team team;           // LDS, shared with the wavefronts that help this one (sorted-set search of a batch that leaves the machine idle)
 };
 
 // The candidates a search expands at a time (tie_free_phase) lie in LDS behind the 64 ids that search lists in s.nbuf.
@@ -146,6 +169,7 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));
 }
+__device__ __forceinline__ unsigned long long first_lanes(int n) { return n < 64 ? (1ull << (n & 63)) - 1ull : ~0ull; }  // (n <= 64)
 __device__ __forceinline__ float wave_min(float x) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) x = fminf(x, __shfl_xor(x, m, 64));
@@ -493,7 +517,7 @@ __device__ __forceinline__ void dist_list_t(const DevIndex& ix, const QVec<QR>& 
   if (QR > 0) {
     constexpr int R = QR > 0 ? QR : 1;
     // groups of 4 rows in flight
-    constexpr int UMAX = R == 1 ? (WIDE >= 4 ? 8 : 4) : (R == 2 ? (WIDE >= 4 ? 8 : (WIDE >= 2 ? 4 : (WIDE >= 1 ? 2 : 1))) : (WIDE >= 4 ? 4 : 1));
+    constexpr int UMAX = R == 1 ? (WIDE >= 4 ? 8 : 4) : (R == 2 ? (WIDE >= 4 ? 8 : (WIDE >= 2 ? 4 : (WIDE >= 1 ? 2 : 1))) : (WIDE >= 4 ? 4 : (WIDE >= 3 ? 2 : 1)));
     int r = 0;
     while (r < n) {
       const int rem = n - r;
@@ -985,6 +1009,28 @@ __device__ __forceinline__ int max_so_far(int x) {
   take(__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
   return x;
 }
+// Smallest value of all lanes (finite, or +inf).
+__device__ __forceinline__ float least_of_all(float x) {
+  auto take = [&](int from) __attribute__((always_inline)) { x = fminf(x, __builtin_bit_cast(float, from)); };
+  const auto bits = [&]() __attribute__((always_inline)) { return __builtin_bit_cast(int, x); };
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x111, 0xF, 0xF, false));  // (as max_so_far: lane 63 has seen all)
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x112, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x114, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x118, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x142, 0xA, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x143, 0xC, 0xF, false));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits(), 63));
+}
+__device__ __forceinline__ int least_of_all_ints(int x) {
+  auto take = [&](int from) __attribute__((always_inline)) { x = from < x ? from : x; };
+  take(__builtin_amdgcn_update_dpp(x, x, 0x111, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(x, x, 0x112, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(x, x, 0x114, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(x, 63);
+}
 // Several offers of a list at once: those of the lanes in `offers` (fewer than 64; not SPARSE: the first lanes, and +inf in
 // the others), whose list lies in ids / keys (LDS), into a set of `size` entries; what does not fit behind ef entries falls off its end.  The offers are put
 // in order (in ids / keys), every entry finds by halving how many of them go before it, and entries and offers go to their
@@ -1164,6 +1210,152 @@ __device__ __forceinline__ int frontier_take_many(Frontier<NS>& f, int want, Hea
   }
   wave_sync();
   return total < want ? total : want;
+}
+// frontier_insert_all<SPARSE> for the wavefront that searches in a team, where latency is all that counts and LDS there is: every entry and
+// every offer is compared with all offers, four keys to an LDS read (halving, a trip to LDS per step, or reading the
+// keys from lanes, a scalar hazard each, takes twice as long); keys and ids move together, and the set stays as it is in its
+// registers until the outcome is known.  Of several offers of one node one counts.  room: 128 * (NS + 1) words.
+template <int NS>
+__device__ __forceinline__ bool frontier_merge(Frontier<NS>& f, unsigned long long offers, int size, int ef, float my_key, uint32_t my_id,
+                                               uint32_t* room, float above, int& count, float& last_key, int lane) {
+  constexpr int N = NS > 0 ? NS : 1;
+  int less = 0;   // offers before this lane's
+  int before[N];  // offers before each of this lane's entries
+  int n, entries;
+  bool mine, equal;
+  while (true) {
+    n = __popcll(offers);
+    mine = __builtin_amdgcn_inverse_ballot_w64(offers);
+    float* const keys = reinterpret_cast<float*>(room);
+    keys[lane] = INFINITY;
+    wave_sync();
+    if (mine) keys[lanes_below(offers)] = my_key;
+    wave_sync();
+    less = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) before[j] = 0;
+    for (int i = 0; i < n; i += 4) {
+      const float4 k = reinterpret_cast<const float4*>(keys)[i >> 2];
+      less += k.x < my_key ? 1 : 0;
+      less += k.y < my_key ? 1 : 0;
+      less += k.z < my_key ? 1 : 0;
+      less += k.w < my_key ? 1 : 0;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        before[j] += k.x < f.k[j] ? 1 : 0;
+        before[j] += k.y < f.k[j] ? 1 : 0;
+        before[j] += k.z < f.k[j] ? 1 : 0;
+        before[j] += k.w < f.k[j] ? 1 : 0;
+      }
+    }
+    wave_sync();
+    // how many entries go before an offer that has so many offers before it (as in frontier_insert_all); and the offers in order,
+    // where one of two equal ones leaves a place empty
+    const int next_first = __builtin_amdgcn_update_dpp(-1, before[0], 0x130, 0xF, 0xF, false);  // wave_shl:1
+    uint32_t* const nth = room + 128;
+    room[lane] = 0u;
+    nth[lane] = 64u;
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int after = j + 1 < N ? before[j + 1 < N ? j + 1 : 0] : next_first;
+      room[after != before[j] ? before[j] : 64 + lane] = (uint32_t)(lane * N + j + 1);
+    }
+    if (mine) nth[less] = (uint32_t)lane;
+    wave_sync();
+    entries = max_so_far((int)room[lane]);
+    const uint32_t at_place = nth[lane], first = nth[mine ? less : 0];
+    equal = __ballot(lane < n && at_place == 64u) != 0ull;
+    if (__builtin_expect(!equal, 1)) break;
+    const uint32_t first_id = (uint32_t)__shfl((int)my_id, (int)first, 64);
+    const unsigned long long again = __ballot(first != (uint32_t)lane && first_id == my_id) & offers;
+    if (again == 0ull) break;
+    offers &= ~again;
+    wave_sync();
+  }
+  bool done = false;
+  if (!equal && n < 64) {
+    const int place = __shfl(entries, less, 64) + less;
+    wave_sync();
+    HeapEnt* const to = reinterpret_cast<HeapEnt*>(room);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      HeapEnt e;
+      e.key = f.k[j];
+      e.id = f.v[j];
+      to[lane * N + j + before[j]] = e;
+    }
+    if (mine) {
+      HeapEnt e;
+      e.key = my_key;
+      e.id = my_id;
+      to[place] = e;
+    }
+    wave_sync();
+    HeapEnt now[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) now[j] = to[lane * N + j];
+    const float last = uni(to[64 * N - ef + (size + n < ef ? size + n : ef) - 1].key);
+    const float next_to = to[mine && place > 0 ? place - 1 : 0].key;
+    // (an offer equal to an entry comes right behind it; those that fall off count as far as they are no farther than the last)
+    done = __ballot(mine && my_key <= last && place > 0 && next_to == my_key) == 0ull && last > above;
+    if (done) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        f.k[j] = now[j].key;
+        f.v[j] = now[j].id;
+      }
+      last_key = last;
+      count = n;
+    }
+    wave_sync();
+  }
+  return done;
+}
+// For a team (team_help): the eight closest entries not yet expanded to the first places of its line, the 24 next
+// ones behind them.  None is marked; returns how many there are in all, rank: waiting entries in the lanes below.  (All
+// writes are unconditional, to a place that nobody reads where there is nothing to write: no exec-mask branches.)
+template <int NS>
+__device__ __forceinline__ int frontier_line_up(const Frontier<NS>& f, const Team& team, int& rank, int lane) {
+  constexpr int N = NS > 0 ? NS : 1;
+  HeapEnt* const line = team.line();
+  int total = 0;
+  rank = 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const unsigned long long open = __ballot((int)f.v[j] >= 0);
+    total += __popcll(open);
+    rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned int)(open >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)open, (unsigned int)rank));
+  }
+  int at = rank;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const bool open = (int)f.v[j] >= 0;
+    HeapEnt e;
+    e.key = f.k[j];
+    e.id = f.v[j];
+    line[open && at < Team::kInLine ? at : Team::kInLine] = e;
+    at += open ? 1 : 0;
+  }
+  if (total < Team::kInLine && lane >= total && lane < Team::kInLine) {
+    HeapEnt none;
+    none.key = INFINITY;
+    none.id = kEmpty;
+    line[lane] = none;
+  }
+  wave_sync();
+  return total;
+}
+// marks the `count` closest entries not yet expanded
+template <int NS>
+__device__ __forceinline__ void frontier_take_first(Frontier<NS>& f, int count, int rank) {
+  constexpr int N = NS > 0 ? NS : 1;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const bool open = (int)f.v[j] >= 0;
+    f.v[j] |= open && rank < count ? kExpanded : 0u;
+    rank += open ? 1 : 0;
+  }
 }
 // key of the entry with this id (which is in the set)
 template <int NS>
@@ -1358,10 +1550,10 @@ __device__ __forceinline__ void search_level_far_lds(const DevIndex& ix, const Q
 // (Four ways rather than two at the same size: on the 1.18 M-point set the neighbourhoods
 // overlap so much that most forgotten nodes were victims of set conflicts, not of capacity —
 // repeated evaluations fell from 31 % to 12 % of the distinct ones.)
-__device__ __forceinline__ void filter_reset(Scratch& s, int lane) {
+__device__ __forceinline__ void filter_reset(Scratch& s, int lane, int lanes = 64) {
   uint4* c4 = reinterpret_cast<uint4*>(s.vcache);
   const int n4 = (s.filter.sets() + 1) >> 1;  // 2 sets per 16 bytes
-  for (int i = lane; i < n4; i += 64) {
+  for (int i = lane; i < n4; i += lanes) {
     const uint32_t a = filter_empty_tag(s.filter, 2u * (uint32_t)i) * 0x10001u, b = filter_empty_tag(s.filter, 2u * (uint32_t)i + 1u) * 0x10001u;
     c4[i] = make_uint4(a, a, b, b);
   }
@@ -1407,6 +1599,20 @@ __device__ __forceinline__ uint32_t filter_find(FilterShape f, uint32_t id, uint
   const uint32_t place = f.more_bits() != 0 ? filter_place<true>(id) : filter_place<false>(id);
   slot = filter_set<true>(f, place);
   return place;
+}
+// the lanes whose id the filter does not know; enters the ids of the lanes in `which` (where two of them fall into one set one is forgotten)
+__device__ __forceinline__ unsigned long long filter_unknown(const Scratch& s, uint32_t id) {
+  uint32_t set;
+  const uint32_t place = filter_find(s.filter, id, set);
+  return filter_misses(reinterpret_cast<const uint2*>(s.vcache)[set], place);
+}
+__device__ __forceinline__ void filter_enter(Scratch& s, uint32_t id, unsigned long long which) {
+  uint2* sets = reinterpret_cast<uint2*>(s.vcache);
+  uint32_t set;
+  const uint32_t place = filter_find(s.filter, id, set);
+  const uint2 w = sets[set];
+  if (__builtin_amdgcn_inverse_ballot_w64(which)) sets[set] = filter_push(w, place);
+  __builtin_amdgcn_wave_barrier();
 }
 __device__ __forceinline__ void visit_lossy_single(Scratch& s, uint32_t id, int lane) {
   if (lane == 0) {
@@ -1464,6 +1670,169 @@ __device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t can
                                                 int& n_ids, unsigned long long& ends, int lane) {
   if (__builtin_expect(s.filter.more_bits() != 0, 0)) return visit_lossy_rows_t<K, true>(ix, cands, rows, level, S, s, n_ids, ends, lane);
   return visit_lossy_rows_t<K, false>(ix, cands, rows, level, S, s, n_ids, ends, lane);
+}
+// ---- a query that a team of wavefronts searches ---------------------------------------------------------------
+// A batch that leaves the machine idle is bound by the chain of its slowest search: fetch the next candidates' link rows, fetch the
+// vectors of their new nodes, put those into the set, choose the next candidates.  The first two are memory latency and
+// arithmetic that nothing but the choice of the candidates waits for, and the choice is mostly known ahead: of the 300
+// candidates that a search expands at ef 300, 274 are among the next sixteen in line two steps before their turn (60 000 x 50; 102 of
+// 128 at ef 128 on integers).  So one wavefront of a workgroup makes the search; in every step it says which candidates are the next
+// in line, and the others fetch their link rows and evaluate the nodes that have not been dealt with, ahead of time.  A
+// candidate whose list is there when its turn comes costs neither fetch; one whose list is not is evaluated by the
+// search itself.  The search's decisions, and what it returns, are its own either way: a list holds every node of the link
+// row but those whose offers it has dealt with for good, with the keys it would have computed.  A helper that
+// finds a node closer than the candidate it came from goes on with that node, which will be the next candidate.
+// (Cycles of a step of one query on 100 000 x 50 at ef 300, a wavefront alone: distances 1 150, the set 2 200, candidates, links and
+// filter 2 090, 112 steps; the search by a team has 69 of them, of which 13 evaluate nodes of their own.)
+//
+// Slots: the owner's id when its list is there, how many eights of nodes it has in bits 28 to 30; the id with kExpanded while it is
+// being made; kNobody: free.  (Ids are below 2^28 where there is a visited filter.)  A helper takes a free slot of the candidate's
+// bucket by compare-and-swap, then looks whether the candidate is still in line and in no other slot (the search writes the line
+// before it looks for lists: one of the two sees the other), and gives the slot back otherwise.  Only the search frees a slot
+// whose list is there.  LDS operations of a wavefront are carried out in order.
+constexpr uint32_t kNobody = 0x7FFFFFFFu, kTeamId = 0x0FFFFFFFu;
+constexpr int kMostListed = 56;  // (seven eights; a longer list is left to the search)
+__device__ __forceinline__ void lds_done() {  // everything this wavefront wrote to LDS is there
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ uint32_t lds_now(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+__device__ __forceinline__ void lds_tell(uint32_t* p, uint32_t x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+// The slots of a node's bucket.  there: the slot its list is in, or -1; eights: of nodes there; making: its list is being made;
+// room: a free slot, or -1.
+struct TeamPlace {
+  int there, eights, room;
+  bool making;
+};
+__device__ __forceinline__ TeamPlace team_look(const Team& team, uint32_t id) {
+  const int first = 4 * (int)team.bucket(id);
+  wave_sync();
+  const uint4 now = *reinterpret_cast<const uint4*>(team.owner() + first);
+  const uint32_t o[4] = {now.x, now.y, now.z, now.w};
+  TeamPlace t;
+  t.there = t.room = -1;
+  t.eights = 0;
+  t.making = false;
+#pragma unroll
+  for (int w = 3; w >= 0; --w) {
+    const bool mine = (o[w] & (kTeamId | kExpanded)) == id;
+    t.there = mine ? first + w : t.there;
+    t.eights = mine ? (int)(o[w] >> 28) : t.eights;
+    t.making = t.making || o[w] == (id | kExpanded);
+    t.room = o[w] == kNobody ? first + w : t.room;
+  }
+  return t;
+}
+
+// Frees the slots of candidates that are not in the line (pushed out of the set, or back in it).
+__device__ __forceinline__ void team_tidy(const Team& team, int lane) {
+  static_assert(kTeamSlots == 128, "two slots per lane");
+  const TeamPlace t = team_look(team, lane < Team::kInLine ? team.line()[lane < Team::kInLine ? lane : 0].id : kEmpty);
+  uint32_t* const kept = team.room();
+  kept[lane] = kept[lane + 64] = 0u;
+  wave_sync();
+  if (t.there >= 0) kept[t.there] = 1u;
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t owner = lds_now(team.owner() + lane + 64 * i);
+    if ((owner & kExpanded) == 0u && owner != kNobody && kept[lane + 64 * i] == 0u) lds_tell(team.owner() + lane + 64 * i, kNobody);
+    __builtin_amdgcn_wave_barrier();
+  }
+  wave_sync();
+}
+// rows in flight (dist_list): sixteen, eight long ones (of 65 to 128 elements thirty-two would take the registers of a wavefront per SIMD)
+template <int QR>
+constexpr int team_wide() {
+  return QR == 4 ? 3 : (QR == 1 ? 1 : 2);
+}
+template <int DT, int QR>
+__device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv, const Scratch& s, int helper, int lane) {
+  const Team& team = s.team;
+  const int S = ix.S0;
+  uint32_t next = kEmpty;  // the node to go on with, whose list nobody has asked for yet
+  float next_key = 0.f;
+  while (uni((int)lds_now(team.over())) == 0) {
+    uint32_t id = next;
+    float key = next_key;
+    int slot;
+    if (next == kEmpty) {
+      const uint32_t* const wish = reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0));
+      const float wish_key = __uint_as_float(lds_now(wish));
+      const uint32_t wish_id = lds_now(wish + 1);
+      const TeamPlace t = team_look(team, wish_id);
+      unsigned long long open = __ballot(lane > 0 && lane < Team::kInLine && wish_id != kEmpty && t.there < 0 && !t.making && t.room >= 0);
+      // (helpers that look at the same time choose different wishes, as far as there are several)
+      if (open != 0ull) {
+        for (int skip = helper % __popcll(open); skip > 0; --skip) open &= open - 1ull;
+        const int i = __builtin_ctzll(open);
+        id = (uint32_t)__builtin_amdgcn_readlane((int)wish_id, i);
+        key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wish_key), i));
+        slot = __builtin_amdgcn_readlane(t.room, i);
+      } else {
+        slot = -1;
+      }
+    } else {
+      const TeamPlace t = team_look(team, next);
+      slot = uni(t.there < 0 && !t.making ? t.room : -1);
+    }
+    const bool asked = next == kEmpty;
+    next = kEmpty;
+    bool mine = false;
+    if (slot >= 0) {
+      if (lane == 0) {
+        uint32_t was = kNobody;
+        mine = __hip_atomic_compare_exchange_strong(team.owner() + slot, &was, id | kExpanded, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (uni(mine ? 1 : 0) != 0) {
+      lds_done();
+      const bool wished = __ballot(lane > 0 && lane < Team::kInLine && lds_now(reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0)) + 1) == id) != 0ull;
+      const int other = 4 * (int)team.bucket(id) + (lane & 3);
+      const uint32_t there = lds_now(team.owner() + other);
+      const bool twice = __ballot(other != slot && ((there & (kTeamId | kExpanded)) == id || there == (id | kExpanded))) != 0ull;
+      uint32_t say = kNobody;
+      if ((wished || !asked) && !twice) {
+        uint32_t* const ids = team.ids(slot);
+        const uint32_t got = scalar_base(ix.links0 + (size_t)id * S)[lane < S ? lane : 0];
+        const uint32_t node = lane < S ? got : kEmpty;
+        const unsigned long long mask = __ballot(node != kEmpty) & filter_unknown(s, node);
+        const int n = __popcll(mask);
+        if (lane < S) ids[lane] = kEmpty;
+        wave_sync();
+        if (__builtin_amdgcn_inverse_ballot_w64(mask)) ids[lanes_below(mask)] = node;
+        wave_sync();
+        dist_list<DT, QR, false, team_wide<QR>()>(ix, qv, s.qlds, ids, n, team.keys(slot), lane);
+        lds_done();
+        if (n <= kMostListed) say = id | ((uint32_t)(n > 0 ? (n + 7) >> 3 : 1) << 28);
+        if (n > 0) {
+          const float my_key = lane < n ? team.keys(slot)[lane < n ? lane : 0] : INFINITY;
+          const float least = least_of_all(my_key);
+          const unsigned long long at = __ballot(my_key == least);
+          if (least < key && at != 0ull) {
+            next = (uint32_t)uni((int)ids[__builtin_ctzll(at)]);
+            next_key = least;
+          }
+        }
+      }
+      if (lane == 0) lds_tell(team.owner() + slot, say);
+      __builtin_amdgcn_wave_barrier();
+    } else if (slot < 0) {
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+}
+
+// Compacts the ids of a link row (of at most 64) that the filter does not know into s.nbuf, without telling it; returns how many.
+__device__ __forceinline__ int visit_unmarked(const uint32_t* row, int S, Scratch& s, int lane) {
+  const uint32_t got = row[lane < S ? lane : 0];
+  const uint32_t id = lane < S ? got : kEmpty;
+  const unsigned long long mask = __ballot(id != kEmpty) & filter_unknown(s, id);
+  if (__builtin_amdgcn_inverse_ballot_w64(mask)) s.nbuf[lanes_below(mask)] = id;
+  __builtin_amdgcn_wave_barrier();
+  return __popcll(mask);
 }
 // Takes the ids of the lanes that say so out of the filter again.  (Two of them may share a word: each makes its own half the
 // set's empty tag with two atomics -- which may come twice for one id, listed twice where the filter lost it in between.)
@@ -1814,6 +2183,193 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
   }
 }
 
+// The tie-free loop where a team helps: as tie_free_phase, but while the set fills and afterwards, and with up to eight candidates
+// considered in every step.  Their lists are there already (the first one may have none: its nodes are evaluated here; the step
+// ends before another without); of the eight, as many are expanded as surely come next whatever their offers do: those before the
+// first one that an offer of an earlier one is closer than.  The others stay where they are, with their lists.  So a step
+// costs no evaluation that a later one repeats, and a search has 60 of them at ef 300 where batches that grow and shrink took 100
+// (CPU model, 60 000 x 50).
+template <int DT, int QR, int NS, bool WATCH>
+__device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv, int ef, int S, Scratch& s, SearchState& st, Frontier<NS>& fr,
+                                          int& n, int& hop_cid, int& resume_at, const TieWatch& watch, int lane) {
+  constexpr int kMergeFrom = 6;  // fewer offers enter the set one by one
+  const int w0 = WATCH ? uni(watch.id0) : -1, w1 = WATCH ? uni(watch.id1) : -1;
+  const int w2 = WATCH ? uni(watch.id2) : -1, w3 = WATCH ? uni(watch.id3) : -1;
+  const float w_hi = WATCH ? uni(watch.hi) : -INFINITY;
+  int rows = 1;                     // candidates considered
+  bool taken = true;                // (the one whose n nodes come first is marked already)
+  int rank = 0, steps = 0;
+  HeapEnt cand;                     // lane r: the r-th; +inf behind the last
+  cand.key = INFINITY;
+  cand.id = kEmpty;
+  float cand_keys[8];               // all of their keys, in each lane
+#pragma unroll
+  for (int c = 0; c < 8; ++c) cand_keys[c] = INFINITY;
+  int row_ends = 64;                // lane r: the first lane behind its nodes
+  int from = 0;                     // each lane: the number of the candidate whose node it holds
+  int slot = -1;                    // lane r: where its list is
+  uint32_t listed_id = kEmpty;      // nodes that came from lists, lane by lane behind the n ids whose keys are still to be computed
+  float listed_key = INFINITY;
+  unsigned long long listed = 0ull; // the lanes that hold one
+  uint2* listed_set = nullptr;      // where the filter has it, what it says there, and what it is to say
+  uint2 listed_word = make_uint2(0u, 0u);
+  uint32_t listed_place = 0u;
+  Trail no_trail;
+  unsigned long long accepted = 0ull;
+  while (true) {
+    if (n > 0) dist_list<DT, QR, false, team_wide<QR>()>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+    wave_sync();
+    float my_key = listed_key;
+    uint32_t my_id = listed_id;
+    unsigned long long valid = listed;
+    if (n > 0) {
+      const int at = lane < n ? lane : n - 1;
+      const float got_key = s.dbuf[at];
+      const uint32_t got_id = s.nbuf[at];
+      my_key = lane < n ? got_key : my_key;
+      my_id = lane < n ? got_id : my_id;
+      valid |= first_lanes(n);
+    }
+    unsigned long long todo = st.n_acc < ef ? valid : valid & __ballot(st.lower > my_key);
+    int good = rows;  // candidates that are expanded now
+    if (todo != 0ull && rows > 1) {
+      // (an offer keeps back the candidates after its own that it is closer than)
+      int kept_back = 0;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) kept_back += cand_keys[c] <= my_key ? 1 : 0;
+      kept_back = kept_back > from ? kept_back : from + 1;
+      const int first_kept = least_of_all_ints(__builtin_amdgcn_inverse_ballot_w64(todo) ? kept_back : 8);
+      good = first_kept < rows ? first_kept : rows;
+    }
+    const unsigned long long now_lanes = good < rows ? first_lanes(__builtin_amdgcn_readlane(row_ends, good - 1)) : ~0ull;
+    todo &= now_lanes;
+    if (!taken) frontier_take_first<NS>(fr, good, rank);
+    const int most = good;
+    if (__popcll(todo) >= kMergeFrom) {
+      int offers = 0;
+      float last_key = 0.f;
+      if (frontier_merge<NS>(fr, todo, st.n_acc < ef ? st.n_acc : ef, ef, my_key, my_id, s.team.room(), w_hi, offers, last_key, lane)) {
+        st.n_acc = st.n_acc + offers;
+        st.maxkey = last_key;
+        st.lower = last_key;
+        todo = 0ull;
+      }
+    }
+    int r = 0, row_end = 64;
+    unsigned long long ends = 64ull;  // row_ends, eight bits each
+    if (todo != 0ull && rows > 1) {
+      ends = 0ull;
+      for (int c = 0; c < good; ++c) ends |= (unsigned long long)(uint32_t)__builtin_amdgcn_readlane(row_ends, c) << (8 * c);
+      row_end = (int)(ends & 0xFFu);
+    }
+    if (todo != 0ull)
+      tie_free_offers<NS, false, false, WATCH, false, true>(st, fr, todo, my_key, my_id, ef, w_hi, cand, ends, hop_cid, r, row_end, good,
+                                                            resume_at, accepted, no_trail, lane);
+    if (resume_at >= 0) {
+      // an equal key: the general loop goes on with this candidate's offers, at the front of the list
+      for (int b = r + 1; b < most; ++b) frontier_untake<NS>(fr, (uint32_t)__builtin_amdgcn_readlane((int)cand.id, b));
+      if (lane <= r && slot >= 0) lds_tell(s.team.owner() + slot, kNobody);
+      __builtin_amdgcn_wave_barrier();
+      if (!taken) {
+        st.n_hops += r + 1;
+        hop_cid = __builtin_amdgcn_readlane((int)cand.id, r);
+      }
+      const int start = r > 0 ? (int)((ends >> (8 * (r - 1))) & 0xFFu) : 0;
+      const unsigned long long of = valid & first_lanes(row_end) & ~first_lanes(start);
+      const unsigned long long before = valid & first_lanes(start);
+      n = __popcll(of);
+      st.n_dist += __popcll(before | of);
+      resume_at = __popcll(of & first_lanes(resume_at));
+      wave_sync();
+      if (__builtin_amdgcn_inverse_ballot_w64(of)) {
+        s.nbuf[lanes_below(of)] = my_id;
+        s.dbuf[lanes_below(of)] = my_key;
+      }
+      filter_enter(s, my_id, before | of);
+      wave_sync();
+      return 1;
+    }
+    // the lists of the candidates that have been expanded are done with, and their nodes dealt with
+    if (lane < good && slot >= 0) lds_tell(s.team.owner() + slot, kNobody);
+    __builtin_amdgcn_wave_barrier();
+    const unsigned long long done = valid & now_lanes;
+    st.n_dist += __popcll(done);
+    if (n > 0) {
+      filter_enter(s, my_id, done);
+    } else if (__builtin_amdgcn_inverse_ballot_w64(done)) {  // (nothing has been entered since)
+      *listed_set = filter_push(listed_word, listed_place);
+    }
+    __builtin_amdgcn_wave_barrier();
+    // every eighth step the lists of candidates that are no longer among the next go
+    if ((++steps & 7) == 0) team_tidy(s.team, lane);
+    if (!taken) st.n_hops += good;
+    taken = false;
+
+    n = 0;
+    const int total = frontier_line_up<NS>(fr, s.team, rank, lane);
+    if (total == 0) return 0;
+    rows = total < 8 ? total : 8;
+    const int nth = lane & 7;
+    cand = s.team.line()[nth];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) cand_keys[c] = s.team.line()[c].key;
+    if (WATCH) {
+      // a watched entry's turn is the general loop's business: the batch ends before it
+      const unsigned long long hit = __ballot(lane < rows && ((int)cand.id == w0 || (int)cand.id == w1 || (int)cand.id == w2 || (int)cand.id == w3));
+      if (hit != 0ull) rows = __builtin_ctzll(hit);
+      if (rows == 0) return 3;
+    }
+    TeamPlace t = team_look(s.team, cand.id);
+    // (lists that are just being made are waited for: each was begun a step ago or earlier)
+    for (int polls = 0; polls < 4096 && __ballot(lane < rows && t.there < 0 && t.making) != 0ull; ++polls) t = team_look(s.team, cand.id);
+    const unsigned long long there = __ballot(lane < rows && t.there >= 0);
+    const unsigned long long stop = first_lanes(rows) & ~there & ~1ull;
+    rows = stop != 0ull ? __builtin_ctzll(stop) : rows;
+    hop_cid = uni((int)cand.id);
+    if ((there & 1ull) == 0ull) {  // the first one has no list: its nodes are the search's own to evaluate
+      n = visit_unmarked(scalar_base(link_row(ix, (uint32_t)hop_cid, 0)), S, s, lane);
+      t.eights = lane == 0 ? (n > 0 ? (n + 7) >> 3 : 1) : t.eights;
+    }
+    // Eight lanes, or more of them, to a list: lane r gets the first eight behind its nodes.
+    const int own = (there & 1ull) == 0ull ? 1 : 0;
+    int upto = lane < rows ? t.eights : 0;
+    const int eights = upto;
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xF, 0xF, true);  // row_shr:1
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xF, 0xF, true);  // row_shr:2
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xF, 0xF, true);  // row_shr:4
+    const unsigned long long over = __ballot(upto > 8) & first_lanes(rows);
+    rows = over != 0ull ? __builtin_ctzll(over) : rows;
+    row_ends = 8 * upto;
+    // whose nodes each eight of lanes holds: the lists' first eights, one bit each, from all of them
+    int begins = lane < rows ? 1 << (upto - eights) : 0;
+    begins |= __builtin_amdgcn_update_dpp(0, begins, 0x111, 0xF, 0xF, true);
+    begins |= __builtin_amdgcn_update_dpp(0, begins, 0x112, 0xF, 0xF, true);
+    begins |= __builtin_amdgcn_update_dpp(0, begins, 0x114, 0xF, 0xF, true);
+    const uint32_t starts = (uint32_t)__builtin_amdgcn_readlane(begins, 7);
+    const int used = __builtin_amdgcn_readlane(upto, rows - 1);
+    const int eight = lane >> 3;
+    const uint32_t mine = starts & ((2u << eight) - 1u);
+    from = __popc(mine) - 1;
+    const int part = eight - (31 - __builtin_clz(mine | 1u));
+    const bool in = eight < used && (own == 0 || from > 0);
+    slot = lane < rows ? t.there : -1;
+    const int where = __shfl(t.there, in ? from : 0, 64);
+    const int place = in ? 8 * part + nth : 0;
+    const uint32_t got = s.team.ids(in ? where : 0)[place];
+    const float got_key = s.team.keys(in ? where : 0)[place];
+    const uint32_t id = in ? got : kEmpty;
+    uint32_t set;
+    listed_place = filter_find(s.filter, id, set);
+    listed_set = reinterpret_cast<uint2*>(s.vcache) + set;
+    listed_word = *listed_set;
+    listed = __ballot(id != kEmpty) & filter_misses(listed_word, listed_place);
+    listed_id = id;
+    listed_key = __builtin_amdgcn_inverse_ballot_w64(listed) ? got_key : INFINITY;
+    cand.key = lane < rows ? cand.key : INFINITY;
+    wave_sync();
+  }
+}
+
 // Best-first search of one level on the sorted set (needs the LDS tag filter).  On entry
 // s.nbuf[0..n_seed) holds the seeds, already entered into the filter.  Returns 0: fr holds the
 // result (st.top_size entries, ascending), all keys were distinct; 2: the same, but equal keys
@@ -1850,12 +2406,12 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
 // far: expand the farthest waiting entry instead of the closest (the reference's
 // reverse_cand); that is no hnswlib search any more, equal keys simply keep their order of
 // arrival and nothing is ever given up.  BUILD likewise never gives up.
-template <int DT, int QR, int NS, bool BUILD, bool TRAILS = false, bool FEW = false>
+template <int DT, int QR, int NS, bool BUILD, bool TRAILS = false, bool FEW = false, bool TEAM = false>
 __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<QR>& qv, int level, int ef, Scratch& s,
                                                   SearchState& st, Frontier<NS>& fr, int n_seed, int lane,
                                                   bool far = false, bool whole_set = false, Trail* trail = nullptr) {
   const int S = row_stride(ix, level);
-  constexpr int kWide = FEW ? 4 : ((QR == 0 && !BUILD && NS <= 8) ? 2 : 1);  // (rows in flight: dist_list)
+  constexpr int kWide = TEAM ? team_wide<QR>() : FEW ? 4 : ((QR == 0 && !BUILD && NS <= 8) ? 2 : 1);  // (rows in flight: dist_list)
   int n = n_seed;
   const bool exact = !BUILD && !far;  // the outcome has to be hnswlib's
   Trail no_trail;
@@ -1883,6 +2439,9 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
       if constexpr (BUILD) {
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
+      } else if constexpr (TEAM) {  // (other wavefronts help)
+        if (!have_tie) how = team_phase<DT, QR, NS, false>(ix, qv, ef, S, s, st, fr, n, hop_cid, resume_at, watch, lane);
+        else how = team_phase<DT, QR, NS, true>(ix, qv, ef, S, s, st, fr, n, hop_cid, resume_at, watch, lane);
       } else if (!have_tie) {
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
@@ -2028,6 +2587,11 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
       hop_cid = cid;
       st.n_hops += 1;
       wave_sync();
+      if constexpr (TEAM) {
+        const TeamPlace t = team_look(s.team, (uint32_t)cid);
+        if (lane == 0 && t.there >= 0) lds_tell(s.team.owner() + t.there, kNobody);
+        __builtin_amdgcn_wave_barrier();
+      }
       n = visit_lossy(scalar_base(link_row(ix, (uint32_t)cid, level)), S, s, lane);
       wave_sync();
       // Equal keys that sit in the set do no harm while none of them that still waits is expanded or pushed out

@@ -602,7 +602,7 @@ class Engine {
     return f;
   }
 
-  // How many wavefronts (workgroups of one) of a kernel the GPU holds.  A workgroup's LDS is handed out in whole steps of
+  // How many workgroups (of one wavefront, or of `waves`) of a kernel the GPU holds.  A workgroup's LDS is handed out in whole steps of
   // kLdsStep bytes, which the runtime's answer leaves out (measured with workgroups that count each other, 160 KB per CU:
   // 5 120 bytes 32 on a CU, 5 184 25, 6 464 21, 7 744 18; the runtime says 32, 31, 25 and 21).  (Asked once per kernel and LDS
   // size: a search wants to know half a dozen of them.)
@@ -610,23 +610,56 @@ class Engine {
   struct Resident {
     const void* kernel;
     size_t lds;
+    int waves;
     int slots;
   };
   std::vector<Resident> resident_known;
   template <typename K>
-  int resident_slots(K kernel, size_t lds) {
+  int resident_slots(K kernel, size_t lds, int waves = 1) {
     const void* const id = reinterpret_cast<const void*>(kernel);
     for (const Resident& r : resident_known)
-      if (r.kernel == id && r.lds == lds) return r.slots;
+      if (r.kernel == id && r.lds == lds && r.waves == waves) return r.slots;
     hipFuncAttributes attr;
     HIP_CHECK(hipFuncGetAttributes(&attr, id));
     const size_t fixed = attr.sharedSizeBytes, whole = (fixed + lds + kLdsStep - 1) / kLdsStep * kLdsStep;
     int per_cu = 0;
-    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, std::max(whole, fixed) - fixed));
-    per_cu = std::max(1, std::min(per_cu, 32));
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, std::max(whole, fixed) - fixed));
+    per_cu = std::max(waves > 1 ? 0 : 1, std::min(per_cu, 32));
     if (resident_known.size() >= 256) resident_known.clear();
-    resident_known.push_back({id, lds, per_cu * num_cus});
+    resident_known.push_back({id, lds, waves, per_cu * num_cus});
     return per_cu * num_cus;
+  }
+
+  // A batch that leaves the machine idle by teams of wavefronts, a workgroup of eight or four per query (kernels.h, team_help);
+  // false: not such a batch.  Eight where the GPU holds them for all queries at once, else four (a number in between puts two of
+  // a workgroup's wavefronts on one SIMD as eight do: 345 678 x 101 in fp16, 400 queries, 5 to 7 of them 319 us, four 229).
+  // A wavefront alone -> by teams, ef 300: 100 000 x 50, one query 267 -> 188 us, 32 335 -> 257, 256 408 -> 301, 512 459 -> 302, 768
+  // 468 -> 357, 1 000 514 -> 502; x 180 301 -> 214, 414 -> 310, 748 -> 548, 815 -> 575, 774 -> 671, 789 -> 745; 500 000 x 96 295 -> 206, 408 ->
+  // 277, 546 -> 413, 551 -> 452, 560 -> 527, 571 -> 576; x 300 237 -> 161, 292 -> 208, 436 -> 323, 466 -> 376, 484 -> 454, 483 -> 452.
+  // Alone as well: long rows where the batch has the memory busy, to which helpers add a quarter (100 000 x 960, 32 queries 522 -> 376
+  // us; 256 653, in eights 629, in fours 568; 400 667, in fours 687).
+  template <typename K, typename Lds>
+  bool launch_teams(K kernel, int qr, int ns, Lds&& search_lds, const DevIndex& ix, SearchArgs a) {
+    constexpr size_t kBusyFrom = (size_t)1100 << 10, kHalfBusyFrom = (size_t)700 << 10;  // bytes of one row for every query
+    const int per_cu = (a.nq + num_cus - 1) / num_cus;
+    const size_t rows = qr == 0 ? (size_t)a.nq * Dp * (storage_half ? 2 : 4) : 0;
+    if (ix.S0 > 64 || filter_entries > 0 || rows > kBusyFrom) return false;
+    const size_t lds = (size_t)160 * 1024 / per_cu / kLdsStep * kLdsStep;
+    const FilterShape least = least_filter(a.ef);
+    a.fc = filter_shape(std::min(8 * least.sets(), 4096), host.N);  // (a forgotten node keeps candidates back)
+    a.team_turn = num_cus;
+    a.team_bucket_bits = 5;
+    auto bytes = [&] { return search_lds(a.fc) + (size_t)Team::words(ns, a.team_bucket_bits, ix.S0) * 4; };
+    while (a.fc.sets() > 2 * least.sets() && bytes() > lds) a.fc = filter_shape(a.fc.sets() / 2, host.N);
+    while (a.team_bucket_bits > 3 && bytes() > lds) --a.team_bucket_bits;
+    if (bytes() > lds) return false;
+    for (int waves = rows > kHalfBusyFrom ? kMostTeam / 2 : kMostTeam; waves >= kMostTeam / 2; waves /= 2) {
+      if (resident_slots(kernel, bytes(), waves) < per_cu * num_cus) continue;
+      hipLaunchKernelGGL(kernel, dim3(a.nq), dim3(64 * waves), bytes(), stream, ix, a);
+      HIP_CHECK(hipGetLastError());
+      return true;
+    }
+    return false;
   }
 
   // ---- search ------------------------------------------------------------------------------

@@ -287,7 +287,8 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       HIP_CHECK(hipGetLastError());
     }
     if (alone) {
-      hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, false, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
+      if (!launch_teams(search_fast_kernel<DT, QR, NS, false, true, true>, QR, NS, fast_lds, ix, a))
+        hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, false, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
     } else if constexpr (QR == 1 || QR == 2) {
       if (keep_trails) hipLaunchKernelGGL((search_fast_kernel<DT, QR, NS, true>), dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);
       else hipLaunchKernelGGL(fast_kernel, dim3(slots), dim3(64), fast_lds_bytes, stream, ix, a);

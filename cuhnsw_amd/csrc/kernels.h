@@ -70,6 +70,8 @@ struct SearchArgs {
   int slot_base;   // first slot of the pool this launch may use (two literal launches can be in flight)
   SlotPool pool;
   int cand_lds, hnswlib_dist;
+  int team_bucket_bits;  // sorted-set pass by teams of wavefronts (struct Team)
+  int team_turn;         // workgroups after which the next one comes to a CU that has one
   int rcap, lcap;  // ids and keys a row buffer holds: those of a link row; literal pass: those of the answer too
   int vc_bits;  // log2 entries of the LDS visited cache of the literal search, 0 = none
   FilterShape fc;  // the LDS visited filter of the sorted-set search (no sets: that search is off)
@@ -485,9 +487,12 @@ __device__ __forceinline__ const Args& fresh_args() {
 // FEW: for batches that leave the machine idle, at most a wavefront per SIMD: twice the rows in flight and more
 // candidates at a time, with the registers that takes (100 000 x 50, ef 300, one query: 0.290 -> 0.278 ms; 100 000 x 960,
 // ef 300, 1 000 queries: 1.35 -> 1.29).
+// TEAM: FEW, and the other wavefronts of the workgroup help the one that searches (device_core.h, team_help; which batches:
+// launch_teams).  Held to 128 registers, four of its wavefronts on a SIMD, on rows of up to 256 elements.
+constexpr int kMostTeam = 8;  // wavefronts per query
 constexpr int fast_waves_of_six(int dt, int qr, bool trails) { return (dt == DIST_DOT ? qr == 1 : trails) ? 6 : 7; }
-template <int DT, int QR, int NS, bool TRAILS, bool FEW = false>
-__global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : NS == 6 ? fast_waves_of_six(DT, QR, TRAILS) : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
+template <int DT, int QR, int NS, bool TRAILS, bool FEW = false, bool TEAM = false>
+__global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 && NS <= 8 ? 4 : 2) : FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 ? 7 : NS == 6 ? fast_waves_of_six(DT, QR, TRAILS) : (NS <= 8 ? 5 : 1)) : (QR == 4 && NS == 5 && DT == DIST_L2) ? 5 : 1) search_fast_kernel(DevIndex ix0, SearchArgs a0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const FastLdsPlan lp = plan_fast_lds(QR, ix0.Dp, a0.rcap, a0.fc, a0.k);
   Scratch s;
@@ -496,13 +501,35 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
   s.qlds = reinterpret_cast<float4*>(smem + lp.qlds);
   s.nbuf = reinterpret_cast<uint32_t*>(smem + lp.nbuf);
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
+  if (TEAM) {
+    // a workgroup per query: its first wavefront searches, the others help
+    s.team.base = reinterpret_cast<uint32_t*>(smem + lp.total);
+    s.team.bucket_bits = a0.team_bucket_bits;
+    s.team.stride = ix0.S0;
+    s.team.lists = Team::lists_at(NS);
+    for (int i = (int)threadIdx.x; i < Team::kRoom; i += (int)blockDim.x)
+      s.team.base[i] = i < (4 << a0.team_bucket_bits) ? kNobody : (i == Team::kOver ? 0u : kEmpty);
+    filter_reset(s, (int)threadIdx.x, (int)blockDim.x);
+    __syncthreads();
+    // (the workgroups that share a CU have their first wavefronts on the same SIMD: another one of each searches)
+    const int waves = (int)blockDim.x >> 6;
+    const int wave = (uni((int)threadIdx.x >> 6) + waves - ((int)blockIdx.x / a0.team_turn) % waves) % waves;
+    if (wave > 0) {
+      const int lane = (int)threadIdx.x & 63;
+      QVec<QR> qv;
+      load_query<QR>(qv, s.qlds, a0.q + (size_t)blockIdx.x * ix0.D, ix0.D, ix0.Dp, lane);
+      team_help<DT, QR>(ix0, qv, s, wave - 1, lane);
+      return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+  }
   // tells a literal pass waiting beside this one that the two kernels do run at the same time
   if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(a0.done + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int trail_buf = (TRAILS && a0.trail) ? (int)blockIdx.x : -1;  // the buffer this wavefront's trails go to
   int share_at = 0;  // the queue this wavefront is at (a.shares)
 
   for (;;) {
-    int lane = fresh((int)threadIdx.x);
+    int lane = fresh((int)threadIdx.x & 63);
     const SearchArgs& in = fresh_args<SearchArgs>();
     const DevIndex& from = fresh_index();
     int qi = 0;
@@ -524,6 +551,8 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
         }
         share_at += 1;
       }
+    } else if (TEAM) {
+      qi = share_at++ == 0 ? (int)blockIdx.x : in.nq;
     } else if (lane == 0) {
       qi = atomicAdd(in.counter, 1);
       if (qi < in.nq && in.order) qi = in.order[qi];
@@ -554,15 +583,27 @@ __global__ void __launch_bounds__(64, FEW ? 1 : (QR >= 1 && QR <= 2) ? (NS <= 5 
     }
 
     lane = fresh(lane);
+    if (TEAM) {
+      // (the first candidate: its list can be made while this wavefront gets ready)
+      HeapEnt e;
+      e.key = INFINITY;
+      e.id = cur;
+      if (lane == 0) s.team.line()[8] = e;
+      __builtin_amdgcn_wave_barrier();
+    }
     Frontier<NS> fr;
     frontier_init<NS>(fr, a0.ef, lane);
-    filter_reset(s, lane);
+    if (!TEAM) filter_reset(s, lane);
     visit_lossy_single(s, cur, lane);
     if (lane == 0) s.nbuf[0] = cur;
     wave_sync();
     // (the flag is made wavefront-uniform explicitly and both outcomes are plain branches)
     const int how =
-        __builtin_amdgcn_readfirstlane(search_level_fast<DT, QR, NS, false, TRAILS, FEW>(ix0, qv, 0, a0.ef, s, st, fr, 1, lane, a0.reverse != 0, a0.k >= a0.ef, TRAILS ? &tr : nullptr));
+        __builtin_amdgcn_readfirstlane(search_level_fast<DT, QR, NS, false, TRAILS, FEW, TEAM>(ix0, qv, 0, a0.ef, s, st, fr, 1, lane, a0.reverse != 0, a0.k >= a0.ef, TRAILS ? &tr : nullptr));
+    if (TEAM) {
+      if (lane == 0) lds_tell(s.team.over(), 1u);
+      __builtin_amdgcn_wave_barrier();
+    }
     lane = fresh(lane);
     const SearchArgs& a = fresh_args<SearchArgs>();
     const DevIndex& ix = fresh_index();

@@ -63,6 +63,8 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_L2, 0, 6, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,6,few>"),
 ]
 OTHERS = [
+    ("search_fast_kernel<DIST_DOT, 1, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,5,team>"),
+    ("search_fast_kernel<DIST_L2, 2, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,5,team>"),
     ("search_kernel<DIST_DOT, 1, 5>(DevIndex, SearchArgs)", "search_kernel<dot,1,5>"),
     ("build_search_kernel<DIST_DOT, 1, 2>(DevIndex, BuildArgs)", "build_search_kernel<dot,1,2>"),
     ("build_search_kernel<DIST_L2, 2, 5>(DevIndex, BuildArgs)", "build_search_kernel<l2,2,5>"),
