@@ -1762,7 +1762,7 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
       const float wish_key = __uint_as_float(lds_now(wish));
       const uint32_t wish_id = lds_now(wish + 1);
       const TeamPlace t = team_look(team, wish_id);
-      unsigned long long open = __ballot(lane > 0 && lane < Team::kInLine && wish_id != kEmpty && t.there < 0 && !t.making && t.room >= 0);
+      unsigned long long open = __ballot(lane < Team::kInLine && wish_id != kEmpty && t.there < 0 && !t.making && t.room >= 0);
       // (helpers that look at the same time choose different wishes, as far as there are several)
       if (open != 0ull) {
         for (int skip = helper % __popcll(open); skip > 0; --skip) open &= open - 1ull;
@@ -1789,7 +1789,7 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
     }
     if (uni(mine ? 1 : 0) != 0) {
       lds_done();
-      const bool wished = __ballot(lane > 0 && lane < Team::kInLine && lds_now(reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0)) + 1) == id) != 0ull;
+      const bool wished = __ballot(lane < Team::kInLine && lds_now(reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0)) + 1) == id) != 0ull;
       const int other = 4 * (int)team.bucket(id) + (lane & 3);
       const uint32_t there = lds_now(team.owner() + other);
       const bool twice = __ballot(other != slot && ((there & (kTeamId | kExpanded)) == id || there == (id | kExpanded))) != 0ull;
@@ -1833,6 +1833,33 @@ __device__ __forceinline__ int visit_unmarked(const uint32_t* row, int S, Scratc
   if (__builtin_amdgcn_inverse_ballot_w64(mask)) s.nbuf[lanes_below(mask)] = id;
   __builtin_amdgcn_wave_barrier();
   return __popcll(mask);
+}
+// The list of a candidate whose turn has come, if there is one: the nodes that the filter does not know, and their keys, to s.nbuf
+// and s.dbuf, their number to n.
+__device__ __forceinline__ bool visit_listed(Scratch& s, uint32_t cid, int S, int& n, int lane) {
+  TeamPlace t = team_look(s.team, cid);
+  for (int polls = 0; polls < 4096 && uni(t.there < 0 && t.making ? 1 : 0) != 0; ++polls) t = team_look(s.team, cid);
+  const int where = uni(t.there);
+  if (where >= 0) {
+    const uint32_t got = s.team.ids(where)[lane < S ? lane : 0];
+    const float key = s.team.keys(where)[lane < S ? lane : 0];
+    const uint32_t id = lane < S ? got : kEmpty;
+    uint2* sets = reinterpret_cast<uint2*>(s.vcache);
+    uint32_t set;
+    const uint32_t place = filter_find(s.filter, id, set);
+    const uint2 w = sets[set];
+    const unsigned long long mask = __ballot(id != kEmpty) & filter_misses(w, place);
+    if (__builtin_amdgcn_inverse_ballot_w64(mask)) {
+      sets[set] = filter_push(w, place);
+      s.nbuf[lanes_below(mask)] = id;
+      s.dbuf[lanes_below(mask)] = key;
+    }
+    __builtin_amdgcn_wave_barrier();
+    n = __popcll(mask);
+    if (lane == 0) lds_tell(s.team.owner() + where, kNobody);
+    __builtin_amdgcn_wave_barrier();
+  }
+  return where >= 0;
 }
 // Takes the ids of the lanes that say so out of the filter again.  (Two of them may share a word: each makes its own half the
 // set's empty tag with two atomics -- which may come twice for one id, listed twice where the filter lost it in between.)
@@ -2191,7 +2218,7 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
 // (CPU model, 60 000 x 50).
 template <int DT, int QR, int NS, bool WATCH>
 __device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv, int ef, int S, Scratch& s, SearchState& st, Frontier<NS>& fr,
-                                          int& n, int& hop_cid, int& resume_at, const TieWatch& watch, int lane) {
+                                          int& n, bool have_keys, int& hop_cid, int& resume_at, const TieWatch& watch, int lane) {
   constexpr int kMergeFrom = 6;  // fewer offers enter the set one by one
   const int w0 = WATCH ? uni(watch.id0) : -1, w1 = WATCH ? uni(watch.id1) : -1;
   const int w2 = WATCH ? uni(watch.id2) : -1, w3 = WATCH ? uni(watch.id3) : -1;
@@ -2217,7 +2244,8 @@ __device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv
   Trail no_trail;
   unsigned long long accepted = 0ull;
   while (true) {
-    if (n > 0) dist_list<DT, QR, false, team_wide<QR>()>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+    if (n > 0 && !have_keys) dist_list<DT, QR, false, team_wide<QR>()>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+    have_keys = false;
     wave_sync();
     float my_key = listed_key;
     uint32_t my_id = listed_id;
@@ -2431,6 +2459,7 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
   // instructions per accepted candidate — and only then moves on to the general loop below, at the very offer
   // that met the equal key (resume_at).
   int resume_at = -1;
+  bool listed = false;  // (TEAM) the keys of the n nodes are there
   bool calm = (exact || (BUILD && !far)) && S <= 64;  // no equal keys are at work (or none matter): the tie-free loop may run
   TieWatch watch;
   while (true) {
@@ -2440,8 +2469,8 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
       } else if constexpr (TEAM) {  // (other wavefronts help)
-        if (!have_tie) how = team_phase<DT, QR, NS, false>(ix, qv, ef, S, s, st, fr, n, hop_cid, resume_at, watch, lane);
-        else how = team_phase<DT, QR, NS, true>(ix, qv, ef, S, s, st, fr, n, hop_cid, resume_at, watch, lane);
+        if (!have_tie) how = team_phase<DT, QR, NS, false>(ix, qv, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
+        else how = team_phase<DT, QR, NS, true>(ix, qv, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
       } else if (!have_tie) {
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
@@ -2468,7 +2497,7 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
     while (true) {
       if ((QR == 1 || (QR == 2 && DT == DIST_DOT)) && NS == 6 && !BUILD && !FEW) lane = fresh(lane);
       if (resume_at < 0) {
-        if (n > 0) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
+        if (n > 0 && !(TEAM && listed)) dist_list<DT, QR, false, kWide>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
         st.n_dist += n;
         wave_sync();
       }
@@ -2587,12 +2616,16 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
       hop_cid = cid;
       st.n_hops += 1;
       wave_sync();
+      listed = false;
       if constexpr (TEAM) {
-        const TeamPlace t = team_look(s.team, (uint32_t)cid);
-        if (lane == 0 && t.there >= 0) lds_tell(s.team.owner() + t.there, kNobody);
-        __builtin_amdgcn_wave_barrier();
+        if (S <= 64) {
+          int rank;
+          frontier_line_up<NS>(fr, s.team, rank, lane);
+          listed = visit_listed(s, (uint32_t)cid, S, n, lane);
+          if ((st.n_hops & 7) == 0) team_tidy(s.team, lane);
+        }
       }
-      n = visit_lossy(scalar_base(link_row(ix, (uint32_t)cid, level)), S, s, lane);
+      if (!listed) n = visit_lossy(scalar_base(link_row(ix, (uint32_t)cid, level)), S, s, lane);
       wave_sync();
       // Equal keys that sit in the set do no harm while none of them that still waits is expanded or pushed out
       // (unless the whole set is the answer): no group can form, and which of two expanded twins an eviction
