@@ -67,6 +67,8 @@ struct Team {
   // the closest candidates; behind them a place that nobody reads
   __device__ __forceinline__ HeapEnt* line() const { return reinterpret_cast<HeapEnt*>(base + kLine); }
   __device__ __forceinline__ uint32_t* over() const { return base + kOver; }
+  // the level that is searched (from bit 16 on), and a number that changes with it: odd while no list may be begun
+  __device__ __forceinline__ uint32_t* level() const { return base + kOver + 1; }
   __device__ __forceinline__ uint32_t* room() const { return base + kRoom; }
   __device__ __forceinline__ uint32_t bucket(uint32_t id) const { return (id * 2654435761u) >> (32 - bucket_bits); }
   __device__ __forceinline__ uint32_t* ids(int slot) const { return base + lists + 2 * slot * stride; }
@@ -1747,17 +1749,49 @@ template <int QR>
 constexpr int team_wide() {
   return QR == 4 ? 3 : (QR == 1 ? 1 : 2);
 }
-template <int DT, int QR>
+// The search of one level is over and another's begins (LEVELS): nobody begins a list any more, those under way are waited
+// for (a helper looks at the level again once it has its slot: it is seen here, or sees that it may not) -- and all slots are free.
+__device__ __forceinline__ void team_close(const Team& team, int lane) {
+  if (lane == 0) lds_tell(team.level(), lds_now(team.level()) | 1u);
+  wave_sync();
+  for (int i = 0; i < 2; ++i) {
+    while (true) {
+      const uint32_t owner = lds_now(team.owner() + lane + 64 * i);
+      if (__ballot((owner & kExpanded) != 0u && owner != kEmpty) == 0ull) {
+        if (owner != kEmpty) lds_tell(team.owner() + lane + 64 * i, kNobody);
+        __builtin_amdgcn_wave_barrier();
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+}
+__device__ __forceinline__ void team_open(const Team& team, int level, int lane) {
+  HeapEnt none;
+  none.key = INFINITY;
+  none.id = kEmpty;
+  if (lane < Team::kInLine) team.line()[lane < Team::kInLine ? lane : 0] = none;
+  wave_sync();
+  if (lane == 0) lds_tell(team.level(), ((uint32_t)level << 16) | (((lds_now(team.level()) & 0xFFFFu) + 1u) & 0xFFFEu));
+  wave_sync();
+}
+template <int DT, int QR, bool LEVELS = false>
 __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv, const Scratch& s, int helper, int lane) {
   const Team& team = s.team;
-  const int S = ix.S0;
+  uint32_t next_at = 0u;  // and the level it was found on
   uint32_t next = kEmpty;  // the node to go on with, whose list nobody has asked for yet
   float next_key = 0.f;
   while (uni((int)lds_now(team.over())) == 0) {
+    const uint32_t at = LEVELS ? (uint32_t)uni((int)lds_now(team.level())) : 0u;
+    if (LEVELS && (at != next_at || (at & 1u) != 0u)) next = kEmpty;
+    next_at = at;
+    const int S = LEVELS ? row_stride(ix, (int)(at >> 16)) : ix.S0;
     uint32_t id = next;
     float key = next_key;
     int slot;
-    if (next == kEmpty) {
+    if (LEVELS && (at & 1u) != 0u) {
+      slot = -1;
+    } else if (next == kEmpty) {
       const uint32_t* const wish = reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0));
       const float wish_key = __uint_as_float(lds_now(wish));
       const uint32_t wish_id = lds_now(wish + 1);
@@ -1793,10 +1827,11 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
       const int other = 4 * (int)team.bucket(id) + (lane & 3);
       const uint32_t there = lds_now(team.owner() + other);
       const bool twice = __ballot(other != slot && ((there & (kTeamId | kExpanded)) == id || there == (id | kExpanded))) != 0ull;
+      const bool still = !LEVELS || (uint32_t)uni((int)lds_now(team.level())) == at;
       uint32_t say = kNobody;
-      if ((wished || !asked) && !twice) {
+      if ((wished || !asked) && !twice && still) {
         uint32_t* const ids = team.ids(slot);
-        const uint32_t got = scalar_base(ix.links0 + (size_t)id * S)[lane < S ? lane : 0];
+        const uint32_t got = scalar_base(LEVELS ? link_row(ix, id, (int)(at >> 16)) : ix.links0 + (size_t)id * S)[lane < S ? lane : 0];
         const uint32_t node = lane < S ? got : kEmpty;
         const unsigned long long mask = __ballot(node != kEmpty) & filter_unknown(s, node);
         const int n = __popcll(mask);
@@ -2216,8 +2251,8 @@ __device__ __forceinline__ int tie_free_phase(const DevIndex& ix, const QVec<QR>
 // first one that an offer of an earlier one is closer than.  The others stay where they are, with their lists.  So a step
 // costs no evaluation that a later one repeats, and a search has 60 of them at ef 300 where batches that grow and shrink took 100
 // (CPU model, 60 000 x 50).
-template <int DT, int QR, int NS, bool WATCH>
-__device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv, int ef, int S, Scratch& s, SearchState& st, Frontier<NS>& fr,
+template <int DT, int QR, int NS, bool WATCH, bool BUILD = false>
+__device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv, int level, int ef, int S, Scratch& s, SearchState& st, Frontier<NS>& fr,
                                           int& n, bool have_keys, int& hop_cid, int& resume_at, const TieWatch& watch, int lane) {
   constexpr int kMergeFrom = 6;  // fewer offers enter the set one by one
   const int w0 = WATCH ? uni(watch.id0) : -1, w1 = WATCH ? uni(watch.id1) : -1;
@@ -2291,7 +2326,7 @@ __device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv
       row_end = (int)(ends & 0xFFu);
     }
     if (todo != 0ull)
-      tie_free_offers<NS, false, false, WATCH, false, true>(st, fr, todo, my_key, my_id, ef, w_hi, cand, ends, hop_cid, r, row_end, good,
+      tie_free_offers<NS, false, false, WATCH, BUILD, true>(st, fr, todo, my_key, my_id, ef, w_hi, cand, ends, hop_cid, r, row_end, good,
                                                             resume_at, accepted, no_trail, lane);
     if (resume_at >= 0) {
       // an equal key: the general loop goes on with this candidate's offers, at the front of the list
@@ -2355,7 +2390,7 @@ __device__ __forceinline__ int team_phase(const DevIndex& ix, const QVec<QR>& qv
     rows = stop != 0ull ? __builtin_ctzll(stop) : rows;
     hop_cid = uni((int)cand.id);
     if ((there & 1ull) == 0ull) {  // the first one has no list: its nodes are the search's own to evaluate
-      n = visit_unmarked(scalar_base(link_row(ix, (uint32_t)hop_cid, 0)), S, s, lane);
+      n = visit_unmarked(scalar_base(link_row(ix, (uint32_t)hop_cid, level)), S, s, lane);
       t.eights = lane == 0 ? (n > 0 ? (n + 7) >> 3 : 1) : t.eights;
     }
     // Eight lanes, or more of them, to a list: lane r gets the first eight behind its nodes.
@@ -2465,12 +2500,14 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
   while (true) {
     if (calm) {
       int how = st.n_acc >= ef ? 2 : 0;
-      if constexpr (BUILD) {
+      if constexpr (BUILD && TEAM) {
+        how = team_phase<DT, QR, NS, false, true>(ix, qv, level, ef, S, s, st, fr, n, false, hop_cid, resume_at, watch, lane);
+      } else if constexpr (BUILD) {
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, false, false, true>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
       } else if constexpr (TEAM) {  // (other wavefronts help)
-        if (!have_tie) how = team_phase<DT, QR, NS, false>(ix, qv, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
-        else how = team_phase<DT, QR, NS, true>(ix, qv, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
+        if (!have_tie) how = team_phase<DT, QR, NS, false>(ix, qv, level, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
+        else how = team_phase<DT, QR, NS, true>(ix, qv, level, ef, S, s, st, fr, n, listed, hop_cid, resume_at, watch, lane);
       } else if (!have_tie) {
         if (how == 0) how = tie_free_phase<DT, QR, NS, false, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
         if (how == 2) how = tie_free_phase<DT, QR, NS, true, TRAILS, false, false, FEW>(ix, qv, level, ef, S, s, st, fr, n, hop_cid, resume_at, accepted, tr, watch, lane);
@@ -2617,7 +2654,7 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
       st.n_hops += 1;
       wave_sync();
       listed = false;
-      if constexpr (TEAM) {
+      if constexpr (TEAM && !BUILD) {
         if (S <= 64) {
           int rank;
           frontier_line_up<NS>(fr, s.team, rank, lane);

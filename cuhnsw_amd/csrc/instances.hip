@@ -505,6 +505,30 @@ void Engine::build_levels() {
   const size_t lds1 = search_lds(a.fc);
   const LdsPlan lp3 = plan_lds(QR, Dp, s_max + cap_in, 0, a.lcap, s_max + cap_in, std::max(m_max, cap_in));
   const int slots1 = resident_slots(k_search, lds1);
+  // Batches that leave the machine idle: a workgroup of wavefronts per node (kernels.h, TEAM), eight or four as in launch_teams.
+  // (A batch of 58 / 222 / 543 nodes of 20 000 x 50: 126 -> 88 us, 203 -> 128, 220 -> 183; the 44 batches 6.70 -> 5.81 ms, 20 003 x 128
+  // 12.6 -> 10.9, 8 000 x 300 12.2 -> 10.8, 6 000 x 960 15.8 -> 14.2, 100 000 x 50 13.0 -> 12.3.)
+  auto k_team = build_search_kernel<DT, QR, (NS > 0 ? NS : 2), true>;
+  const bool teams = NS > 0 && sorted_set && !a.reverse && s_max <= 64 && filter_entries <= 0;
+  auto launch_team = [&](BuildArgs b) {
+    if (!teams || b.count > 4 * num_cus) return false;
+    const int per_cu = (b.count + num_cus - 1) / num_cus;
+    const size_t room = (size_t)160 * 1024 / per_cu / kLdsStep * kLdsStep - 64;  // (the kernel has 64 bytes of its own)
+    const FilterShape least = least_filter(efc);
+    b.fc = filter_shape(std::min(8 * least.sets(), 4096), N);
+    b.team_turn = num_cus;
+    b.team_bucket_bits = 5;
+    auto bytes = [&] { return search_lds(b.fc) + (size_t)Team::words(NS, b.team_bucket_bits, s_max) * 4; };
+    while (b.fc.sets() > 2 * least.sets() && bytes() > room) b.fc = filter_shape(b.fc.sets() / 2, N);
+    while (b.team_bucket_bits > 3 && bytes() > room) --b.team_bucket_bits;
+    if (bytes() > room) return false;
+    for (int waves = kMostTeam; waves >= kMostTeam / 2; waves /= 2) {
+      if (resident_slots(k_team, bytes(), waves) < per_cu * num_cus) continue;
+      hipLaunchKernelGGL(k_team, dim3(b.count + b.n_upper), dim3(64 * waves), bytes(), stream, ix, b);
+      return true;
+    }
+    return false;
+  };
   const int slots3 = resident_slots(k_reverse, lp3.total);
   // the sorted-set search needs no per-wavefront global memory (no bitmap, no undo list, no log)
   if (!sorted_set) ensure_pool(slots1, glob_cap, 2 * glob_cap);
@@ -559,7 +583,7 @@ void Engine::build_levels() {
       a.n_upper = upper_end[batch] - from;
     }
     ++batch;
-    hipLaunchKernelGGL(k_search, dim3(std::min(b, slots1)), dim3(64), lds1, stream, ix, a);
+    if (!launch_team(a)) hipLaunchKernelGGL(k_search, dim3(std::min(b, slots1)), dim3(64), lds1, stream, ix, a);
     HIP_CHECK(hipGetLastError());
     if (cur_max >= 0) {
       long long work = (long long)b * m_max;

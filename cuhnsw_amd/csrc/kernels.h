@@ -114,6 +114,7 @@ struct BuildArgs {
   int cand_lds, lcap;
   int vc_bits;
   FilterShape fc;
+  int team_bucket_bits, team_turn;  // a team of wavefronts per node: as in SearchArgs
   HeapEnt* inbox0;  // N x cap_in
   int* inbox0_cnt;  // N
   HeapEnt* inboxU;  // upper rows x cap_in
@@ -449,6 +450,23 @@ static __global__ void __launch_bounds__(1024) order_scatter_kernel(const uint4*
   }
 }
 
+// The LDS that the wavefronts of a workgroup share to search together (device_core.h, team_help), set up by all of them; returns this
+// one's part: 0 searches, the others help.
+template <int NS>
+__device__ __forceinline__ int gather_team(Scratch& s, unsigned char* lds, int stride, int level, int bucket_bits, int turn) {
+  s.team.base = reinterpret_cast<uint32_t*>(lds);
+  s.team.bucket_bits = bucket_bits;
+  s.team.stride = stride;
+  s.team.lists = Team::lists_at(NS);
+  for (int i = (int)threadIdx.x; i < Team::kRoom; i += (int)blockDim.x)
+    s.team.base[i] = i < (4 << bucket_bits) ? kNobody : (i == Team::kOver ? 0u : (i == Team::kOver + 1 ? (uint32_t)level << 16 : kEmpty));
+  filter_reset(s, (int)threadIdx.x, (int)blockDim.x);
+  __syncthreads();
+  // (the workgroups that share a CU have their first wavefronts on the same SIMD: another one of each searches)
+  const int waves = (int)blockDim.x >> 6;
+  return (uni((int)threadIdx.x >> 6) + waves - ((int)blockIdx.x / turn) % waves) % waves;
+}
+
 // A kernel's arguments read afresh from where the launch put them.  The compiler loads every argument once, when the
 // kernel starts, and keeps it: fifty scalar registers for what is needed once per query, and what does not fit is parked
 // in lanes of vector registers.  Through a pointer it cannot see through the fields are loaded where they are used.
@@ -503,17 +521,7 @@ __global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 &&
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
   if (TEAM) {
     // a workgroup per query: its first wavefront searches, the others help
-    s.team.base = reinterpret_cast<uint32_t*>(smem + lp.total);
-    s.team.bucket_bits = a0.team_bucket_bits;
-    s.team.stride = ix0.S0;
-    s.team.lists = Team::lists_at(NS);
-    for (int i = (int)threadIdx.x; i < Team::kRoom; i += (int)blockDim.x)
-      s.team.base[i] = i < (4 << a0.team_bucket_bits) ? kNobody : (i == Team::kOver ? 0u : kEmpty);
-    filter_reset(s, (int)threadIdx.x, (int)blockDim.x);
-    __syncthreads();
-    // (the workgroups that share a CU have their first wavefronts on the same SIMD: another one of each searches)
-    const int waves = (int)blockDim.x >> 6;
-    const int wave = (uni((int)threadIdx.x >> 6) + waves - ((int)blockIdx.x / a0.team_turn) % waves) % waves;
+    const int wave = gather_team<NS>(s, smem + lp.total, ix0.S0, 0, a0.team_bucket_bits, a0.team_turn);
     if (wave > 0) {
       const int lane = (int)threadIdx.x & 63;
       QVec<QR> qv;
@@ -1193,12 +1201,13 @@ __device__ __forceinline__ void write_row_and_post(const DevIndex& ix, const Bui
 // Phase 1 of a build batch: search, select, write the new rows, post the reverse links.
 // (held to six / five wavefronts per SIMD where the query fits one / two float4 registers: a few
 // spilled registers, 3-4 % off the build time of the 1.18 M x 50 and 10 M x 96 sets)
-template <int DT, int QR, int NS>
-__global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR == 2) ? 5 : 1)) build_search_kernel(DevIndex ix, BuildArgs a) {
+// TEAM: a batch that leaves the machine idle, a workgroup per node (team_help), those of the list first; sorted set only.
+template <int DT, int QR, int NS, bool TEAM = false>
+__global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 && NS <= 8 ? 4 : 2) : (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR == 2) ? 5 : 1)) build_search_kernel(DevIndex ix, BuildArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  int lane = threadIdx.x;
+  int lane = threadIdx.x & 63;
   const int m_max = ix.max_m0 > ix.max_m ? ix.max_m0 : ix.max_m;
-  const bool sorted_set = NS > 0 && a.fc.sets() > 0;
+  const bool sorted_set = TEAM || (NS > 0 && a.fc.sets() > 0);
   const LdsPlan lp = plan_lds(QR, ix.Dp, sorted_set ? -1 : a.efc, a.cand_lds, a.lcap, a.efc, m_max, a.vc_bits, a.fc);
   Scratch s;
   s.vcache = sorted_set ? reinterpret_cast<uint16_t*>(smem + lp.fcache)
@@ -1219,14 +1228,36 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
   bind_slot(s, a.pool, blockIdx.x);
   // this wavefront's share of a.counters (LDS, so that counting costs the kernel no registers when it is off)
   __shared__ unsigned int work[16];
-  if (lane < 16) work[lane] = 0u;
+  if (threadIdx.x < 16) work[threadIdx.x] = 0u;
   wave_sync();
+  int taken = 0;  // (TEAM) nodes this workgroup has dealt with
+  if (TEAM) {
+    const int at = (int)blockIdx.x < a.n_upper ? a.upper[blockIdx.x] : (int)blockIdx.x - a.n_upper;
+    const uint32_t x = (uint32_t)(a.begin + uni(at < a.count ? at : 0));
+    const int lx = ix.levels[x];
+    const int top_level = uni(lx < a.cur_max ? lx : a.cur_max);
+    const bool here = uni(((int)blockIdx.x < a.n_upper || a.n_upper == 0 || lx <= 0) ? 1 : 0) != 0;
+    const int wave = gather_team<NS>(s, smem + lp.total, ix.S0 > ix.SU ? ix.S0 : ix.SU, top_level > 0 ? top_level : 0, a.team_bucket_bits, a.team_turn);
+    if (wave > 0) {
+      if (here && top_level >= 0) {
+        QVec<QR> qv;
+        load_node_query<QR>(qv, s.qlds, ix, x, lane);
+        team_help<DT, QR, true>(ix, qv, s, wave - 1, lane);
+      }
+      return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+  }
 
   for (;;) {
     // first the n_upper nodes of the list, then all by id, the ones of the list passed over
     lane = fresh(lane);
     int b = 0;
-    if (lane == 0) {
+    if (TEAM) {
+      b = (int)blockIdx.x;
+      b = b < a.n_upper ? a.upper[b] : b - a.n_upper + (1 << 30);
+      if (taken++ > 0) b = a.count + (1 << 30);
+    } else if (lane == 0) {
       b = atomicAdd(a.counter, 1);
       b = b < a.n_upper ? a.upper[b] : b - a.n_upper + (1 << 30);
     }
@@ -1260,7 +1291,15 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
         const int evals_before = st.n_dist, hops_before = st.n_hops;
         int T;
         if (sorted_set) {
-          filter_reset(s, lane);
+          if (!TEAM || level < top_level) filter_reset(s, lane);
+          if (TEAM) {
+            if (level < top_level) team_open(s.team, level, lane);
+            HeapEnt e;
+            e.key = INFINITY;
+            e.id = cur;
+            if (lane == 0) s.team.line()[8] = e;
+            __builtin_amdgcn_wave_barrier();
+          }
           // sorted set in registers: the efc best come out in order (equal keys in the order
           // the set placed them, which is deterministic).  The new node itself cannot turn up:
           // nothing links to it before the batch's later phases.
@@ -1269,8 +1308,13 @@ __global__ void __launch_bounds__(64, (NS <= 5 && QR == 1) ? 6 : ((NS <= 5 && QR
           wave_sync();
           Frontier<NS> fr;
           frontier_init<NS>(fr, a.efc, lane);
-          search_level_fast<DT, QR, NS, true>(ix, qv, level, a.efc, s, st, fr, 1, lane, a.reverse != 0);
+          search_level_fast<DT, QR, NS, true, false, TEAM, TEAM>(ix, qv, level, a.efc, s, st, fr, 1, lane, a.reverse != 0);
           T = st.top_size;
+          if (TEAM) {
+            if (level > 0) team_close(s.team, lane);
+            else if (lane == 0) lds_tell(s.team.over(), 1u);
+            __builtin_amdgcn_wave_barrier();
+          }
           wave_sync();
           frontier_dump<NS>(fr, a.efc, T, sid, skey, lane);
           wave_sync();

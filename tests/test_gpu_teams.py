@@ -44,3 +44,34 @@ def test_batches_that_leave_the_machine_idle_match_the_oracle(oracle, tmp_path, 
       g_ids, g_d, g_f, stats = _device_search(e, q[part], k, ef)
       assert (g_f == o_f[part]).all() and (g_ids == o_ids[part]).all() and (g_d == o_d[part]).all(), nq
       assert (stats[:, 1:] == o_cnt[part, 1:4]).all(), nq
+
+
+@pytest.mark.parametrize("n,d,dist,max_m,max_m0,efc,kind,extra", [
+    (5200, 16, "l2", 8, 16, 60, "int", {}),                                   # equal keys everywhere
+    (4500, 100, "dot", 32, 64, 130, "gauss", dict(heuristic_coef=0.25)),      # link rows of 64 ids
+    (2500, 300, "l2", 3, 6, 100, "gauss", dict(save_remains=True)),           # many levels; rows too long for registers
+    (4500, 180, "l2", 16, 32, 700, "scattered", {}),                          # the largest set
+], ids=["ties", "full64", "levels", "large"])
+def test_index_built_by_teams_is_the_one_built_without(tmp_path, n, d, dist, max_m, max_m0, efc, kind, extra):
+  """Batches of a build go through every size up to a quarter of the nodes; a filter of a given size takes the wavefront alone."""
+  if kind == "int":
+    x = integer_vectors(n, d, seed=3, hi=6)
+  elif kind == "scattered":
+    x = np.random.default_rng(4).standard_normal((n, d)).astype(np.float32)
+  else:
+    x = gauss_mixture(n, d, seed=5, normalise=dist == "dot")
+  levels = _levels(n, 1.0 / np.log(max_m), 6)
+  files = []
+  for entries in (0, 16384):
+    options = dict(dict(heuristic_coef=0.0), dist_type=dist, max_m=max_m, max_m0=max_m0, ef_construction=efc)
+    options.update(extra)
+    e = _engine(tmp_path, **options)
+    e.set_tunable("filter_entries", entries)
+    e.set_data(x)
+    e.set_random_levels(levels)
+    print("built by teams", kind, entries, flush=True)
+    e.build_graph()
+    p = tmp_path / "b.idx"
+    e.save_index(str(p))
+    files.append(p.read_bytes())
+  assert files[0] == files[1]
