@@ -700,6 +700,23 @@ __global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 &&
   }
 }
 
+// The accepted entries of a search through hnswlib's result heap.  (64 of the log's records per fetch, handed out lane by lane, and
+// the next 64 fetched meanwhile: one by one each is a trip to memory, a third of what an entry takes.)
+__device__ __forceinline__ void replay_log(const Scratch& s, LdsHeap& top, int& size, int n, int ef, int lane) {
+  HeapEnt next = s.log[lane < n ? lane : 0];
+  for (int base = 0; base < n; base += 64) {
+    const HeapEnt mine = next;
+    const int cnt = n - base < 64 ? n - base : 64;
+    next = s.log[base + 64 + lane < n ? base + 64 + lane : 0];
+    for (int j = 0; j < cnt; ++j) {
+      HeapEnt e;
+      e.key = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.key), j));
+      e.id = (uint32_t)__builtin_amdgcn_readlane((int)mine.id, j);
+      coop_push<false>(top, size, e, lane);
+      if (size > ef) coop_pop<false>(top, size, s.tree, lane);
+    }
+  }
+}
 // Search with literal hnswlib priority queues: the only pass for ef beyond the sorted set's
 // capacity, the second pass (over a.redo) otherwise.
 // NS > 0: result keys in registers (ef <= 64*NS); NS == 0: literal result heap in LDS.
@@ -869,11 +886,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
           seed.id = cur;
           coop_push<false>(top, size, seed, lane);
         }
-        for (int i = 0; i < st.n_acc; ++i) {
-          const HeapEnt e = uniform_ent(s.log[i]);
-          coop_push<false>(top, size, e, lane);
-          if (size > a.ef) coop_pop<false>(top, size, s.tree, lane);
-        }
+        replay_log(s, top, size, st.n_acc, a.ef, lane);
         for (int base = rest_from; base < tmeta.y; base += 64) {
           const int cnt = tmeta.y - base < 64 ? tmeta.y - base : 64;
           const uint4 r = trail[base + (lane < cnt ? lane : 0)];   // 64 records per fetch, handed out lane by lane
@@ -909,11 +922,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
         literal = true;
         LdsHeap top{s.top};
         int size = 0;
-        for (int i = 0; i < st.n_acc; ++i) {
-          const HeapEnt e = uniform_ent(s.log[i]);
-          coop_push<false>(top, size, e, lane);
-          if (size > a.ef) coop_pop<false>(top, size, s.tree, lane);
-        }
+        replay_log(s, top, size, st.n_acc, a.ef, lane);
         st.top_size = size;
       }
       }
@@ -951,11 +960,7 @@ __global__ void __launch_bounds__(64, (QR >= 1 && QR <= 2 && NS > 0 && NS <= 5) 
         literal = true;
         LdsHeap top{s.top};
         int size = 0;
-        for (int i = 0; i < st.n_acc; ++i) {
-          const HeapEnt e = uniform_ent(s.log[i]);
-          coop_push<false>(top, size, e, lane);
-          if (size > a.ef) coop_pop<false>(top, size, s.tree, lane);
-        }
+        replay_log(s, top, size, st.n_acc, a.ef, lane);
         st.top_size = size;
       }
     }
