@@ -172,12 +172,20 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));
 }
 __device__ __forceinline__ unsigned long long first_lanes(int n) { return n < 64 ? (1ull << (n & 63)) - 1ull : ~0ull; }  // (n <= 64)
-__device__ __forceinline__ float wave_min(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x = fminf(x, __shfl_xor(x, m, 64));
-  return uni(x);  // (the same in every lane: said so, or all that depends on it counts as lane-dependent)
-}
 
+// Smallest value of all lanes, wavefront-uniform.  (Through neighbours' registers: as exchanges through LDS it took 720 cycles, a
+// quarter of a step of a descent.)
+__device__ __forceinline__ float least_of_all(float x) {
+  auto take = [&](int from) __attribute__((always_inline)) { x = fminf(x, __builtin_bit_cast(float, from)); };
+  const auto bits = [&]() __attribute__((always_inline)) { return __builtin_bit_cast(int, x); };
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x111, 0xF, 0xF, false));  // (lane 63 has seen all in the end)
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x112, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x114, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x118, 0xF, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x142, 0xA, 0xF, false));
+  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x143, 0xC, 0xF, false));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits(), 63));
+}
 template <int DT>
 __device__ __forceinline__ void acc4(const float4 q, const float4 v, float& ax, float& ay, float& az, float& aw) {
   if (DT == DIST_DOT) {
@@ -1010,18 +1018,6 @@ __device__ __forceinline__ int max_so_far(int x) {
   take(__builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
   take(__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
   return x;
-}
-// Smallest value of all lanes (finite, or +inf).
-__device__ __forceinline__ float least_of_all(float x) {
-  auto take = [&](int from) __attribute__((always_inline)) { x = fminf(x, __builtin_bit_cast(float, from)); };
-  const auto bits = [&]() __attribute__((always_inline)) { return __builtin_bit_cast(int, x); };
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x111, 0xF, 0xF, false));  // (as max_so_far: lane 63 has seen all)
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x112, 0xF, 0xF, false));
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x114, 0xF, 0xF, false));
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x118, 0xF, 0xF, false));
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x142, 0xA, 0xF, false));
-  take(__builtin_amdgcn_update_dpp(bits(), bits(), 0x143, 0xC, 0xF, false));
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits(), 63));
 }
 __device__ __forceinline__ int least_of_all_ints(int x) {
   auto take = [&](int from) __attribute__((always_inline)) { x = from < x ? from : x; };
@@ -2551,7 +2547,7 @@ __device__ __forceinline__ int search_level_fast(const DevIndex& ix, const QVec<
           resume_at = -1;
         }
         // offers turned away while a group of equal keys is being expanded: remember the closest
-        if (exact && in_group) group_edge = uni(fminf(group_edge, wave_min((mine < n && !pass) ? my_key : INFINITY)));
+        if (exact && in_group) group_edge = uni(fminf(group_edge, least_of_all((mine < n && !pass) ? my_key : INFINITY)));
         // (plain if/else nesting, one way out of the loop: `continue` and `return` in here make the
         // compiler thread a state variable through a dozen scalar blocks per accepted candidate)
         while (todo != 0ull) {
@@ -2839,17 +2835,41 @@ __device__ __forceinline__ void search_level_lean(const DevIndex& ix, const QVec
 // scans the neighbour list captured at its start and moves to the strictly
 // closest entry, which for a strict running minimum is the first occurrence of the
 // list minimum.
+// (A chain of fetches: where a node's upper rows are, its row, the neighbours' vectors.  Where the neighbours' rows are is asked for
+// beside their vectors, and so is the node's row one level down, which a sweep that finds nothing closer goes on with.)
 template <int DT, int QR>
 __device__ __forceinline__ void descend(const DevIndex& ix, const QVec<QR>& qv, int from_level, int to_level,
                                         uint32_t& cur, float& dcur, Scratch& s, SearchState& st, int lane) {
+  if (from_level <= to_level) return;
+  const int SU = ix.SU;
+  const int at = lane < SU ? lane : 0;
+  long long first = ix.upper_off[cur];  // the node's row of level 1
+  uint32_t below = kEmpty;              // the first 64 slots of its row one level down, where they have been asked for
+  bool have_below = false;
   for (int level = from_level; level > to_level; --level) {
     bool changed = true;
     while (changed) {
       changed = false;
-      int n = load_row(link_row(ix, cur, level), ix.SU, s, lane);
+      const uint32_t* const row = ix.linksU + (size_t)(first + level - 1) * SU;
+      const uint32_t got = have_below ? below : row[at];
+      const uint32_t mine = lane < SU ? got : kEmpty;
+      have_below = level - 1 > to_level;
+      if (have_below) below = (row - SU)[at];
+      const unsigned long long mask = __ballot(mine != kEmpty);
+      if (mine != kEmpty) s.nbuf[lanes_below(mask)] = mine;
+      __builtin_amdgcn_wave_barrier();
+      int n = __popcll(mask);
+      for (int base = 64; base < SU; base += 64) {
+        const uint32_t id = base + lane < SU ? row[base + lane] : kEmpty;
+        const unsigned long long more = __ballot(id != kEmpty);
+        if (id != kEmpty) s.nbuf[n + lanes_below(more)] = id;
+        __builtin_amdgcn_wave_barrier();
+        n += __popcll(more);
+      }
       wave_sync();
       st.n_sweeps += 1;
       if (n == 0) break;
+      const long long firsts = ix.upper_off[mine != kEmpty ? mine : cur];
       dist_list<DT, QR, false>(ix, qv, s.qlds, s.nbuf, n, s.dbuf, lane);
       st.n_dist_upper += n;
       wave_sync();
@@ -2858,7 +2878,7 @@ __device__ __forceinline__ void descend(const DevIndex& ix, const QVec<QR>& qv, 
       for (int base = 0; base < n; base += 64) {
         int t = base + lane;
         float d = t < n ? s.dbuf[t] : INFINITY;
-        float m = wave_min(d);
+        float m = least_of_all(d);
         if (m < best) {
           best = m;
           unsigned long long mask = __ballot(d == m);
@@ -2868,6 +2888,15 @@ __device__ __forceinline__ void descend(const DevIndex& ix, const QVec<QR>& qv, 
       if (bidx >= 0 && best < dcur) {
         dcur = uni(best);
         cur = (uint32_t)uni((int)s.nbuf[bidx]);
+        const unsigned long long holds = __ballot(mine == cur);
+        if (holds != 0ull) {
+          const int l = __builtin_ctzll(holds);
+          first = (long long)(((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(firsts >> 32), l) << 32) |
+                              (uint32_t)__builtin_amdgcn_readlane((int)firsts, l));
+        } else {
+          first = ix.upper_off[cur];
+        }
+        have_below = false;
         changed = true;
       }
       wave_sync();
