@@ -1254,11 +1254,14 @@ __global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 &&
     const int lx = ix.levels[x];
     const int top_level = uni(lx < a.cur_max ? lx : a.cur_max);
     const bool here = uni(((int)blockIdx.x < a.n_upper || a.n_upper == 0 || lx <= 0) ? 1 : 0) != 0;
+    // (a row that lies in LDS: there before gather_team's barrier, all wavefronts write the same.  The selection puts its picks in its
+    // place, and a helper that came to write it only then would have the picks' tests made against the node.)
+    QVec<QR> qv;
+    if (QR == 0) load_node_query<QR>(qv, s.qlds, ix, x, lane);
     const int wave = gather_team<NS>(s, smem + lp.total, ix.S0 > ix.SU ? ix.S0 : ix.SU, top_level > 0 ? top_level : 0, a.team_bucket_bits, a.team_turn);
     if (wave > 0) {
       if (here && top_level >= 0) {
-        QVec<QR> qv;
-        load_node_query<QR>(qv, s.qlds, ix, x, lane);
+        if (QR != 0) load_node_query<QR>(qv, s.qlds, ix, x, lane);
         team_help<DT, QR, true>(ix, qv, s, wave - 1, lane);
       }
       return;
