@@ -33,6 +33,7 @@
 #include "heap_coop.h"
 #include "index_file.h"
 #include "options.h"
+#include "team_slots.h"
 #include "visited_filter.h"
 
 namespace cuhnsw_amd {
@@ -1683,12 +1684,11 @@ __device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t can
 // (Cycles of a step of one query on 100 000 x 50 at ef 300, a wavefront alone: distances 1 150, the set 2 200, candidates, links and
 // filter 2 090, 112 steps; the search by a team has 69 of them, of which 13 evaluate nodes of their own.)
 //
-// Slots: the owner's id when its list is there, how many eights of nodes it has in bits 28 to 30; the id with kExpanded while it is
-// being made; kNobody: free.  (Ids are below 2^28 where there is a visited filter.)  A helper takes a free slot of the candidate's
+// Slots: team_slots.h.  (Ids are below 2^28 where there is a visited filter.)  A helper takes a free slot of the candidate's
 // bucket by compare-and-swap, then looks whether the candidate is still in line and in no other slot (the search writes the line
 // before it looks for lists: one of the two sees the other), and gives the slot back otherwise.  Only the search frees a slot
 // whose list is there.  LDS operations of a wavefront are carried out in order.
-constexpr uint32_t kNobody = 0x7FFFFFFFu, kTeamId = 0x0FFFFFFFu;
+static_assert(kSlotMaking == kExpanded && kNoSlot == kEmpty, "as the ids in the line and in link rows");
 constexpr int kMostListed = 56;  // (seven eights; a longer list is left to the search)
 __device__ __forceinline__ void lds_done() {  // everything this wavefront wrote to LDS is there
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1735,7 +1735,7 @@ __device__ __forceinline__ void team_tidy(const Team& team, int lane) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const uint32_t owner = lds_now(team.owner() + lane + 64 * i);
-    if ((owner & kExpanded) == 0u && owner != kNobody && kept[lane + 64 * i] == 0u) lds_tell(team.owner() + lane + 64 * i, kNobody);
+    if (slot_holds_list(owner) && kept[lane + 64 * i] == 0u) lds_tell(team.owner() + lane + 64 * i, kNobody);
     __builtin_amdgcn_wave_barrier();
   }
   wave_sync();
@@ -1753,8 +1753,8 @@ __device__ __forceinline__ void team_close(const Team& team, int lane) {
   for (int i = 0; i < 2; ++i) {
     while (true) {
       const uint32_t owner = lds_now(team.owner() + lane + 64 * i);
-      if (__ballot((owner & kExpanded) != 0u && owner != kEmpty) == 0ull) {
-        if (owner != kEmpty) lds_tell(team.owner() + lane + 64 * i, kNobody);
+      if (__ballot(slot_being_made(owner)) == 0ull) {
+        if (slot_holds_list(owner)) lds_tell(team.owner() + lane + 64 * i, kNobody);
         __builtin_amdgcn_wave_barrier();
         break;
       }

@@ -10,10 +10,12 @@
 #pragma once
 #include <stdint.h>
 
+#ifndef CUHNSW_HOST_DEVICE
 #ifndef __HIPCC__
 #define CUHNSW_HOST_DEVICE
 #else
 #define CUHNSW_HOST_DEVICE __host__ __device__
+#endif
 #endif
 
 namespace cuhnsw_amd {
