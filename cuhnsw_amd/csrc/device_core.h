@@ -1689,7 +1689,6 @@ __device__ __forceinline__ int visit_lossy_rows(const DevIndex& ix, uint32_t can
 // before it looks for lists: one of the two sees the other), and gives the slot back otherwise.  Only the search frees a slot
 // whose list is there.  LDS operations of a wavefront are carried out in order.
 static_assert(kSlotMaking == kExpanded && kNoSlot == kEmpty, "as the ids in the line and in link rows");
-constexpr int kMostListed = 56;  // (seven eights; a longer list is left to the search)
 __device__ __forceinline__ void lds_done() {  // everything this wavefront wrote to LDS is there
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -1714,10 +1713,10 @@ __device__ __forceinline__ TeamPlace team_look(const Team& team, uint32_t id) {
   t.making = false;
 #pragma unroll
   for (int w = 3; w >= 0; --w) {
-    const bool mine = (o[w] & (kTeamId | kExpanded)) == id;
+    const bool mine = slot_is_of(o[w], id);
     t.there = mine ? first + w : t.there;
-    t.eights = mine ? (int)(o[w] >> 28) : t.eights;
-    t.making = t.making || o[w] == (id | kExpanded);
+    t.eights = mine ? slot_eights(o[w]) : t.eights;
+    t.making = t.making || o[w] == (id | kSlotMaking);
     t.room = o[w] == kNobody ? first + w : t.room;
   }
   return t;
@@ -1813,7 +1812,7 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
     if (slot >= 0) {
       if (lane == 0) {
         uint32_t was = kNobody;
-        mine = __hip_atomic_compare_exchange_strong(team.owner() + slot, &was, id | kExpanded, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        mine = __hip_atomic_compare_exchange_strong(team.owner() + slot, &was, id | kSlotMaking, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
       __builtin_amdgcn_wave_barrier();
     }
@@ -1822,7 +1821,7 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
       const bool wished = __ballot(lane < Team::kInLine && lds_now(reinterpret_cast<const uint32_t*>(team.line() + (lane < Team::kInLine ? lane : 0)) + 1) == id) != 0ull;
       const int other = 4 * (int)team.bucket(id) + (lane & 3);
       const uint32_t there = lds_now(team.owner() + other);
-      const bool twice = __ballot(other != slot && ((there & (kTeamId | kExpanded)) == id || there == (id | kExpanded))) != 0ull;
+      const bool twice = __ballot(other != slot && (slot_is_of(there, id) || there == (id | kSlotMaking))) != 0ull;
       const bool still = !LEVELS || (uint32_t)uni((int)lds_now(team.level())) == at;
       uint32_t say = kNobody;
       if ((wished || !asked) && !twice && still) {
@@ -1837,7 +1836,7 @@ __device__ __forceinline__ void team_help(const DevIndex& ix, const QVec<QR>& qv
         wave_sync();
         dist_list<DT, QR, false, team_wide<QR>()>(ix, qv, s.qlds, ids, n, team.keys(slot), lane);
         lds_done();
-        if (n <= kMostListed) say = id | ((uint32_t)(n > 0 ? (n + 7) >> 3 : 1) << 28);
+        say = slot_word(id, n);
         if (n > 0) {
           const float my_key = lane < n ? team.keys(slot)[lane < n ? lane : 0] : INFINITY;
           const float least = least_of_all(my_key);

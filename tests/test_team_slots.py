@@ -24,3 +24,8 @@ def test_a_list_has_one_writer_and_one_level(run):
   assert states > 1000 and (clashes, stale) == (0, 0)
   # (the walk does find the two writers where a level's end stores to slots that were free when it looked)
   assert slots(1)[1] > 0
+
+
+def test_a_list_of_any_length_that_a_row_can_have_keeps_its_slot(run):
+  """Rows of 64 ids have lists of up to eight eights."""
+  assert run("words")() == [0, 0]
