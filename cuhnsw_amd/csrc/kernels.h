@@ -295,7 +295,7 @@ __device__ __forceinline__ float entry4_key(const void* rows, uint32_t rowlen, u
   }
   return finish16<DT, false>(ax, ay, az, aw);
 }
-template <int DT, int QR, bool HALF>
+template <int DT, int QR, bool HALF, bool BESIDE>
 __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs& a) {
   const int lane = threadIdx.x, g = lane >> 4, sub = lane & 15;
   const uint32_t rowlen = (uint32_t)ix.Dp >> 2, used = (uint32_t)(ix.D + 3) >> 2;
@@ -314,9 +314,6 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
     bool active = have && level > 0;
     int sweeps = 0, evals = 0;
     uint32_t region = cur;
-    // (as in descend: where the neighbours' rows are is asked for beside their vectors -- in one round of wavefronts; a batch of several
-    // is better off without these fetches.  1.18 M x 50, 10 000 queries 1.743 -> 1.707 ms, 1 M x 96, 100 000 with them 8.87 -> 8.93.)
-    const bool beside = (long long)gridDim.x * 4 >= a.nq;
     long long first = ix.upper_off[cur];
     while (__ballot(active) != 0ull) {
       const uint32_t* row = ix.linksU + (size_t)((active ? first : 0) + (active ? level : 1) - 1) * ix.SU;
@@ -328,7 +325,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
         const uint32_t got = row[base + sub < ix.SU ? base + sub : 0];
         const uint32_t id = (active && base + sub < ix.SU) ? got : kEmpty;
         const unsigned long long valid = __ballot(id != kEmpty);
-        const long long firsts = beside ? ix.upper_off[id != kEmpty ? id : cur] : 0ll;
+        const long long firsts = BESIDE ? ix.upper_off[id != kEmpty ? id : cur] : 0ll;
         int best_at = -1;
         n += __popc((uint32_t)(valid >> (16 * g)) & 0xFFFFu);
         constexpr int B = QR == 1 ? 16 : 8;  // rows in flight per lane: 16 float4 registers' worth
@@ -350,9 +347,11 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
               best_at = p0 + j;
             }
         }
-        const int from = 16 * g + (best_at < 0 ? 0 : best_at);
-        const uint32_t low = (uint32_t)__shfl((int)firsts, from, 64), high = (uint32_t)__shfl((int)(firsts >> 32), from, 64);
-        best_first = best_at < 0 ? best_first : (long long)(((unsigned long long)high << 32) | low);
+        if constexpr (BESIDE) {
+          const int from = 16 * g + (best_at < 0 ? 0 : best_at);
+          const uint32_t low = (uint32_t)__shfl((int)firsts, from, 64), high = (uint32_t)__shfl((int)(firsts >> 32), from, 64);
+          best_first = best_at < 0 ? best_first : (long long)(((unsigned long long)high << 32) | low);
+        }
       }
       if (active) {
         sweeps += 1;
@@ -360,7 +359,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
         if (n > 0 && best < dcur) {
           dcur = best;
           cur = best_id;  // and sweep again on this level
-          first = beside ? best_first : ix.upper_off[best_id];
+          first = BESIDE ? best_first : ix.upper_off[best_id];
         } else {
           if (level == a.region_level) region = cur;
           level -= 1;
@@ -376,10 +375,12 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
     }
   }
 }
-template <int DT, int QR>
+// BESIDE: as in descend, where the neighbours' rows are is asked for beside their vectors.  For batches of one round of
+// wavefronts (the host's choice: instances.hip); its registers cost a wavefront per SIMD, four instead of five.
+template <int DT, int QR, bool BESIDE>
 __global__ void __launch_bounds__(64) entry4_kernel(DevIndex ix, SearchArgs a) {
-  if (uni(ix.half) != 0) entry4_body<DT, QR, true>(ix, a);
-  else entry4_body<DT, QR, false>(ix, a);
+  if (uni(ix.half) != 0) entry4_body<DT, QR, true, BESIDE>(ix, a);
+  else entry4_body<DT, QR, false, BESIDE>(ix, a);
 }
 // counters -> first position of every bucket (exclusive prefix sum over `from` and what lies before; one workgroup of 1024).
 // cut: the longest queries end with the first bucket at which there are `most` of them or more; set to that bucket and to

@@ -62,6 +62,13 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_DOT, 2, 4, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,4,few>"),
     ("search_fast_kernel<DIST_L2, 0, 6, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,6,few>"),
 ]
+# the batch's descents, four to a wavefront (the instances for batches of more than one round of wavefronts)
+DESCENTS = [
+    ("entry4_kernel<DIST_DOT, 1, false>(DevIndex, SearchArgs)", "entry4_kernel<dot,1>"),
+    ("entry4_kernel<DIST_DOT, 2, false>(DevIndex, SearchArgs)", "entry4_kernel<dot,2>"),
+    ("entry4_kernel<DIST_L2, 1, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,1>"),
+    ("entry4_kernel<DIST_L2, 2, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,2>"),
+]
 OTHERS = [
     ("search_fast_kernel<DIST_DOT, 1, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,5,team>"),
     ("search_fast_kernel<DIST_L2, 2, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,5,team>"),
@@ -257,7 +264,7 @@ def compile_kernels(instances):
 
 
 def main():
-  report = compile_kernels(FIRST_PASS + OTHERS)
+  report = compile_kernels(FIRST_PASS + DESCENTS + OTHERS)
   for name, r in report.items():
     print("%-34s VGPRs %3d  waves/SIMD %d  VGPR spills %3d  SGPR spills %3d  scratch %3d B/lane  scratch instrs %3d (in hop loops %d)" % (
         name, r["vgprs"], r["waves_per_simd"], r["vgpr_spills"], r["sgpr_spills"], r["scratch_bytes_per_lane"],
