@@ -572,9 +572,12 @@ class Engine {
   // (Against the next power of two above the least: 500 000 x 128 at ef 128, 256 -> 568 sets, 10 000 queries 1.93 -> 1.81 ms; 1 M x
   // 96, ef 256, topk 100, 512 -> 568 sets, 100 000 queries 9.28 -> 9.14; 1 183 514 x 50 indexed and saved, 256 -> 425, 124.7 ->
   // 123.0.)
+  // (Worked out once per kernel, filter to begin with -- and so to end with -- and LDS beside it, which the sizes without a
+  // filter, with the first and with the last tell: the answer lies over the filter and counts as far as it is longer.)
   struct Fitted {
     const void* kernel;
-    size_t lds;
+    uint32_t first;
+    size_t lds_none, lds_first, lds_last;
     int sets;
   };
   std::vector<Fitted> filters_known;
@@ -582,10 +585,11 @@ class Engine {
   FilterShape fit_filter(K kernel, FilterShape f, Lds&& lds_of) {
     if (filter_entries > 0 || f.sets() == 0) return f;
     const void* const id = reinterpret_cast<const void*>(kernel);
-    const size_t least_lds = lds_of(f);
-    for (const Fitted& k : filters_known)
-      if (k.kernel == id && k.lds == least_lds) return filter_shape(k.sets, host.N);
     const int most = std::min(4 * f.sets(), kMostFilterSets);
+    Fitted now{id, f.code, lds_of(FilterShape()), lds_of(f), lds_of(filter_shape(most, host.N)), 0};
+    for (const Fitted& k : filters_known)
+      if (k.kernel == id && k.first == now.first && k.lds_none == now.lds_none && k.lds_first == now.lds_first && k.lds_last == now.lds_last)
+        return filter_shape(k.sets, host.N);
     while (true) {
       const FilterShape half = filter_shape(f.sets() / 2, host.N);
       if (half.sets() >= f.sets() || resident_slots(kernel, lds_of(half)) * 20 < resident_slots(kernel, lds_of(f)) * 23) break;
@@ -598,7 +602,8 @@ class Engine {
       else high = (low + high) / 2;
     }
     if (filters_known.size() >= 64) filters_known.clear();
-    filters_known.push_back({id, least_lds, f.sets()});
+    now.sets = f.sets();
+    filters_known.push_back(now);
     return f;
   }
 
