@@ -19,7 +19,7 @@ SYMBOLS = [
     "cuhnsw_search_knn_device_noalloc", "cuhnsw_last_build_dropped_links", "cuhnsw_debug_link_keys0",
     "cuhnsw_last_build_counters", "cuhnsw_debug_gather_probe", "cuhnsw_last_search_trails",
     "cuhnsw_last_search_side_by_side", "cuhnsw_literal_fallbacks", "cuhnsw_trails_available",
-    "cuhnsw_num_deleted", "cuhnsw_search_knn_taking",
+    "cuhnsw_num_deleted", "cuhnsw_search_knn_taking", "cuhnsw_last_search_team", "cuhnsw_last_build_team_batches",
 ]
 
 _lib = None
@@ -61,6 +61,8 @@ def load():
   l.cuhnsw_last_search_repeats.argtypes = [vp]
   l.cuhnsw_last_search_trails.argtypes = [vp]
   l.cuhnsw_last_search_side_by_side.argtypes = [vp]
+  l.cuhnsw_last_search_team.argtypes = [vp]
+  l.cuhnsw_last_build_team_batches.argtypes = [vp]
   l.cuhnsw_literal_fallbacks.argtypes = [vp]
   l.cuhnsw_trails_available.argtypes = [vp]
   l.cuhnsw_num_deleted.argtypes = [vp]
@@ -185,6 +187,8 @@ class Engine:
   last_build_seconds = property(lambda s: s._l.cuhnsw_last_build_seconds(s._h))
   last_search_repeats = property(lambda s: s._l.cuhnsw_last_search_repeats(s._h))
   last_search_trails = property(lambda s: s._l.cuhnsw_last_search_trails(s._h))
+  last_search_team = property(lambda s: s._l.cuhnsw_last_search_team(s._h))
+  last_build_team_batches = property(lambda s: s._l.cuhnsw_last_build_team_batches(s._h))
   last_search_side_by_side = property(lambda s: bool(s._l.cuhnsw_last_search_side_by_side(s._h)))
   literal_fallbacks = property(lambda s: s._l.cuhnsw_literal_fallbacks(s._h))
   trails_available = property(lambda s: bool(s._l.cuhnsw_trails_available(s._h)))

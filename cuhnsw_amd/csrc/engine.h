@@ -187,6 +187,8 @@ class Engine {
   int sequential_left = 0;       // searches still to run one pass after the other
   int literal_fallbacks = 0;     // how often that happened on this index
   int last_side_by_side = 0;     // the last search ran its literal pass beside the first pass
+  int last_team = 0;             // wavefronts that searched each of its queries together (launch_teams); 0 = one alone
+  int last_team_batches = 0;     // batches of the last build whose nodes were searched so
   bool trails_unavailable = false;  // the trail buffers could not be allocated: searches go on without trails
   int filter_entries = 0;  // entries of the sorted-set search's visited filter (0 = automatic)
   int first_pass_waves = 0;  // wavefronts per CU of the first pass (0 = as many as fit)
@@ -444,7 +446,7 @@ class Engine {
     recent_queries = recent_repeats = 0.0;
     sequential_left = 0;
     literal_fallbacks = 0;
-    last_side_by_side = 0;
+    last_side_by_side = last_team = 0;
     last_repeats = last_trails = 0;
   }
 
@@ -662,6 +664,7 @@ class Engine {
       if (resident_slots(kernel, bytes(), waves) < per_cu * num_cus) continue;
       hipLaunchKernelGGL(kernel, dim3(a.nq), dim3(64 * waves), bytes(), stream, ix, a);
       HIP_CHECK(hipGetLastError());
+      last_team = waves;
       return true;
     }
     return false;

@@ -164,6 +164,8 @@ int cuhnsw_num_deleted(cuhnsw_engine* e) { return e ? e->impl.host.n_deleted : 0
 int cuhnsw_last_search_repeats(cuhnsw_engine* e) { return e ? e->impl.last_repeats : 0; }
 int cuhnsw_last_search_trails(cuhnsw_engine* e) { return e ? e->impl.last_trails : 0; }
 int cuhnsw_last_search_side_by_side(cuhnsw_engine* e) { return e ? e->impl.last_side_by_side : 0; }
+int cuhnsw_last_search_team(cuhnsw_engine* e) { return e ? e->impl.last_team : 0; }
+int cuhnsw_last_build_team_batches(cuhnsw_engine* e) { return e ? e->impl.last_team_batches : 0; }
 int cuhnsw_literal_fallbacks(cuhnsw_engine* e) { return e ? e->impl.literal_fallbacks : 0; }
 int cuhnsw_trails_available(cuhnsw_engine* e) { return e ? (e->impl.trails_unavailable ? 0 : 1) : 0; }
 int cuhnsw_set_tunable(cuhnsw_engine* e, const char* name, double value) {

@@ -56,7 +56,7 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
   a.report = nullptr;
   last_repeats = 0;
   last_trails = 0;
-  last_side_by_side = 0;
+  last_side_by_side = last_team = 0;
   if (use_static) {
     launch_search_static<DT, QR, NS>(ix, a, ms);
     return;
@@ -516,6 +516,7 @@ void Engine::build_levels() {
   const size_t lds1 = search_lds(a.fc);
   const LdsPlan lp3 = plan_lds(QR, Dp, s_max + cap_in, 0, a.lcap, s_max + cap_in, std::max(m_max, cap_in));
   const int slots1 = resident_slots(k_search, lds1);
+  last_team_batches = 0;
   // Batches that leave the machine idle: a workgroup of wavefronts per node (kernels.h, TEAM), eight or four as in launch_teams.
   // (A batch of 58 / 222 / 543 nodes of 20 000 x 50: 126 -> 88 us, 203 -> 128, 220 -> 183; the 44 batches 6.70 -> 5.81 ms, 20 003 x 128
   // 12.6 -> 10.9, 8 000 x 300 12.2 -> 10.8, 6 000 x 960 15.8 -> 14.2, 100 000 x 50 13.0 -> 12.3.)
@@ -536,6 +537,7 @@ void Engine::build_levels() {
     for (int waves = kMostTeam; waves >= kMostTeam / 2; waves /= 2) {
       if (resident_slots(k_team, bytes(), waves) < per_cu * num_cus) continue;
       hipLaunchKernelGGL(k_team, dim3(b.count + b.n_upper), dim3(64 * waves), bytes(), stream, ix, b);
+      last_team_batches += 1;
       return true;
     }
     return false;

@@ -174,6 +174,10 @@ int cuhnsw_last_search_trails(cuhnsw_engine* e);
 /* 1 if the last search ran its literal pass beside the first pass (on a second stream), 0 if after it.
  * No counterpart in the reference (one kernel, one stream, cpp/src/cuhnsw_build.cu:254-275). */
 int cuhnsw_last_search_side_by_side(cuhnsw_engine* e);
+/* How many wavefronts searched each query of the last search together (batches that leave the GPU idle), 0 if one did; and how
+ * many of the last build's batches had their nodes searched so.  No counterpart in the reference (one block per query). */
+int cuhnsw_last_search_team(cuhnsw_engine* e);
+int cuhnsw_last_build_team_batches(cuhnsw_engine* e);
 /* How often, since the index became resident, a literal wavefront's bounded wait for the first pass ran out
  * (the two streams were not running side by side: a profiler that serialises kernels, a saturated device).
  * Each time the batch is answered after its first pass instead, and the next 8 searches run their passes one
