@@ -69,9 +69,25 @@ DESCENTS = [
     ("entry4_kernel<DIST_L2, 1, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,1>"),
     ("entry4_kernel<DIST_L2, 2, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,2>"),
 ]
-OTHERS = [
+# a workgroup of wavefronts per query or node (held to 128 registers, or 256 on long rows and the largest sets)
+TEAMS = [
+    ("search_fast_kernel<DIST_DOT, 1, 2, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,2,team>"),
     ("search_fast_kernel<DIST_DOT, 1, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,5,team>"),
+    ("search_fast_kernel<DIST_DOT, 1, 8, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,1,8,team>"),
+    ("search_fast_kernel<DIST_L2, 2, 2, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,2,team>"),
     ("search_fast_kernel<DIST_L2, 2, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,2,5,team>"),
+    ("search_fast_kernel<DIST_DOT, 2, 8, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,8,team>"),
+    ("search_fast_kernel<DIST_L2, 4, 4, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,4,4,team>"),
+    ("search_fast_kernel<DIST_L2, 4, 8, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,4,8,team>"),
+    ("search_fast_kernel<DIST_L2, 0, 5, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,5,team>"),
+    ("search_fast_kernel<DIST_L2, 0, 16, false, true, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,16,team>"),
+    ("build_search_kernel<DIST_DOT, 1, 2, true>(DevIndex, BuildArgs)", "build_search_kernel<dot,1,2,team>"),
+    ("build_search_kernel<DIST_DOT, 2, 3, true>(DevIndex, BuildArgs)", "build_search_kernel<dot,2,3,team>"),
+    ("build_search_kernel<DIST_L2, 2, 4, true>(DevIndex, BuildArgs)", "build_search_kernel<l2,2,4,team>"),
+    ("build_search_kernel<DIST_L2, 4, 4, true>(DevIndex, BuildArgs)", "build_search_kernel<l2,4,4,team>"),
+    ("build_search_kernel<DIST_L2, 0, 4, true>(DevIndex, BuildArgs)", "build_search_kernel<l2,0,4,team>"),
+]
+OTHERS = [
     ("search_kernel<DIST_DOT, 1, 5>(DevIndex, SearchArgs)", "search_kernel<dot,1,5>"),
     ("build_search_kernel<DIST_DOT, 1, 2>(DevIndex, BuildArgs)", "build_search_kernel<dot,1,2>"),
     ("build_search_kernel<DIST_L2, 2, 5>(DevIndex, BuildArgs)", "build_search_kernel<l2,2,5>"),
@@ -264,7 +280,7 @@ def compile_kernels(instances):
 
 
 def main():
-  report = compile_kernels(FIRST_PASS + DESCENTS + OTHERS)
+  report = compile_kernels(FIRST_PASS + DESCENTS + TEAMS + OTHERS)
   for name, r in report.items():
     print("%-34s VGPRs %3d  waves/SIMD %d  VGPR spills %3d  SGPR spills %3d  scratch %3d B/lane  scratch instrs %3d (in hop loops %d)" % (
         name, r["vgprs"], r["waves_per_simd"], r["vgpr_spills"], r["sgpr_spills"], r["scratch_bytes_per_lane"],
