@@ -637,14 +637,39 @@ class Engine {
     return per_cu * num_cus;
   }
 
+  // Whether teams of `waves` wavefronts are faster than a wavefront alone per query: what helpers evaluate ahead must be what the search
+  // comes to.  A short search ends before it has got to most of the 32 candidates in line, and the less the rows and the other teams
+  // leave of a CU the longer a search it takes to make up for that.  A long one on a CU that teams share has its wavefronts busy and its
+  // memory as well; rows of 129 to 256 elements spill in teams on top.  Bounds of ef by row (up to 64, 128, 256 elements, longer) and
+  // load (a team of eight for every fourth CU or fewer, for every CU or fewer, two on a CU; teams of four).
+  // Time by teams over time alone, 100 000 to 1 M elements, fp32 and fp16, dot and L2 -- inside the bounds 0.6 to 1.03.  Outside:
+  // x 50 ef 16 1.02 to 1.1, ef 1 000 256 queries 0.95 and 1.09, fours 0.97 to 1.19; 500 000 x 96 ef 30 64 to 1 024 queries 1.04 to
+  // 1.13, ef 500 fours 1.07 and 1.12; 400 000 x 200 ef 20 1.06 to 1.46, ef 64 400 to 1 024 queries 1.1 to 1.2, fours at ef 128 0.96 to
+  // 1.1, 440 1.01 to 1.13, 512 1.07 to 1.16, x 180 in fp16 0.98 to 1.04, 1.09 to 1.15, 1.09 to 1.18; 300 000 x 200 L2, 1 024 queries 1.0 to
+  // 1.3; 90 000 x 960 ef 20 128 and more 1.09 to 1.19.
+  static bool teams_pay(int qr, int ef, int nq, int cus, int waves, bool half) {
+    struct Bounds { int from, to; };
+    constexpr Bounds bounds[4][4] = {{{32, 960}, {32, 928}, {40, 512}, {40, 704}},
+                                     {{40, 960}, {48, 928}, {56, 512}, {72, 640}},
+                                     {{56, 960}, {72, 704}, {100, 512}, {128, 320}},
+                                     {{40, 960}, {48, 928}, {48, 512}, {48, 640}}};
+    const bool fours = waves < kMostTeam;
+    const int row = qr == 0 ? 3 : qr >> 1;
+    const Bounds b = bounds[row][fours ? 3 : 4 * nq <= cus ? 0 : nq <= cus ? 1 : 2];
+    if (fours && qr == 4 && (half || nq > 3 * cus)) return false;
+    if (fours && qr == 2 && nq > 2 * cus && ef > 448) return false;
+    return ef >= b.from && (ef <= b.to || 32 * nq <= cus);  // (few enough, and the longest search of the batch is an ordinary one)
+  }
+
   // A batch that leaves the machine idle by teams of wavefronts, a workgroup of eight or four per query (kernels.h, team_help);
   // false: not such a batch.  Eight where the GPU holds them for all queries at once, else four (a number in between puts two of
   // a workgroup's wavefronts on one SIMD as eight do: 345 678 x 101 in fp16, 400 queries, 5 to 7 of them 319 us, four 229).
-  // A wavefront alone -> by teams, ef 300: 100 000 x 50, one query 267 -> 188 us, 32 335 -> 257, 256 408 -> 301, 512 459 -> 302, 768
-  // 468 -> 357, 1 000 514 -> 502; x 180 301 -> 214, 414 -> 310, 748 -> 548, 815 -> 575, 774 -> 671, 789 -> 745; 500 000 x 96 295 -> 206, 408 ->
-  // 277, 546 -> 413, 551 -> 452, 560 -> 527, 571 -> 576; x 300 237 -> 161, 292 -> 208, 436 -> 323, 466 -> 376, 484 -> 454, 483 -> 452.
-  // Alone as well: long rows where the batch has the memory busy, to which helpers add a quarter (100 000 x 960, 32 queries 522 -> 376
-  // us; 256 653, in eights 629, in fours 568; 400 667, in fours 687).
+  // A wavefront alone -> by teams, ef 300, us, 1 / 32 / 256 / 512 / 768 / 1 000 queries: 100 000 x 50 264 -> 182, 320 -> 232, 451 -> 323,
+  // 512 -> 377, 554 -> 454, 584 -> 538; 500 000 x 96 273 -> 191, 386 -> 284, 507 -> 408, 542 -> 420, 558 -> 501, 580 -> 560; 100 000 x 180
+  // 275 -> 204, 348 -> 258, 393 -> 314, 444 -> 367, 468 -> 436.  On long rows the GPU holds no teams for more than 512 queries:
+  // x 300 343 -> 239, 424 -> 305, 493 -> 374, 517 -> 455; x 512 317 -> 226, 397 -> 301, 666 -> 542, 705 -> 639.
+  // Alone as well: long rows where the batch has the memory busy, to which helpers add a quarter (100 000 x 960, 32 queries 551 -> 366
+  // us; 256 646, in eights 618, in fours 582; 400 667, in fours 687; 512 710, in fours 817).
   template <typename K, typename Lds>
   bool launch_teams(K kernel, int qr, int ns, Lds&& search_lds, const DevIndex& ix, SearchArgs a) {
     constexpr size_t kBusyFrom = (size_t)1100 << 10, kHalfBusyFrom = (size_t)700 << 10;  // bytes of one row for every query
@@ -661,7 +686,7 @@ class Engine {
     while (a.team_bucket_bits > 3 && bytes() > lds) --a.team_bucket_bits;
     if (bytes() > lds) return false;
     for (int waves = rows > kHalfBusyFrom ? kMostTeam / 2 : kMostTeam; waves >= kMostTeam / 2; waves /= 2) {
-      if (resident_slots(kernel, bytes(), waves) < per_cu * num_cus) continue;
+      if (!teams_pay(qr, a.ef, a.nq, num_cus, waves, storage_half) || resident_slots(kernel, bytes(), waves) < per_cu * num_cus) continue;
       hipLaunchKernelGGL(kernel, dim3(a.nq), dim3(64 * waves), bytes(), stream, ix, a);
       HIP_CHECK(hipGetLastError());
       last_team = waves;

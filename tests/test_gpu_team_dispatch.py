@@ -19,14 +19,26 @@ def _built(tmp_path, n, d, dist, entries=0, max_m0=32, efc=80):
 
 
 # (256 CUs: the wavefronts that the GPU holds of a kernel of 128 registers are four teams of four, or two of eight, on each; long rows
-# take 256 registers: half as many; and their bytes in all)
+# take 256 registers: half as many; and their bytes in all.  And a wavefront alone where teams are the slower way: short searches, long
+# ones on a GPU that many teams share, teams of four on rows of 129 to 256 elements but for a middle range)
 @pytest.mark.parametrize("d,dist,ef,teams", [
     (50, "dot", 300, {1: 8, 256: 8, 257: 8, 512: 8, 513: 4, 768: 4, 1024: 4, 1025: 0}),
+    (50, "dot", 31, {1: 0, 64: 0, 512: 0, 1024: 0}),
+    (50, "dot", 32, {1: 8, 256: 8, 257: 0, 513: 0}),
+    (50, "dot", 512, {64: 8, 512: 8, 1024: 4}),
+    (50, "dot", 930, {8: 8, 64: 8, 65: 0, 300: 0}),
+    (50, "dot", 1000, {8: 8, 9: 0, 256: 0}),
     (128, "l2", 128, {1: 8, 256: 8, 512: 8, 513: 4, 1024: 4, 1025: 0}),
-    (180, "l2", 200, {1: 8, 256: 8, 512: 8, 513: 4, 1024: 4, 1025: 0}),
+    (100, "l2", 50, {1: 8, 64: 8, 256: 8, 257: 0, 513: 0}),
+    (100, "dot", 450, {512: 8, 513: 0, 1024: 0}),
+    (180, "l2", 200, {1: 8, 256: 8, 512: 8, 513: 4, 768: 4, 769: 0, 1024: 0}),
+    (180, "l2", 60, {1: 8, 64: 8, 65: 0, 512: 0, 700: 0}),
+    (180, "dot", 100, {65: 8, 512: 8, 513: 0}),
+    (180, "dot", 330, {512: 8, 513: 0}),
     (300, "l2", 150, {1: 8, 256: 8, 257: 4, 512: 4, 513: 0}),
+    (300, "l2", 39, {1: 0, 300: 0}),
     (960, "l2", 150, {1: 8, 186: 8, 187: 4, 293: 4, 294: 0}),
-], ids=["dot50", "l2_128", "l2_180", "l2_300", "l2_960"])
+])
 def test_batches_that_leave_the_machine_idle_go_by_teams(tmp_path, d, dist, ef, teams):
   e = _built(tmp_path, 2000, d, dist)
   q = gauss_mixture(1025, d, seed=3, normalise=dist == "dot")
@@ -36,7 +48,7 @@ def test_batches_that_leave_the_machine_idle_go_by_teams(tmp_path, d, dist, ef, 
     got[nq] = e.last_search_team
   assert got == teams
   e.set_tunable("filter_entries", 16384)
-  _device_search(e, q[:100], 10, ef)
+  _device_search(e, q[:1], 10, ef)
   assert e.last_search_team == 0
 
 
