@@ -651,7 +651,7 @@ class Engine {
     struct Bounds { int from, to; };
     constexpr Bounds bounds[4][4] = {{{32, 960}, {32, 928}, {40, 512}, {40, 704}},
                                      {{40, 960}, {48, 928}, {56, 512}, {72, 640}},
-                                     {{56, 960}, {72, 704}, {100, 512}, {128, 320}},
+                                     {{48, 960}, {72, 704}, {100, 512}, {128, 320}},
                                      {{40, 960}, {48, 928}, {48, 512}, {48, 640}}};
     const bool fours = waves < kMostTeam;
     const int row = qr == 0 ? 3 : qr >> 1;
