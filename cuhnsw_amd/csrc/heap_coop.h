@@ -27,11 +27,12 @@
 
 namespace cuhnsw_amd {
 
-// Every kernel here runs one wavefront per workgroup, and a wavefront's LDS (and global)
-// instructions execute in program order, so lanes exchange data through memory without
-// waiting: what is needed between a write by one lane and a read by another is only that
-// the compiler keeps their order.  (__syncthreads() would also drain every outstanding
-// global access — a full memory round trip per call.)
+// A wavefront's LDS (and global) instructions execute in program order, so its lanes exchange data
+// through memory without waiting: what is needed between a write by one lane and a read by another
+// is only that the compiler keeps their order.  (__syncthreads() would also drain every outstanding
+// global access — a full memory round trip per call.)  This orders one wavefront and nothing else:
+// where several share a workgroup (the teams, and the kernels that sort a batch), what they
+// share is behind a barrier, or handed over through a team's slots (team_slots.h).
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(TEAM ? 64 * kMostTeam : 64, TEAM ? (QR != 0 &&
   s.nbuf = reinterpret_cast<uint32_t*>(smem + lp.nbuf);
   s.dbuf = reinterpret_cast<float*>(smem + lp.dbuf);
   if (TEAM) {
-    // a workgroup per query: its first wavefront searches, the others help
+    // a workgroup per query: one wavefront searches (gather_team says which), the others help
     const int wave = gather_team<NS>(s, smem + lp.total, ix0.S0, 0, a0.team_bucket_bits, a0.team_turn);
     if (wave > 0) {
       const int lane = (int)threadIdx.x & 63;

@@ -58,7 +58,7 @@ CUHNSW_HOST_DEVICE inline uint32_t filter_set(FilterShape f, uint32_t place) {
 #endif
 }
 // 16 bits that no number of the set ends in: those of the middle of its stretch with the highest of them turned (a stretch is
-// at most 64 528 << more_bits long, and the middle is found within a few)
+// at most 64 528 long whatever more_bits is, as the fewest sets grow with it, and the middle is found within a few)
 CUHNSW_HOST_DEVICE inline uint32_t filter_empty_tag(FilterShape f, uint32_t set) {
   const float stretch = (float)(1u << 24) / (float)f.sets() * (float)(1 << f.more_bits());
   return ((uint32_t)(((float)set + 0.5f) * stretch) ^ 0x8000u) & 0xFFFFu;
