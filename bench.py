@@ -34,7 +34,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
-KERNEL_SOURCES = ["device_core.h", "heap_coop.h", "kernels.h", "engine.h", "instances.hip"]
+KERNEL_SOURCES = ["device_core.h", "heap_coop.h", "team_slots.h", "visited_filter.h", "kernels.h", "engine.h", "instances.hip"]
 
 
 def kernel_source_digest():
