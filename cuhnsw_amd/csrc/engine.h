@@ -571,9 +571,8 @@ class Engine {
   // ... and the one it gets: what the wavefronts that the kernel's registers allow leave of LDS is the filter's, as far as it
   // needs it (four times the least: next to nothing is forgotten then).  Nor must it be what limits the wavefronts: half the
   // filter repeats more evaluations, but is the faster choice wherever it buys 15 % more of them.
-  // (Against the next power of two above the least: 500 000 x 128 at ef 128, 256 -> 568 sets, 10 000 queries 1.93 -> 1.81 ms; 1 M x
-  // 96, ef 256, topk 100, 512 -> 568 sets, 100 000 queries 9.28 -> 9.14; 1 183 514 x 50 indexed and saved, 256 -> 425, 124.7 ->
-  // 123.0.)
+  // (Against the next power of two above the least: 500 000 x 128 at ef 128, 256 -> 568 sets, 10 000 queries 1.93 -> 1.81 ms; 150 000
+  // x 100 L2, 1 500 to 6 500 queries, ef 180 0.92 to 0.96 of the time, ef 300 0.95 to 0.98; dot rows of 64 elements 1.0 to 1.03.)
   // (Worked out once per kernel, filter to begin with -- and so to end with -- and LDS beside it, which the sizes without a
   // filter, with the first and with the last tell: the answer lies over the filter and counts as far as it is longer.)
   struct Fitted {

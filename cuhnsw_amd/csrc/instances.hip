@@ -261,20 +261,17 @@ void Engine::launch_search(const DevIndex& ix, SearchArgs& a, int max_slots_over
       }
       if constexpr (QR == 1 || QR == 2) {
         // four queries per wavefront, one per group of 16 lanes
-        auto k_entry = entry4_kernel<DT, QR, false>;
-        auto k_beside = entry4_kernel<DT, QR, true>;
+        auto k_entry = entry4_kernel<DT, QR>;
         const int groups = std::max(1, (a.nq + 3) / 4);
-        // Five wavefronts on a SIMD, or four with their neighbours' rows asked for ahead where these take the batch in one round
-        // (1.18 M x 50, 10 000 queries: 1.743 -> 1.707 ms).  Two rounds are of equal length: a full one and a short one take as
-        // long, and the full one's wavefronts are in each other's way.  More rounds of longer L2 rows: four again.
+        // Two rounds of wavefronts are of equal length: a full one and a short one take as long, and the full one's wavefronts are
+        // in each other's way.  More than two, of longer L2 rows: four wavefronts on a SIMD instead of the five it holds.
         // Every batch by four wavefronts / this, us: 1 M x 50 dot, 20 000 queries 104 / 101, 24 000 113 / 118, 33 000 161 / 139,
         // 60 000 256 / 240, 100 000 435 / 394; 600 000 x 96 dot 131 / 127, 142 / 140 (a full and a short round: 155), 202 / 179,
         // 314 / 298, 528 / 490; 300 000 x 128 L2 135 / 127, 147 / 137, 178 / 178, 285 / 285 (five wavefronts: 294), 454 / 454 (478).
-        const bool beside = groups <= resident_slots(k_beside, 0);
-        const int slots_now = resident_slots(k_entry, 0);
-        int entry_grid = groups <= slots_now || beside ? groups : groups <= 2 * slots_now ? (groups + 1) / 2 : slots_now;
-        if (DT == DIST_L2 && QR == 2 && groups > 2 * slots_now) entry_grid = std::min(entry_grid, 4 * 4 * num_cus);
-        hipLaunchKernelGGL(beside ? k_beside : k_entry, dim3(entry_grid), dim3(64), 0, stream, ix, a);
+        const int entry_slots = resident_slots(k_entry, 0);
+        int entry_grid = groups <= entry_slots ? groups : groups <= 2 * entry_slots ? (groups + 1) / 2 : entry_slots;
+        if (DT == DIST_L2 && QR == 2 && groups > 2 * entry_slots) entry_grid = std::min(entry_grid, 4 * 4 * num_cus);
+        hipLaunchKernelGGL(k_entry, dim3(entry_grid), dim3(64), 0, stream, ix, a);
       } else {
         auto k_entry = entry_kernel<DT, QR>;
         const size_t entry_lds = plan_fast_lds(QR, ix.Dp, a.rcap, FilterShape(), 0).total;

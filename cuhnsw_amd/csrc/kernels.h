@@ -295,7 +295,7 @@ __device__ __forceinline__ float entry4_key(const void* rows, uint32_t rowlen, u
   }
   return finish16<DT, false>(ax, ay, az, aw);
 }
-template <int DT, int QR, bool HALF, bool BESIDE>
+template <int DT, int QR, bool HALF>
 __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs& a) {
   const int lane = threadIdx.x, g = lane >> 4, sub = lane & 15;
   const uint32_t rowlen = (uint32_t)ix.Dp >> 2, used = (uint32_t)(ix.D + 3) >> 2;
@@ -319,14 +319,11 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
       const uint32_t* row = ix.linksU + (size_t)((active ? first : 0) + (active ? level : 1) - 1) * ix.SU;
       float best = INFINITY;
       uint32_t best_id = cur;
-      long long best_first = first;
       int n = 0;
       for (int base = 0; base < ix.SU; base += 16) {
         const uint32_t got = row[base + sub < ix.SU ? base + sub : 0];
         const uint32_t id = (active && base + sub < ix.SU) ? got : kEmpty;
         const unsigned long long valid = __ballot(id != kEmpty);
-        const long long firsts = BESIDE ? ix.upper_off[id != kEmpty ? id : cur] : 0ll;
-        int best_at = -1;
         n += __popc((uint32_t)(valid >> (16 * g)) & 0xFFFFu);
         constexpr int B = QR == 1 ? 16 : 8;  // rows in flight per lane: 16 float4 registers' worth
 #pragma unroll
@@ -344,13 +341,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
             if (ids[j] != kEmpty && keys[j] < best) {  // strictly closer: the first occurrence of the minimum wins
               best = keys[j];
               best_id = ids[j];
-              best_at = p0 + j;
             }
-        }
-        if constexpr (BESIDE) {
-          const int from = 16 * g + (best_at < 0 ? 0 : best_at);
-          const uint32_t low = (uint32_t)__shfl((int)firsts, from, 64), high = (uint32_t)__shfl((int)(firsts >> 32), from, 64);
-          best_first = best_at < 0 ? best_first : (long long)(((unsigned long long)high << 32) | low);
         }
       }
       if (active) {
@@ -359,7 +350,7 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
         if (n > 0 && best < dcur) {
           dcur = best;
           cur = best_id;  // and sweep again on this level
-          first = BESIDE ? best_first : ix.upper_off[best_id];
+          first = ix.upper_off[best_id];
         } else {
           if (level == a.region_level) region = cur;
           level -= 1;
@@ -375,12 +366,13 @@ __device__ __forceinline__ void entry4_body(const DevIndex& ix, const SearchArgs
     }
   }
 }
-// BESIDE: as in descend, where the neighbours' rows are is asked for beside their vectors.  For batches of one round of
-// wavefronts (the host's choice: instances.hip); its registers cost a wavefront per SIMD, four instead of five.
-template <int DT, int QR, bool BESIDE>
+// (Where the neighbours' rows are, asked for beside their vectors as in descend, is not worth it here, for a wavefront per SIMD less:
+// 10 000 / 16 000 queries with it and without, us: 1.18 M x 50 67, 90 and 65, 90; 600 000 x 96 77, 106 and 78, 104; 300 000 x 128 L2 76,
+// 107 and 71, 101.)
+template <int DT, int QR>
 __global__ void __launch_bounds__(64) entry4_kernel(DevIndex ix, SearchArgs a) {
-  if (uni(ix.half) != 0) entry4_body<DT, QR, true, BESIDE>(ix, a);
-  else entry4_body<DT, QR, false, BESIDE>(ix, a);
+  if (uni(ix.half) != 0) entry4_body<DT, QR, true>(ix, a);
+  else entry4_body<DT, QR, false>(ix, a);
 }
 // counters -> first position of every bucket (exclusive prefix sum over `from` and what lies before; one workgroup of 1024).
 // cut: the longest queries end with the first bucket at which there are `most` of them or more; set to that bucket and to

@@ -62,12 +62,12 @@ FIRST_PASS = [
     ("search_fast_kernel<DIST_DOT, 2, 4, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<dot,2,4,few>"),
     ("search_fast_kernel<DIST_L2, 0, 6, false, true>(DevIndex, SearchArgs)", "search_fast_kernel<l2,0,6,few>"),
 ]
-# the batch's descents, four to a wavefront (the instances for batches of more than one round of wavefronts)
+# the batch's descents, four to a wavefront
 DESCENTS = [
-    ("entry4_kernel<DIST_DOT, 1, false>(DevIndex, SearchArgs)", "entry4_kernel<dot,1>"),
-    ("entry4_kernel<DIST_DOT, 2, false>(DevIndex, SearchArgs)", "entry4_kernel<dot,2>"),
-    ("entry4_kernel<DIST_L2, 1, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,1>"),
-    ("entry4_kernel<DIST_L2, 2, false>(DevIndex, SearchArgs)", "entry4_kernel<l2,2>"),
+    ("entry4_kernel<DIST_DOT, 1>(DevIndex, SearchArgs)", "entry4_kernel<dot,1>"),
+    ("entry4_kernel<DIST_DOT, 2>(DevIndex, SearchArgs)", "entry4_kernel<dot,2>"),
+    ("entry4_kernel<DIST_L2, 1>(DevIndex, SearchArgs)", "entry4_kernel<l2,1>"),
+    ("entry4_kernel<DIST_L2, 2>(DevIndex, SearchArgs)", "entry4_kernel<l2,2>"),
 ]
 # a workgroup of wavefronts per query or node (held to 128 registers, or 256 on long rows and the largest sets)
 TEAMS = [

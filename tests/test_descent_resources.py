@@ -1,5 +1,5 @@
 """The register budget of the kernel that makes a batch's descents four to a wavefront, on the compiler's own output (no GPU
-needed): batches of more than one round of its wavefronts have five of them on a SIMD, 20 480 queries a round."""
+needed): five of its wavefronts on a SIMD, 20 480 queries a round."""
 import shutil
 
 import pytest

@@ -1,4 +1,4 @@
-"""A batch's descents, four queries to a wavefront, at the batch sizes where the kernel or its grid changes (256 CUs: one round of four
+"""A batch's descents, four queries to a wavefront, at the batch sizes where its grid changes (256 CUs: one round of four
 wavefronts on a SIMD, of five, two rounds of five, and one query more than each): ids, found counts and the counters of the
 descents against the oracle."""
 import numpy as np
