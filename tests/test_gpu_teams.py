@@ -51,8 +51,7 @@ def test_batches_that_leave_the_machine_idle_match_the_oracle(oracle, tmp_path, 
     (4500, 100, "dot", 32, 64, 130, "gauss", dict(heuristic_coef=0.25)),      # link rows of 64 ids
     (2500, 300, "l2", 3, 6, 100, "gauss", dict(save_remains=True)),           # many levels; rows too long for registers
     (4500, 180, "l2", 16, 32, 700, "scattered", {}),                          # the largest set
-    (1200, 960, "l2", 16, 32, 12, "gauss", {}),   # the selection soon after the start, its picks where the node's long row was
-], ids=["ties", "full64", "levels", "large", "long"])
+], ids=["ties", "full64", "levels", "large"])
 def test_index_built_by_teams_is_the_one_built_without(tmp_path, n, d, dist, max_m, max_m0, efc, kind, extra):
   """Batches of a build go through every size up to a quarter of the nodes; a filter of a given size takes the wavefront alone."""
   if kind == "int":
